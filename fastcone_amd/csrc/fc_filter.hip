@@ -24,6 +24,7 @@
 // completely before it writes either, so the filter may run in place.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -249,55 +250,69 @@ __global__ __launch_bounds__(kFT) void row_filter_kernel(FiltArgs a) {
 
 // ---- tables (FP64) ---------------------------------------------------------------------------
 
-// Taps kern[q], q = d + nw - 1, d in [-(nw-1), nw-1].
-__global__ __launch_bounds__(256) void filt_taps(int kind, double p0, int nw,
-                                                 double* __restrict__ kern) {
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= 2 * nw - 1) return;
-  const long long d = (long long)q - (nw - 1);
-  const long long ad = d < 0 ? -d : d;
-  double v = 0.0;
+// Tap kern[d], d in [0, nw); kern[-d] = kern[d] (ramp) or -kern[d] (Hilbert). Ramp: irfft of H over
+// n = 2 nw bins, (1/n) [H0 + 2 sum_{k=1}^{nw-1} H_k cos(2 pi k d / n) + H_nw cos(pi d)] with
+// H_k = c k, H0 = c / 8, c = pi / n. The sum has a closed form: with t = pi d / nw,
+// sum k cos(k t) = -nw / 2 for even d > 0 and nw / 2 - 1 / (2 sin^2(t / 2)) for odd d.
+__device__ __forceinline__ double filt_tap(int kind, double p0, int nw, int d) {
   if (kind == FC_FILTER_RAMP) {
-    // irfft of H over n = 2 nw bins: (1/n) [H0 + 2 sum_{k=1}^{nw-1} H_k cos(2 pi k d / n)
-    //                                      + H_nw cos(pi d)],  H_k = (pi / n) k, H0 = (pi / n) / 8
-    const long long n = 2LL * nw;
+    const double n = 2.0 * (double)nw, c = M_PI / n;
+    double v = 0.125 * c;
+    if (d == 0) {
+      v += c * (double)nw * (double)nw;
+    } else if (d & 1) {
+      const double s = sinpi((double)d / n);
+      v -= c / (s * s);
+    }
+    return p0 * v / n;
+  }
+  if (!(d & 1)) return 0.0;
+  const double x = (double)d * p0;
+  return 2.0 / (M_PI * (double)d) * (x / sin(x));
+}
+
+// cos(2 pi m / L) from the table of its first quarter, q[j] = cos(2 pi j / L), j in [0, L/4].
+__device__ __forceinline__ double cos_table(const double* q, int L, int m) {
+  m &= L - 1;
+  if (m > L / 2) m = L - m;
+  return m > L / 4 ? -q[L / 2 - m] : q[m];
+}
+
+// Twiddles tw[m] = e^{-2 pi i m / L} and multipliers mult[k] = (1/L) sum_d kern[d] e^{-2 pi i k d / L}
+// in FP64, rounded to FP32. Every block holds the taps and a quarter wave of the length-L cosine in
+// LDS; a wave owns a bin k <= L/2 (its lanes share the taps' sum, k d mod L being an exact mask) and
+// writes it and its conjugate at L - k.
+// Bound by latency: a few FP64 transcendentals per thread, then one LDS gather and FMA per term. The
+// three kernels this replaces evaluated a sum of nw cosines per tap and 2 nw - 1 FP64 sine/cosine
+// pairs with a 64-bit remainder per bin, one thread each: 108 us at nw = 96 (L = 256) and 850 us at
+// nw = 768 (L = 2048) against 4.2 and 6.1 us
+// for this one.
+__global__ __launch_bounds__(256) void filt_tables(int kind, double p0, int nw, int L,
+                                                   float2* __restrict__ tw,
+                                                   float2* __restrict__ mult) {
+  extern __shared__ double lds_tab[];
+  double* quarter = lds_tab;               // L/4 + 1
+  double* taps = lds_tab + L / 4 + 1;      // nw
+  for (int j = threadIdx.x; j <= L / 4; j += 256) quarter[j] = cospi(2.0 * (double)j / (double)L);
+  for (int d = threadIdx.x; d < nw; d += 256) taps[d] = filt_tap(kind, p0, nw, d);
+  __syncthreads();
+  for (int m = blockIdx.x * 256 + threadIdx.x; m < L; m += gridDim.x * 256)
+    tw[m] = make_float2((float)cos_table(quarter, L, m), (float)-cos_table(quarter, L, m - L / 4));
+  const int lane = threadIdx.x & 63;
+  const int shift = kind == FC_FILTER_RAMP ? 0 : L / 4;  // sum of cosines or of sines
+  for (int k = blockIdx.x * 4 + (threadIdx.x >> 6); k <= L / 2; k += gridDim.x * 4) {
     double s = 0.0;
-    for (long long k = 1; k < nw; ++k) s += (double)k * cospi(2.0 * (double)((k * ad) % n) / (double)n);
-    const double c = M_PI / (double)n;
-    v = p0 * (0.125 * c + 2.0 * c * s + c * (double)nw * ((ad & 1) ? -1.0 : 1.0)) / (double)n;
-  } else if (ad & 1) {
-    const double x = (double)d * p0;
-    v = 2.0 / (M_PI * (double)d) * (x / sin(x));
+    for (int d = 1 + lane; d < nw; d += 64)
+      s = fma(taps[d], cos_table(quarter, L, k * d - shift), s);
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) {
+      float2 v;
+      if (kind == FC_FILTER_RAMP) v = make_float2((float)((taps[0] + 2.0 * s) / L), 0.0f);
+      else v = make_float2(0.0f, (float)(-2.0 * s / L));
+      mult[k] = v;
+      if (k > 0 && k < L / 2) mult[L - k] = make_float2(v.x, -v.y);
+    }
   }
-  kern[q] = v;
-}
-
-// mult[k] = (1/L) sum_d kern[d] e^{-2 pi i k d / L}, with exact integer reduction of k d mod L.
-__global__ __launch_bounds__(256) void filt_multiplier(const double* __restrict__ kern, int nw,
-                                                       int L, float2* __restrict__ mult) {
-  const int k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= L) return;
-  double re = 0.0, im = 0.0;
-  for (int q = 0; q < 2 * nw - 1; ++q) {
-    const double c0 = kern[q];
-    if (c0 == 0.0) continue;
-    const long long d = (long long)q - (nw - 1);
-    long long m = ((long long)k * d) % L;
-    if (m < 0) m += L;
-    double s, c;
-    sincospi(2.0 * (double)m / (double)L, &s, &c);
-    re = fma(c0, c, re);
-    im = fma(-c0, s, im);
-  }
-  mult[k] = make_float2((float)(re / L), (float)(im / L));
-}
-
-__global__ __launch_bounds__(256) void filt_twiddles(int L, float2* __restrict__ tw) {
-  const int m = blockIdx.x * 256 + threadIdx.x;
-  if (m >= L) return;
-  double s, c;
-  sincospi(2.0 * (double)m / (double)L, &s, &c);
-  tw[m] = make_float2((float)c, (float)-s);
 }
 
 int filter_log2(int nw) {
@@ -309,9 +324,8 @@ int filter_log2(int nw) {
 inline constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Tables of the widest supported row (FC_FILTER_MAX_COLS columns, FFT length 8192): twiddles and
-// multipliers (8192 float2 each) and the 8191 FP64 taps. Every row filter needs at most this.
-constexpr size_t kMaxTableBytes = 2 * align256((size_t)8192 * sizeof(float2)) +
-                                  align256((2 * (size_t)FC_FILTER_MAX_COLS - 1) * sizeof(double));
+// multipliers (8192 float2 each). Every row filter needs at most this.
+constexpr size_t kMaxTableBytes = 2 * align256((size_t)8192 * sizeof(float2));
 
 // Device-resident tables for fc_fdk_filter_noalloc_dev (one copy per GPU, held until the process
 // ends). In host code the name is only a stand-in: the device address comes from
@@ -345,7 +359,7 @@ int scratch_address(int device, void** out) {
 
 size_t filter_table_bytes(int nw) {
   const size_t L = (size_t)1 << filter_log2(nw);
-  return 2 * align256(L * sizeof(float2)) + align256((2 * (size_t)nw - 1) * sizeof(double));
+  return 2 * align256(L * sizeof(float2));
 }
 
 int launch_row_filter(const void* in, int in_dt, void* out, int out_dt, int nw, int nh,
@@ -360,10 +374,10 @@ int launch_row_filter(const void* in, int in_dt, void* out, int out_dt, int nw, 
   char* base = static_cast<char*>(tables);
   float2* tw = reinterpret_cast<float2*>(base);
   float2* mult = reinterpret_cast<float2*>(base + align256((size_t)L * sizeof(float2)));
-  double* kern = reinterpret_cast<double*>(base + 2 * align256((size_t)L * sizeof(float2)));
-  filt_taps<<<(2 * nw - 1 + 255) / 256, 256, 0, stream>>>(kind, p0, nw, kern);
-  filt_twiddles<<<(L + 255) / 256, 256, 0, stream>>>(L, tw);
-  filt_multiplier<<<(L + 255) / 256, 256, 0, stream>>>(kern, nw, L, mult);
+  // one bin per wave up to L = 2048, at most a block per CU (its LDS holds up to 49 KB of tables)
+  const int tblocks = std::min(256, (L / 2 + 4) / 4);
+  filt_tables<<<tblocks, 256, (L / 4 + 1 + (size_t)nw) * sizeof(double), stream>>>(kind, p0, nw, L,
+                                                                                   tw, mult);
   FiltArgs a;
   a.in = in;
   a.out = out;
