@@ -4,10 +4,10 @@
 // (tap = 9 dz + 3 dy + dx, zero padding 1); accumulation FP32.
 //
 //  * forward (and input gradient): implicit GEMM  Y[voxel][co] = sum_k P[voxel][k] Wt[k][co],
-//    k = tap * Cin + ci, with v_mfma_f32_16x16x32_bf16: a wave owns 16 consecutive voxels of an
-//    x row and all output channels; each lane feeds 8 consecutive k (one 16-byte load of 8
-//    channels of one tap). Bias and ReLU are fused in the epilogue. The input gradient is the
-//    same kernel on dY with the flipped, transposed weights  W'[ci][26 - tap][co] = W[co][tap][ci].
+//    k = tap * Cin + ci, with v_mfma_f32_16x16x32_bf16 on input planes staged in LDS; each lane
+//    feeds 8 consecutive k (8 channels of one tap). Bias and ReLU are fused in the epilogue. The
+//    input gradient is the same kernel on dY with the flipped, transposed weights
+//    W'[ci][26 - tap][co] = W[co][tap][ci].
 //  * weight gradient: dW[co][k] = sum_voxel dY[voxel][co] P[voxel][k] with
 //    v_mfma_f32_16x16x32_bf16 fed the raw BF16 bits (products exact in FP32): a block per (group
 //    of x rows, 64 k), one 16-column slice of K per wave; each row's output gradient is staged
@@ -24,6 +24,7 @@
 //   result D lane l, register r holds D[4 (l / 16) + r][l % 16].
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "fc_device.h"
@@ -35,64 +36,213 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+// output stores: the caller's buffer may start at any element
+typedef unsigned int u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 // ---- forward / input-gradient implicit GEMM --------------------------------------------------
+// A block owns a tile of XT x YT voxels in x and y and walks a chunk of z planes. Three input planes
+// (the tile with its one-voxel halo, zero outside the volume) are resident in LDS; the next one is
+// loaded into registers while a plane is computed. A wave owns V groups of 16 consecutive x voxels
+// and all output channels: the weights are the MFMA's A operand (16 channels x 32 k), the patches
+// its B operand (32 k x 16 voxels, one 16-byte LDS read per lane), so a lane ends with four
+// consecutive channels of one voxel, an 8-byte store. The order of every output's sum is k
+// ascending, 32 per instruction.
+//
+// Each weight fragment feeds V instructions; where the whole weight set fits (kWReg) it stays in
+// registers over the walk, otherwise it comes from L1 once per V instructions. A voxel's channels
+// are padded by 16 bytes in LDS: the pitch is an odd number of 16-byte units, so the eight voxels of
+// a quarter of a read lie in different banks.
+//
+// Bound by the LDS reads of the patches (1 KB per instruction) in the 16- and 48-channel layers and
+// by the weights' way from L1 in the 64- and 96-channel ones. Before, a wave owned one group and
+// read patches and weights from L1 for every instruction. Time at 256^3: 16 -> 16 channels 1.49 ->
+// 0.32 ms (1.07 GB of activations: 0.23 ms at the rate of a large copy), 48 -> 16 5.29 -> 0.98 ms;
+// at 128^3: 96 -> 32 2.26 -> 0.96 ms, 32 -> 32 0.64 -> 0.17 ms; at 64^3: 64 -> 64 0.47 -> 0.21 ms.
+template <int CIN, int COUT>
+struct ConvTile {
+  static constexpr int XT = (CIN == 16 && COUT <= 32) || (CIN == 32 && COUT >= 32) ? 32 : 16;
+  static constexpr int YT = 8;
+  static constexpr int V = XT * YT / 16 / 4;          // groups of 16 voxels per wave
+  static constexpr int PITCH = 2 * CIN + 16;          // bytes per voxel
+  static constexpr int ROWB = (XT + 2) * PITCH, PLANEB = (YT + 2) * ROWB;
+  static constexpr int K = 27 * CIN, KSTEPS = (K + 31) / 32, NB = COUT / 16;
+  static constexpr bool kWReg = KSTEPS * NB <= 42;    // 168 VGPRs
+  static constexpr int G = NB <= 2 ? 4 : (NB <= 4 ? 2 : 1);  // steps of weights loaded ahead
+  // LDS offset of k's tap and channel in its plane, and its plane
+  static constexpr int off(int k) {
+    const int tap = k / CIN;
+    return ((tap / 3) % 3 * (XT + 2) + tap % 3) * PITCH + 2 * (k % CIN);
+  }
+  static constexpr int dz(int k) { return k / CIN / 9; }
+};
+
 template <int CIN, int COUT, bool RELU>
-__global__ __launch_bounds__(256) void conv_fwd_mfma(const uint16_t* __restrict__ x,
-                                                     const uint16_t* __restrict__ w,
-                                                     const float* __restrict__ bias,
-                                                     uint16_t* __restrict__ y, int D, int H,
-                                                     int W) {
+__global__ __launch_bounds__(256, 2) void conv_fwd_mfma(const uint16_t* __restrict__ x,
+                                                        const uint16_t* __restrict__ w,
+                                                        const float* __restrict__ bias,
+                                                        uint16_t* __restrict__ y, int D, int H,
+                                                        int W, int tx, int ty, int zc, int nzc) {
   static_assert(CIN % 16 == 0 && COUT % 16 == 0, "channel counts must be multiples of 16");
-  constexpr int K = 27 * CIN;
-  constexpr int KSTEPS = (K + 31) / 32;
-  constexpr int NB = COUT / 16;
+  using T = ConvTile<CIN, COUT>;
+  constexpr int XT = T::XT, YT = T::YT, V = T::V, PITCH = T::PITCH, ROWB = T::ROWB;
+  constexpr int K = T::K, KSTEPS = T::KSTEPS, NB = T::NB;
+  constexpr int C8 = CIN / 8, UNITS = (XT + 2) * (YT + 2) * C8, NU = (UNITS + 255) / 256;
+  __shared__ __align__(16) char ring[3 * T::PLANEB];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int xb = blockIdx.x * 64 + wave * 16;
-  const int yv = blockIdx.y;
-  const int n = blockIdx.z / D, z = blockIdx.z - (blockIdx.z / D) * D;
-  const int xv = xb + m;
-  f32x4 acc[NB];
+  const bool hi = g >= 2;
+  int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int bx = b % tx; b /= tx;
+  const int by = b % ty; b /= ty;
+  const int bz = b % nzc, n = b / nzc;
+  const int xb = bx * XT, yb = by * YT, z0 = bz * zc, z1 = min(D, z0 + zc);
+
+  // this thread's 16-byte units of a plane: voxel offset from the tile's corner (-1: outside the
+  // volume in x or y, or no unit) and LDS address
+  int vox[NU], dst[NU], ch[NU];
 #pragma unroll
-  for (int cb = 0; cb < NB; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bf16x8 zero8 = {};
-  for (int s = 0; s < KSTEPS; ++s) {
-    const int k = s * 32 + g * 8;
-    bf16x8 a = zero8;
-    bf16x8 b[NB];
+  for (int q = 0; q < NU; ++q) {
+    const int u = (int)threadIdx.x + 256 * q;
+    const int v = u / C8, c8 = u - v * C8, yy = v / (XT + 2), xx = v - yy * (XT + 2);
+    const int gx = xb + xx - 1, gy = yb + yy - 1;
+    vox[q] = u < UNITS && gx >= 0 && gx < W && gy >= 0 && gy < H ? (yy * W + xx) : -1;
+    dst[q] = u < UNITS ? v * PITCH + 16 * c8 : -1;
+    ch[q] = 8 * c8;
+  }
+  u32x4 pf[NU];
+  auto fetch = [&](int z) {
+    // element (z, yb - 1, xb - 1) of batch n; only units inside the volume are read
+    const uint16_t* p = x + ((((long long)n * D + z) * H + (yb - 1)) * W + (xb - 1)) * CIN;
+    const bool zin = z >= 0 && z < D;
 #pragma unroll
-    for (int cb = 0; cb < NB; ++cb) b[cb] = zero8;
-    if (k < K) {
-      const int tap = k / CIN, ci = k - (k / CIN) * CIN;
-      const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
-      const int zz = z + dz - 1, yy = yv + dy - 1, xx = xv + dx - 1;
-      if (zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 && xx < W && xv < W)
-        a = *reinterpret_cast<const bf16x8*>(
-            x + ((((size_t)n * D + zz) * H + yy) * W + xx) * CIN + ci);
+    for (int q = 0; q < NU; ++q) {
+      pf[q] = u32x4{0u, 0u, 0u, 0u};
+      if (zin && vox[q] >= 0)
+        pf[q] = *reinterpret_cast<const u32x4*>(p + (long long)vox[q] * CIN + ch[q]);
+    }
+  };
+  auto put = [&](int slot) {
+#pragma unroll
+    for (int q = 0; q < NU; ++q)
+      if (dst[q] >= 0) *reinterpret_cast<u32x4*>(ring + slot * T::PLANEB + dst[q]) = pf[q];
+  };
+  // weight fragment (step s, block cb): row cb 16 + m, k = 32 s + 8 g; zero past K
+  const int wlane = m * K + g * 8;
+  auto wfrag = [&](int s, int cb, int from) {
+    u32x4 q = u32x4{0u, 0u, 0u, 0u};
+    if (K % 32 == 0 || s + 1 < KSTEPS || !hi)
+      q = *reinterpret_cast<const u32x4*>(w + from + cb * 16 * K + s * 32);
+    return __builtin_bit_cast(bf16x8, q);
+  };
+  constexpr int G = T::kWReg ? KSTEPS : T::G;
+  bf16x8 wr[T::kWReg ? KSTEPS * NB : 2 * G * NB];
+  if constexpr (T::kWReg) {
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) wr[s * NB + cb] = wfrag(s, cb, wlane);
+  }
+  f32x4 bb[NB];
+#pragma unroll
+  for (int cb = 0; cb < NB; ++cb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bb[cb][r] = bias ? bias[cb * 16 + 4 * g + r] : 0.0f;
+
+  // group v of wave `wave`: row (wave V + v) 16 / XT, x offset 16 ((wave V + v) % (XT / 16))
+  constexpr int GX = XT / 16;
+  static_assert(V % GX == 0, "a wave owns whole rows");
+  const int lane0 = (wave * (V / GX) * (XT + 2) + m) * PITCH + 16 * g;
+  // weights not held in registers come G steps ahead, in alternating halves of wr; the empty asm
+  // keeps the compiler from loading them earlier (it would hoist them all and spill)
+  auto ahead = [&](int s0) {
+    int from = wlane;
+    asm volatile("" : "+v"(from));
+#pragma unroll
+    for (int q = 0; q < G; ++q)
 #pragma unroll
       for (int cb = 0; cb < NB; ++cb)
-        b[cb] = *reinterpret_cast<const bf16x8*>(w + (size_t)(cb * 16 + m) * K + k);
+        if (s0 + q < KSTEPS) wr[((s0 / G % 2) * G + q) * NB + cb] = wfrag(s0 + q, cb, from);
+  };
+  int slot[3] = {0, 1, 2};  // ring slots of planes z - 1, z, z + 1
+  for (int d = 0; d < 3; ++d) {
+    fetch(z0 - 1 + d);
+    put(d);
+  }
+  __syncthreads();
+  for (int z = z0; z < z1; ++z) {
+    if (z + 1 < z1) fetch(z + 2);
+    int base[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) base[d] = lane0 + slot[d] * T::PLANEB;
+    f32x4 acc[V][NB];
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) acc[v][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (!T::kWReg) ahead(0);
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) {
+      if constexpr (!T::kWReg) {
+        if (s % G == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (s + G < KSTEPS) ahead(s + G);
+        }
+      }
+      // lanes g = 0, 1 hold k0 .. k0 + 15 and lanes g = 2, 3 k1 .. k1 + 15: the second half is
+      // either the next 16 channels of the same tap, another tap, or past the end (zero)
+      const int k0 = 32 * s, k1 = 32 * s + 16;
+      const int o0 = T::off(k0), d0 = T::dz(k0);
+      int addr = base[d0];
+      if (k1 >= K) {
+        addr -= hi ? 32 : 0;
+      } else if (T::dz(k1) != d0) {
+        addr = hi ? base[T::dz(k1)] + (T::off(k1) - 32 - o0) : addr;
+      } else if (T::off(k1) - o0 != 32) {
+        addr += hi ? T::off(k1) - 32 - o0 : 0;
+      }
+      bf16x8 a[NB];
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb)
+        a[cb] = wr[(T::kWReg ? s : s / G % 2 * G + s % G) * NB + cb];
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const int gofs = (v / GX) * ROWB + (v % GX) * 16 * PITCH;
+        u32x4 q = *reinterpret_cast<const u32x4*>(ring + addr + (o0 + gofs));
+        if (k1 >= K && hi) q = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb)
+          acc[v][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[cb], __builtin_bit_cast(bf16x8, q),
+                                                               acc[v][cb], 0, 0, 0);
+      }
     }
 #pragma unroll
-    for (int cb = 0; cb < NB; ++cb)
-      acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[cb], acc[cb], 0, 0, 0);
-  }
-  const size_t rowbase = (((size_t)n * D + z) * H + yv) * W;
+    for (int v = 0; v < V; ++v) {
+      const int vy = yb + wave * (V / GX) + v / GX, vx = xb + (v % GX) * 16 + m;
+      if (vy < H && vx < W) {
+        uint16_t* o = y + ((((size_t)n * D + z) * H + vy) * W + vx) * COUT + 4 * g;
 #pragma unroll
-  for (int cb = 0; cb < NB; ++cb) {
-    const int co = cb * 16 + m;
-    const float bb = bias ? bias[co] : 0.0f;
+        for (int cb = 0; cb < NB; ++cb) {
+          uint32_t h[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int vx = xb + g * 4 + r;
-      if (vx < W) {
-        float v = acc[cb][r] + bb;
-        if (RELU) v = fmaxf(v, 0.0f);
-        y[(rowbase + vx) * COUT + co] = f32_to_bf16_bits(v);
+          for (int r = 0; r < 4; ++r) {
+            float f = acc[v][cb][r] + bb[cb][r];
+            if (RELU) f = fmaxf(f, 0.0f);
+            h[r] = f32_to_bf16_bits(f);
+          }
+          *reinterpret_cast<u32x2_a2*>(o + cb * 16) = u32x2_a2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+        }
       }
+    }
+    __syncthreads();  // plane z - 1 is no longer read
+    if (z + 1 < z1) {
+      put(slot[0]);
+      const int s0 = slot[0];
+      slot[0] = slot[1];
+      slot[1] = slot[2];
+      slot[2] = s0;
+      __syncthreads();
     }
   }
 }
@@ -385,13 +535,20 @@ __global__ __launch_bounds__(64) void mfma_probe(const uint16_t* __restrict__ A3
 template <int CIN, int COUT>
 bool launch_fwd_t(const void* x, const void* w, const float* b, void* y, int N, int D, int H,
                   int W, int relu, hipStream_t s) {
-  dim3 grid((W + 63) / 64, H, N * D);
+  using T = ConvTile<CIN, COUT>;
+  const int tx = (W + T::XT - 1) / T::XT, ty = (H + T::YT - 1) / T::YT;
+  // planes per block: as many as leave about 2048 blocks (eight per CU), at most 32 (the two halo
+  // planes are then 6 % of the planes loaded)
+  const long long tiles = (long long)tx * ty * N;
+  const int zc = (int)std::max(1LL, std::min(32LL, tiles * D / 2048));
+  const int nzc = (D + zc - 1) / zc;
+  const unsigned grid = (unsigned)(tiles * nzc);
   if (relu)
-    conv_fwd_mfma<CIN, COUT, true><<<grid, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)w,
-                                                        b, (uint16_t*)y, D, H, W);
+    conv_fwd_mfma<CIN, COUT, true><<<grid, 256, 0, s>>>(
+        (const uint16_t*)x, (const uint16_t*)w, b, (uint16_t*)y, D, H, W, tx, ty, zc, nzc);
   else
-    conv_fwd_mfma<CIN, COUT, false><<<grid, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)w,
-                                                         b, (uint16_t*)y, D, H, W);
+    conv_fwd_mfma<CIN, COUT, false><<<grid, 256, 0, s>>>(
+        (const uint16_t*)x, (const uint16_t*)w, b, (uint16_t*)y, D, H, W, tx, ty, zc, nzc);
   return true;
 }
 

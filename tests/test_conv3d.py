@@ -235,3 +235,24 @@ def test_unet_training_fits_a_representable_target(gpu):
     print("representable target: training MSE at iterations 300, 350, 400: "
           + ", ".join(f"{r:.3f}" for r in ratios) + " of the identity start's")
     assert min(ratios) < 0.2
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 32), (32, 32), (48, 16), (64, 64), (96, 32)])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 5, 8, 32), (2, 9, 17, 33)])
+def test_conv_tile_edges(gpu, cin, cout, shape):
+    # one voxel, whole tiles, and one voxel past a tile in every direction (tiles of 16 or 32 x 8
+    # voxels, chunks of planes). Both results are rounded to BF16 (relative 2^-9
+    # each, the sums in FP32): rel. L2 < 2^-8
+    from fastcone_amd.unet import conv3d
+    g = torch.Generator().manual_seed(cin + cout + sum(shape))
+    x = torch.randn(shape + (cin,), generator=g).to(torch.bfloat16)
+    w = (torch.randn((cout, 27, cin), generator=g) / np.sqrt(27 * cin)).to(torch.bfloat16).float()
+    gy = torch.randn(shape + (cout,), generator=g).to(torch.bfloat16)
+    xg = x.to(gpu).requires_grad_(True)
+    y = conv3d(xg, w.to(gpu), torch.zeros(cout, device=gpu), False)
+    y.backward(gy.to(gpu))
+    xr = x.float().permute(0, 4, 1, 2, 3).requires_grad_(True)
+    yr = torch.nn.functional.conv3d(xr, _torch_w(w), padding=1)
+    yr.backward(gy.float().permute(0, 4, 1, 2, 3))
+    assert rel(y.float().cpu(), yr.detach().permute(0, 2, 3, 4, 1)) < 2.0 ** -8
+    assert rel(xg.grad.float().cpu(), xr.grad.permute(0, 2, 3, 4, 1)) < 2.0 ** -8
