@@ -8,12 +8,10 @@
 //    feeds 8 consecutive k (8 channels of one tap). Bias and ReLU are fused in the epilogue. The
 //    input gradient is the same kernel on dY with the flipped, transposed weights
 //    W'[ci][26 - tap][co] = W[co][tap][ci].
-//  * weight gradient: dW[co][k] = sum_voxel dY[voxel][co] P[voxel][k] with
-//    v_mfma_f32_16x16x32_bf16 fed the raw BF16 bits (products exact in FP32): a block per (group
-//    of x rows, 64 k), one 16-column slice of K per wave; each row's output gradient is staged
-//    once per block in LDS, transposed to channel-major in chunks of 256 voxels, so a lane's 8
-//    voxels of one channel are one 16-byte LDS read; the input is gathered per tap. Each block
-//    adds its partial dW to the FP32 master gradient with float atomics.
+//  * weight gradient: dW[co][tap][ci] = sum_voxel dY[voxel][co] x[voxel + tap][ci] with
+//    v_mfma_f32_16x16x32_bf16 fed the raw BF16 bits (products exact in FP32), voxels as k: a wave
+//    per 16 x 16 channels and x segment, walking rows. Each block adds its sums to the FP32 master
+//    gradient with float atomics.
 //  * 1-channel layers (first layer Cin = 1, last layer Cout = 1): direct FP32 VALU kernels
 //    (forward, input gradient, weight gradient).
 //
@@ -26,6 +24,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <utility>
 
 #include "fc_device.h"
 #include "fc_internal.h"
@@ -260,93 +259,168 @@ __global__ __launch_bounds__(256) void flip_transpose_weights(const uint16_t* __
 }
 
 // ---- weight gradient -------------------------------------------------------------------------
-// grid.x: groups of kRows x-rows (n, z, y); grid.y: blocks of 64 k, one 16-column slice per wave.
-// The row's output gradient is staged once per block in LDS (channel-major, 256-voxel chunks) and
-// read by all four waves, so it is fetched from HBM / L2 once per 64 columns of K. dW (FP32) is
-// accumulated.
-constexpr int kRows = 8;
-constexpr int kWgChunk = 256;            // voxels of a row staged at once
-constexpr int kWgPitch = kWgChunk + 8;    // LDS row pitch (elements): 16-byte aligned rows
-template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void conv_wgrad_mfma(const uint16_t* __restrict__ x,
-                                                       const uint16_t* __restrict__ dy,
-                                                       float* __restrict__ dw, int N, int D,
-                                                       int H, int W) {
-  constexpr int K = 27 * CIN;
-  constexpr int NB = (COUT + 15) / 16;
-  // the output-gradient chunk of the current row, transposed: T[co][voxel - chunk start]
-  __shared__ __align__(16) uint16_t T[NB * 16][kWgPitch];
+// dW[co][tap][ci] for 16 output and 16 input channels per wave: 27 accumulators of 16 x 16, one per
+// tap, with the voxels as the MFMA's k. A wave owns 32 consecutive x voxels of the input and walks
+// rows y at fixed (n, z); per row of the output gradient it stages three new input rows (z - 1, z,
+// z + 1) and the gradient row in its own LDS, as they lie in memory (16 channels per voxel), and
+// reads them back transposed (ds_read_b64_tr_b16: four voxels of one channel per lane). The taps'
+// shift along x is applied to the gradient row (three fragments), so an input fragment serves its
+// three dx; along y it is kept in registers for the three rows that use it. A row then costs 27
+// instructions, 6 KB of LDS reads and no barrier. The waves of a block add their sums in LDS and the
+// block adds them to dW with float atomics.
+//
+// Bound by the matrix instructions (27 x 16 clocks per row and wave) with two waves per SIMD (108
+// accumulator registers). Before, every lane gathered its eight voxels one by one for each tap:
+// a training step's seven layers (4 x 128^3) took 19.1 ms; 48 -> 16 channels at 4 x 128^3 7.88 ->
+// 0.52 ms, 16 -> 16 2.24 -> 0.17 ms, 96 -> 32 at 4 x 64^3 2.12 -> 0.22 ms.
+constexpr int kWgSeg = 32;                        // input voxels per wave and row
+constexpr int kWgWaveB = 3 * kWgSeg * 32 + 34 * 32;  // LDS bytes per wave: three rows, gradient row
+constexpr int kWgRed = 4;                         // accumulators reduced at once
+
+struct WgArgs {
+  const uint16_t* x;
+  const uint16_t* dy;
+  float* dw;
+  long long units;  // (n, z, y chunk, x segment)
+  int D, H, W, cin, cout;
+  int nseg, nyc, yc;
+};
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// input rows: the caller's buffer may start at any element
+typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+
+// Eight voxels of one channel per lane from voxels of 32 bytes (16 channels): lane (m, g) gets
+// channel m of voxels 8 g .. 8 g + 7. A transposed read takes, per 16 lanes, four voxels: lane j
+// addresses voxel j / 4, channels 4 (j % 4) .. + 3, and receives channel j of all four.
+__device__ __forceinline__ bf16x8 read_channel(const char* row, int lane) {
+  typedef __attribute__((address_space(3))) s16x4* lds_p;
+  const char* p = row + (8 * (lane >> 4) + ((lane & 15) >> 2)) * 32 + (lane & 3) * 8;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_p)p);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_p)(p + 4 * 32));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// Orders a wave's LDS writes before its lanes' later reads, and reads before later writes. LDS
+// operations of one wave execute in order; this only keeps the compiler from moving them.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
+  __shared__ __align__(16) char lds[4 * kWgWaveB];
+  static_assert(4 * kWgRed * 1024 <= 4 * kWgWaveB, "the reduction reuses the rows' LDS");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int kk = blockIdx.y * 64 + wave * 16 + m;  // B column of this lane
-  const bool kvalid = kk < K;
-  const int tap = kvalid ? kk / CIN : 0, ci = kvalid ? kk - (kk / CIN) * CIN : 0;
-  const int dz = tap / 9, dyy = (tap / 3) % 3, dx = tap % 3;
-  const int nrows = N * D * H;
-  f32x4 acc[NB];
+  const int ncb = a.cin / 16, nco = a.cout / 16;
+  int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int ci0 = b % ncb * 16; b /= ncb;
+  const int co0 = b % nco * 16; b /= nco;
+  const long long unit = (long long)b * 4 + wave;
+  f32x4 acc[3][3][3];  // [dz][dy][dx]
 #pragma unroll
-  for (int cb = 0; cb < NB; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int rr = 0; rr < kRows; ++rr) {
-    const int row = blockIdx.x * kRows + rr;
-    if (row >= nrows) break;  // uniform over the block
-    const int yv = row % H, nz = row / H;
-    const int z = nz % D, n = nz / D;
-    const int zz = z + dz - 1, yy = yv + dyy - 1;
-    const bool rvalid = kvalid && zz >= 0 && zz < D && yy >= 0 && yy < H;
-    const size_t xrow = (((size_t)n * D + zz) * H + yy) * W;
-    const size_t yrow = (((size_t)n * D + z) * H + yv) * W;
-    for (int xc = 0; xc < W; xc += kWgChunk) {
-      const int nv = min(kWgChunk, W - xc);
-      const int nvp = (nv + 31) & ~31;  // the x0 loop reads whole 32-voxel steps
-      __syncthreads();  // the previous chunk is no longer read
-      // stage: 8 consecutive channels of one voxel per 16-byte load, zero past the row's end
-      for (int e = threadIdx.x; e < nvp * (COUT / 8); e += 256) {
-        const int v = e / (COUT / 8), c8 = (e - v * (COUT / 8)) * 8;
-        u32x4 q = u32x4{0u, 0u, 0u, 0u};
-        if (v < nv) q = *reinterpret_cast<const u32x4*>(dy + (yrow + xc + v) * COUT + c8);
+  for (int q = 0; q < 27; ++q) acc[q / 9][q / 3 % 3][q % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (unit < a.units) {
+    long long u = unit;
+    const int x0 = (int)(u % a.nseg) * kWgSeg; u /= a.nseg;
+    const int y0 = (int)(u % a.nyc) * a.yc; u /= a.nyc;
+    const int z = (int)(u % a.D);
+    const long long n = u / a.D;
+    const int y1 = min(a.H, y0 + a.yc);
+    char* xr = lds + wave * kWgWaveB;
+    char* gr = xr + 3 * kWgSeg * 32;
+    const int xv = x0 + (lane >> 1);                     // input voxel of this lane's 16 bytes
+    const int gv0 = x0 - 1 + (lane >> 1), gv1 = gv0 + 32;  // gradient voxels (gv1: lanes 0 - 3)
+    const bool xok = xv < a.W, g0ok = gv0 >= 0 && gv0 < a.W, g1ok = lane < 4 && gv1 < a.W;
+    u32x4 px[3], pg0, pg1;
+    // input rows yy of the three planes, and gradient row yg, as zeros outside the volume
+    auto fetch_x = [&](int yy) {
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          T[c8 + 2 * h][v] = (uint16_t)(q[h] & 0xffffu);
-          T[c8 + 2 * h + 1][v] = (uint16_t)(q[h] >> 16);
-        }
+      for (int d = 0; d < 3; ++d) {
+        const int zz = z + d - 1;
+        px[d] = u32x4{0u, 0u, 0u, 0u};
+        if (xok && zz >= 0 && zz < a.D && yy >= 0 && yy < a.H)
+          px[d] = *reinterpret_cast<const u32x4_a2*>(
+              a.x + (((n * a.D + zz) * a.H + yy) * a.W + xv) * a.cin + ci0 + 8 * (lane & 1));
       }
-      __syncthreads();
-      // 32 voxels per step: lane (m, g) supplies voxels x0 + 8 g + q, q = 0..7, of its output
-      // channel (A, one 16-byte LDS read) and of its K column (B, gathered) as raw BF16 bits
-      for (int x0 = 0; x0 < nv; x0 += 32) {
-        uint32_t bw[4];
+    };
+    auto fetch_g = [&](int yg) {
+      const uint16_t* p = a.dy + ((n * a.D + z) * a.H + yg) * a.W * a.cout + co0 + 8 * (lane & 1);
+      pg0 = pg1 = u32x4{0u, 0u, 0u, 0u};
+      if (g0ok) pg0 = *reinterpret_cast<const u32x4*>(p + (long long)gv0 * a.cout);
+      if (g1ok) pg1 = *reinterpret_cast<const u32x4*>(p + (long long)gv1 * a.cout);
+    };
+    auto put_x = [&]() {
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          uint32_t pr = 0u;
+      for (int d = 0; d < 3; ++d)
+        *reinterpret_cast<u32x4*>(xr + d * kWgSeg * 32 + lane * 16) = px[d];
+    };
+    bf16x8 B[3][3];  // [dz][row mod 3]
+    auto read_x = [&](int slot) {
 #pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const int xv = xc + x0 + g * 8 + 2 * h + e;
-            const int xx = xv + dx - 1;
-            uint32_t v = 0u;
-            if (rvalid && xv < W && xx >= 0 && xx < W) v = x[(xrow + xx) * CIN + ci];
-            pr |= v << (16 * e);
-          }
-          bw[h] = pr;
+      for (int d = 0; d < 3; ++d) B[d][slot] = read_channel(xr + d * kWgSeg * 32, lane);
+    };
+    fetch_x(y0 - 1);
+    put_x();
+    wave_sync();
+    read_x(0);
+    fetch_x(y0);
+    wave_sync();
+    put_x();
+    wave_sync();
+    read_x(1);
+    wave_sync();
+    fetch_x(y0 + 1);
+    fetch_g(y0);
+    for (int y = y0; y < y1;) {
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {  // rows y - 1, y, y + 1 are in slots r, r + 1, r + 2 mod 3
+        if (y >= y1) break;
+        put_x();
+        *reinterpret_cast<u32x4*>(gr + lane * 16) = pg0;
+        if (lane < 4) *reinterpret_cast<u32x4*>(gr + (64 + lane) * 16) = pg1;
+        wave_sync();
+        if (y + 1 < y1) {
+          fetch_x(y + 2);
+          fetch_g(y + 1);
         }
-        const bf16x8 bv = __builtin_bit_cast(bf16x8, u32x4{bw[0], bw[1], bw[2], bw[3]});
+        read_x((r + 2) % 3);
+        bf16x8 A[3];
 #pragma unroll
-        for (int cb = 0; cb < NB; ++cb) {
-          const u32x4 aq = *reinterpret_cast<const u32x4*>(&T[cb * 16 + m][x0 + g * 8]);
-          acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, aq), bv,
-                                                            acc[cb], 0, 0, 0);
-        }
+        for (int dx = 0; dx < 3; ++dx) A[dx] = read_channel(gr + (2 - dx) * 32, lane);
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+              acc[d][dy][dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  A[dx], B[d][(r + dy) % 3], acc[d][dy][dx], 0, 0, 0);
+        wave_sync();
+        ++y;
       }
     }
   }
+  // sum over the block's waves, kWgRed taps at a time: part[wave][tap][co][ci]
+  float* part = reinterpret_cast<float*>(lds);
 #pragma unroll
-  for (int cb = 0; cb < NB; ++cb)
+  for (int q0 = 0; q0 < 27; q0 += kWgRed) {
+    __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float v = acc[cb][r];
-      const int co = cb * 16 + g * 4 + r;                  // D row
-      const int kc = blockIdx.y * 64 + wave * 16 + m;      // D column
-      if (co < COUT && kc < K && v != 0.0f) unsafeAtomicAdd(dw + (size_t)co * K + kc, v);
+    for (int q = q0; q < q0 + kWgRed && q < 27; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[((wave * kWgRed + q - q0) * 16 + 4 * g + r) * 16 + m] = acc[q / 9][q / 3 % 3][q % 3][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < kWgRed * 256 && q0 + e / 256 < 27; e += 256) {
+      const int co = co0 + e / 16 % 16, ci = ci0 + e % 16;
+      const float v = part[e] + part[e + kWgRed * 256] + part[e + 2 * kWgRed * 256] +
+                      part[e + 3 * kWgRed * 256];
+      if (v != 0.0f)
+        unsafeAtomicAdd(a.dw + ((size_t)co * 27 + (q0 + e / 256)) * a.cin + ci, v);
     }
+  }
 }
 
 // ---- 1-channel layers (FP32 VALU) ------------------------------------------------------------
@@ -566,19 +640,28 @@ bool launch_fwd(int cin, int cout, const void* x, const void* w, const float* b,
 
 bool launch_wgrad(int cin, int cout, const void* x, const void* dy, float* dw, int N, int D,
                   int H, int W, hipStream_t s) {
-  const int K = 27 * cin;
-  const int rows = N * D * H;
-  dim3 grid((rows + kRows - 1) / kRows, (K + 63) / 64);
-#define FC_WG_CASE(ci, co)                                                                   \
-  if (cin == ci && cout == co) {                                                             \
-    conv_wgrad_mfma<ci, co><<<grid, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)dy, dw, \
-                                                 N, D, H, W);                                \
-    return true;                                                                             \
-  }
-  FC_WG_CASE(16, 16) FC_WG_CASE(16, 32) FC_WG_CASE(32, 32) FC_WG_CASE(32, 64)
-  FC_WG_CASE(64, 64) FC_WG_CASE(96, 32) FC_WG_CASE(48, 16)
-#undef FC_WG_CASE
-  return false;
+  bool known = false;  // the network's layers
+  for (const auto& p : {std::pair<int, int>{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64},
+                        {96, 32}, {48, 16}})
+    known = known || (p.first == cin && p.second == cout);
+  if (!known) return false;
+  WgArgs a;
+  a.x = (const uint16_t*)x;
+  a.dy = (const uint16_t*)dy;
+  a.dw = dw;
+  a.D = D; a.H = H; a.W = W; a.cin = cin; a.cout = cout;
+  a.nseg = (W + kWgSeg - 1) / kWgSeg;
+  // about 4096 waves (two rounds of two per SIMD), at least eight rows each: a wave's first two
+  // input rows and its share of the final sum are then a small part
+  const int combos = cin / 16 * (cout / 16);
+  const long long columns = (long long)N * D * a.nseg * combos;
+  const int want = (int)std::min<long long>((H + 7) / 8, (4096 + columns - 1) / columns);
+  a.yc = (H + want - 1) / want;
+  a.nyc = (H + a.yc - 1) / a.yc;
+  a.units = (long long)N * D * a.nseg * a.nyc;
+  const long long blocks = (a.units + 3) / 4 * combos;
+  conv_wgrad_mfma<<<(unsigned)blocks, 256, 0, s>>>(a);
+  return true;
 }
 
 }  // namespace

@@ -256,3 +256,23 @@ def test_conv_tile_edges(gpu, cin, cout, shape):
     yr.backward(gy.float().permute(0, 4, 1, 2, 3))
     assert rel(y.float().cpu(), yr.detach().permute(0, 2, 3, 4, 1)) < 2.0 ** -8
     assert rel(xg.grad.float().cpu(), xr.grad.permute(0, 2, 3, 4, 1)) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 16), (48, 16), (32, 64)])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 2, 8, 32), (2, 9, 17, 33), (1, 3, 26, 65)])
+def test_weight_gradient_segment_edges(gpu, cin, cout, shape):
+    # rows of one voxel, one whole segment of 32 and one voxel past a segment; one row, and row
+    # chunks that leave a remainder. The products are exact in FP32 and the sums differ from the
+    # FP64 reference by their FP32 rounding: below sqrt(terms) 2^-24 of the sum of magnitudes, so
+    # rel. L2 < 1e-5 for these few thousand terms
+    from fastcone_amd.unet import conv3d
+    g = torch.Generator().manual_seed(cin + cout + sum(shape))
+    x = torch.randn(shape + (cin,), generator=g).to(torch.bfloat16)
+    gy = torch.randn(shape + (cout,), generator=g).to(torch.bfloat16)
+    w = torch.zeros((cout, 27, cin), device=gpu, requires_grad=True)
+    conv3d(x.to(gpu), w, torch.zeros(cout, device=gpu), False).backward(gy.to(gpu))
+    wr = torch.zeros((cout, cin, 3, 3, 3), dtype=torch.float64, requires_grad=True)
+    yr = torch.nn.functional.conv3d(x.double().permute(0, 4, 1, 2, 3), wr, padding=1)
+    yr.backward(gy.double().permute(0, 4, 1, 2, 3))
+    ref = wr.grad.permute(0, 2, 3, 4, 1).reshape(cout, 27, cin)
+    assert rel(w.grad.cpu(), ref) < 1e-5
