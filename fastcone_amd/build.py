@@ -20,7 +20,7 @@ ARCH = os.environ.get("FASTCONE_ARCH", "gfx950")
 
 HIP_SOURCES = ["fc_runtime.hip", "fc_project.hip", "fc_backproject.hip", "fc_util.hip",
                "fc_filter.hip",
-               "fc_geometry.cpp", "fc_katsevich.hip", "fc_conv3d.hip"]
+               "fc_geometry.cpp", "fc_katsevich.hip", "fc_conv3d.hip", "fc_net.hip"]
 C_SOURCES = ["wrapper.c"]
 
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

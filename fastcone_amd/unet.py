@@ -7,7 +7,8 @@ nearest-neighbour upsampling up with channel concatenation of the skip connectio
 correction from the FDK reconstruction to the CGLS reconstruction.
 
 Convolutions (forward, input gradient, weight gradient) run in fc_conv3d_* (MFMA); pooling,
-upsampling, concatenation, ReLU masks and the loss are torch element-wise glue. Master weights and
+upsampling with concatenation, their gradients and the ReLU mask with the bias gradient in
+fc_net_*; the loss is torch's. Master weights and
 Adam state are FP32; the kernels read BF16 copies.
 """
 import math
@@ -32,6 +33,12 @@ def _stream(t):
     return ctypes.c_void_p(int(torch.cuda.current_stream(t.device).cuda_stream))
 
 
+def _packed(t):
+    """t, contiguous and 16-byte aligned (a gradient may come as any view)."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 class _Conv(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w32, b32, cin, cout, relu):
@@ -54,15 +61,25 @@ class _Conv(torch.autograd.Function):
         x, wb, y = ctx.saved_tensors
         cin, cout, relu = ctx.cfg
         N, D, H, W, _ = x.shape
-        if relu:
-            gy = gy * (y > 0)
-        gy = gy.to(torch.float32 if cout == 1 else torch.bfloat16).contiguous()
         L = _native.lib()
+        db = None
+        if relu and gy.dtype == torch.bfloat16 and not torch.is_grad_enabled():
+            # mask and bias gradient in one pass
+            g0, gy = _packed(gy), torch.empty_like(y)
+            db = torch.zeros(cout, dtype=torch.float32, device=y.device)
+            _native.check(L.fc_net_relu_grad_dev(y.device.index, g0.data_ptr(), y.data_ptr(),
+                                                 gy.data_ptr(), db.data_ptr(), N * D * H * W,
+                                                 cout, _stream(y)))
+        else:
+            if relu:
+                gy = gy * (y > 0)
+            gy = gy.to(torch.float32 if cout == 1 else torch.bfloat16).contiguous()
         dw = torch.zeros((cout, 27, cin), dtype=torch.float32, device=x.device)
         rc = L.fc_conv3d_wgrad_dev(x.device.index, x.data_ptr(), gy.data_ptr(), dw.data_ptr(),
                                    N, D, H, W, cin, cout, _stream(x))
         _native.check(rc)
-        db = gy.float().sum(dim=(0, 1, 2, 3))
+        if db is None:
+            db = gy.float().sum(dim=(0, 1, 2, 3))
         dx = None
         if ctx.needs_input_grad[0]:
             dx = torch.empty_like(x)
@@ -89,6 +106,59 @@ def upsample2(x):
     N, D, H, W, C = x.shape
     return x[:, :, None, :, None, :, None, :].expand(N, D, 2, H, 2, W, 2, C).reshape(
         N, 2 * D, 2 * H, 2 * W, C)
+
+
+class _Pool(torch.autograd.Function):
+    """A level's output for its skip connection and, average-pooled (avgpool2), for the next level.
+    One function for both uses, so that their gradients are added in the pooling's backward pass."""
+
+    @staticmethod
+    def forward(ctx, x):
+        N, D, H, W, C = x.shape
+        y = torch.empty((N, D // 2, H // 2, W // 2, C), dtype=x.dtype, device=x.device)
+        _native.check(_native.lib().fc_net_pool_dev(x.device.index, x.data_ptr(), y.data_ptr(), N,
+                                                    D, H, W, C, _stream(x)))
+        return x.view_as(x), y
+
+    @staticmethod
+    def backward(ctx, gs, gp):
+        N, D, H, W, C = gs.shape
+        # the skip gradient is a channel slice of the concatenation's: voxels at a fixed pitch
+        pitch = gs.stride(3)
+        if gs.stride() != (D * H * W * pitch, H * W * pitch, W * pitch, pitch, 1) or pitch % 8 \
+                or gs.data_ptr() % 16:
+            gs, pitch = _packed(gs), C
+        gp = _packed(gp)
+        g = torch.empty((N, D, H, W, C), dtype=gs.dtype, device=gs.device)
+        _native.check(_native.lib().fc_net_skip_pool_grad_dev(
+            gs.device.index, gs.data_ptr(), pitch, gp.data_ptr(), g.data_ptr(), N, D, H, W, C,
+            _stream(gs)))
+        return g
+
+
+class _UpCat(torch.autograd.Function):
+    """upsample2(a) and b concatenated along the channels."""
+
+    @staticmethod
+    def forward(ctx, a, b):
+        N, D, H, W, cb = b.shape
+        ctx.ca = a.shape[4]
+        out = torch.empty((N, D, H, W, ctx.ca + cb), dtype=b.dtype, device=b.device)
+        _native.check(_native.lib().fc_net_up_cat_dev(b.device.index, a.data_ptr(), b.data_ptr(),
+                                                      out.data_ptr(), N, D, H, W, ctx.ca, cb,
+                                                      _stream(b)))
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        N, D, H, W, C = g.shape
+        ca = ctx.ca
+        g = _packed(g)
+        ga = torch.empty((N, D // 2, H // 2, W // 2, ca), dtype=g.dtype, device=g.device)
+        _native.check(_native.lib().fc_net_up_cat_grad_dev(g.device.index, g.data_ptr(),
+                                                           ga.data_ptr(), N, D, H, W, ca, C - ca,
+                                                           _stream(g)))
+        return ga, g[..., ca:]
 
 
 class UNet3D(torch.nn.Module):
@@ -118,11 +188,11 @@ class UNet3D(torch.nn.Module):
             if s % 4:
                 raise ValueError("volume sides must be multiples of 4")
         x = (vol * self.SCALE).to(torch.bfloat16)[..., None].contiguous()
-        e1 = self._c(self._c(x, "e1a"), "e1b")
-        e2 = self._c(self._c(avgpool2(e1), "e2a"), "e2b")
-        bt = self._c(self._c(avgpool2(e2), "b_a"), "b_b")
-        d2 = self._c(self._c(torch.cat([upsample2(bt), e2], dim=-1).contiguous(), "d2a"), "d2b")
-        d1 = self._c(self._c(torch.cat([upsample2(d2), e1], dim=-1).contiguous(), "d1a"), "d1b")
+        e1, p1 = _Pool.apply(self._c(self._c(x, "e1a"), "e1b"))
+        e2, p2 = _Pool.apply(self._c(self._c(p1, "e2a"), "e2b"))
+        bt = self._c(self._c(p2, "b_a"), "b_b")
+        d2 = self._c(self._c(_UpCat.apply(bt, e2), "d2a"), "d2b")
+        d1 = self._c(self._c(_UpCat.apply(d2, e1), "d1a"), "d1b")
         out = vol + self._c(d1, "out")[..., 0] / self.SCALE
         return out[0] if single else out
 

@@ -208,6 +208,23 @@ int fc_conv3d_dgrad_dev(int device, const void* dy, const void* w, void* wt, voi
 /* dw (FP32 [cout][27][cin]) += weight gradient for input x and output gradient dy. */
 int fc_conv3d_wgrad_dev(int device, const void* x, const void* dy, float* dw, int N, int D, int H,
                         int W, int cin, int cout, void* stream);
+/* The network's element-wise steps on the same BF16 layout (16-byte aligned; D, H, W even and the
+ * fine sizes). fc_net_pool_dev: y = mean over 2x2x2 voxels, c = 16 or 32. fc_net_up_cat_dev: out =
+ * (a upsampled by 2, nearest; b) along the channels, ca + cb = 64 + 32 or 32 + 16.
+ * fc_net_up_cat_grad_dev: ga = the gradient with respect to a for output gradient g (b's is a channel
+ * slice of g). fc_net_skip_pool_grad_dev: g = gs + the pooling's gradient for gp, gs holding c
+ * channels of every gs_pitch. fc_net_relu_grad_dev: gm = gy where y > 0, else 0, and db[c] (FP32) +=
+ * its sum over the voxels, c = 16, 32 or 64. No counterpart in the reference. */
+int fc_net_pool_dev(int device, const void* x, void* y, int N, int D, int H, int W, int c,
+                    void* stream);
+int fc_net_up_cat_dev(int device, const void* a, const void* b, void* out, int N, int D, int H,
+                      int W, int ca, int cb, void* stream);
+int fc_net_up_cat_grad_dev(int device, const void* g, void* ga, int N, int D, int H, int W,
+                           int ca, int cb, void* stream);
+int fc_net_skip_pool_grad_dev(int device, const void* gs, int gs_pitch, const void* gp, void* g,
+                              int N, int D, int H, int W, int c, void* stream);
+int fc_net_relu_grad_dev(int device, const void* gy, const void* y, void* gm, float* db,
+                         long long voxels, int c, void* stream);
 /* One 16x16x32 BF16 and one 16x16x4 FP32 MFMA product of row-major A, B (single wave): checks the
  * operand / result lane layouts the convolution kernels assume. */
 int fc_mfma_layout_probe(int device, const void* A32, const void* B32, const float* A4,

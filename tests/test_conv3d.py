@@ -276,3 +276,55 @@ def test_weight_gradient_segment_edges(gpu, cin, cout, shape):
     yr.backward(gy.double().permute(0, 4, 1, 2, 3))
     ref = wr.grad.permute(0, 2, 3, 4, 1).reshape(cout, 27, cin)
     assert rel(w.grad.cpu(), ref) < 1e-5
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 2, 2), (2, 4, 6, 10), (1, 6, 2, 130)])
+@pytest.mark.parametrize("ca,cb", [(32, 16), (64, 32)])
+def test_pool_and_up_cat_match_torch(gpu, shape, ca, cb):
+    # rows shorter and longer than a block of 256 units; the layers' results are those of avgpool2,
+    # upsample2 and torch.cat, and their gradients those of torch's backward pass up to one BF16
+    # rounding of a sum (2^-8 relative)
+    from fastcone_amd.unet import _Pool, _UpCat, avgpool2, upsample2
+    N, D, H, W = shape
+    g = torch.Generator().manual_seed(ca + sum(shape))
+    bf = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).to(gpu)
+    e, a = bf(N, D, H, W, cb), bf(N, D // 2, H // 2, W // 2, ca)
+    gc, gp = bf(N, D, H, W, ca + cb), bf(N, D // 2, H // 2, W // 2, cb)
+    out = []
+    for ours in (True, False):
+        x, y = e.clone().requires_grad_(True), a.clone().requires_grad_(True)
+        skip, pool = _Pool.apply(x) if ours else (x, avgpool2(x))
+        c = _UpCat.apply(y, skip) if ours else torch.cat([upsample2(y), skip], dim=-1)
+        torch.autograd.backward([c, pool], [gc, gp])
+        out.append((c.detach(), pool.detach(), y.grad, x.grad))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert rel(out[0][2].cpu(), out[1][2].cpu()) < 2.0 ** -8
+    assert rel(out[0][3].cpu(), out[1][3].cpu()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("voxels", [1, 127, 4097, 70001])
+@pytest.mark.parametrize("c", [16, 32, 64])
+def test_relu_gradient_kernel(gpu, voxels, c):
+    # one block and several, with remainders; the masked gradient is exact, a NaN or infinite
+    # gradient of a masked value is NaN, and the bias gradient differs from the FP64 sum by FP32
+    # rounding: at most sqrt(voxels) 2^-24 of the sum of magnitudes
+    import ctypes
+    from fastcone_amd import _native
+    g = torch.Generator().manual_seed(voxels + c)
+    gy = torch.randn((voxels, c), generator=g).to(torch.bfloat16)
+    y = torch.randn((voxels, c), generator=g).to(torch.bfloat16)
+    ref = gy * (y > 0)
+    gd, yd = gy.to(gpu), y.to(gpu)
+    gm = torch.empty_like(gd)
+    db = torch.zeros(c, device=gpu)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    L = _native.lib()
+    _native.check(L.fc_net_relu_grad_dev(gpu.index, gd.data_ptr(), yd.data_ptr(), gm.data_ptr(),
+                                         db.data_ptr(), voxels, c, st))
+    assert torch.equal(gm.cpu(), ref)
+    bound = ref.double().abs().sum(0) * (voxels ** 0.5 + 1.0) * 2.0 ** -24 + 1e-30
+    assert bool(((db.double().cpu() - ref.double().sum(0)).abs() <= bound).all())
+    gd[0, 0], yd[0, 0] = float("inf"), -1.0
+    _native.check(L.fc_net_relu_grad_dev(gpu.index, gd.data_ptr(), yd.data_ptr(), gm.data_ptr(),
+                                         db.data_ptr(), voxels, c, st))
+    assert bool(gm[0, 0].isnan()) and bool(db[0].isnan())
