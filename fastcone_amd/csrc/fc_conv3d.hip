@@ -12,8 +12,9 @@
 //    v_mfma_f32_16x16x32_bf16 fed the raw BF16 bits (products exact in FP32), voxels as k: a wave
 //    per 16 x 16 channels and x segment, walking rows. Each block adds its sums to the FP32 master
 //    gradient with float atomics.
-//  * 1-channel layers (first layer Cin = 1, last layer Cout = 1): direct FP32 VALU kernels
-//    (forward, input gradient, weight gradient).
+//  * 1-channel layers (first layer Cin = 1, last layer Cout = 1): forward passes and the last
+//    layer's input gradient are FP32 FMAs in ascending order of k; both weight gradients are MFMAs
+//    over the voxels.
 //
 // Operand / result lane layouts of the MFMA form used (checked by fc_mfma_layout_probe, which also
 // checks the 16x16x4 FP32 form):
@@ -24,6 +25,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 #include <utility>
 
 #include "fc_device.h"
@@ -35,8 +37,9 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-// output stores: the caller's buffer may start at any element
+// the caller's buffers may start at any element
 typedef unsigned int u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void conv_fwd_mfma(const uint16_t* __restri
     for (int q = 0; q < NU; ++q) {
       pf[q] = u32x4{0u, 0u, 0u, 0u};
       if (zin && vox[q] >= 0)
-        pf[q] = *reinterpret_cast<const u32x4*>(p + (long long)vox[q] * CIN + ch[q]);
+        pf[q] = *reinterpret_cast<const u32x4_a2*>(p + (long long)vox[q] * CIN + ch[q]);
     }
   };
   auto put = [&](int slot) {
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(256, 2) void conv_fwd_mfma(const uint16_t* __restri
   auto wfrag = [&](int s, int cb, int from) {
     u32x4 q = u32x4{0u, 0u, 0u, 0u};
     if (K % 32 == 0 || s + 1 < KSTEPS || !hi)
-      q = *reinterpret_cast<const u32x4*>(w + from + cb * 16 * K + s * 32);
+      q = *reinterpret_cast<const u32x4_a2*>(w + from + cb * 16 * K + s * 32);
     return __builtin_bit_cast(bf16x8, q);
   };
   constexpr int G = T::kWReg ? KSTEPS : T::G;
@@ -223,14 +226,14 @@ __global__ __launch_bounds__(256, 2) void conv_fwd_mfma(const uint16_t* __restri
         uint16_t* o = y + ((((size_t)n * D + z) * H + vy) * W + vx) * COUT + 4 * g;
 #pragma unroll
         for (int cb = 0; cb < NB; ++cb) {
-          uint32_t h[4];
+          float f[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            float f = acc[v][cb][r] + bb[cb][r];
-            if (RELU) f = fmaxf(f, 0.0f);
-            h[r] = f32_to_bf16_bits(f);
+            f[r] = acc[v][cb][r] + bb[cb][r];
+            if (RELU) f[r] = fmaxf(f[r], 0.0f);
           }
-          *reinterpret_cast<u32x2_a2*>(o + cb * 16) = u32x2_a2{h[0] | h[1] << 16, h[2] | h[3] << 16};
+          *reinterpret_cast<u32x2_a2*>(o + cb * 16) =
+              u32x2_a2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
         }
       }
     }
@@ -287,9 +290,6 @@ struct WgArgs {
 };
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-// input rows: the caller's buffer may start at any element
-typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-
 // Eight voxels of one channel per lane from voxels of 32 bytes (16 channels): lane (m, g) gets
 // channel m of voxels 8 g .. 8 g + 7. A transposed read takes, per 16 lanes, four voxels: lane j
 // addresses voxel j / 4, channels 4 (j % 4) .. + 3, and receives channel j of all four.
@@ -423,163 +423,390 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
   }
 }
 
-// ---- 1-channel layers (FP32 VALU) ------------------------------------------------------------
-// Cin = 1: y[v][co] = act(b[co] + sum_tap w[co][tap] x[v + tap]); one thread per voxel.
-template <int COUT, bool RELU>
-__global__ __launch_bounds__(256) void conv_fwd_cin1(const uint16_t* __restrict__ x,
-                                                     const uint16_t* __restrict__ w,
-                                                     const float* __restrict__ bias,
-                                                     uint16_t* __restrict__ y, int N, int D,
-                                                     int H, int W) {
-  __shared__ float ws[COUT * 27];
-  for (int q = threadIdx.x; q < COUT * 27; q += 256) ws[q] = bf2f(w[q]);
-  __syncthreads();
-  const size_t nvox = (size_t)N * D * H * W;
-  const size_t v = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (v >= nvox) return;
-  const int xv = (int)(v % W), yv = (int)((v / W) % H), z = (int)((v / ((size_t)W * H)) % D);
-  const size_t n = v / ((size_t)W * H * D);
-  float acc[COUT];
-#pragma unroll
-  for (int co = 0; co < COUT; ++co) acc[co] = bias ? bias[co] : 0.0f;
-  for (int tap = 0; tap < 27; ++tap) {
-    const int zz = z + tap / 9 - 1, yy = yv + (tap / 3) % 3 - 1, xx = xv + tap % 3 - 1;
-    if (zz < 0 || zz >= D || yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
-    const float xvv = bf2f(x[((n * D + zz) * H + yy) * W + xx]);
-#pragma unroll
-    for (int co = 0; co < COUT; ++co) acc[co] = fmaf(ws[co * 27 + tap], xvv, acc[co]);
-  }
-#pragma unroll
-  for (int co = 0; co < COUT; ++co) {
-    float o = acc[co];
-    if (RELU) o = fmaxf(o, 0.0f);
-    y[v * COUT + co] = f32_to_bf16_bits(o);
-  }
-}
+// ---- 1-channel layers ------------------------------------------------------------------------
+// Sixteen channels from one: y[v][c] = act(b[c] + sum_tap w[c][tap] x[v + tap]) (the first layer) or,
+// with FLIP, sum_tap w[tap][c] x[v - tap] (the input gradient of the last layer), FP32 FMAs in
+// ascending order of the taps that lie in the volume. A thread computes kOneZ consecutive z of one
+// (x, y): an input value serves three outputs and the weights of a tap, read from LDS for the whole
+// wave, 16 kOneZ FMAs. Bound by the 432 FMAs per voxel (0.2 ms at 256^3; two, three or four waves per
+// SIMD and kOneZ = 2 or 4 take the same time). With one voxel per thread, a branch per tap and the
+// integer BF16 rounding it took 0.74 ms at 256^3, now 0.27 ms; the input gradient at 4 x 128^3 0.37
+// -> 0.14 ms.
+constexpr int kOneZ = 2;
 
-// Cout = 1: y[v] = b + sum_{tap, ci} w[tap][ci] x[v + tap][ci]  (output FP32, no activation).
-// Also the input gradient of a Cin = 1 layer reads like this with the flipped weights.
-template <int CIN>
-__global__ __launch_bounds__(256) void conv_fwd_cout1(const uint16_t* __restrict__ x,
+template <bool FLIP>
+struct OneIn {
+  using T = uint16_t;
+  static __device__ __forceinline__ float load(const T* p) { return bf2f(*p); }
+};
+template <>
+struct OneIn<true> {
+  using T = float;
+  static __device__ __forceinline__ float load(const T* p) { return *p; }
+};
+
+template <bool FLIP, bool RELU>
+__global__ __launch_bounds__(256) void conv_one_to_16(const void* __restrict__ xin,
                                                       const uint16_t* __restrict__ w,
                                                       const float* __restrict__ bias,
-                                                      float* __restrict__ y, int N, int D, int H,
-                                                      int W) {
-  __shared__ float ws[27 * CIN];
-  for (int q = threadIdx.x; q < 27 * CIN; q += 256) ws[q] = bf2f(w[q]);
-  __syncthreads();
-  const size_t nvox = (size_t)N * D * H * W;
-  const size_t v = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (v >= nvox) return;
-  const int xv = (int)(v % W), yv = (int)((v / W) % H), z = (int)((v / ((size_t)W * H)) % D);
-  const size_t n = v / ((size_t)W * H * D);
-  float acc = bias ? bias[0] : 0.0f;
-  for (int tap = 0; tap < 27; ++tap) {
-    const int zz = z + tap / 9 - 1, yy = yv + (tap / 3) % 3 - 1, xx = xv + tap % 3 - 1;
-    if (zz < 0 || zz >= D || yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
-    const uint16_t* px = x + (((n * D + zz) * H + yy) * W + xx) * CIN;
-#pragma unroll
-    for (int ci = 0; ci < CIN; ++ci) acc = fmaf(ws[tap * CIN + ci], bf2f(px[ci]), acc);
+                                                      uint16_t* __restrict__ y, int D, int H,
+                                                      int W, int nzc) {
+  using In = OneIn<FLIP>;
+  __shared__ __align__(16) float ws[27][16];
+  bool finite = true;
+  for (int q = threadIdx.x; q < 27 * 16; q += 256) {
+    const float f = bf2f(w[q]);
+    finite = finite && fabsf(f) <= 3.402823466e38f;
+    if (FLIP) ws[q / 16][q % 16] = f;
+    else ws[q % 27][q / 27] = f;
   }
-  y[v] = acc;
-}
-
-// Input gradient of a Cout = 1 layer: dx[v][ci] = sum_tap w[tap][ci] dy[v - tap] (dy FP32).
-template <int CIN>
-__global__ __launch_bounds__(256) void conv_dgrad_cout1(const float* __restrict__ dy,
-                                                        const uint16_t* __restrict__ w,
-                                                        uint16_t* __restrict__ dx, int N, int D,
-                                                        int H, int W) {
-  __shared__ float ws[27 * CIN];
-  for (int q = threadIdx.x; q < 27 * CIN; q += 256) ws[q] = bf2f(w[q]);
-  __syncthreads();
-  const size_t nvox = (size_t)N * D * H * W;
-  const size_t v = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (v >= nvox) return;
-  const int xv = (int)(v % W), yv = (int)((v / W) % H), z = (int)((v / ((size_t)W * H)) % D);
-  const size_t n = v / ((size_t)W * H * D);
-  float acc[CIN];
+  // a tap outside the volume is left out of the sum; its value is 0 here, so with finite weights it
+  // may as well be added, and the taps need no branches
+  finite = __syncthreads_and(finite);
+  const long long plane = (long long)H * W;
+  const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (p >= plane) return;
+  const int n = blockIdx.y / nzc, z0 = (blockIdx.y - n * nzc) * kOneZ;
+  const int yv = plane < (1ll << 31) ? (int)((uint32_t)p / (uint32_t)W) : (int)(p / W);
+  const int xv = (int)(p - (long long)yv * W);
+  const typename In::T* x = static_cast<const typename In::T*>(xin) + (long long)n * D * plane;
+  // v[q][t]: plane z0 - 1 + q, offset t of the 3 x 3 neighbourhood; zero outside the volume (the
+  // load then reads the thread's own voxel or the nearest plane)
+  bool ok[9];
+  float v[kOneZ + 2][9];
 #pragma unroll
-  for (int ci = 0; ci < CIN; ++ci) acc[ci] = 0.0f;
-  for (int tap = 0; tap < 27; ++tap) {
-    // dy at v - (tap - 13): the output voxel whose tap `tap` reads voxel v
-    const int zz = z - (tap / 9 - 1), yy = yv - ((tap / 3) % 3 - 1), xx = xv - (tap % 3 - 1);
-    if (zz < 0 || zz >= D || yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
-    const float g = dy[((n * D + zz) * H + yy) * W + xx];
+  for (int t = 0; t < 9; ++t) {
+    const int yy = yv + t / 3 - 1, xx = xv + t % 3 - 1;
+    ok[t] = yy >= 0 && yy < H && xx >= 0 && xx < W;
+    const typename In::T* px = x + p + (ok[t] ? (long long)(t / 3 - 1) * W + (t % 3 - 1) : 0);
 #pragma unroll
-    for (int ci = 0; ci < CIN; ++ci) acc[ci] = fmaf(ws[tap * CIN + ci], g, acc[ci]);
+    for (int q = 0; q < kOneZ + 2; ++q) {
+      const int zz = z0 - 1 + q;
+      const float f = In::load(px + min(max(zz, 0), D - 1) * plane);
+      v[q][t] = ok[t] && zz >= 0 && zz < D ? f : 0.0f;
+    }
   }
+  float acc[kOneZ][16];
 #pragma unroll
-  for (int ci = 0; ci < CIN; ++ci) dx[v * CIN + ci] = f32_to_bf16_bits(acc[ci]);
-}
-
-// Weight gradient of a Cout = 1 layer with FP32 dy: dw[tap][ci] = sum_v dy[v] x[v + tap][ci].
-// One block per (tap, chunk of voxels); each thread a subset of voxels for all ci.
-template <int CIN>
-__global__ __launch_bounds__(256) void conv_wgrad_cout1(const uint16_t* __restrict__ x,
-                                                        const float* __restrict__ dy,
-                                                        float* __restrict__ dw, int N, int D,
-                                                        int H, int W, int chunk) {
-  __shared__ float red[CIN][256];
-  const int tap = blockIdx.y;
-  const int dz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const size_t nvox = (size_t)N * D * H * W;
-  float acc[CIN];
+  for (int r = 0; r < kOneZ; ++r)
 #pragma unroll
-  for (int ci = 0; ci < CIN; ++ci) acc[ci] = 0.0f;
-  const size_t v0 = (size_t)blockIdx.x * chunk;
-  for (size_t v = v0 + threadIdx.x; v < v0 + chunk && v < nvox; v += 256) {
-    const int xv = (int)(v % W), yv = (int)((v / W) % H), z = (int)((v / ((size_t)W * H)) % D);
-    const size_t n = v / ((size_t)W * H * D);
-    const int zz = z + dz, yy = yv + dyy, xx = xv + dx;
-    if (zz < 0 || zz >= D || yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
-    const float g = dy[v];
-    const uint16_t* px = x + (((n * D + zz) * H + yy) * W + xx) * CIN;
+    for (int c = 0; c < 16; ++c) acc[r][c] = bias ? bias[c] : 0.0f;
+  auto taps = [&](auto tag) {
+    constexpr bool CHECK = decltype(tag)::value;
 #pragma unroll
-    for (int ci = 0; ci < CIN; ++ci) acc[ci] = fmaf(g, bf2f(px[ci]), acc[ci]);
-  }
+    for (int tap = 0; tap < 27; ++tap) {
+      const int dz = FLIP ? 2 - tap / 9 : tap / 9, t = FLIP ? 8 - tap % 9 : tap % 9;
+      float wt[16];
 #pragma unroll
-  for (int ci = 0; ci < CIN; ++ci) red[ci][threadIdx.x] = acc[ci];
-  __syncthreads();
-  if (threadIdx.x < CIN) {
-    float s = 0.0f;
-    for (int q = 0; q < 256; ++q) s += red[threadIdx.x][q];
-    unsafeAtomicAdd(dw + tap * CIN + threadIdx.x, s);
+      for (int c = 0; c < 16; ++c) wt[c] = ws[tap][c];
+#pragma unroll
+      for (int r = 0; r < kOneZ; ++r) {
+        const int zz = z0 + r + dz - 1;
+        if (CHECK && !(ok[t] && zz >= 0 && zz < D)) continue;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) acc[r][c] = fmaf(wt[c], v[r + dz][t], acc[r][c]);
+      }
+    }
+  };
+  if (finite) taps(std::false_type{});
+  else taps(std::true_type{});
+#pragma unroll
+  for (int r = 0; r < kOneZ; ++r) {
+    if (z0 + r >= D) break;
+    uint16_t* o = y + (((long long)n * D + z0 + r) * plane + p) * 16;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4_a2 q;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float f0 = acc[r][8 * h + 2 * e], f1 = acc[r][8 * h + 2 * e + 1];
+        if (RELU) f0 = fmaxf(f0, 0.0f), f1 = fmaxf(f1, 0.0f);
+        q[e] = pack_bf16(f0, f1);
+      }
+      *reinterpret_cast<u32x4_a2*>(o + 8 * h) = q;
+    }
   }
 }
 
-// Weight gradient of a Cin = 1 layer: dw[co][tap] = sum_v dy[v][co] x[v + tap].
-template <int COUT>
-__global__ __launch_bounds__(256) void conv_wgrad_cin1(const uint16_t* __restrict__ x,
-                                                       const uint16_t* __restrict__ dy,
-                                                       float* __restrict__ dw, int N, int D,
-                                                       int H, int W, int chunk) {
-  __shared__ float red[COUT][256];
-  const int tap = blockIdx.y;
-  const int dz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-  const size_t nvox = (size_t)N * D * H * W;
-  float acc[COUT];
-#pragma unroll
-  for (int co = 0; co < COUT; ++co) acc[co] = 0.0f;
-  const size_t v0 = (size_t)blockIdx.x * chunk;
-  for (size_t v = v0 + threadIdx.x; v < v0 + chunk && v < nvox; v += 256) {
-    const int xv = (int)(v % W), yv = (int)((v / W) % H), z = (int)((v / ((size_t)W * H)) % D);
-    const size_t n = v / ((size_t)W * H * D);
-    const int zz = z + dz, yy = yv + dyy, xx = xv + dx;
-    if (zz < 0 || zz >= D || yy < 0 || yy >= H || xx < 0 || xx >= W) continue;
-    const float xs = bf2f(x[((n * D + zz) * H + yy) * W + xx]);
-    const uint16_t* pg = dy + v * COUT;
-#pragma unroll
-    for (int co = 0; co < COUT; ++co) acc[co] = fmaf(bf2f(pg[co]), xs, acc[co]);
-  }
-#pragma unroll
-  for (int co = 0; co < COUT; ++co) red[co][threadIdx.x] = acc[co];
+template <bool FLIP, bool RELU>
+void launch_one_to_16(const void* x, const void* w, const float* b, void* y, int N, int D, int H,
+                      int W, hipStream_t s) {
+  const int nzc = (D + kOneZ - 1) / kOneZ;
+  const dim3 grid((unsigned)(((long long)H * W + 255) / 256), N * nzc);
+  conv_one_to_16<FLIP, RELU><<<grid, 256, 0, s>>>(x, (const uint16_t*)w, b, (uint16_t*)y, D, H, W,
+                                                  nzc);
+}
+
+// One FP32 channel from sixteen (the last layer): y[v] = b + sum_{tap, c} w[tap][c] x[v + tap][c], one
+// chain of FMAs per voxel in ascending order over the taps that lie in the volume. A thread computes
+// kOneY consecutive y of one (x, z): an input voxel is loaded and converted once per plane for the
+// up to three outputs that use it, and the nine taps of a plane stay in registers (144) over the
+// thread's rows; the next row's voxels are in flight meanwhile. Bound by its 432 FMAs and 216
+// conversions per voxel: 0.33 ms at 256^3, 0.66 ms with one voxel per thread (every tap's weights
+// from LDS and its input converted again). As an implicit GEMM with one used row it takes 0.25 ms,
+// but the other order of the sums changes the loss gradient's last bits, and they the BF16
+// gradients of all layers.
+constexpr int kOneY = 4;
+
+__global__ __launch_bounds__(256, 2) void conv_16_to_one(const uint16_t* __restrict__ x,
+                                                         const uint16_t* __restrict__ w,
+                                                         const float* __restrict__ bias,
+                                                         float* __restrict__ y, int D, int H,
+                                                         int W) {
+  __shared__ __align__(16) float ws[27 * 16];
+  for (int q = threadIdx.x; q < 27 * 16; q += 256) ws[q] = bf2f(w[q]);
   __syncthreads();
-  if (threadIdx.x < COUT) {
-    float s = 0.0f;
-    for (int q = 0; q < 256; ++q) s += red[threadIdx.x][q];
-    unsafeAtomicAdd(dw + threadIdx.x * 27 + tap, s);
+  const int hg = (H + kOneY - 1) / kOneY;
+  const long long cols = (long long)hg * W;
+  const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (p >= cols) return;
+  const int yg = cols < (1ll << 31) ? (int)((uint32_t)p / (uint32_t)W) : (int)(p / W);
+  const int xv = (int)(p - (long long)yg * W), y0 = yg * kOneY;
+  const int n = blockIdx.y / D, z = blockIdx.y - n * D;
+  const uint16_t* vol = x + (long long)n * D * H * W * 16;
+  constexpr int NR = kOneY + 2;  // input rows per plane
+  const bool xok[3] = {xv > 0, true, xv + 1 < W};
+  u32x4 cur[3][2], nxt[3][2];
+  // row j of plane z - 1 + d; voxels outside the volume read one inside (and are not used)
+  auto fetch = [&](int d, int j) {
+    const int zz = min(max(z - 1 + d, 0), D - 1), yy = min(max(y0 - 1 + j, 0), H - 1);
+    const uint16_t* row = vol + (((long long)zz * H + yy) * W + xv) * 16;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const u32x4_a2* q = reinterpret_cast<const u32x4_a2*>(row + (xok[t] ? (t - 1) * 16 : 0));
+      nxt[t][0] = q[0];
+      nxt[t][1] = q[1];
+    }
+  };
+  float acc[kOneY];
+#pragma unroll
+  for (int r = 0; r < kOneY; ++r) acc[r] = bias ? bias[0] : 0.0f;
+  fetch(0, 0);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    float wt[9][16];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int c = 0; c < 16; ++c) wt[t][c] = ws[(9 * d + t) * 16 + c];
+    const bool zok = z - 1 + d >= 0 && z - 1 + d < D;  // uniform
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t) cur[t][0] = nxt[t][0], cur[t][1] = nxt[t][1];
+      if (d < 2 || j + 1 < NR) fetch(j + 1 < NR ? d : d + 1, j + 1 < NR ? j + 1 : 0);
+      const int yy = y0 - 1 + j;
+      if (!zok || yy < 0 || yy >= H) continue;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        if (!xok[t]) continue;
+        float f[16];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const uint32_t u = cur[t][q / 4][q % 4];
+          f[2 * q] = __uint_as_float(u << 16);
+          f[2 * q + 1] = __uint_as_float(u & 0xffff0000u);
+        }
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+#pragma unroll
+          for (int r = 0; r < kOneY; ++r) {
+            const int dy = j - r;  // output row y0 + r uses this row as its tap dy
+            if (dy >= 0 && dy < 3) acc[r] = fmaf(wt[3 * dy + t][c], f[c], acc[r]);
+          }
+      }
+    }
   }
+#pragma unroll
+  for (int r = 0; r < kOneY; ++r)
+    if (y0 + r < H) y[(((long long)n * D + z) * H + y0 + r) * W + xv] = acc[r];
+}
+
+void launch_16_to_one(const void* x, const void* w, const float* b, float* y, int N, int D, int H,
+                      int W, hipStream_t s) {
+  const long long cols = (long long)((H + kOneY - 1) / kOneY) * W;
+  conv_16_to_one<<<dim3((unsigned)((cols + 255) / 256), N * D), 256, 0, s>>>(
+      (const uint16_t*)x, (const uint16_t*)w, b, y, D, H, W);
+}
+
+// Weight gradient of a 1-channel layer: one tensor has 16 channels per voxel ("wide", BF16), the
+// other one ("narrow": the first layer's BF16 input, or with FLIP the last layer's FP32 output
+// gradient). dW[tap][c] = sum over narrow voxels v of narrow[v] wide[v + shift(tap)][c], as MFMAs with
+// the voxels as k: the rows of A are the narrow rows (dz, dy) around the wide row, B its 16 channels
+// read transposed (as in conv_wgrad_mfma) at the three shifts along x. FP32 narrow values are split
+// into three BF16 parts of eight significant bits each (their sum is exact), one row of A per part:
+// the products are exact in FP32 and only the order of the sums differs from FP32 FMAs.
+// A wave owns 32 narrow x voxels and walks rows y at fixed (n, z). Bound by the reading of the wide
+// tensor (0.27 GB at 4 x 128^3: 0.06 ms at the rate of a large copy). Before, a block per tap read
+// both tensors again: first layer 1.05 -> 0.11 ms, last layer 1.11 -> 0.07 ms there.
+constexpr int kNrPitch = 80;  // bytes of 32 BF16 values, padded: rows four apart share no bank
+constexpr int kNrWaves = 16;  // waves per block: few blocks keep the chain of atomic sums short
+
+struct WgNarrowArgs {
+  const uint16_t* wide;
+  const void* narrow;
+  float* dw;
+  long long units;  // (n, z, y chunk, x segment)
+  int D, H, W;
+  int nseg, nyc, yc;
+};
+
+template <bool FLIP>
+__global__ __launch_bounds__(64 * kNrWaves) void conv_wgrad_narrow(WgNarrowArgs a) {
+  constexpr int PARTS = FLIP ? 3 : 1, ROWS = 9 * PARTS, MT = (ROWS + 15) / 16;
+  constexpr int kNarrowB = 9 * PARTS * kNrPitch, kWaveB = kNarrowB + 34 * 32;
+  constexpr int kRedB = kNrWaves * MT * 1024;  // one shift's accumulators
+  __shared__ __align__(16) char lds[kNrWaves * kWaveB > kRedB ? kNrWaves * kWaveB : kRedB];
+  __shared__ float sums[27 * 16];              // as dW lies in memory
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const long long unit = (long long)xcd_remap(blockIdx.x, gridDim.x) * kNrWaves + wave;
+  f32x4 acc[MT][3];
+#pragma unroll
+  for (int q = 0; q < 3 * MT; ++q) acc[q / 3][q % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (unit < a.units) {
+    long long u = unit;
+    const int x0 = (int)(u % a.nseg) * kWgSeg; u /= a.nseg;
+    const int y0 = (int)(u % a.nyc) * a.yc; u /= a.nyc;
+    const int z = (int)(u % a.D);
+    const long long n = u / a.D;
+    const int y1 = min(a.H, y0 + a.yc);
+    char* nr = lds + wave * kWaveB;       // [plane z - 1 + d][row mod 3][part]
+    char* wr = nr + kNarrowB;             // wide voxels x0 - 1 .. x0 + 32
+    const int wv0 = x0 - 1 + (lane >> 1), wv1 = wv0 + 32;
+    const bool w0ok = wv0 >= 0 && wv0 < a.W, w1ok = lane < 4 && wv1 < a.W;
+    u32x4 pw0, pw1;
+    float pn[2];
+    auto fetch_w = [&](int yy) {
+      const uint16_t* p = a.wide + ((n * a.D + z) * a.H + yy) * a.W * 16 + 8 * (lane & 1);
+      pw0 = pw1 = u32x4{0u, 0u, 0u, 0u};
+      if (w0ok) pw0 = *reinterpret_cast<const u32x4_a2*>(p + (long long)wv0 * 16);
+      if (w1ok) pw1 = *reinterpret_cast<const u32x4_a2*>(p + (long long)wv1 * 16);
+    };
+    // value q of this lane: plane (lane + 64 q) / 32, voxel (lane + 64 q) % 32 of row yy
+    auto fetch_n = [&](int yy) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int e = lane + 64 * q, zz = z - 1 + e / 32, xx = x0 + e % 32;
+        pn[q] = 0.0f;
+        if (e < 96 && zz >= 0 && zz < a.D && yy >= 0 && yy < a.H && xx < a.W) {
+          const long long i = ((n * a.D + zz) * a.H + yy) * a.W + xx;
+          pn[q] = FLIP ? static_cast<const float*>(a.narrow)[i]
+                       : bf2f(static_cast<const uint16_t*>(a.narrow)[i]);
+        }
+      }
+    };
+    auto put_n = [&](int slot) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int e = lane + 64 * q;
+        if (e >= 96) continue;
+        uint16_t* o = reinterpret_cast<uint16_t*>(nr + ((e / 32 * 3 + slot) * PARTS) * kNrPitch) +
+                      e % 32;
+        uint32_t b = __float_as_uint(pn[q]);
+        if constexpr (FLIP) {
+          // parts by truncation; an infinite value has no further parts, a NaN stays one
+          const bool fin = (b & 0x7f800000u) != 0x7f800000u;
+          if ((b & 0x7fffffffu) > 0x7f800000u) b |= 0x400000u;
+          const float r1 = fin ? pn[q] - __uint_as_float(b & 0xffff0000u) : 0.0f;
+          const uint32_t b1 = __float_as_uint(r1) & 0xffff0000u;
+          const float r2 = r1 - __uint_as_float(b1);
+          o[kNrPitch / 2] = (uint16_t)(b1 >> 16);
+          o[kNrPitch] = (uint16_t)(__float_as_uint(r2) >> 16);
+        }
+        o[0] = (uint16_t)(b >> 16);
+      }
+    };
+    // A row m of tile i is row j = 16 i + m: part j / 9 of the narrow row (dz, dy) = j % 9. Its
+    // address when rows y - 1, y, y + 1 are in slots r, r + 1, r + 2 mod 3; rows past the last are
+    // not used and repeat the first
+    int arow[MT][3];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int j = 16 * i + m < ROWS ? 16 * i + m : 0;
+      const int part = j / 9, d = j % 9;
+      const int zi = FLIP ? 2 - d / 3 : d / 3, yi = FLIP ? 2 - d % 3 : d % 3;
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+        arow[i][r] = ((zi * 3 + (r + yi) % 3) * PARTS + part) * kNrPitch + 16 * g;
+    }
+    fetch_n(y0 - 1);
+    put_n(0);
+    fetch_n(y0);
+    put_n(1);
+    fetch_n(y0 + 1);
+    fetch_w(y0);
+    for (int y = y0; y < y1;) {
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        if (y >= y1) break;
+        put_n((r + 2) % 3);
+        *reinterpret_cast<u32x4*>(wr + lane * 16) = pw0;
+        if (lane < 4) *reinterpret_cast<u32x4*>(wr + (64 + lane) * 16) = pw1;
+        wave_sync();
+        if (y + 1 < y1) {
+          fetch_n(y + 2);
+          fetch_w(y + 1);
+        }
+        bf16x8 B[3];
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) B[dx] = read_channel(wr + (FLIP ? dx : 2 - dx) * 32, lane);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const bf16x8 A =
+              __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(nr + arow[i][r]));
+#pragma unroll
+          for (int dx = 0; dx < 3; ++dx)
+            acc[i][dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[dx], acc[i][dx], 0, 0, 0);
+        }
+        wave_sync();
+        ++y;
+      }
+    }
+  }
+  // sum over the block's waves and the parts, one shift at a time: part[wave][row][channel]
+  float* part = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int dx = 0; dx < 3; ++dx) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[((wave * MT + i) * 16 + 4 * g + r) * 16 + m] = acc[i][dx][r];
+    __syncthreads();
+    if (threadIdx.x < 9 * 16) {
+      const int d = threadIdx.x / 16, c = threadIdx.x % 16;
+      float v = 0.0f;
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q)
+#pragma unroll
+        for (int k = 0; k < kNrWaves; ++k) v += part[(k * MT * 16 + q * 9 + d) * 16 + c];
+      const int tap = 3 * d + dx;
+      sums[FLIP ? tap * 16 + c : c * 27 + tap] = v;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 27 * 16) unsafeAtomicAdd(a.dw + threadIdx.x, sums[threadIdx.x]);
+}
+
+template <bool FLIP>
+void launch_wgrad_narrow(const void* wide, const void* narrow, float* dw, int N, int D, int H,
+                         int W, hipStream_t s) {
+  WgNarrowArgs a;
+  a.wide = (const uint16_t*)wide;
+  a.narrow = narrow;
+  a.dw = dw;
+  a.D = D; a.H = H; a.W = W;
+  a.nseg = (W + kWgSeg - 1) / kWgSeg;
+  // about 4096 waves (a block of 16 per CU), at least sixteen rows each
+  const long long columns = (long long)N * D * a.nseg;
+  const int want = (int)std::min<long long>((H + 15) / 16, (4096 + columns - 1) / columns);
+  a.yc = (H + want - 1) / want;
+  a.nyc = (H + a.yc - 1) / a.yc;
+  a.units = columns * a.nyc;
+  conv_wgrad_narrow<FLIP>
+      <<<(unsigned)((a.units + kNrWaves - 1) / kNrWaves), 64 * kNrWaves, 0, s>>>(a);
 }
 
 // MFMA lane-layout probe: D = A B for one 16x16x32 BF16 and one 16x16x4 FP32 product, with
@@ -680,15 +907,13 @@ int fc_conv3d_fwd_dev(int device, const void* x, const void* w, const float* bia
   int rc = select_device(device);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long nvox = (long)N * D * H * W;
-  const int blocks = (int)((nvox + 255) / 256);
   int tok = prof_begin("conv3d_fwd", s);
   if (cin == 1 && cout == 16) {
-    if (relu) conv_fwd_cin1<16, true><<<blocks, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)w, bias, (uint16_t*)y, N, D, H, W);
-    else conv_fwd_cin1<16, false><<<blocks, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)w, bias, (uint16_t*)y, N, D, H, W);
+    if (relu) launch_one_to_16<false, true>(x, w, bias, y, N, D, H, W, s);
+    else launch_one_to_16<false, false>(x, w, bias, y, N, D, H, W, s);
   } else if (cout == 1 && cin == 16) {
     FC_CHECK_ARG(!relu, "the Cout = 1 layer has no activation and writes FP32");
-    conv_fwd_cout1<16><<<blocks, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)w, bias, (float*)y, N, D, H, W);
+    launch_16_to_one(x, w, bias, (float*)y, N, D, H, W, s);
   } else if (!launch_fwd(cin, cout, x, w, bias, y, N, D, H, W, relu, s)) {
     prof_end(tok, s);
     FC_CHECK_ARG(false, "unsupported channel pair %d -> %d", cin, cout);
@@ -708,11 +933,9 @@ int fc_conv3d_dgrad_dev(int device, const void* dy, const void* w, void* wt, voi
   int rc = select_device(device);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long nvox = (long)N * D * H * W;
-  const int blocks = (int)((nvox + 255) / 256);
   int tok = prof_begin("conv3d_dgrad", s);
   if (cout == 1 && cin == 16) {
-    conv_dgrad_cout1<16><<<blocks, 256, 0, s>>>((const float*)dy, (const uint16_t*)w, (uint16_t*)dx, N, D, H, W);
+    launch_one_to_16<true, false>(dy, w, nullptr, dx, N, D, H, W, s);
   } else {
     FC_CHECK_ARG(wt, "null weight workspace");
     const int total = cout * 27 * cin;
@@ -737,16 +960,11 @@ int fc_conv3d_wgrad_dev(int device, const void* x, const void* dy, float* dw, in
   int rc = select_device(device);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long nvox = (long)N * D * H * W;
   int tok = prof_begin("conv3d_wgrad", s);
   if (cin == 1 && cout == 16) {
-    const int chunk = 16384;
-    dim3 grid((unsigned)((nvox + chunk - 1) / chunk), 27);
-    conv_wgrad_cin1<16><<<grid, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)dy, dw, N, D, H, W, chunk);
+    launch_wgrad_narrow<false>(dy, x, dw, N, D, H, W, s);
   } else if (cout == 1 && cin == 16) {
-    const int chunk = 16384;
-    dim3 grid((unsigned)((nvox + chunk - 1) / chunk), 27);
-    conv_wgrad_cout1<16><<<grid, 256, 0, s>>>((const uint16_t*)x, (const float*)dy, dw, N, D, H, W, chunk);
+    launch_wgrad_narrow<true>(x, dy, dw, N, D, H, W, s);
   } else if (!launch_wgrad(cin, cout, x, dy, dw, N, D, H, W, s)) {
     prof_end(tok, s);
     FC_CHECK_ARG(false, "unsupported channel pair %d -> %d", cin, cout);

@@ -27,12 +27,16 @@ struct Store<FC_F16> {
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
 
-// FP32 -> BF16 with round-to-nearest-even; NaN stays NaN.
+// FP32 -> BF16 with round-to-nearest-even, NaN stays NaN (payload's high bits, quiet): one
+// v_cvt_pk_bf16_f32 for two values. Equal to the integer rounding u + 0x7fff + (u >> 16 & 1) for
+// all 2^32 inputs.
+typedef float fc_f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 fc_bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(fc_f32x2{a, b}, fc_bf16x2));
+}
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
 
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t b) {
@@ -103,6 +107,7 @@ __device__ __forceinline__ float hi16(uint32_t w) {
 
 template <int DT>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
+  if constexpr (DT == FC_BF16) return pack_bf16(a, b);
   return (uint32_t)to_bits16<DT>(a) | ((uint32_t)to_bits16<DT>(b) << 16);
 }
 

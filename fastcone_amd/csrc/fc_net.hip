@@ -22,12 +22,9 @@ namespace {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// The two channels of word q of a 16-byte unit as FP32, and back with one rounding each.
+// The two channels of word q of a 16-byte unit as FP32.
 __device__ __forceinline__ float lo_bf16(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float hi_bf16(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  return (uint32_t)f32_to_bf16_bits(a) | (uint32_t)f32_to_bf16_bits(b) << 16;
-}
 
 // Sum over the 2 x 2 x 2 voxels of a coarse voxel, FP32: units p + dz sz + dy sy + dx sx.
 __device__ __forceinline__ void sum8(const u32x4* p, size_t sx, size_t sy, size_t sz, float s[8]) {

@@ -328,3 +328,31 @@ def test_relu_gradient_kernel(gpu, voxels, c):
     _native.check(L.fc_net_relu_grad_dev(gpu.index, gd.data_ptr(), yd.data_ptr(), gm.data_ptr(),
                                          db.data_ptr(), voxels, c, st))
     assert bool(gm[0, 0].isnan()) and bool(db[0].isnan())
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 2, 16, 32), (2, 5, 17, 33), (1, 3, 35, 70)])
+def test_one_channel_layers(gpu, shape):
+    # z chunks, 32-voxel segments and 16-row chunks whole and with remainders. First layer: BF16
+    # output (one rounding, 2^-9 each side: rel. L2 < 2^-8); last layer: FP32 sums of 432 exact
+    # products (sqrt(432) 2^-24 = 1.2e-6, bound 1e-5), its BF16 input gradient < 2^-8; weight
+    # gradients, the last layer's from FP32 output gradients with all 24 bits, < 1e-5 as above
+    from fastcone_amd.unet import conv3d
+    g = torch.Generator().manual_seed(sum(shape))
+    for cin, cout in ((1, 16), (16, 1)):
+        x = torch.randn(shape + (cin,), generator=g).to(torch.bfloat16)
+        w = (torch.randn((cout, 27, cin), generator=g) / np.sqrt(27 * cin)).to(torch.bfloat16).float()
+        b = torch.randn(cout, generator=g)
+        gy = torch.randn(shape + (cout,), generator=g)
+        gy = gy.to(torch.bfloat16) if cout != 1 else gy
+        xg = x.to(gpu).requires_grad_(cin != 1)
+        wg = w.to(gpu).requires_grad_(True)
+        y = conv3d(xg, wg, b.to(gpu), False)
+        y.backward(gy.to(gpu))
+        xr = x.double().permute(0, 4, 1, 2, 3).requires_grad_(True)
+        wr = _torch_w(w).double().requires_grad_(True)
+        yr = torch.nn.functional.conv3d(xr, wr, b.double(), padding=1)
+        yr.backward(gy.double().permute(0, 4, 1, 2, 3))
+        assert rel(y.cpu(), yr.detach().permute(0, 2, 3, 4, 1)) < (1e-5 if cout == 1 else 2.0 ** -8)
+        assert rel(wg.grad.cpu(), wr.grad.permute(0, 2, 3, 4, 1).reshape(cout, 27, cin)) < 1e-5
+        if cin != 1:
+            assert rel(xg.grad.cpu(), xr.grad.permute(0, 2, 3, 4, 1)) < 2.0 ** -8
