@@ -946,47 +946,55 @@ struct AdjVArgs {
   int nbx, nby, nbz;
   int nsplit;          // view ranges per brick (grid z = nbz * nsplit)
   int max_steps;
+  int tiles_w, tiles_h;  // 16 x 16 pixel tiles of a view (adj_rays)
 };
 
 // One thread per ray (view, row, column): the ray's FP32 first sample, step and sample count
 // exactly as the projector computes them (ray_segment), and its datum y h norm, stored once so
 // that every brick the ray crosses reads 32 bytes instead of redoing the FP64 set-up; plus
-// max |y h norm| over the stack as the bits of a non-negative float (ordered like the value):
-// a block-wide maximum, then one integer atomic per block.
+// max |y h norm| over the stack as the bits of a non-negative float (ordered like the value): a
+// block-wide maximum, then one integer atomic per block that exceeds the maximum so far (an atomic
+// from every block serialises on its one address). Records lie column by column, [view][column][row],
+// as the bricks read them; a block takes a 16 x 16 pixel tile, so a wave reads eight row pieces of 32
+// bytes and writes eight column pieces of 256.
 template <int DT>
 __global__ __launch_bounds__(256) void adj_rays(AdjVArgs a) {
-  __shared__ float red[256];
-  const size_t per_view = (size_t)a.nw * a.nh;
-  const size_t total = per_view * (size_t)a.nviews;
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+  __shared__ float red[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int per_view = a.tiles_w * a.tiles_h;
+  const int t = (int)(blockIdx.x / (unsigned)per_view), tile = (int)blockIdx.x - t * per_view;
+  const int ty = tile / a.tiles_w, tx = tile - ty * a.tiles_w;
+  const int j = tx * kTile + (wave & 1) * 8 + (lane >> 3);
+  const int i = ty * kTile + (wave >> 1) * 8 + (lane & 7);
   float m = 0.0f;
-  if (idx < total) {
-    const int t = (int)(idx / per_view);
-    const int rem = (int)(idx - (size_t)t * per_view);
-    const int i = rem / a.nw, j = rem - i * a.nw;
-    const float y = load_elem<DT>(a.proj, idx) * (a.norm ? a.norm[t] : 1.0f) * (float)a.h;
+  if (j < a.nw && i < a.nh) {
+    const float y = load_elem<DT>(a.proj, ((size_t)t * a.nh + i) * a.nw + j) *
+                    (a.norm ? a.norm[t] : 1.0f) * (float)a.h;
     RaySeg r;
     r.nk = 0;
     r.px = r.py = r.pz = r.sx = r.sy = r.sz = 0.0f;
     if (y != 0.0f)
       r = ray_segment(a.views + (size_t)t * FC_VIEW_DOUBLES, j, i, a.ox, a.oy, a.oz, a.nx, a.ny,
                       a.nz, a.h, a.max_steps, 2.0f);
-    a.rays[2 * idx] = make_float4(r.px, r.py, r.pz, r.sx);
-    a.rays[2 * idx + 1] =
-        make_float4(r.sy, r.sz, __int_as_float(r.nk), r.nk > 0 && fabsf(y) <= 3.402823466e38f ? y : 0.0f);
+    float4* rec = a.rays + 2 * (((size_t)t * a.nw + j) * a.nh + i);
+    rec[0] = make_float4(r.px, r.py, r.pz, r.sx);
+    rec[1] = make_float4(r.sy, r.sz, __int_as_float(r.nk),
+                         r.nk > 0 && fabsf(y) <= 3.402823466e38f ? y : 0.0f);
     // a non-finite datum on a ray that reaches the block cannot be held by the fixed-point
     // accumulator: it is flagged (the whole output becomes NaN) and kept out of the maximum
     const bool bad = r.nk > 0 && !(fabsf(y) <= 3.402823466e38f);
     if (bad) atomicOr(a.ymax + 1, 1u);
     m = r.nk > 0 && !bad ? fabsf(y) : 0.0f;
   }
-  red[threadIdx.x] = m;
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  if (lane == 0) red[wave] = m;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t bits =
+        __float_as_uint(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    if (bits > __hip_atomic_load(a.ymax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(a.ymax, bits);
   }
-  if (threadIdx.x == 0) atomicMax(a.ymax, __float_as_uint(red[0]));
 }
 
 // One thread per (brick, view): the detector pixels whose rays can carry samples with a base cell
@@ -1061,36 +1069,39 @@ __global__ __launch_bounds__(kAT) void adjoint_vox_kernel(AdjVArgs a) {
   // base-cell range in the padded sample frame (voxel index + 2)
   const int lox = kAB * bx + 1, loy = kAB * by + 1, loz = kAB * bz + 1;
   const float flx = (float)lox, fly = (float)loy, flz = (float)loz;
+  const uint32_t cell0 = (uint32_t)((loz * kAL + loy) * kAL + lox);  // the accumulator's first cell
   const uint2* W = a.win + ((size_t)(bz * a.nby + by) * a.nbx + bx) * (size_t)a.nviews;
   int t = tbeg, start = 0;
   uint2 w = tbeg < tend ? W[tbeg] : make_uint2(0u, 0u);
-  // Items are dealt in chunks of kAT: wave pair (2 q, 2 q + 1) takes items 128 q .. 128 q + 127
-  // of each chunk, lane l of wave 2 q + b item 128 q + 2 l + b, so the 64 lanes of a wave hold
-  // rays 2 pixels apart: far enough apart that they rarely add to the same LDS word at once
-  // (same-address atomics serialise), close enough that their in-brick segments have similar
-  // lengths (the wave runs for its longest). Timed at 256^3 x 360 views x 384^2: 1 pixel apart
-  // 92.7 ms, 2 apart 78.7, 4 apart 86.3, 8 apart 89.0.
+  // A view's items run down the columns of its window, and are dealt in chunks of kAT: wave pair
+  // (2 q, 2 q + 1) takes items 128 q .. 128 q + 127 of each chunk, lane l of wave 2 q + b item
+  // 128 q + 2 l + b. Rays of one column cross the brick in nearly the same plane, so the lanes of a
+  // wave have in-brick segments of nearly the same length (the wave runs for its longest) and change
+  // cells at nearly the same samples; along rows the lengths vary from nothing to the brick's
+  // diagonal. Two rows apart they rarely add to the same LDS word at once (same-address atomics
+  // serialise). Timed at 256^3 x 360 views x 384^2, this kernel and its rays: along rows 2 apart 76.7
+  // ms, along columns 1, 2, 3 and 4 apart 88.3, 61.2, 72.0 and 69.3 ms (columns also 2 apart: 63.4).
   const int perm =
       ((threadIdx.x >> 7) << 7) | ((threadIdx.x & 63) << 1) | ((threadIdx.x >> 6) & 1);
   for (int g = perm;; g += kAT) {
-    int Wj = (int)(w.y & 0xffffu), npix = Wj * (int)(w.y >> 16);
+    int Wi = (int)(w.y >> 16), npix = Wi * (int)(w.y & 0xffffu);
     while (t < tend && g >= start + npix) {
       start += npix;
       if (++t < tend) {
         w = W[t];
-        Wj = (int)(w.y & 0xffffu);
-        npix = Wj * (int)(w.y >> 16);
+        Wi = (int)(w.y >> 16);
+        npix = Wi * (int)(w.y & 0xffffu);
       }
     }
     if (t >= tend) break;
     const int p = g - start;
-    // p / Wj from a 1-ulp reciprocal, exact for p < 2^21: (p + 0.5) / Wj lies at least 0.5 / Wj
-    // from an integer and the roundings move it by less than 2^-2 / Wj (integer division for
+    // p / Wi from a 1-ulp reciprocal, exact for p < 2^21: (p + 0.5) / Wi lies at least 0.5 / Wi
+    // from an integer and the roundings move it by less than 2^-2 / Wi (integer division for
     // larger windows)
-    const int pi = p < (1 << 21) ? (int)(((float)p + 0.5f) * __builtin_amdgcn_rcpf((float)Wj))
-                                 : p / Wj;
-    const int i = (int)(w.x >> 16) + pi, j = (int)(w.x & 0xffffu) + (p - pi * Wj);
-    const size_t ray = ((size_t)t * a.nh + i) * a.nw + j;
+    const int pj = p < (1 << 21) ? (int)(((float)p + 0.5f) * __builtin_amdgcn_rcpf((float)Wi))
+                                 : p / Wi;
+    const int j = (int)(w.x & 0xffffu) + pj, i = (int)(w.x >> 16) + (p - pj * Wi);
+    const size_t ray = ((size_t)t * a.nw + j) * a.nh + i;
     const float4 r1 = a.rays[2 * ray + 1];
     if (r1.w == 0.0f) continue;  // zero datum or a ray that misses the block
     const float4 r0 = a.rays[2 * ray];
@@ -1117,7 +1128,19 @@ __global__ __launch_bounds__(kAT) void adjoint_vox_kernel(AdjVArgs a) {
     clip(r.py, r.sy, fly);
     clip(r.pz, r.sz, flz);
     if (!(khi >= klo)) continue;
-    const int k0 = max(0, (int)ceilf(klo)), k1 = min(r.nk - 1, (int)floorf(khi));
+    // Every sample coordinate is monotone in k, so the samples of the brick are consecutive: drop
+    // those outside it at both ends, and the loop needs no test. The index counts in FP32 (exact:
+    // k < 2^24), the same values as (float)k.
+    float kf = fmaxf(ceilf(klo), 0.0f), kf1 = fminf(floorf(khi), (float)(r.nk - 1));
+    auto inside = [&](float k) {
+      const int cx = (int)fmaf(k, r.sx, r.px) - lox, cy = (int)fmaf(k, r.sy, r.py) - loy,
+                cz = (int)fmaf(k, r.sz, r.pz) - loz;
+      return (uint32_t)cx < (uint32_t)kAB && (uint32_t)cy < (uint32_t)kAB &&
+             (uint32_t)cz < (uint32_t)kAB;
+    };
+    while (kf <= kf1 && !inside(kf)) kf += 1.0f;
+    while (kf <= kf1 && !inside(kf1)) kf1 -= 1.0f;
+    if (!(kf <= kf1)) continue;
     // Consecutive samples (0.5 voxel apart) often share a base cell: their weights are summed in
     // registers and added to LDS when the cell changes. A sum must stay below 2^31 in the 2^28
     // fixed-point scale, so at most 7 samples. The step h along a unit direction advances the
@@ -1127,10 +1150,15 @@ __global__ __launch_bounds__(kAT) void adjoint_vox_kernel(AdjVArgs a) {
     float A[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) A[c] = 0.0f;
-    uint32_t cur = 0xffffffffu;
+    auto cell_of = [&](float qx, float qy, float qz) {
+      return mad_u24(mad_u24((uint32_t)(int)qz, (uint32_t)kAL, (uint32_t)(int)qy), (uint32_t)kAL,
+                     (uint32_t)(int)qx);
+    };
+    uint32_t cur = cell_of(fmaf(kf, r.sx, r.px), fmaf(kf, r.sy, r.py), fmaf(kf, r.sz, r.pz));
     int run = 0;
     auto flush = [&]() {
-      unsigned long long* L = acc + cur;
+      unsigned long long* L = reinterpret_cast<unsigned long long*>(
+          reinterpret_cast<char*>(acc) + ((cur << 3) - (cell0 << 3)));
       // round to the nearest integer, sign-extend, add in 64-bit two's complement
       auto add = [](unsigned long long* p, float v) {
         atomicAdd(p, (unsigned long long)(long long)__float2int_rn(v));
@@ -1139,33 +1167,28 @@ __global__ __launch_bounds__(kAT) void adjoint_vox_kernel(AdjVArgs a) {
       add(L + kAL * kAL, A[4]); add(L + kAL * kAL + 1, A[5]);
       add(L + kAL * kAL + kAL, A[6]); add(L + kAL * kAL + kAL + 1, A[7]);
     };
-    // the sample index counts in FP32 (exact: k < 2^24), the same values as (float)k, so one add
-    // and one compare per sample control the loop
-    const float kf1 = (float)k1;
-    for (float kf = (float)k0; kf <= kf1; kf += 1.0f) {
+    for (; kf <= kf1; kf += 1.0f) {
       const float qx = fmaf(kf, r.sx, r.px), qy = fmaf(kf, r.sy, r.py), qz = fmaf(kf, r.sz, r.pz);
-      const uint32_t cx = (uint32_t)((int)qx - lox), cy = (uint32_t)((int)qy - loy),
-                     cz = (uint32_t)((int)qz - loz);
-      if (cx >= (uint32_t)kAB || cy >= (uint32_t)kAB || cz >= (uint32_t)kAB) continue;
-      const float ax = __builtin_amdgcn_fractf(qx), ay = __builtin_amdgcn_fractf(qy),
-                  az = __builtin_amdgcn_fractf(qz);
-      const uint32_t cell = (cz * kAL + cy) * kAL + cx;
-      const float wz1 = y * az, wz0 = y - wz1;
-      const float w10 = wz0 * ay, w00 = wz0 - w10, w11 = wz1 * ay, w01 = wz1 - w11;
-      const float w[8] = {w00 - w00 * ax, w00 * ax, w10 - w10 * ax, w10 * ax,
-                          w01 - w01 * ax, w01 * ax, w11 - w11 * ax, w11 * ax};
+      const uint32_t cell = cell_of(qx, qy, qz);
       if (cell != cur || (CAPRUN && run == kRun)) {
-        if (cur != 0xffffffffu) flush();
+        flush();
         cur = cell;
-        if constexpr (CAPRUN) run = 0;
 #pragma unroll
         for (int c = 0; c < 8; ++c) A[c] = 0.0f;
+        if constexpr (CAPRUN) run = 0;
       }
       if constexpr (CAPRUN) ++run;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) A[c] += w[c];
+      const float ax = __builtin_amdgcn_fractf(qx), ay = __builtin_amdgcn_fractf(qy),
+                  az = __builtin_amdgcn_fractf(qz);
+      const float bx = 1.0f - ax;
+      const float wz1 = y * az, wz0 = y - wz1;
+      const float w10 = wz0 * ay, w00 = wz0 - w10, w11 = wz1 * ay, w01 = wz1 - w11;
+      A[0] = fmaf(bx, w00, A[0]); A[1] = fmaf(ax, w00, A[1]);
+      A[2] = fmaf(bx, w10, A[2]); A[3] = fmaf(ax, w10, A[3]);
+      A[4] = fmaf(bx, w01, A[4]); A[5] = fmaf(ax, w01, A[5]);
+      A[6] = fmaf(bx, w11, A[6]); A[7] = fmaf(ax, w11, A[7]);
     }
-    if (cur != 0xffffffffu) flush();
+    flush();
   }
   __syncthreads();
   // LDS element (ex, ey, ez) is voxel (16 b - 1 + e) of the block; voxels outside [0, n) are the
@@ -1585,7 +1608,9 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
   a.ymax = reinterpret_cast<unsigned int*>(static_cast<char*>(ws) + moff);
   int tok = prof_begin("adjoint", stream);
   zero_fill<unsigned int><<<1, 256, 0, stream>>>(a.ymax, 2);  // max |y| bits, non-finite flag
-  const unsigned rblocks = (unsigned)((nrays + 255) / 256);
+  a.tiles_w = (a.nw + kTile - 1) / kTile;
+  a.tiles_h = (a.nh + kTile - 1) / kTile;
+  const unsigned rblocks = (unsigned)((long long)a.tiles_w * a.tiles_h * a.nviews);
   if (dt == FC_F32) adj_rays<FC_F32><<<rblocks, 256, 0, stream>>>(a);
   else if (dt == FC_BF16) adj_rays<FC_BF16><<<rblocks, 256, 0, stream>>>(a);
   else adj_rays<FC_F16><<<rblocks, 256, 0, stream>>>(a);
