@@ -15,23 +15,31 @@
 // 16 x 16 x 16 voxel cube. Per view the block stages, in LDS, the detector window that the cube
 // projects onto (rows of the raw projection, zero outside the detector), double-buffered: while
 // the block accumulates view t from one buffer, the rows of view t+1 are already in flight (FP32
-// storage: copied straight into the other buffer; 16-bit storage: into registers, written to the
-// other buffer at the top of the next iteration), so one barrier per view suffices and the load
-// latency hides behind the arithmetic. Per view and column the
-// projective terms are evaluated once in FP64; when the detector columns do not depend on z
-// (untilted detectors) each voxel then costs one FMA for its row, a clamp and a bilinear
-// interpolation from LDS (two ds_read2 pairs).
+// storage: copied straight into the other buffer, 16 bytes per lane; 16-bit storage: into registers,
+// converted and written to the other buffer at the top of the next iteration), so one barrier per
+// view suffices and the load latency hides behind the arithmetic. Per view and column the projective
+// terms are a few FMAs on the view's table entry (below); when the detector columns do not depend on
+// z (untilted detectors) each voxel then costs one FMA for its row and a bilinear interpolation from
+// LDS (two ds_read2 pairs, one multiply-add for the address).
 //
-// The windows come from a pre-pass (bp_windows, one thread per block and view): the projective
-// image of a box lies in the box of its eight corners' images, so the corners' FP64 (u, v) widened
-// by a pixel each side bound every tap. A view whose window does not fit the LDS tile is gathered
-// from global memory with explicit bounds (rare: very short source distances); a view that misses
-// the detector entirely is skipped.
+// View table: every kTab views the block computes, one thread per view and in FP64, the window of its
+// cube — the projective image of a box lies in the box of its eight corners' images, so the corners'
+// (u, v) widened by a pixel each side bound every tap — and the view's projective forms relative to
+// the window's and the cube's corner, A' = A - u0 C, B' = B - v0 C and C as linear functions of the
+// offset in the cube. There they are small (|A'| < 64 |C|), so rounding them to FP32 moves a tile
+// coordinate by about 4e-6 pixel, less than the FP32 rounding of an absolute coordinate. A view whose
+// window does not fit the LDS tile is gathered from global memory with explicit bounds (rare: very
+// short source distances); a view that misses the detector entirely is skipped.
+//
+// Small volumes leave compute units idle or the last round of blocks nearly empty: the views are
+// then split over several blocks per cube, whose sums go to partial volumes that bp_reduce adds in
+// order (launch_backproject).
 //
 // "Quad" staging (stage_quads: the four bilinear corners of every base pixel stored together) is
 // kept for the Katsevich backprojector's filtered data.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -70,81 +78,100 @@ __global__ __launch_bounds__(256) void stage_quads(const void* __restrict__ proj
   }
 }
 
-constexpr int kTileW = 64;                 // widest staged window (one pixel per lane)
-constexpr int kPre = 12;                   // rows per wave and view: window height <= 4 kPre
+constexpr int kTileW = 64;                 // widest staged window
+constexpr int kTileH = 48;                 // tallest staged window
 // Row pitch of a staged window (floats): fixed, so a bilinear sample's two row pairs are one
 // base address with immediate offsets {0, 1, kTileP, kTileP + 1}. 76 = 12 mod 32 banks: timed at
 // 512^3 x 720 against pitches 65-80, it leaves the fewest bank conflicts between the lanes' rows
-// (65: 51.5 ms, 68: 49.9, 70: 48.6, 72: 48.2, 74-78: 47.7, 80: 48.0).
+// (65: 51.5 ms, 68: 49.9, 70: 48.6, 72: 48.2, 74-78: 47.7, 80: 48.0). It is also 19 units of 16
+// bytes, the load-to-LDS copy's unit per lane.
 constexpr uint32_t kTileP = 76;
-constexpr int kTileCap = kTileP * 4 * kPre;  // floats per LDS buffer (14.3 KiB)
+constexpr uint32_t kUnits = kTileP / 4;    // 16-byte units per row
+constexpr int kTileCap = kTileP * kTileH;  // floats per LDS buffer (14.3 KiB)
+constexpr int kRowsW = 64 / (int)kUnits;   // rows per wave and copy instruction (57 lanes)
+constexpr int kRowsB = 4 * kRowsW;         // and per block
+constexpr int kCopies = kTileH / kRowsB;   // copies per thread of the tallest window
+static_assert(kTileH % kRowsB == 0, "whole copies");
 constexpr uint32_t kWinSkip = 0u;          // window word y: the cube misses the detector
 constexpr uint32_t kWinGlobal = 0xffffu;   // window word y low half: gather from global memory
+constexpr int kTab = 48;                   // views per table: five blocks fit a CU's LDS
 
 struct BpArgs {
-  float* vol;
+  float* vol;          // accumulated; with nsplit > 1 the partial volumes, one per split, stored
   const void* proj;    // [nviews][nh][nw] in the storage dtype
   const float* norm;   // per-view scale or null
   const double* views;
-  const uint2* win;    // per (block, view): x = u0 | v0 << 16 (int16 each), y = Wu | Wv << 16
   double ox, oy, oz;
   int nx, ny, nz;
   int nw, nh, nviews;
-  int nbx, nby;
+  int nbz, nsplit;
 };
 
-struct WinArgs {
-  const double* views;
-  uint2* win;
-  double ox, oy, oz;
-  int nx, ny, nz;
-  int nw, nh, nviews;
-  int nbx, nby, nbz;
+// One view for one cube: with (dx, dy, dz) a voxel's offset from the cube's first voxel,
+// A' = a0 + a1 dx + a2 dy + a3 dz, likewise B' and C; u - u0 = A' / C, v - v0 = B' / C.
+struct ViewEntry {
+  float a[4], b[4], c[4];
+  float s;       // norm
+  uint32_t org;  // window origin u0 | v0 << 16 (int16 each)
+  uint32_t size; // Wu | Wv << 16, or kWinSkip / kWinGlobal
+  uint32_t tilted;  // a3 or c3 nonzero
 };
 
-// One thread per (block, view): the detector window of the block's voxel cube. Window pixels
-// [u0, u0 + Wu) x [v0, v0 + Wv) with u0 = floor(min u) - 1 and Wu = floor(max u) - u0 + 3, so every
-// tap (iu, iu + 1) of a voxel in the cube lies at least one pixel inside; likewise v.
-__global__ __launch_bounds__(256) void bp_windows(WinArgs a) {
-  const size_t total = (size_t)a.nbx * a.nby * a.nbz * a.nviews;
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
-  const int t = (int)(idx % (size_t)a.nviews);
-  const size_t b = idx / (size_t)a.nviews;
-  const int bx = (int)(b % a.nbx), by = (int)((b / a.nbx) % a.nby), bz = (int)(b / ((size_t)a.nbx * a.nby));
-  const double xs[2] = {bx * kBXY + a.ox, min(bx * kBXY + kBXY - 1, a.nx - 1) + a.ox};
-  const double ys[2] = {by * kBXY + a.oy, min(by * kBXY + kBXY - 1, a.ny - 1) + a.oy};
-  const double zs[2] = {bz * kZR + a.oz, min(bz * kZR + kZR - 1, a.nz - 1) + a.oz};
+// Window pixels [u0, u0 + Wu) x [v0, v0 + Wv) with u0 = floor(min u) - 1 and Wu = floor(max u) - u0
+// + 3, so every tap (iu, iu + 1) of a voxel in the cube lies at least one pixel inside; likewise v.
+__device__ __forceinline__ ViewEntry view_entry(const BpArgs& a, int t, int x0, int y0, int z0) {
   const double* M = a.views + (size_t)t * FC_VIEW_DOUBLES + 12;
+  const double X0 = x0 + a.ox, Y0 = y0 + a.oy, Z0 = z0 + a.oz;
+  const double ex = min(kBXY - 1, a.nx - 1 - x0), ey = min(kBXY - 1, a.ny - 1 - y0),
+               ez = min(kZR - 1, a.nz - 1 - z0);
+  const double A0 = M[0] * X0 + M[1] * Y0 + M[2] * Z0 + M[3];
+  const double B0 = M[4] * X0 + M[5] * Y0 + M[6] * Z0 + M[7];
+  const double C0 = M[8] * X0 + M[9] * Y0 + M[10] * Z0 + M[11];
   double umin = 1e300, umax = -1e300, vmin = 1e300, vmax = -1e300;
   bool ok = true;
-#pragma unroll
+  // the matrix is reread per corner: held in registers, it would spill the block's accumulators
+#pragma unroll 1
   for (int c = 0; c < 8; ++c) {
-    const double X = xs[c & 1], Y = ys[(c >> 1) & 1], Z = zs[c >> 2];
-    const double C = M[8] * X + M[9] * Y + M[10] * Z + M[11];
+    asm volatile("" : "+v"(M));
+    const double dx = c & 1 ? ex : 0.0, dy = c & 2 ? ey : 0.0, dz = c & 4 ? ez : 0.0;
+    const double C = C0 + M[8] * dx + M[9] * dy + M[10] * dz;
     ok = ok && C > 0.0;
-    const double u = (M[0] * X + M[1] * Y + M[2] * Z + M[3]) / C;
-    const double v = (M[4] * X + M[5] * Y + M[6] * Z + M[7]) / C;
+    const double rc = 1.0 / C;
+    const double u = (A0 + M[0] * dx + M[1] * dy + M[2] * dz) * rc;
+    const double v = (B0 + M[4] * dx + M[5] * dy + M[6] * dz) * rc;
     umin = fmin(umin, u); umax = fmax(umax, u);
     vmin = fmin(vmin, v); vmax = fmax(vmax, v);
   }
-  uint2 w;
-  w.x = 0u;
-  w.y = kWinGlobal;
+  ViewEntry e;
+  e.s = a.norm ? a.norm[t] : 1.0f;
+  e.org = 0u;
+  e.size = kWinGlobal;
+  e.tilted = M[2] != 0.0 || M[10] != 0.0;
+  int u0 = 0, v0 = 0;
   if (ok && umin > -1e6 && umax < 1e6 && vmin > -1e6 && vmax < 1e6) {
     if (umax <= -1.0 || umin >= (double)a.nw || vmax <= -1.0 || vmin >= (double)a.nh) {
-      w.y = kWinSkip;  // zero-extended data: every sample of the cube is 0
+      e.size = kWinSkip;  // zero-extended data: every sample of the cube is 0
     } else {
-      const int u0 = (int)floor(umin) - 1, v0 = (int)floor(vmin) - 1;
+      u0 = (int)floor(umin) - 1;
+      v0 = (int)floor(vmin) - 1;
       const int Wu = (int)floor(umax) - u0 + 3, Wv = (int)floor(vmax) - v0 + 3;
-      if (Wu <= kTileW && Wv <= 4 * kPre && u0 >= -32768 && u0 <= 32767 && v0 >= -32768 &&
+      if (Wu <= kTileW && Wv <= kTileH && u0 >= -32768 && u0 <= 32767 && v0 >= -32768 &&
           v0 <= 32767) {
-        w.x = ((uint32_t)u0 & 0xffffu) | ((uint32_t)v0 << 16);
-        w.y = (uint32_t)Wu | ((uint32_t)Wv << 16);
+        e.org = ((uint32_t)u0 & 0xffffu) | ((uint32_t)v0 << 16);
+        e.size = (uint32_t)Wu | ((uint32_t)Wv << 16);
       }
     }
   }
-  a.win[idx] = w;
+  e.a[0] = (float)(A0 - u0 * C0);
+  e.b[0] = (float)(B0 - v0 * C0);
+  e.c[0] = (float)C0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    e.a[1 + k] = (float)(M[k] - u0 * M[8 + k]);
+    e.b[1 + k] = (float)(M[4 + k] - v0 * M[8 + k]);
+    e.c[1 + k] = (float)M[8 + k];
+  }
+  return e;
 }
 
 // Zero-extended bilinear sample of one view straight from global memory (window fallback).
@@ -165,269 +192,344 @@ __device__ __forceinline__ float bilinear_global(const void* proj, size_t vbase,
   return lerp(lerp(p[0], p[1], au), lerp(p[2], p[3], au), av);
 }
 
-// Clamp to [lo, hi]; NaN maps to lo (fmaxf returns the non-NaN operand).
+// Clamp to [lo, hi], one instruction; NaN maps to lo (the median of a NaN and two numbers is the
+// smaller number).
 __device__ __forceinline__ float clampf(float v, float lo, float hi) {
-  return fminf(fmaxf(v, lo), hi);
+  return __builtin_amdgcn_fmed3f(v, lo, hi);
 }
 
-// Bilinear sample at tile coordinates (u, v) >= 0 of an LDS window (row pitch kTileP).
-__device__ __forceinline__ float tile_bilinear(const float* T, uint32_t iu, float au, float v) {
-  const uint32_t iv = (uint32_t)(int)v;
+// LDS byte address of a pointer into a __shared__ array.
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(size_t)p; }
+
+// Bilinear sample of an LDS window (row pitch kTileP) at row coordinate v >= 0 and fraction au of
+// the column at LDS byte address `col` (row 0).
+__device__ __forceinline__ float tile_bilinear(uint32_t col, float au, float v) {
+  typedef __attribute__((address_space(3))) const float* lds_p;
   const float av = __builtin_amdgcn_fractf(v);
-  const float* p = T + mad_u24(iv, kTileP, iu);
+  const lds_p p = (lds_p)mad_u24((uint32_t)(int)v, 4u * kTileP, col);
   return lerp(lerp(p[0], p[1], au), lerp(p[kTileP], p[kTileP + 1], au), av);
 }
 
-// One dword per active lane from global memory at row + lane_bytes (row wave-uniform, in scalar
-// registers: the scalar-base form of the instruction, so a row costs no vector arithmetic) into
-// LDS at lds_dst + 4 lane (lds_dst wave-uniform), by the load-to-LDS path: no registers hold the
-// data and no LDS write instruction is issued. Written as assembly rather than the compiler
-// builtin, with which the compiler waits for every outstanding load-to-LDS before each later LDS
-// read (it cannot tell that the reads address the other window buffer). The instruction has no
-// register outputs, its address registers are read at issue, and the LDS it writes is read only
-// after the explicit s_waitcnt and the barrier of the next view. Loads complete in order, so the
-// compiler's own vmcnt waits stay conservative with these loads outstanding.
-// M0 is declared clobbered; the compiler reports that it reserves M0, and it uses M0 nowhere
-// else in this kernel.
+// acc[k] += wt times the bilinear sample at row vb + k dv of the column at LDS byte address `col`;
+// rows clamped to [0, vmax] if CLAMP. Two samples' reads are issued before the previous two are
+// used.
+template <bool CLAMP>
+__device__ __forceinline__ void column_samples(float* acc, uint32_t col, float au, float vb,
+                                               float dv, float wt, float vmax) {
+  typedef __attribute__((address_space(3))) const float* lds_p;
+  constexpr int kG = 2;
+  float p[2][kG][4], av[2][kG];
+  auto read = [&](int g) {
+#pragma unroll
+    for (int q = 0; q < kG; ++q) {
+      float v = fmaf((float)(g * kG + q), dv, vb);
+      if (CLAMP) v = clampf(v, 0.0f, vmax);
+      av[g & 1][q] = __builtin_amdgcn_fractf(v);
+      const lds_p a = (lds_p)mad_u24((uint32_t)(int)v, 4u * kTileP, col);
+      p[g & 1][q][0] = a[0];
+      p[g & 1][q][1] = a[1];
+      p[g & 1][q][2] = a[kTileP];
+      p[g & 1][q][3] = a[kTileP + 1];
+    }
+  };
+  read(0);
+#pragma unroll
+  for (int g = 0; g < kZR / kG; ++g) {
+    if (g + 1 < kZR / kG) read(g + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < kG; ++q) {
+      const float* r = p[g & 1][q];
+      acc[g * kG + q] = fmaf(wt, lerp(lerp(r[0], r[1], au), lerp(r[2], r[3], au), av[g & 1][q]),
+                             acc[g * kG + q]);
+    }
+  }
+}
+
+// 16 bytes (or one dword) per active lane from global memory at base + lane_bytes (base
+// wave-uniform, in scalar registers: the scalar-base form of the instruction, so a copy costs no
+// vector address arithmetic) into LDS at lds_dst + 16 lane (+ 4 lane; lds_dst wave-uniform), by the
+// load-to-LDS path: no registers hold the data and no LDS write instruction is issued. Written as
+// assembly rather than the compiler builtin, with which the compiler waits for every outstanding
+// load-to-LDS before each later LDS read (it cannot tell that the reads address the other window
+// buffer). The instruction has no register outputs, its address registers are read at issue, and
+// the LDS it writes is read only after the explicit s_waitcnt and the barrier of the next view.
+// Loads complete in order, so the compiler's own vmcnt waits stay conservative with these loads
+// outstanding. M0 is declared clobbered; the compiler reports that it reserves M0, and it uses M0
+// nowhere else in this kernel.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void copy_dword_to_lds(const float* row, uint32_t lane_bytes,
-                                                  float* lds_dst) {
-  const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)lds_dst);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(m0), "v"(lane_bytes),
-               "s"(row)
+__device__ __forceinline__ void copy_units_to_lds(const void* base, uint32_t lane_bytes,
+                                                  uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
+                   __builtin_amdgcn_readfirstlane(lds_dst)),
+               "v"(lane_bytes), "s"(base)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void copy_dword_to_lds(const void* base, uint32_t lane_bytes,
+                                                  uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(
+                   __builtin_amdgcn_readfirstlane(lds_dst)),
+               "v"(lane_bytes), "s"(base)
                : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
-// The per-view words every lane of a block needs (the view's 3 x 4 matrix, the next view's
-// window word and the view's weight), by scalar loads waited for in the same statement. With
-// the copies above in the loop the compiler cannot prove these words unchanged and reads them
-// with vector loads; vector loads count down in issue order, so waiting for one issued after
-// the next view's copies would also wait for every copy, and the view would not overlap them.
-typedef unsigned int fc_u32x8 __attribute__((ext_vector_type(8)));
-typedef unsigned int fc_u32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ void load_view_words(const double* M, const uint2* Wn, const float* S,
-                                                double m[12], uint2& wn, float& s) {
-  fc_u32x16 lo;
-  fc_u32x8 hi;
-  unsigned long long w;
-  unsigned int sv;
-  asm volatile(
-      "s_load_dwordx16 %0, %4, 0x0\n\t"
-      "s_load_dwordx8 %1, %4, 0x40\n\t"
-      "s_load_dwordx2 %2, %5, 0x0\n\t"
-      "s_load_dword %3, %6, 0x0\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&s"(lo), "=&s"(hi), "=&s"(w), "=&s"(sv)
-      : "s"(M), "s"(Wn), "s"(S)
-      : "memory");
+// The same for a tilted detector: column, row and weight by voxel, from the view's forms at the
+// column's first voxel.
+template <int MODE, bool CLAMP>
+__device__ __forceinline__ void tilted_samples(float* acc, uint32_t T0, float A, float B, float C,
+                                               const ViewEntry& E, float umax, float vmax) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) m[i] = __hiloint2double((int)lo[2 * i + 1], (int)lo[2 * i]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) m[8 + i] = __hiloint2double((int)hi[2 * i + 1], (int)hi[2 * i]);
-  wn = make_uint2((unsigned)w, (unsigned)(w >> 32));
-  s = __uint_as_float(sv);
+  for (int k = 0; k < kZR; ++k) {
+    if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four samples at a time in registers
+    const float kf = (float)k;
+    const float rc = __builtin_amdgcn_rcpf(fmaf(kf, E.c[3], C));  // 1 ulp, as the positions
+    float u = fmaf(kf, E.a[3], A) * rc, v = fmaf(kf, E.b[3], B) * rc;
+    if (CLAMP) u = clampf(u, 0.0f, umax), v = clampf(v, 0.0f, vmax);
+    float wt = E.s;
+    if constexpr (MODE == FC_BP_FDK) wt = E.s * rc * rc;
+    if constexpr (MODE == FC_BP_KATSEVICH) wt = E.s * rc;
+    acc[k] = fmaf(wt, tile_bilinear(T0 + 4u * (uint32_t)(int)u, __builtin_amdgcn_fractf(u), v), acc[k]);
+  }
 }
 
+typedef uint32_t fc_u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+// Bound by VALU issue (0.95-1.0 instructions per CU clock, 15.8 -> 13.4 per voxel-view at 512^3 x 720)
+// with the LDS busy 64 % of the time; five blocks per CU for FP32 storage (96 registers), four for
+// 16-bit storage, whose staging registers would spill at five. Against per-view FP64 terms by column
+// and dword copies row by row: 512^3 x 720 FP32 39.2 -> 37.0 ms, 256^3 x 360 BF16 3.3 -> 3.1 ms,
+// 150 x 333 x 290 x 275 tilted FP16 2.84 -> 2.75 ms. Keeping two samples' reads ahead (column_samples)
+// is part of that: with four ahead the registers allow only four blocks (38.0 ms).
 template <int DT, int MODE>
-__global__ __launch_bounds__(256) void bp_kernel(BpArgs a) {
-  __shared__ float tile[2][kTileCap];
+__global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a) {
+  __shared__ __align__(16) float tile[2][kTileCap];
+  __shared__ __align__(16) ViewEntry tab[kTab + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int x = blockIdx.x * kBXY + (wave & 1) * 8 + (lane & 7);
-  const int y = blockIdx.y * kBXY + (wave >> 1) * 8 + (lane >> 3);
-  const int z0 = blockIdx.z * kZR;
-  const double X = (double)x + a.ox, Y = (double)y + a.oy, Z0 = (double)z0 + a.oz;
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int ix = (wave & 1) * 8 + (lane & 7), iy = (wave >> 1) * 8 + (lane >> 3);
+  const int bx0 = blockIdx.x * kBXY, by0 = blockIdx.y * kBXY;
+  const int split = blockIdx.z / a.nbz, z0 = (int)(blockIdx.z - split * a.nbz) * kZR;
+  const int x = bx0 + ix, y = by0 + iy;
+  const float dx = (float)ix, dy = (float)iy;
+  const int tbeg = (int)((long long)a.nviews * split / a.nsplit);
+  const int tend = (int)((long long)a.nviews * (split + 1) / a.nsplit);
   // the whole 16 x 16 x 16 cube lies in the volume (no clamping of tile coordinates needed)
-  const bool inner = (int)(blockIdx.x + 1) * kBXY <= a.nx &&
-                     (int)(blockIdx.y + 1) * kBXY <= a.ny && z0 + kZR <= a.nz;
-  const uint2* W = a.win + ((size_t)(blockIdx.z * a.nby + blockIdx.y) * a.nbx + blockIdx.x) *
-                               (size_t)a.nviews;
+  const bool inner = bx0 + kBXY <= a.nx && by0 + kBXY <= a.ny && z0 + kZR <= a.nz;
   float acc[kZR];
 #pragma unroll
   for (int k = 0; k < kZR; ++k) acc[k] = 0.0f;
 
-  // Rows of a view's window, staged as (row wave + 4 q, column lane); zero outside the detector.
-  // 16-bit storage: registers hold the raw storage bits (converting at commit keeps the loads in
-  // flight); FP32 storage copies straight into LDS (issue_lds below). The row phase is
-  // wave-uniform, so row checks are scalar branches and addresses advance by a scalar stride.
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
-  uint32_t pre[kPre];
-  auto issue = [&](int t, uint2 w) {
-    const uint32_t Wu = w.y & 0xffffu, Wv = w.y >> 16;
-    if (Wu == kWinSkip || Wu == kWinGlobal) return;
-    const int u0 = (int)(int16_t)(w.x & 0xffffu), v0 = (int)(int16_t)(w.x >> 16);
-    const int pu = u0 + lane;
-    const bool colok = (uint32_t)lane < Wu && pu >= 0 && pu < a.nw;
-    const int pv0 = v0 + wv;
-    const long long row0 = ((long long)t * a.nh + pv0) * a.nw;  // element index of (pv0, 0)
-    // row wv + 4 q is in the window when 4 q < rows: compared with an immediate, so no register
-    // holds a per-row constant across the view loop
-    const int rows = (int)Wv - wv;
-#pragma unroll
-    for (int q = 0; q < kPre; ++q) {
-      pre[q] = 0u;  // +0 in every storage format
-      if (4 * q < rows && (uint32_t)(pv0 + 4 * q) < (uint32_t)a.nh && colok)
-        pre[q] = load_bits<DT>(a.proj, (size_t)(row0 + (long long)(4 * q) * a.nw + pu));
-    }
+  // A window is copied in units of four pixels, kUnits per row: lane l of a wave takes unit l mod
+  // kUnits of row kRowsW wave + l / kUnits + kRowsB i, so a wave's units are consecutive in LDS.
+  // Units past the window's last column (rounded up) are left out; they are never read.
+  constexpr uint32_t kSize = DT == FC_F32 ? 4u : 2u;  // bytes per pixel
+  const uint32_t lrow = (uint32_t)lane / kUnits;
+  const uint32_t col = lane < kRowsW * (int)kUnits ? 4u * ((uint32_t)lane - lrow * kUnits) : 0xffffu;
+  const uint32_t off = (lrow * (uint32_t)a.nw + col) * kSize;
+  // whole units of the window lie on the detector
+  auto whole = [&](int u0, int v0, uint32_t Wu, uint32_t Wv) {
+    return u0 >= 0 && u0 + (int)((Wu + 3u) & ~3u) <= a.nw && v0 >= 0 && v0 + (int)Wv <= a.nh;
   };
-  auto commit = [&](float* T, uint2 w) {
-    const uint32_t Wu = w.y & 0xffffu, Wv = w.y >> 16;
+  // FP32 storage: global memory -> LDS buffer
+  auto issue_lds = [&](int t, uint32_t org, uint32_t size, uint32_t buf) {
+    const uint32_t Wu = size & 0xffffu, Wv = size >> 16;
     if (Wu == kWinSkip || Wu == kWinGlobal) return;
-    float* Tw = T + (uint32_t)wv * kTileP + (uint32_t)lane;
-    const int rows = (int)Wv - wv;
+    const int u0 = (int)(int16_t)(org & 0xffffu), v0 = (int)(int16_t)(org >> 16);
+    // the window's first pixel (it may lie before the detector, but only pixels on it are loaded)
+    const float* win = static_cast<const float*>(a.proj) + ((long long)t * a.nh + v0) * a.nw + u0;
+    if (whole(u0, v0, Wu, Wv)) {
+      const int rows = (int)Wv - kRowsW * wv;  // of this wave's copies
+      if (col < Wu) {
 #pragma unroll
-    for (int q = 0; q < kPre; ++q) {
-      if (4 * q < rows && (uint32_t)lane < Wu)
-        Tw[4u * kTileP * (uint32_t)q] = bits_to_f32<DT>(pre[q]);
+        for (int i = 0; i < kCopies; ++i)
+          if (kRowsB * i < rows && (int)lrow < rows - kRowsB * i)
+            copy_units_to_lds(win + (long long)(kRowsW * wv + kRowsB * i) * a.nw, off,
+                              buf + 4u * kTileP * (uint32_t)(kRowsW * wv + kRowsB * i));
+      }
+      return;
     }
-  };
-
-  // FP32 storage: the window rows go straight from global memory into the LDS buffer (rows of
-  // lanes < Wu; pixels outside the detector are stored as zero), with no staging registers.
-  auto issue_lds = [&](int t, uint2 w, float* Tn) {
-    const uint32_t Wu = w.y & 0xffffu, Wv = w.y >> 16;
-    if (Wu == kWinSkip || Wu == kWinGlobal) return;
-    const int u0 = (int)(int16_t)(w.x & 0xffffu), v0 = (int)(int16_t)(w.x >> 16);
+    // a window over the detector's edge, row by row: row wv + 4 q, column = lane; pixels outside the
+    // detector are stored as zero by the lanes themselves
     const int pu = u0 + lane;
     const bool colok = pu >= 0 && pu < a.nw;
-    const int pv0 = v0 + wv;
-    // the window row's first pixel (wave-uniform; it may lie before the detector row, but only
-    // lanes with a pixel on the detector load) and each lane's byte offset from it
-    const float* row0 = static_cast<const float*>(a.proj) + ((long long)t * a.nh + pv0) * a.nw + u0;
-    const uint32_t lane_bytes = 4u * (uint32_t)lane;
-    // row wv + 4 q is in the window when 4 q < rows: compared with an immediate, so no register
-    // holds a per-row constant across the view loop
-    const int rows = (int)Wv - wv;
-    float* Tw = Tn + (uint32_t)wv * kTileP;
     if ((uint32_t)lane < Wu) {
-#pragma unroll
-      for (int q = 0; q < kPre; ++q) {
-        if (4 * q < rows) {
-          // pixels outside the detector are written as zero by the lanes themselves
-          float* dst = Tw + 4u * kTileP * (uint32_t)q;
-          if (colok && (uint32_t)(pv0 + 4 * q) < (uint32_t)a.nh)
-            copy_dword_to_lds(row0 + (long long)(4 * q) * a.nw, lane_bytes, dst);
-          else
-            dst[lane] = 0.0f;
+      for (uint32_t r = (uint32_t)wv; r < Wv; r += 4u) {
+        const uint32_t dst = buf + 4u * kTileP * r;
+        if (colok && (uint32_t)(v0 + (int)r) < (uint32_t)a.nh) {
+          copy_dword_to_lds(win + (long long)r * a.nw, 4u * (uint32_t)lane, dst);
+        } else {
+          typedef __attribute__((address_space(3))) float* lds_p;
+          *(lds_p)(dst + 4u * (uint32_t)lane) = 0.0f;
         }
       }
     }
   };
-
-  uint2 wn = make_uint2(0u, kWinSkip);
-  if (a.nviews > 0) {
-    wn = W[0];
-    if constexpr (DT == FC_F32) issue_lds(0, wn, tile[0]);
-    else issue(0, wn);
-  }
-  for (int t = 0; t < a.nviews; ++t) {
-    const uint2 w = wn;
-    float* T = tile[t & 1];
-    const bool more = t + 1 < a.nviews;
-    const uint32_t Wu = w.y & 0xffffu, Wv = w.y >> 16;
-    const double* Mp = a.views + (size_t)t * FC_VIEW_DOUBLES + 12;
-    double M[12];
-    float s;
-    if constexpr (DT == FC_F32) {
-      // the view's words first (they do not depend on the barrier: a wave that finishes view
-      // t - 1 early waits for them while the others still compute); without norms the weight's
-      // load reads the matrix's first word, and the weight is 1
-      load_view_words(Mp, W + (more ? t + 1 : t),
-                      a.norm ? a.norm + t : reinterpret_cast<const float*>(Mp), M, wn, s);
-      if (!a.norm) s = 1.0f;
-      // this wave's copies of view t have landed; the barrier then covers every wave's
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    } else {
-      // the other buffer's readers (view t-1) all passed the previous barrier before this write
-      commit(T, w);
-    }
-    __syncthreads();
-    // the next view's rows are in flight while view t is accumulated; the other buffer's readers
-    // (view t-1) all passed the barrier above
-    if constexpr (DT == FC_F32) {
-      if (more) issue_lds(t + 1, wn, tile[(t + 1) & 1]);
-    } else {
-      if (more) {
-        wn = W[t + 1];
-        issue(t + 1, wn);
-      }
+  // 16-bit storage: registers hold the raw bits of a unit (converting at commit keeps the loads in
+  // flight). A unit over the detector's edge is loaded from the nearest place on it and shifted into
+  // place at commit; zero bits are +0 in every storage format.
+  uint2 pre[kCopies];
+  auto issue = [&](int t, uint32_t org, uint32_t size) {
+    const uint32_t Wu = size & 0xffffu, Wv = size >> 16;
+    if (Wu == kWinSkip || Wu == kWinGlobal) return;
+    const int u0 = (int)(int16_t)(org & 0xffffu), v0 = (int)(int16_t)(org >> 16);
+    const int rows = (int)Wv - kRowsW * wv;
+    const int vlo = min(max(v0, 0), a.nh - 1);
+    const uint16_t* base = static_cast<const uint16_t*>(a.proj) + ((long long)t * a.nh + vlo) * a.nw;
+    const int cs = min(max(u0 + (int)col, 0), max(a.nw - 4, 0));
 #pragma unroll
-      for (int i = 0; i < 12; ++i) M[i] = Mp[i];
-      s = a.norm ? a.norm[t] : 1.0f;
-    }
-    if (Wu == kWinSkip) continue;  // uniform: the cube misses the detector in this view
-    const double A = M[0] * X + M[1] * Y + M[2] * Z0 + M[3];
-    const double B = M[4] * X + M[5] * Y + M[6] * Z0 + M[7];
-    const double C = M[8] * X + M[9] * Y + M[10] * Z0 + M[11];
-    if (Wu == kWinGlobal) {
-      const size_t vbase = (size_t)t * a.nh * a.nw;
-      const float af = (float)A, bf = (float)B, cf = (float)C;
-      const float da = (float)M[2], db = (float)M[6], dc = (float)M[10];
-#pragma unroll
-      for (int k = 0; k < kZR; ++k) {
-        const float kf = (float)k;
-        const float rc = 1.0f / fmaf(kf, dc, cf);
-        float wt = s;
-        if constexpr (MODE == FC_BP_FDK) wt = s * rc * rc;
-        if constexpr (MODE == FC_BP_KATSEVICH) wt = s * rc;
-        acc[k] = fmaf(wt, bilinear_global<DT>(a.proj, vbase, a.nw, a.nh, fmaf(kf, da, af) * rc,
-                                              fmaf(kf, db, bf) * rc), acc[k]);
-      }
-      continue;
-    }
-    const float u0f = (float)(int16_t)(w.x & 0xffffu), v0f = (float)(int16_t)(w.x >> 16);
-    // Tile coordinates. Valid voxels lie >= 1 pixel inside the window; the clamps only keep
-    // voxels outside the volume (partial blocks) and NaN inside the buffer.
-    const float umax = (float)Wu - 2.0f, vmax = (float)Wv - 2.0f;
-    if (M[2] == 0.0 && M[10] == 0.0) {  // uniform per view
-      // Columns independent of z: u and the weight are per column, the row is linear in z.
-      // FP32 reciprocal refined by one FP64 Newton step: relative error ~2^-44
-      double rc = (double)__builtin_amdgcn_rcpf((float)C);
-      rc = rc * fma(-C, rc, 2.0);
-      const float u = clampf((float)(A * rc) - u0f, 0.0f, umax);
-      const float vb = (float)(B * rc) - v0f;
-      const float dv = (float)(M[6] * rc);
-      float wt = s;
-      if constexpr (MODE == FC_BP_FDK) wt = s * (float)(rc * rc);
-      if constexpr (MODE == FC_BP_KATSEVICH) wt = s * (float)rc;
-      const uint32_t iu = (uint32_t)(int)u;
-      const float au = __builtin_amdgcn_fractf(u);
-      if (inner) {
-        // every voxel of the cube is in the volume: its taps lie >= 1 pixel inside the window
-#pragma unroll
-        for (int k = 0; k < kZR; ++k)
-          acc[k] = fmaf(wt, tile_bilinear(T, iu, au, fmaf((float)k, dv, vb)), acc[k]);
-      } else {
-#pragma unroll
-        for (int k = 0; k < kZR; ++k) {
-          const float v = clampf(fmaf((float)k, dv, vb), 0.0f, vmax);
-          acc[k] = fmaf(wt, tile_bilinear(T, iu, au, v), acc[k]);
+    for (int i = 0; i < kCopies; ++i) {
+      if (kRowsB * i < rows && (int)lrow < rows - kRowsB * i && col < Wu) {
+        const int r = min(max(v0 + kRowsW * wv + kRowsB * i + (int)lrow, vlo), a.nh - 1) - vlo;
+        const uint16_t* p = base + (uint32_t)(r * a.nw + cs);
+        if (a.nw >= 4) {
+          const fc_u32x2_a2 q = *reinterpret_cast<const fc_u32x2_a2*>(p);
+          pre[i] = make_uint2(q.x, q.y);
+        } else {  // rows of one to three pixels, zeros after them
+          const uint32_t h1 = a.nw > 1 ? p[1] : 0u, h2 = a.nw > 2 ? p[2] : 0u;
+          pre[i] = make_uint2((uint32_t)p[0] | h1 << 16, h2);
         }
       }
-    } else {
-      const float af = (float)A, bf = (float)B, cf = (float)C;
-      const float da = (float)M[2], db = (float)M[6], dc = (float)M[10];
+    }
+  };
+  auto commit = [&](float* T, uint32_t org, uint32_t size) {
+    const uint32_t Wu = size & 0xffffu, Wv = size >> 16;
+    if (Wu == kWinSkip || Wu == kWinGlobal) return;
+    const int u0 = (int)(int16_t)(org & 0xffffu), v0 = (int)(int16_t)(org >> 16);
+    const int rows = (int)Wv - kRowsW * wv;
+    const bool all = whole(u0, v0, Wu, Wv);
 #pragma unroll
-      for (int k = 0; k < kZR; ++k) {
-        const float kf = (float)k;
-        const float rc = __builtin_amdgcn_rcpf(fmaf(kf, dc, cf));  // 1 ulp, as the positions
-        const float u = clampf(fmaf(kf, da, af) * rc - u0f, 0.0f, umax);
-        const float v = clampf(fmaf(kf, db, bf) * rc - v0f, 0.0f, vmax);
-        float wt = s;
-        if constexpr (MODE == FC_BP_FDK) wt = s * rc * rc;
-        if constexpr (MODE == FC_BP_KATSEVICH) wt = s * rc;
-        acc[k] = fmaf(wt, tile_bilinear(T, (uint32_t)(int)u, __builtin_amdgcn_fractf(u), v),
-                      acc[k]);
+    for (int i = 0; i < kCopies; ++i)
+      if (kRowsB * i < rows && (int)lrow < rows - kRowsB * i && col < Wu) {
+        const int r = kRowsW * wv + kRowsB * i + (int)lrow;
+        uint2 q = pre[i];
+        if (!all) {
+          // pixel k of the unit is pixel k + d of what was loaded
+          const int d = u0 + (int)col - min(max(u0 + (int)col, 0), max(a.nw - 4, 0));
+          unsigned long long b = (unsigned long long)q.y << 32 | q.x;
+          b = d >= 0 ? b >> (16 * min(d, 3)) : b << (16 * min(-d, 3));
+          if (d <= -4 || d >= 4 || (uint32_t)(v0 + r) >= (uint32_t)a.nh) b = 0ull;
+          q = make_uint2((uint32_t)b, (uint32_t)(b >> 32));
+        }
+        *reinterpret_cast<float4*>(T + kTileP * (uint32_t)r + col) =
+            make_float4(bits_to_f32<DT>(q.x & 0xffffu), bits_to_f32<DT>(q.x >> 16),
+                        bits_to_f32<DT>(q.y & 0xffffu), bits_to_f32<DT>(q.y >> 16));
+      }
+  };
+
+  for (int tb = tbeg; tb < tend; tb += kTab) {
+    const int n = min(kTab, tend - tb);
+    __syncthreads();  // the previous table is no longer read
+    // one entry more than the table's views: the next view's window
+    if ((int)threadIdx.x <= n && tb + (int)threadIdx.x < tend)
+      tab[threadIdx.x] = view_entry(a, tb + (int)threadIdx.x, bx0, by0, z0);
+    __syncthreads();
+    if (tb == tbeg) {
+      const uint32_t org = __builtin_amdgcn_readfirstlane(tab[0].org),
+                     size = __builtin_amdgcn_readfirstlane(tab[0].size);
+      if constexpr (DT == FC_F32) issue_lds(tb, org, size, lds_address(tile[0]));
+      else issue(tb, org, size);
+    }
+    for (int i = 0; i < n; ++i) {
+      const int t = tb + i;
+      float* T = tile[(t - tbeg) & 1];
+      const bool more = t + 1 < tend;
+      // the entries first (they do not depend on the barrier: a wave that finishes view t - 1 early
+      // waits for them while the others still compute)
+      const ViewEntry E = tab[i];
+      const ViewEntry* next = tab + (more ? i + 1 : i);
+      const uint32_t norg = __builtin_amdgcn_readfirstlane(next->org),
+                     nsize = __builtin_amdgcn_readfirstlane(next->size);
+      const uint32_t org = __builtin_amdgcn_readfirstlane(E.org),
+                     size = __builtin_amdgcn_readfirstlane(E.size);
+      if constexpr (DT == FC_F32) {
+        // this wave's copies of view t have landed; the barrier then covers every wave's
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      } else {
+        // the other buffer's readers (view t-1) all passed the previous barrier before this write
+        commit(T, org, size);
+      }
+      __syncthreads();
+      // the next view's rows are in flight while view t is accumulated; the other buffer's readers
+      // (view t-1) all passed the barrier above
+      if (more) {
+        if constexpr (DT == FC_F32) issue_lds(t + 1, norg, nsize, lds_address(tile[(t + 1 - tbeg) & 1]));
+        else issue(t + 1, norg, nsize);
+      }
+      const uint32_t Wu = size & 0xffffu, Wv = size >> 16;
+      if (Wu == kWinSkip) continue;  // uniform: the cube misses the detector in this view
+      if (Wu == kWinGlobal) {
+        const double* M = a.views + (size_t)t * FC_VIEW_DOUBLES + 12;
+        const double X = (double)x + a.ox, Y = (double)y + a.oy, Z0 = (double)z0 + a.oz;
+        const float af = (float)(M[0] * X + M[1] * Y + M[2] * Z0 + M[3]);
+        const float bf = (float)(M[4] * X + M[5] * Y + M[6] * Z0 + M[7]);
+        const float cf = (float)(M[8] * X + M[9] * Y + M[10] * Z0 + M[11]);
+        const size_t vbase = (size_t)t * a.nh * a.nw;
+        const float da = (float)M[2], db = (float)M[6], dc = (float)M[10];
+#pragma unroll 1
+        for (int k = 0; k < kZR; ++k) {
+          const float kf = (float)k;
+          const float rc = 1.0f / fmaf(kf, dc, cf);
+          float wt = E.s;
+          if constexpr (MODE == FC_BP_FDK) wt = E.s * rc * rc;
+          if constexpr (MODE == FC_BP_KATSEVICH) wt = E.s * rc;
+          const float add = wt * bilinear_global<DT>(a.proj, vbase, a.nw, a.nh,
+                                                     fmaf(kf, da, af) * rc, fmaf(kf, db, bf) * rc);
+#pragma unroll
+          for (int q = 0; q < kZR; ++q) acc[q] += q == k ? add : 0.0f;
+        }
+        continue;
+      }
+      // Tile coordinates. Valid voxels lie >= 1 pixel inside the window; the clamps only keep
+      // voxels outside the volume (partial blocks) and NaN inside the buffer.
+      const float umax = (float)Wu - 2.0f, vmax = (float)Wv - 2.0f;
+      const uint32_t T0 = lds_address(T);
+      const float A = fmaf(dx, E.a[1], fmaf(dy, E.a[2], E.a[0]));
+      const float B = fmaf(dx, E.b[1], fmaf(dy, E.b[2], E.b[0]));
+      const float C = fmaf(dx, E.c[1], fmaf(dy, E.c[2], E.c[0]));
+      if (__builtin_amdgcn_readfirstlane(E.tilted) == 0u) {
+        // Columns independent of z: u and the weight are per column, the row is linear in z.
+        // A 1-ulp reciprocal refined by one Newton step
+        float rc = __builtin_amdgcn_rcpf(C);
+        rc = fmaf(rc, fmaf(-C, rc, 1.0f), rc);
+        const float u = clampf(A * rc, 0.0f, umax);
+        const float vb = B * rc, dv = E.b[3] * rc;
+        float wt = E.s;
+        if constexpr (MODE == FC_BP_FDK) wt = E.s * rc * rc;
+        if constexpr (MODE == FC_BP_KATSEVICH) wt = E.s * rc;
+        const uint32_t col0 = T0 + 4u * (uint32_t)(int)u;
+        const float au = __builtin_amdgcn_fractf(u);
+        // Voxels outside the volume (partial cubes) are kept inside the buffer by clamping; in whole
+        // cubes every voxel's taps lie >= 1 pixel inside the window
+        if (inner) column_samples<false>(acc, col0, au, vb, dv, wt, 0.0f);
+        else column_samples<true>(acc, col0, au, vb, dv, wt, vmax);
+      } else {
+        tilted_samples<MODE, true>(acc, T0, A, B, C, E, umax, vmax);
       }
     }
   }
   if (x < a.nx && y < a.ny) {
+    const size_t plane = (size_t)a.nx * a.ny;
+    float* o = a.vol + (a.nsplit > 1 ? (size_t)split * plane * a.nz : 0) + (size_t)y * a.nx + x;
 #pragma unroll
     for (int k = 0; k < kZR; ++k) {
-      int z = z0 + k;
-      if (z < a.nz) a.vol[((size_t)z * a.ny + y) * a.nx + x] += acc[k];
+      const int z = z0 + k;
+      if (z >= a.nz) break;
+      if (a.nsplit > 1) o[(size_t)z * plane] = acc[k];
+      else o[(size_t)z * plane] += acc[k];
     }
+  }
+}
+
+// vol += sum over the splits' partial volumes, in order.
+__global__ __launch_bounds__(256) void bp_reduce(const float* __restrict__ part, int nsplit,
+                                                 size_t n, float* __restrict__ vol) {
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
+    float s = part[i];
+    for (int k = 1; k < nsplit; ++k) s += part[(size_t)k * n + i];
+    vol[i] += s;
   }
 }
 
@@ -448,7 +550,7 @@ __global__ __launch_bounds__(256) void gather_bench_bp(const float* __restrict__
     const float u = (float)(s >> 8) * su;
     s = s * 1664525u + 1013904223u;
     const float v = (float)(s >> 8) * sv;
-    acc = fmaf(1.0001f, tile_bilinear(T, (uint32_t)(int)u, __builtin_amdgcn_fractf(u), v), acc);
+    acc = fmaf(1.0001f, tile_bilinear(lds_address(T + (int)u), __builtin_amdgcn_fractf(u), v), acc);
   }
   if (acc == 12345.678f) sink[0] = acc;
 }
@@ -478,11 +580,11 @@ __global__ __launch_bounds__(256) void gather_bench_bp_ray(const float* __restri
     const float u = clampf(2.0f + 0.7f * xl + 0.3f * yl + 0.05f * tt, 0.0f, 62.0f);
     const float vb = 2.0f + 0.2f * xl + 0.1f * yl + 0.05f * tt;
     const float wt = 1.0f + 0.001f * tt;
-    const uint32_t iu = (uint32_t)(int)u;
+    const uint32_t col0 = lds_address(T + (int)u);
     const float au = __builtin_amdgcn_fractf(u);
 #pragma unroll
     for (int k = 0; k < kZR; ++k) {
-      acc[k] = fmaf(wt, tile_bilinear(T, iu, au, fmaf((float)k, 1.3f, vb)), acc[k]);
+      acc[k] = fmaf(wt, tile_bilinear(col0, au, fmaf((float)k, 1.3f, vb)), acc[k]);
     }
   }
   float sum = 0.0f;
@@ -502,6 +604,17 @@ int dispatch_bp(const BpArgs& a, int mode, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
+// Splits of the views. Blocks run in rounds of five per CU (1280): fewer cubes than that leave CUs
+// idle, and a few rounds waste much of the last one. A split costs its partial volume's write and
+// read, so it needs enough views. Timed (1 split against the number chosen): 64^3 x 60 views 92 -> 31
+// us (12 splits), 96^3 x 120 176 -> 82 (8), 128^3 x 180 289 -> 212 (4), 150 x 200 x 210 x 200 701 ->
+// 653 (3), 256^3 x 360 2649 -> 2513 (3), 240 x 300^2 x 360 3324 -> 3233 (3); at 320 x 400^2 x 200
+// (12500 cubes) 2 and 3 splits lose 3 and 5 %.
+int bp_splits(long long nblocks, int nviews) {
+  if (nblocks < 1280) return (int)std::max(1LL, std::min<long long>(2560 / nblocks, nviews / 5));
+  return nblocks < 8192 && nviews >= 128 ? 3 : 1;
+}
+
 int launch_backproject(int device, float* vol, const int vs[3], const double origin[3],
                        const void* proj, int dt, const int ps[3], const double* views,
                        const float* norm, int mode, hipStream_t stream) {
@@ -510,37 +623,43 @@ int launch_backproject(int device, float* vol, const int vs[3], const double ori
   const int nbx = (vs[0] + kBXY - 1) / kBXY, nby = (vs[1] + kBXY - 1) / kBXY,
             nbz = (vs[2] + kZR - 1) / kZR;
   FC_CHECK_ARG(nby <= 65535 && nbz <= 65535, "volume too large for the grid");
-  const size_t nwin = (size_t)nbx * nby * nbz * nv;
-  void* ws = nullptr;
-  int rc = acquire_ws(device, SLOT_QUAD, nwin * sizeof(uint2), stream, &ws);
-  if (rc) return rc;
-  WinArgs w;
-  w.views = views;
-  w.win = static_cast<uint2*>(ws);
-  w.ox = origin[0]; w.oy = origin[1]; w.oz = origin[2];
-  w.nx = vs[0]; w.ny = vs[1]; w.nz = vs[2];
-  w.nw = nw; w.nh = nh; w.nviews = nv;
-  w.nbx = nbx; w.nby = nby; w.nbz = nbz;
+  const size_t n = (size_t)vs[0] * vs[1] * vs[2];
   BpArgs a;
   a.vol = vol;
   a.proj = proj;
   a.norm = norm;
   a.views = views;
-  a.win = w.win;
   a.ox = origin[0]; a.oy = origin[1]; a.oz = origin[2];
   a.nx = vs[0]; a.ny = vs[1]; a.nz = vs[2];
   a.nw = nw; a.nh = nh; a.nviews = nv;
-  a.nbx = nbx; a.nby = nby;
-  const dim3 grid(nbx, nby, nbz);
+  a.nbz = nbz;
+  a.nsplit = std::min(bp_splits((long long)nbx * nby * nbz, nv), 65535 / nbz);
+  void* ws = nullptr;
+  if (a.nsplit > 1) {
+    int rc = acquire_ws(device, SLOT_QUAD, (size_t)a.nsplit * n * sizeof(float), stream, &ws);
+    if (rc == FC_ERR_MEMORY) {  // no room for the partial volumes: one block per cube
+      clear_error();
+      a.nsplit = 1;
+    } else if (rc) {
+      return rc;
+    } else {
+      a.vol = static_cast<float*>(ws);
+    }
+  }
+  const dim3 grid(nbx, nby, nbz * a.nsplit);
   int tok = prof_begin("backproject", stream);
-  bp_windows<<<(unsigned)((nwin + 255) / 256), 256, 0, stream>>>(w);
   int r2;
   if (dt == FC_F32) r2 = dispatch_bp<FC_F32>(a, mode, grid, stream);
   else if (dt == FC_BF16) r2 = dispatch_bp<FC_BF16>(a, mode, grid, stream);
   else r2 = dispatch_bp<FC_F16>(a, mode, grid, stream);
+  if (a.nsplit > 1) {
+    bp_reduce<<<(unsigned)std::min<size_t>((n + 255) / 256, 4096), 256, 0, stream>>>(
+        a.vol, a.nsplit, n, vol);
+  }
   prof_end(tok, stream);
   if (r2) return r2;
-  return release_ws(device, SLOT_QUAD, stream);
+  FC_HIP(hipGetLastError());
+  return a.nsplit > 1 ? release_ws(device, SLOT_QUAD, stream) : FC_OK;
 }
 
 int launch_stage_quads(const void* proj, int dt, int nw, int nh, int nv, const float* norm,
