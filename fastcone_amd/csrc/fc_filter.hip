@@ -15,26 +15,30 @@
 // Method. The linear convolution equals a circular one of any length L >= 2 nw - 1, so each row
 // is zero-padded to L = 2^p (64 <= L <= 8192), and two rows share one complex transform (row a in
 // the real part, row b in the imaginary part: the kernel is real, so the two convolutions do not
-// mix). The transform is a radix-8 (then 4 or 2) Stockham FFT in LDS; the spectrum is multiplied
-// by DFT_L(kern) / L and conjugated, transformed forward again and conjugated back
-// (ifft(X) = conj(fft(conj(X))) / L): the result's real part is row a, minus its imaginary part
-// row b. DFT_L(kern) is evaluated on the device in FP64 from the closed-form taps (not from the
-// length-2nw bins, which zero padding to L would not reproduce), and rounded to FP32; so are the
-// twiddles exp(-2 pi i m / L). A 256-thread block owns one pair of rows at a time and reads both
-// completely before it writes either, so the filter may run in place.
+// mix). L / 16 threads transform a pair of rows, sixteen elements each in registers: the forward
+// transform is decimated in frequency, radix 16 and a last radix of 2 to 16, and leaves the spectrum
+// in digit-reversed order in registers; there it is multiplied by DFT_L(kern) / L (loaded in that
+// order) and conjugated; that DFT is real (RAMP) or imaginary (HILBERT: then row a goes in as the
+// imaginary and row b as the real part, which turns the factor i into one sign of the output), so
+// the product is two multiplications; the same stages transposed, in reverse order, transform it back to natural
+// order (ifft(X) = conj(fft(conj(X))) / L): the result's real part is row a, minus its imaginary part
+// row b (HILBERT: plus). A stage writes to LDS exactly the elements it read, so one barrier per exchange suffices and
+// none separates two pairs. DFT_L(kern) is evaluated on the device in FP64 from the closed-form taps
+// (not from the length-2nw bins, which zero padding to L would not reproduce), and rounded to FP32;
+// so are the twiddles exp(-2 pi i m / L). Both rows of a pair are read completely before either is
+// written, so the filter may run in place.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "fc_device.h"
 #include "fc_internal.h"
 
 namespace fc {
 namespace {
-
-constexpr int kFT = 256;  // threads per block
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) {
   return make_float2(a.x + b.x, a.y + b.y);
@@ -85,49 +89,196 @@ __device__ __forceinline__ void dft<8>(float2* v) {
   }
 }
 
-// One Stockham stage of radix R after sub-transforms of length NS, in place in LDS: every item j
-// reads buf[j + r L/R], applies the twiddles of its position k = j mod NS, transforms, and writes
-// buf[(j - k) R + k + r NS]. All reads finish (barrier) before any write.
-template <int L, int R, int NS>
-__device__ __forceinline__ void stockham(float2* buf, const float2* __restrict__ tw) {
-  constexpr int NI = L / R;
-  constexpr int PER = (NI + kFT - 1) / kFT;
-  float2 v[PER][R];
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int j = (int)threadIdx.x + kFT * q;
-    if (NI % kFT == 0 || j < NI) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) v[q][r] = buf[j + r * NI];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const int j = (int)threadIdx.x + kFT * q;
-    if (NI % kFT == 0 || j < NI) {
-      const int k = j & (NS - 1);
-      if constexpr (NS > 1) {
-#pragma unroll
-        for (int r = 1; r < R; ++r) v[q][r] = cmul(v[q][r], tw[k * r * (L / (NS * R))]);
-      }
-      dft<R>(v[q]);
-      const int base = (j - k) * R + k;
-#pragma unroll
-      for (int r = 0; r < R; ++r) buf[base + r * NS] = v[q][r];
-    }
-  }
-  __syncthreads();
+// v W16 and v W16^3, W16 = cos - i sin of pi/8. cos is applied as 1 - 0.076..: rounded to FP32 by
+// itself it is 3.1e-8 too small, an error that all the transform's stages would share.
+__device__ __forceinline__ float2 rot16(float2 v) {
+  const float d = 0.07612046748871326f, s = 0.38268343236508977f;
+  return make_float2(fmaf(-d, v.x, fmaf(s, v.y, v.x)), fmaf(-d, v.y, fmaf(-s, v.x, v.y)));
+}
+__device__ __forceinline__ float2 rot16_3(float2 v) {
+  const float d = 0.07612046748871326f, s = 0.38268343236508977f;
+  return make_float2(fmaf(-d, v.y, fmaf(s, v.x, v.y)), fmaf(d, v.x, fmaf(s, v.y, -v.x)));
 }
 
-// Forward length-L FFT: radix 8 while at least 8 points remain per sub-transform, then 4 or 2.
-template <int L, int NS>
-__device__ __forceinline__ void fft_pass(float2* buf, const float2* __restrict__ tw) {
-  if constexpr (NS < L) {
-    constexpr int R = (L / NS) >= 8 ? 8 : L / NS;
-    stockham<L, R, NS>(buf, tw);
-    fft_pass<L, NS * R>(buf, tw);
+// c + a b and c - a b
+__device__ __forceinline__ float2 cfma(float2 a, float2 b, float2 c) {
+  return make_float2(fmaf(a.x, b.x, fmaf(-a.y, b.y, c.x)), fmaf(a.x, b.y, fmaf(a.y, b.x, c.y)));
+}
+__device__ __forceinline__ float2 cfms(float2 a, float2 b, float2 c) {
+  return make_float2(fmaf(-a.x, b.x, fmaf(a.y, b.y, c.x)), fmaf(-a.x, b.y, fmaf(-a.y, b.x, c.y)));
+}
+
+// dft<16> of v[0], w[0] v[1], .., w[14] v[15] (w null: of v itself). Half of the twiddles are
+// factors of the first butterflies' FMAs: as many instructions, one rounding less. HALF: v[8..15]
+// are zeros.
+template <bool HALF = false>
+__device__ __forceinline__ void dft16(float2* v, const float2* w) {
+  // 4 x 4: columns n1 + 4 n2 over n2, twiddles W16^(n1 k2), rows over n1; X[4 k1 + k2]
+  const float r = 0.70710678118654752f;
+  float2 t[4][4];
+#pragma unroll
+  for (int n1 = 0; n1 < 4; ++n1) {
+    if (w) {
+      const float2 p0 = n1 ? cmul(w[n1 - 1], v[n1]) : v[0], p1 = cmul(w[n1 + 3], v[n1 + 4]);
+      const float2 t0 = cfma(w[n1 + 7], v[n1 + 8], p0), t1 = cfms(w[n1 + 7], v[n1 + 8], p0);
+      const float2 t2 = cfma(w[n1 + 11], v[n1 + 12], p1),
+                   t3 = mul_mi(cfms(w[n1 + 11], v[n1 + 12], p1));
+      t[n1][0] = cadd(t0, t2);
+      t[n1][2] = csub(t0, t2);
+      t[n1][1] = cadd(t1, t3);
+      t[n1][3] = csub(t1, t3);
+    } else if (HALF) {
+      const float2 p1 = mul_mi(v[n1 + 4]);
+      t[n1][0] = cadd(v[n1], v[n1 + 4]);
+      t[n1][2] = csub(v[n1], v[n1 + 4]);
+      t[n1][1] = cadd(v[n1], p1);
+      t[n1][3] = csub(v[n1], p1);
+    } else {
+#pragma unroll
+      for (int n2 = 0; n2 < 4; ++n2) t[n1][n2] = v[n1 + 4 * n2];
+      dft<4>(t[n1]);
+    }
   }
+  t[1][1] = rot16(t[1][1]);
+  t[1][2] = make_float2(r * (t[1][2].x + t[1][2].y), r * (t[1][2].y - t[1][2].x));
+  t[1][3] = rot16_3(t[1][3]);
+  t[2][1] = make_float2(r * (t[2][1].x + t[2][1].y), r * (t[2][1].y - t[2][1].x));
+  t[2][2] = mul_mi(t[2][2]);
+  t[2][3] = make_float2(r * (t[2][3].y - t[2][3].x), -r * (t[2][3].x + t[2][3].y));
+  t[3][1] = rot16_3(t[3][1]);
+  t[3][2] = make_float2(r * (t[3][2].y - t[3][2].x), -r * (t[3][2].x + t[3][2].y));
+  t[3][3] = rot16(t[3][3]);  // times -W16: the sign is in its use
+  t[3][3] = make_float2(-t[3][3].x, -t[3][3].y);
+#pragma unroll
+  for (int k2 = 0; k2 < 4; ++k2) {
+    float2 u[4] = {t[0][k2], t[1][k2], t[2][k2], t[3][k2]};
+    dft<4>(u);
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) v[4 * k1 + k2] = u[k1];
+  }
+}
+
+template <>
+__device__ __forceinline__ void dft<16>(float2* v) {
+  dft16(v, nullptr);
+}
+
+// Length-L transforms by L / 16 threads, sixteen elements each (file header). A stage works on
+// sub-blocks of M elements: thread `tid` has elements j + r M / 16 of sub-block tid / (M / 16), with
+// j = tid mod M / 16; the last one (M < 16, or M = 16) has 16 / M whole sub-blocks, tid + b L / 16.
+constexpr int kE = 16;
+
+template <int L, int M>
+__device__ __forceinline__ constexpr int element(int tid, int r) {
+  if constexpr (M >= kE) {
+    constexpr int S = M / kE;
+    return tid / S * M + tid % S + r * S;
+  } else {
+    return (tid + r / M * (L / kE)) * M + r % M;
+  }
+}
+
+// LDS slot of an element: one float2 of padding after every 16, so that a stage's reads and writes
+// (strides of a power of two) use all banks. element(tid, 0) and element(0, r) share no carry into
+// bit 4, so slot(element(tid, r)) is the sum of their slots and r costs no address arithmetic.
+__device__ __forceinline__ constexpr int slot(int i) { return i + (i >> 4); }
+
+template <int L, int M>
+__device__ __forceinline__ void put(float2* buf, const float2* v, int tid) {
+  float2* b = buf + slot(element<L, M>(tid, 0));
+#pragma unroll
+  for (int r = 0; r < kE; ++r) b[slot(element<L, M>(0, r))] = v[r];
+}
+template <int L, int M>
+__device__ __forceinline__ void get(float2* v, const float2* buf, int tid) {
+  const float2* b = buf + slot(element<L, M>(tid, 0));
+#pragma unroll
+  for (int r = 0; r < kE; ++r) v[r] = b[slot(element<L, M>(0, r))];
+}
+
+// Twiddles of the stage with sub-blocks of M elements.
+template <int L, int M>
+__device__ __forceinline__ void stage_twiddles(float2* t, const float2* __restrict__ tw, int tid) {
+  if constexpr (M > kE) {
+    const int j = tid % (M / kE);
+#pragma unroll
+    for (int q = 1; q < kE; ++q) t[q - 1] = tw[j * q * (L / M)];
+  }
+}
+
+// Those of the first stage are in registers (t0); the others are loaded where they are used, from a
+// few distinct addresses per wave.
+template <int L, int M>
+__device__ __forceinline__ void twiddles(float2* t, const float2* t0, const float2* __restrict__ tw,
+                                         int tid) {
+  if constexpr (M == L) {
+#pragma unroll
+    for (int q = 0; q < kE - 1; ++q) t[q] = t0[q];
+  } else {
+    asm volatile("" : "+v"(tid));  // not kept in registers from pair to pair
+    stage_twiddles<L, M>(t, tw, tid);
+  }
+}
+
+// Sub-block length of the last stage.
+constexpr int last_block(int M) { return M > kE ? last_block(M / kE) : M; }
+
+// Forward stages from sub-blocks of M elements down: v ends as the spectrum in the last stage's
+// elements.
+template <int L, int M>
+__device__ __forceinline__ void fft_down(float2* v, float2* buf, const float2* t0,
+                                         const float2* __restrict__ tw, int tid) {
+  if constexpr (M > kE) {
+    dft16<M == L>(v, nullptr);  // rows fill at most half of the length
+    float2 t[kE - 1];
+    twiddles<L, M>(t, t0, tw, tid);
+#pragma unroll
+    for (int q = 1; q < kE; ++q) v[q] = cmul(v[q], t[q - 1]);
+    put<L, M>(buf, v, tid);
+    __syncthreads();
+    get<L, M / kE>(v, buf, tid);
+    fft_down<L, M / kE>(v, buf, t0, tw, tid);
+  } else {
+#pragma unroll
+    for (int g = 0; g < kE / M; ++g) dft<M>(v + g * M);
+  }
+}
+
+// The same stages transposed, from the last one up to sub-blocks of M elements: v ends as the
+// transform's natural order, elements j + r L / 16.
+template <int L, int M>
+__device__ __forceinline__ void fft_up(float2* v, float2* buf, const float2* t0,
+                                       const float2* __restrict__ tw, int tid) {
+  if constexpr (M > kE) {
+    fft_up<L, M / kE>(v, buf, t0, tw, tid);
+    put<L, M / kE>(buf, v, tid);
+    __syncthreads();
+    get<L, M>(v, buf, tid);
+    float2 t[kE - 1];
+    twiddles<L, M>(t, t0, tw, tid);
+    dft16(v, t);
+  } else {
+#pragma unroll
+    for (int g = 0; g < kE / M; ++g) dft<M>(v + g * M);
+  }
+}
+
+// Frequency of element p after fft_down: the digits of p (radix 16 from the top, the last one the
+// remaining radix) in reverse order.
+template <int L>
+__device__ __forceinline__ int frequency(int p) {
+  int k = 0, mul = 1, size = L;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    if (size > 1) {
+      const int radix = size < kE ? size : kE, sub = size / radix;
+      k += p / sub * mul;
+      p %= sub;
+      mul *= radix;
+      size = sub;
+    }
+  }
+  return k;
 }
 
 struct FiltArgs {
@@ -135,51 +286,50 @@ struct FiltArgs {
   void* out;
   const double* views;  // flat-detector view records for the cosine weight, or null
   const float2* tw;     // L twiddles
-  const float2* mult;   // L multipliers DFT_L(kern) / L
+  const float* mult;    // L multipliers: DFT_L(kern) / L, or its imaginary part (hilbert)
+  bool hilbert;         // DFT_L(kern) is imaginary (else real)
   long long nrows;
   int nw, nh;
   int in_dt, out_dt;
 };
 
-__device__ __forceinline__ float load_any(const void* p, int dt, size_t i) {
-  if (dt == FC_F32) return load_elem<FC_F32>(p, i);
-  if (dt == FC_BF16) return load_elem<FC_BF16>(p, i);
-  return load_elem<FC_F16>(p, i);
+// fn called with the storage type dt as a constant, once for all of a thread's elements.
+template <class F>
+__device__ __forceinline__ void by_type(int dt, F&& fn) {
+  if (dt == FC_F32) fn(std::integral_constant<int, FC_F32>());
+  else if (dt == FC_BF16) fn(std::integral_constant<int, FC_BF16>());
+  else fn(std::integral_constant<int, FC_F16>());
 }
 
-__device__ __forceinline__ void store_any(void* p, int dt, size_t i, float v) {
-  if (dt == FC_F32) static_cast<float*>(p)[i] = v;
-  else if (dt == FC_BF16) static_cast<uint16_t*>(p)[i] = f32_to_bf16_bits(v);
+template <int DT>
+__device__ __forceinline__ void store_elem(void* p, size_t i, float v) {
+  if constexpr (DT == FC_F32) static_cast<float*>(p)[i] = v;
+  else if constexpr (DT == FC_BF16) static_cast<uint16_t*>(p)[i] = f32_to_bf16_bits(v);
   else static_cast<uint16_t*>(p)[i] = f32_to_f16_bits(v);
 }
 
-// Cosine pre-weight of row r: pixel j of the row sits at b + j u (relative to the source, FP64);
-// its weight is dperp / |b + j u|, dperp the source's distance from the detector plane.
+// Cosine pre-weight of a row: pixel j sits at b + j u (relative to the source, FP64); its weight is
+// dperp / |b + j u|, dperp the source's distance from the detector plane. |b + j u|^2 is kept as a
+// polynomial in j.
 struct RowWeight {
-  double bx, by, bz, ux, uy, uz;
+  double c0, c1, c2;
   float dperp;
-  bool on;
 };
 
 __device__ __forceinline__ RowWeight row_weight(const FiltArgs& a, long long r) {
-  RowWeight w;
-  w.on = a.views != nullptr;
-  w.bx = w.by = w.bz = w.ux = w.uy = w.uz = 0.0;
-  w.dperp = 1.0f;
-  if (!w.on) return w;
   const long long t = r / a.nh;
   const double i = (double)(r - t * a.nh);
   const double* V = a.views + (size_t)t * FC_VIEW_DOUBLES;
   const double r0x = V[3] - V[0], r0y = V[4] - V[1], r0z = V[5] - V[2];
-  w.bx = r0x + i * V[9];
-  w.by = r0y + i * V[10];
-  w.bz = r0z + i * V[11];
-  w.ux = V[6];
-  w.uy = V[7];
-  w.uz = V[8];
+  const double bx = r0x + i * V[9], by = r0y + i * V[10], bz = r0z + i * V[11];
+  const double ux = V[6], uy = V[7], uz = V[8];
   const double nx = V[7] * V[11] - V[8] * V[10], ny = V[8] * V[9] - V[6] * V[11],
                nz = V[6] * V[10] - V[7] * V[9];
   const double nn = sqrt(nx * nx + ny * ny + nz * nz);
+  RowWeight w;
+  w.c0 = bx * bx + by * by + bz * bz;
+  w.c1 = 2.0 * (bx * ux + by * uy + bz * uz);
+  w.c2 = ux * ux + uy * uy + uz * uz;
   // only flat-detector records carry the plane geometry this weight needs
   w.dperp = V[24] == (double)FC_DET_FLAT ? (float)(fabs(r0x * nx + r0y * ny + r0z * nz) / nn)
                                          : __builtin_nanf("");
@@ -187,64 +337,124 @@ __device__ __forceinline__ RowWeight row_weight(const FiltArgs& a, long long r) 
 }
 
 __device__ __forceinline__ float weight_at(const RowWeight& w, int j) {
-  if (!w.on) return 1.0f;
   const double jd = (double)j;
-  const double x = fma(jd, w.ux, w.bx), y = fma(jd, w.uy, w.by), z = fma(jd, w.uz, w.bz);
-  return w.dperp * rsqrtf((float)(x * x + y * y + z * z));
+  return w.dperp * __builtin_amdgcn_rsqf((float)fma(jd, fma(jd, w.c2, w.c1), w.c0));
 }
 
+// Element r of a thread lies within the row whatever its length: L / 4 < nw for all L but the
+// smallest, which also serves shorter rows.
+template <int L>
+__device__ __forceinline__ constexpr bool in_row(int r) {
+  return L > 64 && r < kE / 4;
+}
+
+// Threads per block: one pair, or the pairs of one wave.
+constexpr int filt_threads(int L) { return L / kE > 64 ? L / kE : 64; }
+
+// Per pair and wave (2048 points, cosine weights): about 1600 VALU and 72 double LDS instructions
+// against 32 to 48 memory ones. Three waves per SIMD hide the exchanges' and loads' latency best
+// (166 registers; 3.46 GB of FP32 rows of 768 columns, in ms: two waves 2.27, three 2.14, three with
+// the loads issued after the round begins 2.18); about 60 % VALU busy, 1.6 TB/s. The radix-8
+// Stockham stages with every exchange, load and the spectrum product through LDS that this replaces
+// took 3.82 ms; rows of 384 columns 0.56 -> 0.29, 3000 columns 1.36 -> 0.67, and 200000 rows of 31
+// columns 0.29 -> 0.028 (one pair per block left most threads idle there).
+// Relative error against FP64 (white rows of 31 to 3000 columns): 0.83e-7 to 1.23e-7, before
+// 0.87e-7 to 1.26e-7.
+constexpr int kWaves = 3;  // per SIMD
+
 template <int LOG2L>
-__global__ __launch_bounds__(kFT) void row_filter_kernel(FiltArgs a) {
-  constexpr int L = 1 << LOG2L;
-  constexpr int PERM = (L + kFT - 1) / kFT;  // spectrum bins per thread
-  __shared__ float2 buf[L];
-  float2 h[PERM];
+__global__ __launch_bounds__((filt_threads(1 << LOG2L)), kWaves) void row_filter_kernel(FiltArgs a) {
+  constexpr int L = 1 << LOG2L, T = L / kE, NT = filt_threads(L), P = NT / T;
+  constexpr int H = kE / 2;  // a row has at most L / 2 values: elements r < 8 of the first stage
+  __shared__ float2 lds[P][L + L / 16];
+  __shared__ RowWeight wt[2][2 * P];  // both rows of each pair, for this round and the next
+  const int tid = P == 1 ? threadIdx.x : threadIdx.x % T, sub = P == 1 ? 0 : threadIdx.x / T;
+  float2* buf = lds[sub];
+  float h[kE];
+  float2 t0[kE - 1];
+  constexpr int ML = last_block(L);
 #pragma unroll
-  for (int q = 0; q < PERM; ++q) {
-    const int m = (int)threadIdx.x + kFT * q;
-    h[q] = m < L ? a.mult[m] : make_float2(0.0f, 0.0f);
-  }
-  const long long npairs = (a.nrows + 1) / 2;
-  for (long long p = blockIdx.x; p < npairs; p += gridDim.x) {
-    const long long r0 = 2 * p, r1 = r0 + 1;
-    const bool two = r1 < a.nrows;
-    const RowWeight w0 = row_weight(a, r0);
-    const RowWeight w1 = row_weight(a, two ? r1 : r0);
-    const size_t o0 = (size_t)r0 * (size_t)a.nw, o1 = o0 + (size_t)a.nw;
+  for (int r = 0; r < kE; ++r) h[r] = a.mult[frequency<L>(element<L, ML>(tid, r))];
+  stage_twiddles<L, L>(t0, a.tw, tid);
+  const long long npairs = (a.nrows + 1) / 2, step = (long long)gridDim.x * P;
+  // weights of round p0's rows, into half s
+  auto weights = [&](long long p0, int s) {
+    if (a.views && threadIdx.x < 2 * P) {
+      const long long r = 2 * p0 + threadIdx.x;
+      if (r < a.nrows) wt[s][threadIdx.x] = row_weight(a, r);
+    }
+  };
+  // The pair's rows; columns and rows that do not exist hold some other element's value.
+  float f0[H], f1[H];
+  auto fetch = [&](long long pair) {
+    const long long r0 = std::min(2 * pair, a.nrows - 1), r1 = std::min(r0 + 1, a.nrows - 1);
+    const long long x = a.hilbert ? r1 : r0, y = a.hilbert ? r0 : r1;
+    by_type(a.in_dt, [&](auto dt) {
+      constexpr int B = dt() == FC_F32 ? 4 : 2;
+      const char* px = static_cast<const char*>(a.in) + (size_t)x * (size_t)a.nw * B;
+      const char* py = static_cast<const char*>(a.in) + (size_t)y * (size_t)a.nw * B;
 #pragma unroll
-    for (int q = 0; q < PERM; ++q) {
-      const int m = (int)threadIdx.x + kFT * q;
-      if (m < L) {
-        float2 v = make_float2(0.0f, 0.0f);
-        if (m < a.nw) {
-          v.x = load_any(a.in, a.in_dt, o0 + m) * weight_at(w0, m);
-          if (two) v.y = load_any(a.in, a.in_dt, o1 + m) * weight_at(w1, m);
+      for (int r = 0; r < H; ++r) {
+        const unsigned m = in_row<L>(r) ? tid + r * T : std::min(tid + r * T, a.nw - 1);
+        f0[r] = load_elem<dt()>(px + m * B, 0);
+        f1[r] = load_elem<dt()>(py + m * B, 0);
+      }
+    });
+  };
+  long long p0 = (long long)blockIdx.x * P;
+  weights(p0, 0);
+  fetch(p0 + sub);
+  __syncthreads();
+  int s = 0;
+  for (; p0 < npairs; p0 += step, s ^= 1) {
+    const long long r0 = 2 * (p0 + sub);
+    float2 v[kE];
+    int lt = tid;
+    asm volatile("" : "+v"(lt));  // the FP64 columns are not kept in registers from pair to pair
+    if (a.views) {
+      const RowWeight w0 = wt[s][2 * sub + a.hilbert], w1 = wt[s][2 * sub + 1 - a.hilbert];
+#pragma unroll
+      for (int r = 0; r < H; ++r) {
+        f0[r] *= weight_at(w0, lt + r * T);
+        f1[r] *= weight_at(w1, lt + r * T);
+      }
+    }
+    const bool two = r0 + 1 < a.nrows;
+    if (!two) {
+#pragma unroll
+      for (int r = 0; r < H; ++r) (a.hilbert ? f0[r] : f1[r]) = 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < H; ++r) {
+      const bool in = in_row<L>(r) || lt + r * T < a.nw;
+      v[r] = make_float2(in ? f0[r] : 0.0f, in ? f1[r] : 0.0f);
+    }
+    if (p0 + step < npairs) {
+      weights(p0 + step, s ^ 1);  // read after the exchanges' barriers
+      fetch(p0 + step + sub);
+    }
+    fft_down<L, L>(v, buf, t0, a.tw, tid);
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      v[r] = make_float2(h[r] * v[r].x, -h[r] * v[r].y);
+    }
+    fft_up<L, L>(v, buf, t0, a.tw, tid);
+    if (r0 < a.nrows) {
+      const float sign1 = a.hilbert ? 1.0f : -1.0f;
+      by_type(a.out_dt, [&](auto dt) {
+        constexpr int B = dt() == FC_F32 ? 4 : 2;
+        char* q0 = static_cast<char*>(a.out) + (size_t)r0 * (size_t)a.nw * B;
+        char* q1 = q0 + (size_t)a.nw * B;
+#pragma unroll
+        for (int r = 0; r < H; ++r) {
+          const unsigned j = tid + r * T;
+          if (in_row<L>(r) || (int)j < a.nw) {
+            store_elem<dt()>(q0 + j * B, 0, v[r].x);
+            if (two) store_elem<dt()>(q1 + j * B, 0, sign1 * v[r].y);
+          }
         }
-        buf[m] = v;
-      }
+      });
     }
-    __syncthreads();
-    fft_pass<L, 1>(buf, a.tw);
-#pragma unroll
-    for (int q = 0; q < PERM; ++q) {
-      const int m = (int)threadIdx.x + kFT * q;
-      if (m < L) {
-        const float2 z = cmul(h[q], buf[m]);
-        buf[m] = make_float2(z.x, -z.y);
-      }
-    }
-    __syncthreads();
-    fft_pass<L, 1>(buf, a.tw);
-#pragma unroll
-    for (int q = 0; q < PERM; ++q) {
-      const int j = (int)threadIdx.x + kFT * q;
-      if (j < a.nw) {
-        const float2 z = buf[j];
-        store_any(a.out, a.out_dt, o0 + j, z.x);
-        if (two) store_any(a.out, a.out_dt, o1 + j, -z.y);
-      }
-    }
-    __syncthreads();  // the next pair overwrites buf
   }
 }
 
@@ -289,7 +499,7 @@ __device__ __forceinline__ double cos_table(const double* q, int L, int m) {
 // for this one.
 __global__ __launch_bounds__(256) void filt_tables(int kind, double p0, int nw, int L,
                                                    float2* __restrict__ tw,
-                                                   float2* __restrict__ mult) {
+                                                   float* __restrict__ mult) {
   extern __shared__ double lds_tab[];
   double* quarter = lds_tab;               // L/4 + 1
   double* taps = lds_tab + L / 4 + 1;      // nw
@@ -306,11 +516,10 @@ __global__ __launch_bounds__(256) void filt_tables(int kind, double p0, int nw, 
       s = fma(taps[d], cos_table(quarter, L, k * d - shift), s);
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if (lane == 0) {
-      float2 v;
-      if (kind == FC_FILTER_RAMP) v = make_float2((float)((taps[0] + 2.0 * s) / L), 0.0f);
-      else v = make_float2(0.0f, (float)(-2.0 * s / L));
+      const bool ramp = kind == FC_FILTER_RAMP;
+      const float v = (float)((ramp ? taps[0] + 2.0 * s : -2.0 * s) / L);
       mult[k] = v;
-      if (k > 0 && k < L / 2) mult[L - k] = make_float2(v.x, -v.y);
+      if (k > 0 && k < L / 2) mult[L - k] = ramp ? v : -v;
     }
   }
 }
@@ -324,8 +533,11 @@ int filter_log2(int nw) {
 inline constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Tables of the widest supported row (FC_FILTER_MAX_COLS columns, FFT length 8192): twiddles and
-// multipliers (8192 float2 each). Every row filter needs at most this.
-constexpr size_t kMaxTableBytes = 2 * align256((size_t)8192 * sizeof(float2));
+// multipliers (8192 float2 and floats). Every row filter needs at most this.
+constexpr size_t table_bytes(size_t L) {
+  return align256(L * sizeof(float2)) + align256(L * sizeof(float));
+}
+constexpr size_t kMaxTableBytes = table_bytes(8192);
 
 // Device-resident tables for fc_fdk_filter_noalloc_dev (one copy per GPU, held until the process
 // ends). In host code the name is only a stand-in: the device address comes from
@@ -334,9 +546,11 @@ static __device__ __align__(256) unsigned char scratch[kMaxTableBytes];
 
 template <int LOG2L>
 void launch_rows(const FiltArgs& a, hipStream_t s) {
-  const long long npairs = (a.nrows + 1) / 2;
-  const int blocks = (int)(npairs < 2048 ? npairs : 2048);
-  row_filter_kernel<LOG2L><<<blocks, kFT, 0, s>>>(a);
+  constexpr int NT = filt_threads(1 << LOG2L), P = NT / ((1 << LOG2L) / kE);
+  const long long rounds = ((a.nrows + 1) / 2 + P - 1) / P;
+  // the blocks that are resident at once: each loads its multipliers and twiddles once
+  const int blocks = (int)std::min(rounds, 256LL * (4 * kWaves / (NT / 64)));
+  row_filter_kernel<LOG2L><<<blocks, NT, 0, s>>>(a);
 }
 
 std::mutex g_scratch_mutex;
@@ -358,8 +572,7 @@ int scratch_address(int device, void** out) {
 }  // namespace
 
 size_t filter_table_bytes(int nw) {
-  const size_t L = (size_t)1 << filter_log2(nw);
-  return 2 * align256(L * sizeof(float2));
+  return table_bytes((size_t)1 << filter_log2(nw));
 }
 
 int launch_row_filter(const void* in, int in_dt, void* out, int out_dt, int nw, int nh,
@@ -373,7 +586,7 @@ int launch_row_filter(const void* in, int in_dt, void* out, int out_dt, int nw, 
   const int L = 1 << p;
   char* base = static_cast<char*>(tables);
   float2* tw = reinterpret_cast<float2*>(base);
-  float2* mult = reinterpret_cast<float2*>(base + align256((size_t)L * sizeof(float2)));
+  float* mult = reinterpret_cast<float*>(base + align256((size_t)L * sizeof(float2)));
   // one bin per wave up to L = 2048, at most a block per CU (its LDS holds up to 49 KB of tables)
   const int tblocks = std::min(256, (L / 2 + 4) / 4);
   filt_tables<<<tblocks, 256, (L / 4 + 1 + (size_t)nw) * sizeof(double), stream>>>(kind, p0, nw, L,
@@ -384,6 +597,7 @@ int launch_row_filter(const void* in, int in_dt, void* out, int out_dt, int nw, 
   a.views = views;
   a.tw = tw;
   a.mult = mult;
+  a.hilbert = kind == FC_FILTER_HILBERT;
   a.nrows = nrows;
   a.nw = nw;
   a.nh = nh;

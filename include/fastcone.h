@@ -171,7 +171,7 @@ int fc_fdk_filter_dev(int device, const void* proj, int proj_dtype, void* out, i
 
 /* fc_fdk_filter_dev without any device allocation, for callers that cannot allocate (code under
  * HIP graph capture, tight serving loops). No counterpart in the reference. The filter's tables
- * (twiddles and multipliers: at most 128 KiB, enough for FC_FILTER_MAX_COLS columns) live in a
+ * (twiddles and multipliers: at most 96 KiB, enough for FC_FILTER_MAX_COLS columns) live in a
  * static device array, one per GPU, held until the process ends; widths beyond FC_FILTER_MAX_COLS
  * are rejected (FC_ERR_ARGUMENT). Every call rewrites the tables it reads, on its stream; calls
  * that overlap on one GPU (different streams or threads) share the array and race. Same results
