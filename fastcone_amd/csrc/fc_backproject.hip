@@ -34,9 +34,6 @@
 // Small volumes leave compute units idle or the last round of blocks nearly empty: the views are
 // then split over several blocks per cube, whose sums go to partial volumes that bp_reduce adds in
 // order (launch_backproject).
-//
-// "Quad" staging (stage_quads: the four bilinear corners of every base pixel stored together) is
-// kept for the Katsevich backprojector's filtered data.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,31 +49,6 @@ namespace {
 
 constexpr int kZR = 16;   // z voxels per thread
 constexpr int kBXY = 16;  // 16x16 columns per 256-thread block (8x8 per wave)
-
-template <int DT_IN>
-__global__ __launch_bounds__(256) void stage_quads(const void* __restrict__ proj, int nw, int nh,
-                                                   const float* __restrict__ norm,
-                                                   void* __restrict__ quad, int QW, int QH) {
-  int c = blockIdx.x * 256 + threadIdx.x;
-  int r = blockIdx.y, t = blockIdx.z;
-  if (c >= QW) return;
-  int w0 = c - 1, h0 = r - 1;
-  float s = norm ? norm[t] : 1.0f;
-  const size_t vbase = (size_t)t * nw * nh;
-  float v[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    int w = w0 + (q & 1), h = h0 + (q >> 1);
-    bool in = w >= 0 && w < nw && h >= 0 && h < nh;
-    v[q] = in ? s * load_elem<DT_IN>(proj, vbase + (size_t)h * nw + w) : 0.0f;
-  }
-  size_t o = ((size_t)t * QH + r) * QW + c;
-  if constexpr (DT_IN == FC_F32) {
-    static_cast<float4*>(quad)[o] = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-    static_cast<uint2*>(quad)[o] = make_uint2(pack2<DT_IN>(v[0], v[1]), pack2<DT_IN>(v[2], v[3]));
-  }
-}
 
 constexpr int kTileW = 64;                 // widest staged window
 constexpr int kTileH = 48;                 // tallest staged window
@@ -245,35 +217,6 @@ __device__ __forceinline__ void column_samples(float* acc, uint32_t col, float a
     }
   }
 }
-
-// 16 bytes (or one dword) per active lane from global memory at base + lane_bytes (base
-// wave-uniform, in scalar registers: the scalar-base form of the instruction, so a copy costs no
-// vector address arithmetic) into LDS at lds_dst + 16 lane (+ 4 lane; lds_dst wave-uniform), by the
-// load-to-LDS path: no registers hold the data and no LDS write instruction is issued. Written as
-// assembly rather than the compiler builtin, with which the compiler waits for every outstanding
-// load-to-LDS before each later LDS read (it cannot tell that the reads address the other window
-// buffer). The instruction has no register outputs, its address registers are read at issue, and
-// the LDS it writes is read only after the explicit s_waitcnt and the barrier of the next view.
-// Loads complete in order, so the compiler's own vmcnt waits stay conservative with these loads
-// outstanding. M0 is declared clobbered; the compiler reports that it reserves M0, and it uses M0
-// nowhere else in this kernel.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void copy_units_to_lds(const void* base, uint32_t lane_bytes,
-                                                  uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
-                   __builtin_amdgcn_readfirstlane(lds_dst)),
-               "v"(lane_bytes), "s"(base)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void copy_dword_to_lds(const void* base, uint32_t lane_bytes,
-                                                  uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(
-                   __builtin_amdgcn_readfirstlane(lds_dst)),
-               "v"(lane_bytes), "s"(base)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
 
 // The same for a tilted detector: column, row and weight by voxel, from the view's forms at the
 // column's first voxel.
@@ -660,19 +603,6 @@ int launch_backproject(int device, float* vol, const int vs[3], const double ori
   if (r2) return r2;
   FC_HIP(hipGetLastError());
   return a.nsplit > 1 ? release_ws(device, SLOT_QUAD, stream) : FC_OK;
-}
-
-int launch_stage_quads(const void* proj, int dt, int nw, int nh, int nv, const float* norm,
-                       void* quad, hipStream_t stream) {
-  const int QW = nw + 2, QH = nh + 2;
-  FC_CHECK_ARG(QH <= 65535 && nv <= 65535, "projection stack too large for the staging grid");
-  if (nv == 0) return FC_OK;
-  dim3 sg((QW + 255) / 256, QH, nv);
-  if (dt == FC_F32) stage_quads<FC_F32><<<sg, 256, 0, stream>>>(proj, nw, nh, norm, quad, QW, QH);
-  else if (dt == FC_BF16) stage_quads<FC_BF16><<<sg, 256, 0, stream>>>(proj, nw, nh, norm, quad, QW, QH);
-  else stage_quads<FC_F16><<<sg, 256, 0, stream>>>(proj, nw, nh, norm, quad, QW, QH);
-  FC_HIP(hipGetLastError());
-  return FC_OK;
 }
 
 int launch_gather_bench_bp(int device, int dt, int ray, double* samples_per_s) {

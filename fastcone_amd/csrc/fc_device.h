@@ -113,11 +113,46 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 
 __device__ __forceinline__ float lerp(float a, float b, float t) { return fmaf(t, b - a, a); }
 
+// 16 bytes (or one dword) per active lane from global memory at base + lane_bytes (base
+// wave-uniform, in scalar registers: the scalar-base form of the instruction, so a copy costs no
+// vector address arithmetic) into LDS at lds_dst + 16 lane (+ 4 lane; lds_dst wave-uniform), by the
+// load-to-LDS path: no registers hold the data and no LDS write instruction is issued. Written as
+// assembly rather than the compiler builtin, with which the compiler waits for every outstanding
+// load-to-LDS before each later LDS read (it cannot tell that the reads address the other window
+// buffer). The instruction has no register outputs, its address registers are read at issue, and
+// the LDS it writes must be read only after an explicit s_waitcnt vmcnt(0) and a barrier.
+// Loads complete in order, so the compiler's own vmcnt waits stay conservative with these loads
+// outstanding. M0 is declared clobbered; the compiler reports that it reserves M0, and it uses M0
+// nowhere else in the kernels that copy this way.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void copy_units_to_lds(const void* base, uint32_t lane_bytes,
+                                                  uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
+                   __builtin_amdgcn_readfirstlane(lds_dst)),
+               "v"(lane_bytes), "s"(base)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void copy_dword_to_lds(const void* base, uint32_t lane_bytes,
+                                                  uint32_t lds_dst) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(
+                   __builtin_amdgcn_readfirstlane(lds_dst)),
+               "v"(lane_bytes), "s"(base)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 // a[23:0] * b[23:0] + c (low 32 bits), one full-rate VALU instruction. The compiler lowers the
 // equivalent C expression with a variable multiplier to the multi-pass v_mad_u64_u32.
 __device__ __forceinline__ uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t r;
   asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// The same for signed 24-bit factors.
+__device__ __forceinline__ uint32_t mad_i24(int a, int b, uint32_t c) {
+  uint32_t r;
+  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
 // mad_u24 with a wave-uniform multiplier read from a scalar register (an operand the vector

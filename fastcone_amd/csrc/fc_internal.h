@@ -84,9 +84,6 @@ int launch_backproject(int device, float* vol, const int vol_shape[3], const dou
 int launch_sample_count(int device, const int vol_shape[3], const double origin[3],
                         const int proj_shape[3], const double* views, double step,
                         long long* counts, hipStream_t stream);
-// Stage projections into the backprojector's quad layout (norm may be NULL).
-int launch_stage_quads(const void* proj, int dt, int nw, int nh, int nv, const float* norm,
-                       void* quad, hipStream_t stream);
 int launch_gather_bench_fp(int device, int dt, int plain, double* samples_per_s);
 int launch_gather_bench_bp(int device, int dt, int ray, double* samples_per_s);
 // Row filter (fc_filter.hip): out[r, j] = sum_m kern[j - m] wgt(r, m) in[r, m] over nrows rows

@@ -19,11 +19,12 @@
 // psi cot psi sin g), psi_m uniform on [-(pi/2 + am), pi/2 + am], am = largest |fan angle|.
 //
 // Layout: every stage is a dense [view][row][column] FP32 array in HBM (c2: 0.57 GB per stage,
-// 1.1 GB for the kappa-line stages); the backprojector reads g5 through the quad layout of
-// fc_backproject.hip. The Hilbert stage is the FFT row filter of fc_filter.hip (one convolution
+// 1.1 GB for the kappa-line stages); the backprojector reads g5 as pairs of a value and the step to
+// the next column's, with a border of zeros (kat_stage). The Hilbert stage is the FFT row filter of fc_filter.hip (one convolution
 // per kappa line), the other filter stages are elementwise gathers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "fc_device.h"
@@ -81,29 +82,30 @@ __global__ __launch_bounds__(256) void kat_derivative(const void* __restrict__ p
 
 // Tables: fwd[m][j] = detector row coordinate of kappa line m at column j;
 // bwd[i][j] = (m + t) with w_k(g_j, psi_m..m+1) bracketing row i's height, or -1 outside.
-__global__ __launch_bounds__(256) void kat_tables(KatGeom g, float* __restrict__ fwd,
-                                                  float* __restrict__ bwd) {
-  int j = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(64) void kat_tables(KatGeom g, float* __restrict__ fwd,
+                                                 float* __restrict__ bwd) {
+  const int j = blockIdx.y * 64 + threadIdx.x;
   if (j >= g.nw) return;
   const double gam = ((double)j - g.col_c) * g.dg;
-  for (int m = 0; m < g.npsi; ++m)
+  const int m = blockIdx.x;
+  if (m < g.npsi) {
     fwd[(size_t)m * g.nw + j] = (float)(kappa_w(g, gam, -g.pmax + m * g.dpsi) / g.drow + g.row_c);
-  const double wlo = kappa_w(g, gam, -g.pmax), whi = kappa_w(g, gam, g.pmax);
-  for (int i = 0; i < g.nh; ++i) {
-    double w = ((double)i - g.row_c) * g.drow;
-    float r = -1.0f;
-    if (w >= wlo && w <= whi) {
-      int lo = 0, hi = g.npsi - 1;  // w_k is increasing in psi for every detector column
-      while (hi - lo > 1) {
-        int mid = (lo + hi) / 2;
-        if (kappa_w(g, gam, -g.pmax + mid * g.dpsi) <= w) lo = mid; else hi = mid;
-      }
-      double wl = kappa_w(g, gam, -g.pmax + lo * g.dpsi);
-      double wh = kappa_w(g, gam, -g.pmax + hi * g.dpsi);
-      r = (float)((double)lo + (w - wl) / (wh - wl));
-    }
-    bwd[(size_t)i * g.nw + j] = r;
+    return;
   }
+  const int i = m - g.npsi;
+  const double w = ((double)i - g.row_c) * g.drow;
+  float r = -1.0f;
+  if (w >= kappa_w(g, gam, -g.pmax) && w <= kappa_w(g, gam, g.pmax)) {
+    int lo = 0, hi = g.npsi - 1;  // w_k is increasing in psi for every detector column
+    while (hi - lo > 1) {
+      int mid = (lo + hi) / 2;
+      if (kappa_w(g, gam, -g.pmax + mid * g.dpsi) <= w) lo = mid; else hi = mid;
+    }
+    double wl = kappa_w(g, gam, -g.pmax + lo * g.dpsi);
+    double wh = kappa_w(g, gam, -g.pmax + hi * g.dpsi);
+    r = (float)((double)lo + (w - wl) / (wh - wl));
+  }
+  bwd[(size_t)i * g.nw + j] = r;
 }
 
 // g3[k][m][j] = g2[k][row(m, j)][j], linear in the row, zero outside.
@@ -127,37 +129,69 @@ __global__ __launch_bounds__(256) void kat_forward_rebin(const float* __restrict
 // h[n] = 2/(pi n) * n dg / sin(n dg), is the FFT row filter's FC_FILTER_HILBERT kernel.
 constexpr int kMaxCols = 2048;  // detector columns (FFT length <= 4096 in the Hilbert stage)
 
-// g5[k][i][j] = g4 interpolated between kappa lines bracketing row i at column j.
-__global__ __launch_bounds__(256) void kat_backward_rebin(const float* __restrict__ g4, KatGeom g,
-                                                          const float* __restrict__ bwd,
-                                                          float* __restrict__ g5) {
-  int j = blockIdx.x * 256 + threadIdx.x;
-  int i = blockIdx.y, k = blockIdx.z;
-  if (j >= g.nw) return;
-  float r = bwd[(size_t)i * g.nw + j];
-  float v = 0.0f;
-  if (r >= 0.0f) {
-    int m0 = min((int)r, g.npsi - 2);
-    float t = r - (float)m0;
-    const float* col = g4 + (size_t)k * g.npsi * g.nw + j;
-    v = (1.0f - t) * col[(size_t)m0 * g.nw] + t * col[(size_t)(m0 + 1) * g.nw];
+// g5[k][i][j] = g4 interpolated between the kappa lines bracketing row i at column j, staged for the
+// backprojection: element (r, c) of a view is the pixel p = g5(r - 1, c - 1) and the step to the next
+// column's, (p, g5(r - 1, c) - p); pixels off the detector are zero. A wave owns 63 columns and
+// kStageRows rows: a lane interpolates its own column's pixel and takes the next column's from its
+// neighbour. g5 itself is written only if the caller wants it.
+// Bound by memory (2.3 GB read and written for 4320 views of 64 x 512): 0.7 ms; the interpolation and
+// the staging of 16-byte quads in kernels of their own took 0.4 and 1.1 ms.
+constexpr int kStageRows = 22;
+__host__ __device__ constexpr int stage_pitch(int nw) { return (nw + 3) & ~1; }  // 16-byte rows
+__global__ __launch_bounds__(256) void kat_stage(const float* __restrict__ g4, KatGeom g,
+                                                 const float* __restrict__ bwd,
+                                                 float2* __restrict__ pairs,
+                                                 float* __restrict__ g5) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int pitch = stage_pitch(g.nw), rows = g.nh + 3;
+  const int c = (blockIdx.x * 4 + wave) * 63 + lane, j = c - 1;  // element and pixel column
+  const int ra = blockIdx.y * kStageRows, rb = min(ra + kStageRows, rows), k = blockIdx.z;
+  const bool col = j >= 0 && j < g.nw;
+  const float* line = g4 + (size_t)k * g.npsi * g.nw + j;
+  for (int r = ra; r < rb; ++r) {
+    const int i = r - 1;
+    float p = 0.0f;
+    if (col && i >= 0 && i < g.nh) {
+      const float b = bwd[(size_t)i * g.nw + j];
+      if (b >= 0.0f) {
+        const int m0 = min((int)b, g.npsi - 2);
+        const float t = b - (float)m0;
+        p = (1.0f - t) * line[(size_t)m0 * g.nw] + t * line[(size_t)(m0 + 1) * g.nw];
+      }
+      if (g5 && lane < 63) g5[((size_t)k * g.nh + i) * g.nw + j] = p;
+    }
+    const float d = __shfl_down(p, 1, 64) - p;
+    if (lane < 63 && c < pitch) pairs[((size_t)k * rows + r) * pitch + c] = make_float2(p, d);
   }
-  g5[((size_t)k * g.nh + i) * g.nw + j] = v;
 }
 
-// PI-window backprojection. One thread per column (x, y) and kZR consecutive z voxels; per view
-// and column: v* = R - x cos l - y sin l, g* = atan(u* / v*), the column coordinate and the
-// Tam-Danielsson row bounds; per voxel: the row (linear in z), the window test, one quad gather.
-// Each block visits only the views whose source height can see its z range through the window.
-constexpr int kZR = 16;
+// PI-window backprojection. A block owns 16 x 16 columns (8 x 8 per wave, a thread per column) and
+// SLABS * kZR consecutive z; per view and column: v* = R - x cos l - y sin l, g* = atan(u* / v*), the
+// column coordinate and the Tam-Danielsson row bounds; per voxel: the row (linear in z), the window
+// test, one bilinear sample. Views go by in chunks of kViews: a thread per view bounds what the
+// block's columns need of it (KatEntry) and the views that no voxel sees through its window drop out;
+// the others' detector windows are copied to LDS one view ahead.
+constexpr int kZR = 8;
+constexpr int kViews = 128;
+constexpr int kWinW = 40;                 // window columns
+constexpr uint32_t kWinB = kWinW * 8;     // bytes per window row: 16 banks on from the row above
+constexpr int win_rows(int slabs) { return 6 + 10 * slabs; }
 struct KatBpArgs {
   float* vol;
-  const float4* quad;    // g5 staged as bilinear quads, (nh+2) x (nw+2) per view
+  const float2* pairs;   // staged g5: (nh + 3) x stage_pitch(nw) per view
   const float4* vtab;    // per view: cos l, sin l, source z, 0
   KatGeom g;
   float ox, oy, oz;
   int nx, ny, nz;
   double zmax;  // largest |z - zs| a voxel can have inside the window (voxels)
+};
+// A view as a block sees it: every sample's column coordinate lies in [ulo, uhi] and its row in
+// [vlo, vhi]; those of the detector elements from (row, col) on, `units` 16-byte units long.
+struct KatEntry {
+  float cosl, sinl, zs;
+  int k;
+  float ulo, uhi, vlo, vhi;
+  int row, col, units, lds;  // lds: the window fits the LDS buffers
 };
 
 __global__ __launch_bounds__(256) void kat_view_table(KatGeom g, float4* __restrict__ vt) {
@@ -167,64 +201,240 @@ __global__ __launch_bounds__(256) void kat_view_table(KatGeom g, float4* __restr
   vt[k] = make_float4((float)cos(l), (float)sin(l), (float)(g.zs0 + k * g.dl * g.hp), 0.0f);
 }
 
-__global__ __launch_bounds__(256) void kat_bp_kernel(KatBpArgs a) {
+// 1 / b, a / b and the square root of x, correctly rounded like the operators, in 3, 3 more and 8
+// instructions (the operators' 10, 10 and 14 also scale against overflow and underflow of their
+// intermediate values, which no volume and helix of finite voxel coordinates gets near).
+__device__ __forceinline__ float recip(float b) {
+  const float y = __builtin_amdgcn_rcpf(b);
+  return fmaf(fmaf(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float quotient(float a, float b, float recip_b) {
+  const float q = a * recip_b;
+  return fmaf(fmaf(-b, q, a), recip_b, q);
+}
+__device__ __forceinline__ float square_root(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  float s = x * y, h = 0.5f * y;
+  const float r = fmaf(-h, s, 0.5f);
+  s = fmaf(s, r, s);
+  h = fmaf(h, r, h);
+  return fmaf(fmaf(-s, s, x), h, s);
+}
+__device__ __forceinline__ int floor_int(float x) {
+  int i;
+  asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(i) : "v"(x));
+  return i;
+}
+
+// Bounds of what the columns within `rad` of (X, Y), z in [z0, z1], need of view k; false if none of
+// their voxels projects into its window. Margins of 0.05 element (and 1e-5 of the row) cover the
+// rounding of this bound and of the samples' own coordinates.
+__device__ __forceinline__ bool kat_entry(const KatBpArgs& a, int k, float X, float Y, float rad,
+                                          float z0, float z1, int max_rows, KatEntry& e) {
   const KatGeom& g = a.g;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int x = blockIdx.x * 16 + (wave & 1) * 8 + (lane & 7);
-  const int y = blockIdx.y * 16 + (wave >> 1) * 8 + (lane >> 3);
-  const int z0 = blockIdx.z * kZR;
-  const float X = (float)x + a.ox, Y = (float)y + a.oy, Z0 = (float)z0 + a.oz;
-  // views whose source height lies within zmax of the block's z range (block-uniform)
-  const double dz = g.hp * g.dl;
-  int klo = (int)floor(((double)z0 + a.oz - a.zmax - g.zs0) / dz) - 1;
-  int khi = (int)ceil(((double)z0 + a.oz + kZR - 1 + a.zmax - g.zs0) / dz) + 1;
-  klo = max(klo, 0);
-  khi = min(khi, g.nv - 1);
-  const int QW = g.nw + 2, QH = g.nh + 2;
-  const float wmax = (float)g.nw, hmax = (float)g.nh;
+  const float4 vt = a.vtab[k];
+  e.cosl = vt.x, e.sinl = vt.y, e.zs = vt.z, e.k = k;
+  const float vs = (float)g.R - X * vt.x - Y * vt.y, us = Y * vt.x - X * vt.y;
+  const float dist = sqrtf(vs * vs + us * us), dg = (float)g.dg;
+  e.ulo = -1.0f, e.uhi = (float)g.nw, e.vlo = -1.0f, e.vhi = (float)g.nh;
+  e.row = e.col = e.units = e.lds = 0;
+  if (!(dist > 1.05f * rad)) return true;  // next to the source: no bound
+  const float gam = atan2f(us, vs), half = rad / sqrtf((dist - rad) * (dist + rad));  // >= asin
+  const float ga = gam - half, gb = gam + half;
+  // (pi/2 - g) / cos g falls with g: the window's ends are largest at the tile's ends
+  const float sd = (float)(g.SDD / g.drow), ch = (float)(g.SDD * g.hp / g.R / g.drow);
+  const float rowc = (float)g.row_c, hpi = 1.57079632679489662f;
+  float lo = z0 - vt.z, hi = z1 - vt.z;
+  lo = sd * lo / (lo < 0.0f ? dist - rad : dist + rad);
+  hi = sd * hi / (hi > 0.0f ? dist - rad : dist + rad);
+  if (ga > -1.5f) hi = fminf(hi, ch * (hpi - ga) / cosf(fminf(ga, 1.5f)));
+  if (gb < 1.5f) lo = fmaxf(lo, -ch * (hpi + gb) / cosf(fmaxf(gb, -1.5f)));
+  lo -= 0.05f + 1e-5f * fabsf(lo), hi += 0.05f + 1e-5f * fabsf(hi);
+  if (lo > hi) return false;
+  e.vlo = fminf(fmaxf(lo + rowc, -1.0f), e.vhi);
+  e.vhi = fminf(fmaxf(hi + rowc, -1.0f), e.vhi);
+  const float cc = (float)g.col_c;
+  e.ulo = fminf(fmaxf(ga / dg + cc - 0.05f, -1.0f), e.uhi);
+  e.uhi = fminf(fmaxf(gb / dg + cc + 0.05f, -1.0f), e.uhi);
+  e.row = (int)floorf(e.vlo) + 1;
+  e.col = ((int)floorf(e.ulo) + 1) & ~1;
+  const int rows = (int)floorf(e.vhi) + 3 - e.row;
+  e.lds = rows <= max_rows && (int)floorf(e.uhi) + 1 - e.col < kWinW;
+  e.units = rows * (kWinW / 2);
+  return true;
+}
+
+// kZR voxels of a column at rows rr = (q + qa) dr + r0: acc[q] += wgt * sample if rbot <= rr <= rtop. The
+// sample is bilinear between the elements at `at` + row * pitch and the next row's, `at` standing for
+// row 0 of the column, an LDS or a global address. [lo, hi] is the window within the copied rows;
+// INSIDE: all rows of all lanes are inside it.
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(3))) f2* lds_f2;
+template <bool LDS, class P>
+__device__ __forceinline__ void kat_samples(float* acc, P at, uint32_t pitch, float au, float dr,
+                                            float r0, int qa, float lo, float hi, float wgt) {
+  constexpr int B = LDS ? 4 : 1;  // samples in flight; the rare global path gets no registers
+#pragma unroll
+  for (int q0 = 0; q0 < kZR; q0 += B) {
+    f2 p[B], n[B];
+    float av[B], w[B];
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const float rr = fmaf((float)(qa + q0 + q), dr, r0);
+      const float v = __builtin_amdgcn_fmed3f(rr, lo, hi);
+      w[q] = v == rr ? wgt : 0.0f;
+      av[q] = __builtin_amdgcn_fractf(v);
+      const int row = floor_int(v);
+      if constexpr (LDS) {
+        const lds_f2 src = (lds_f2)(size_t)mad_i24(row, (int)kWinB, at);
+        p[q] = src[0], n[q] = src[kWinW];
+      } else {
+        const char* src = at + (long long)row * pitch;
+        p[q] = *reinterpret_cast<const f2*>(src), n[q] = *reinterpret_cast<const f2*>(src + pitch);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < B; ++q) {
+      const float top = fmaf(au, p[q].y, p[q].x), bot = fmaf(au, n[q].y, n[q].x);
+      acc[q0 + q] = fmaf(w[q], lerp(top, bot, av[q]), acc[q0 + q]);
+    }
+  }
+}
+
+// Bound by VALU issue: about 65 instructions per view and column (division, atan, square root) and
+// 12.5 per sample, of which the helix's geometry makes a fifth miss their own window in a group of
+// eight; the LDS reads (16 bytes per sample, without conflicts) take half of that time. 512 x 512 x
+// 256 voxels, 4320 views of 64 x 512: 15.2 ms against 38.9 ms for gathering 16-byte quads of every
+// visited view from global memory (20 L1 accesses per wave and sample: L1-bound at best, 21.6 ms, once
+// the views outside the window were skipped).
+template <int SLABS>
+__global__ __launch_bounds__(256, 4) void kat_bp_kernel(KatBpArgs a) {
+  constexpr int NZ = SLABS * kZR, ROWS = win_rows(SLABS), SLOTS = (ROWS * kWinW / 2 + 255) / 256;
+  __shared__ float4 win[2][ROWS * kWinW / 2];
+  __shared__ KatEntry table[kViews];
+  __shared__ int count[kViews / 64];
+  const KatGeom& g = a.g;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // columns beyond the volume repeat its last ones
+  const int xb = blockIdx.x * 16, yb = blockIdx.y * 16;
+  const int x = xb + (wave & 1) * 8 + (lane & 7), y = yb + (wave >> 1) * 8 + (lane >> 3);
+  const float X = (float)min(x, a.nx - 1) + a.ox, Y = (float)min(y, a.ny - 1) + a.oy;
+  const float hx = 0.5f * (float)(min(xb + 15, a.nx - 1) - xb);
+  const float hy = 0.5f * (float)(min(yb + 15, a.ny - 1) - yb);
+  const float Xc = (float)xb + a.ox + hx, Yc = (float)yb + a.oy + hy;
+  const float rad = 1.001f * sqrtf(hx * hx + hy * hy) + 0.01f;
+  const int pitch = stage_pitch(g.nw);
+  const uint32_t pitchB = (uint32_t)pitch * 8u;
+  const size_t viewB = (size_t)(g.nh + 3) * pitchB;
+  const char* pairs = reinterpret_cast<const char*>(a.pairs);
+  const uint32_t win0 = (uint32_t)(size_t)(lds_f2)&win[0][0];
+  uint32_t off[SLOTS];  // bytes from the window's first element to this thread's units
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) {
+    const uint32_t unit = threadIdx.x + 256u * i;
+    off[i] = unit / (kWinW / 2) * pitchB + unit % (kWinW / 2) * 16u;
+  }
   const float Rf = (float)g.R, inv_dg = (float)(1.0 / g.dg), colc = (float)g.col_c;
-  const float rowc = (float)g.row_c, inv_drow = (float)(1.0 / g.drow);
+  const float rowc = (float)g.row_c;
   const float sdd_drow = (float)(g.SDD / g.drow);
   const float c0r = (float)(g.SDD * g.hp / g.R / g.drow);
   const float hpi = 1.57079632679489662f;
-  float acc[kZR];
+  const double dz = g.hp * g.dl;
+  for (int z0 = blockIdx.z * NZ; z0 < a.nz; z0 += gridDim.z * NZ) {
+    // views whose source height lies within zmax of the block's z range (block-uniform)
+    int klo = (int)floor(((double)z0 + a.oz - a.zmax - g.zs0) / dz) - 1;
+    int khi = (int)ceil(((double)z0 + a.oz + NZ - 1 + a.zmax - g.zs0) / dz) + 1;
+    klo = max(klo, 0);
+    khi = min(khi, g.nv - 1);
+    float acc[NZ];
 #pragma unroll
-  for (int q = 0; q < kZR; ++q) acc[q] = 0.0f;
-  (void)inv_drow;
-  for (int k = klo; k <= khi; ++k) {
-    const float4 vt = a.vtab[k];
-    const float vs = fmaf(-X, vt.x, fmaf(-Y, vt.y, Rf));  // R - x cos l - y sin l
-    const float us = fmaf(-X, vt.y, Y * vt.x);            // -x sin l + y cos l
-    const float t = us / vs;
-    const float gam = atanf(t);
-    const float sec = sqrtf(fmaf(t, t, 1.0f));              // 1 / cos g
-    // w* / drow = SDD (z - zs) cos g / (v* drow): the row is linear in the voxel index
-    const float dr = sdd_drow / (vs * sec);
-    const float r0 = fmaf(Z0 - vt.z, dr, rowc);
-    const float rtop = fmaf(c0r * (hpi - gam), sec, rowc);
-    const float rbot = fmaf(-c0r * (hpi + gam), sec, rowc);
-    const float wgt = 1.0f / vs;
-    const float u = fminf(fmaxf(fmaf(gam, inv_dg, colc), -1.0f), wmax);
-    const float fu = floorf(u), au = u - fu;
-    const uint32_t iu = (uint32_t)((int)fu + 1);
-    const float4* base = a.quad + (size_t)k * QW * QH;
+    for (int q = 0; q < NZ; ++q) acc[q] = 0.0f;
+    for (int kc = klo; kc <= khi; kc += kViews) {
+      __syncthreads();  // the previous chunk's table and windows are no longer read
+      KatEntry e;
+      bool used = false;
+      const int k = kc + (int)threadIdx.x;
+      if (threadIdx.x < kViews && k <= khi)
+        used = kat_entry(a, k, Xc, Yc, rad, (float)z0 + a.oz, (float)(z0 + NZ - 1) + a.oz, ROWS, e);
+      const unsigned long long mask = __ballot(used);
+      if (lane == 0 && wave < kViews / 64) count[wave] = __popcll(mask);
+      __syncthreads();
+      int first = 0, n = 0;
 #pragma unroll
-    for (int q = 0; q < kZR; ++q) {
-      const float rr = fmaf((float)q, dr, r0);
-      const float w = (rr >= rbot && rr <= rtop) ? wgt : 0.0f;
-      const float v = fminf(fmaxf(rr, -1.0f), hmax);
-      const float fv = floorf(v), av = v - fv;
-      const float4 p = base[(uint32_t)((int)fv + 1) * (uint32_t)QW + iu];
-      const float top = lerp(p.x, p.y, au), bot = lerp(p.z, p.w, au);
-      acc[q] = fmaf(w, lerp(top, bot, av), acc[q]);
+      for (int i = 0; i < kViews / 64; ++i) {
+        if (i < wave) first += count[i];
+        n += count[i];
+      }
+      if (used) table[first + __popcll(mask & ((1ull << lane) - 1))] = e;
+      __syncthreads();
+      n = __builtin_amdgcn_readfirstlane(n);
+      auto copy = [&](int i) {
+        const int units = __builtin_amdgcn_readfirstlane(table[i].lds ? table[i].units : 0);
+        const char* src = pairs + (size_t)__builtin_amdgcn_readfirstlane(table[i].k) * viewB +
+                          (size_t)__builtin_amdgcn_readfirstlane(table[i].row) * pitchB +
+                          (size_t)__builtin_amdgcn_readfirstlane(table[i].col) * 8u;
+        const uint32_t dst = win0 + (i & 1) * (uint32_t)sizeof(win[0]);
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+          if ((int)threadIdx.x + 256 * s < units)
+            copy_units_to_lds(src, off[s], dst + 16u * (256u * s + 64u * wave));
+      };
+      if (n > 0) copy(0);
+      for (int i = 0; i < n; ++i) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // view i is in LDS, and nobody reads view i - 1's buffer any more
+        if (i + 1 < n) copy(i + 1);
+        const KatEntry t = table[i];
+        const float vs = fmaf(-X, t.cosl, fmaf(-Y, t.sinl, Rf));  // R - x cos l - y sin l
+        const float us = fmaf(-X, t.sinl, Y * t.cosl);            // -x sin l + y cos l
+        const float wgt = recip(vs);
+        const float tg = quotient(us, vs, wgt);
+        const float gam = atanf(tg);
+        const float sec = square_root(fmaf(tg, tg, 1.0f));  // 1 / cos g
+        // w* / drow = SDD (z - zs) cos g / (v* drow): the row is linear in the voxel index
+        const float vsec = vs * sec, dr = quotient(sdd_drow, vsec, recip(vsec));
+        const float rtop = fmaf(c0r * (hpi - gam), sec, rowc);
+        const float rbot = fmaf(-c0r * (hpi + gam), sec, rowc);
+        const float u = __builtin_amdgcn_fmed3f(fmaf(gam, inv_dg, colc), t.ulo, t.uhi);
+        const float au = u - floorf(u);
+        const int iu = floor_int(u) + 1;
+        // the window within [vlo, vhi]: in-window rows lie strictly inside these
+        const float lo = __builtin_amdgcn_fmed3f(rbot, t.vlo, t.vhi);
+        const float hi = __builtin_amdgcn_fmed3f(rtop, t.vlo, t.vhi);
+        const uint32_t at = win0 + (i & 1) * (uint32_t)sizeof(win[0]) +
+                            (uint32_t)((iu - t.col) * 8 + (1 - t.row) * (int)kWinB);
+        // the rows of a slab count from the sixteenth voxel below it, whatever the slabs
+        auto row0 = [&](int zs, int& qa) {
+          qa = SLABS > 1 ? (zs - z0) & 15 : zs & 15;
+          return fmaf((float)(zs - qa) + a.oz - t.zs, dr, rowc);
+        };
+        int qa;
+        const bool big = !__builtin_amdgcn_readfirstlane(t.lds);
+#pragma unroll
+        for (int s = 0; s < SLABS; ++s) {
+          const float r0 = row0(z0 + s * kZR, qa);
+          const float ra = fmaf((float)qa, dr, r0), rb = fmaf((float)(qa + kZR - 1), dr, r0);
+          if (big || !__any(ra <= rtop && rb >= rbot)) continue;  // the rows rise with z
+          kat_samples<true>(acc + s * kZR, at, 0, au, dr, r0, qa, lo, hi, wgt);
+        }
+        if (big) {
+          const char* src = pairs + (size_t)t.k * viewB + pitchB + (size_t)(uint32_t)iu * 8u;
+#pragma unroll
+          for (int s = 0; s < SLABS; ++s) {
+            const float r0 = row0(z0 + s * kZR, qa);
+            kat_samples<false>(acc + s * kZR, src, pitchB, au, dr, r0, qa, lo, hi, wgt);
+          }
+        }
+      }
     }
-  }
-  if (x < a.nx && y < a.ny) {
-    const float s = (float)(g.dl / (2.0 * M_PI));
+    if (x < a.nx && y < a.ny) {
+      const float s = (float)(g.dl / (2.0 * M_PI));
 #pragma unroll
-    for (int q = 0; q < kZR; ++q) {
-      const int z = z0 + q;
-      if (z < a.nz) a.vol[((size_t)z * a.ny + y) * a.nx + x] += s * acc[q];
+      for (int q = 0; q < NZ; ++q) {
+        const int z = z0 + q;
+        if (z < a.nz) a.vol[((size_t)z * a.ny + y) * a.nx + x] += s * acc[q];
+      }
     }
   }
 }
@@ -289,7 +499,7 @@ extern "C" int fc_katsevich_dev(int device, const void* proj, int proj_dtype, in
 
   int tok = prof_begin("katsevich_filter", stream);
   const int bx = (nw + 255) / 256;
-  kat_tables<<<bx, 256, 0, stream>>>(g, fwd, bwd);
+  kat_tables<<<dim3(npsi + nh, (nw + 63) / 64), 64, 0, stream>>>(g, fwd, bwd);
   float* g2 = static_cast<float*>(A);
   if (proj_dtype == FC_F32) kat_derivative<FC_F32><<<dim3(bx, nh, nviews), 256, 0, stream>>>(proj, g, g2);
   else if (proj_dtype == FC_BF16) kat_derivative<FC_BF16><<<dim3(bx, nh, nviews), 256, 0, stream>>>(proj, g, g2);
@@ -301,22 +511,20 @@ extern "C" int fc_katsevich_dev(int device, const void* proj, int proj_dtype, in
   if ((rc = launch_row_filter(g3, FC_F32, g4, FC_F32, nw, npsi, (long long)npsi * nviews, nullptr,
                               FC_FILTER_HILBERT, dgamma, ftab, stream)))
     return rc;
-  float* g5 = static_cast<float*>(B);  // g3 is no longer needed
-  kat_backward_rebin<<<dim3(bx, nh, nviews), 256, 0, stream>>>(g4, g, bwd, g5);
+  // g5, staged in element pairs for the backprojection over the PI windows; its last window row may
+  // be copied kWinW elements beyond the end
+  FC_CHECK_ARG(nh + 2 <= 65535, "projection stack too large for the staging grid");
+  void* Q = nullptr;
+  const int pitch = stage_pitch(nw);
+  const size_t qbytes = ((size_t)pitch * (nh + 3) * nviews + kWinW) * sizeof(float2);
+  if ((rc = acquire_ws(device, SLOT_QUAD, qbytes, stream, &Q))) return rc;
+  kat_stage<<<dim3((pitch + 251) / 252, (nh + 3 + kStageRows - 1) / kStageRows, nviews), 256, 0,
+              stream>>>(g4, g, bwd, static_cast<float2*>(Q), g5_out);
   prof_end(tok, stream);
   FC_HIP(hipGetLastError());
-  if (g5_out)
-    FC_HIP(hipMemcpyAsync(g5_out, g5, (size_t)nviews * plane * sizeof(float),
-                          hipMemcpyDeviceToDevice, stream));
-
-  // stage g5 as quads and backproject over the PI windows
-  void* Q = nullptr;
-  const size_t qbytes = (size_t)(nw + 2) * (nh + 2) * nviews * 16;
-  if ((rc = acquire_ws(device, SLOT_QUAD, qbytes, stream, &Q))) return rc;
-  if ((rc = launch_stage_quads(g5, FC_F32, nw, nh, nviews, nullptr, Q, stream))) return rc;
   KatBpArgs a;
   a.vol = vol;
-  a.quad = static_cast<const float4*>(Q);
+  a.pairs = static_cast<const float2*>(Q);
   a.vtab = vtab;
   a.g = g;
   a.ox = (float)origin[0]; a.oy = (float)origin[1]; a.oz = (float)origin[2];
@@ -324,10 +532,18 @@ extern "C" int fc_katsevich_dev(int device, const void* proj, int proj_dtype, in
   a.nx = vol_shape[0]; a.ny = vol_shape[1]; a.nz = vol_shape[2];
   // |z - zs| <= (hp/R) (pi/2 + am) / cos^2(am) * v*,  v* <= R + rmax
   a.zmax = hp / R * (M_PI / 2 + am) / (cos(am) * cos(am)) * (R + rmax) + 2.0 * drow;
-  dim3 grid((a.nx + 15) / 16, (a.ny + 15) / 16, (a.nz + kZR - 1) / kZR);
-  FC_CHECK_ARG(grid.y <= 65535 && grid.z <= 65535, "volume too large for the grid");
+  FC_CHECK_ARG((a.ny + 15) / 16 <= 65535 && (a.nz + 15) / 16 <= 65535,
+               "volume too large for the grid");
+  const auto slabs = [&](int n) { return (a.nz + n * kZR - 1) / (n * kZR); };
+  dim3 grid((a.nx + 15) / 16, (a.ny + 15) / 16, slabs(4));
+  // Four slabs per block share a view's bounds and per-column terms; one slab gives four times the
+  // blocks, each with fewer views. The line lies where four still fill the chip (4 against 1, ms:
+  // 20 blocks 1.03 / 0.43, 144: 1.59 / 0.87, 544: 4.00 / 3.81, 816: 2.42 / 2.60, 1800: 7.0 / 7.8).
+  const bool tall = (size_t)grid.x * grid.y * grid.z >= 768;
+  if (!tall) grid.z = std::min(slabs(1), 65535);
   tok = prof_begin("katsevich_bp", stream);
-  kat_bp_kernel<<<grid, 256, 0, stream>>>(a);
+  if (tall) kat_bp_kernel<4><<<grid, 256, 0, stream>>>(a);
+  else kat_bp_kernel<1><<<grid, 256, 0, stream>>>(a);
   prof_end(tok, stream);
   FC_HIP(hipGetLastError());
   if ((rc = release_ws(device, SLOT_QUAD, stream))) return rc;

@@ -140,3 +140,53 @@ def test_katsevich_parity(gpu):
     assert e_f < 1e-4
     assert e_v < 1e-3
     assert e_p < 0.01
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nw,nh,dg,drow,nz,ny,nx,origin,vpt", [
+    (96, 32, 0.0052, 1.0, 9, 17, 33, (-16.0, -8.0, -4.0), 90),     # ragged tiles and slabs
+    (96, 12, 0.0052, 1.0, 16, 32, 32, (-16.0, -16.0, -8.0), 90),   # detector shorter than the window
+    (40, 32, 0.0052, 1.0, 8, 40, 40, (-20.0, -20.0, -4.0), 90),    # columns off the detector
+    (480, 160, 0.00104, 0.2, 12, 20, 20, (-10.0, -10.0, -6.0), 60),  # windows too large for the LDS
+    (96, 32, 0.0052, 1.0, 20, 16, 16, (74.0, -8.0, -10.0), 90),    # close to the source path
+    (64, 24, 0.008, 2.0, 318, 138, 139, (-69.0, -69.0, -159.0), 24),  # four slabs per block
+])
+def test_katsevich_backprojector_branches(gpu, nw, nh, dg, drow, nz, ny, nx, origin, vpt):
+    """Every branch of the backprojector against the oracle, on smooth data (a random field over
+    about eight views, rows and columns). A view that a voxel meets exactly at its window's edge (by
+    symmetry: voxels on the axis, with a view at a quarter turn) counts or not by rounding, in FP64 as
+    in FP32: voxels that differ by more than 1e-4 of the largest value must be such (next to the
+    source FP32 coordinates are good to 3 * 2^-24 R, that is 4e-4 of a row or 1e-4 of these data's
+    amplitude at one voxel's distance), every other agrees within the filtered data's tolerance of
+    test_katsevich_parity."""
+    import torch
+    from fastcone_amd.katsevich import HelixScan, katsevich
+    hp = 0.8 * nh * drow * R / SDD / (2 * math.pi)
+    lam = 2 * math.pi * np.arange(2 * vpt) / vpt
+    hx = oracle.Helix(lam, hp * (lam - lam.mean()), R, SDD, dg, drow, nw, nh, hp)
+    rng = np.random.default_rng(nw + nh)
+    k, i, j = np.meshgrid(np.arange(hx.n), np.arange(nh), np.arange(nw), indexing="ij")
+    proj = sum(rng.normal() * np.cos(0.1 * rng.normal() * k + 6.0 / nh * rng.normal() * i
+                                     + 9.0 / nw * rng.normal() * j) for _ in range(4))
+    scan = HelixScan(hx.n, hx.dl, hx.lambdas[0], hx.zs[0], hp, R, SDD, dg, drow, nw, nh)
+    rec, g5 = katsevich(torch.from_numpy(proj.astype(np.float32)).to(gpu), scan, (nz, ny, nx),
+                        origin=origin, return_filtered=True)
+    rec = rec.cpu().numpy().astype(np.float64)
+    ref, g5_ref = oracle.katsevich(hx, proj, (nz, ny, nx), np.array(origin), return_g5=True)
+    assert _rel(g5.cpu().numpy(), g5_ref) < 1e-4
+    off = np.abs(rec - ref) > 1e-4 * np.abs(ref).max()
+    assert np.linalg.norm((rec - ref)[~off]) < 1e-4 * np.linalg.norm(ref)
+    assert off.sum() < 20
+    for z, y, x in np.argwhere(off):
+        px, py, pz = x + origin[0], y + origin[1], z + origin[2]
+        v = R - px * np.cos(hx.lambdas) - py * np.sin(hx.lambdas)
+        u = py * np.cos(hx.lambdas) - px * np.sin(hx.lambdas)
+        gam = np.arctan2(u, v)
+        dist = np.hypot(u, v)
+        row = SDD * (pz - hx.zs) / dist / drow
+        edge = SDD * hp / R / drow / np.cos(gam) * np.stack([math.pi / 2 - gam, -math.pi / 2 - gam])
+        # FP32 coordinates relative to the source are good to about three roundings of R
+        rel = 1e-6 + 3 * 2.0**-24 * R / dist
+        tol = rel * (np.abs(row) + np.abs(edge) * (1 + np.abs(np.tan(gam)))
+                     + SDD * hp / R / drow / np.cos(gam))
+        assert (np.abs(row - edge) < tol).any()
