@@ -44,8 +44,8 @@ int select_device(int device);
 // A call that uses a workspace on a stream other than the one its previous user ran on first
 // makes the new stream wait on an event recorded after that previous use, so reuse is ordered.
 enum Slot { SLOT_OCTET = 0, SLOT_QUAD = 1, SLOT_H2D_VOL = 2, SLOT_H2D_PROJ = 3,
-            SLOT_H2D_VIEWS = 4, SLOT_H2D_NORM = 5, SLOT_KAT_A = 6, SLOT_KAT_B = 7,
-            SLOT_KAT_TAB = 8, SLOT_FILTER = 9, SLOT_COUNT = 10 };
+            SLOT_H2D_VIEWS = 4, SLOT_H2D_NORM = 5, SLOT_KAT = 6, SLOT_KAT_TAB = 7,
+            SLOT_FILTER = 8, SLOT_COUNT = 9 };
 
 struct Workspace {
   void* ptr = nullptr;
