@@ -81,8 +81,9 @@ __global__ __launch_bounds__(256) void stage_octets(const void* __restrict__ vol
 template <int DT_IN>
 __global__ __launch_bounds__(256) void stage_plain(const void* __restrict__ vol, int nx, int ny,
                                                    int nz, float* __restrict__ out, int PX,
-                                                   int PY) {
+                                                   int PY, unsigned long long* total) {
   int px = blockIdx.x * 256 + threadIdx.x;
+  if (total && px < 2 && blockIdx.y == 0 && blockIdx.z == 0) total[px] = 0ull;
   int py = blockIdx.y, pz = blockIdx.z;
   if (px >= PX) return;
   int x = px - 2, y = py - 2, z = pz - 2;
@@ -95,8 +96,9 @@ __global__ __launch_bounds__(256) void stage_plain(const void* __restrict__ vol,
 template <int DT_IN>
 __global__ __launch_bounds__(256) void stage_plain16(const void* __restrict__ vol, int nx, int ny,
                                                      int nz, uint16_t* __restrict__ out, int PX,
-                                                     int PY) {
+                                                     int PY, unsigned long long* total) {
   int px = blockIdx.x * 256 + threadIdx.x;
+  if (total && px < 2 && blockIdx.y == 0 && blockIdx.z == 0) total[px] = 0ull;
   int py = blockIdx.y, pz = blockIdx.z;
   if (px >= PX) return;
   int x = px - 2, y = py - 2, z = pz - 2;
@@ -252,11 +254,10 @@ __global__ __launch_bounds__(256) void fp_kernel(FpArgs a) {
 // quarters, which costs 30 % fewer brick elements per ray sample than a brick per quarter. When
 // the views are far apart (sparse angular sampling) the union is wide, and the quad is left to
 // fp_lds_kernel, where each 256-thread block takes the whole 16x16 tile of one view (6 waves per
-// SIMD, 24 KiB bricks). fp_quad_kernel decides per quad from the brick elements of both layouts
-// summed over every fourth slab (a brick over its budget counting 4x; a quad whose grid rays do
-// not all advance along the dominant axis always goes to fp_lds_kernel) and records the decision
-// in a byte per
-// quad that fp_lds_kernel, launched next on the same stream, reads.
+// SIMD, 24 KiB bricks). fp_decide chooses for the whole call from the brick elements of both layouts
+// (a brick over its budget counting 4x). A quad whose grid rays do not all advance along the
+// dominant axis always goes to fp_lds_kernel: fp_quad_kernel records that in a byte per quad that
+// fp_lds_kernel, launched next on the same stream, reads.
 // Bricks larger than the LDS budget (or tiles whose rays do not all advance along the dominant
 // axis) fall back to gathering from the staged volume in global memory, with the same arithmetic.
 
@@ -738,18 +739,78 @@ __device__ __forceinline__ float march(const FpArgs& a, float* brick, int4* tab,
   return acc;
 }
 
-// Shared-mode quads. Blocks (quad, half) decide the mode and record it; single-mode quads are
-// left to fp_lds_kernel. `mode` = 0: cost decision, 1: always shared. Launched with half as many
+// The work layout of a whole call, decided once from a sample of its quads: brick elements of both
+// layouts summed over every fourth slab of kSamples quads (pseudo-random ones, a wave each), into
+// total[0] (shared) and total[1] (single), cleared by the staging kernel.
+constexpr int kSamples = 256;
+template <int S>
+__global__ __launch_bounds__(64) void fp_decide(FpArgs a, unsigned long long* __restrict__ total) {
+  constexpr int DP = S + 3;
+  __shared__ QuadGrid G;
+  const unsigned nq = (unsigned)((a.nviews + kQuad - 1) / kQuad), n = nq * a.tiles_per_view;
+  const unsigned pick = n <= kSamples ? blockIdx.x : (blockIdx.x * 2654435761u) % n;
+  const int t0 = (int)(pick / a.tiles_per_view) * kQuad, tile = (int)(pick % a.tiles_per_view);
+  const int j0 = tile % a.tiles_w * kTile, i0 = tile / a.tiles_w * kTile;
+  const int cap_shared = a.lds_cap >= kLdsCap ? kHalfCap : a.lds_cap;
+  const SlabAxes X = slab_axes<S>(a, a.views + (size_t)t0 * FC_VIEW_DOUBLES, j0, i0);
+  const int v = threadIdx.x >> 4, p = threadIdx.x & 15, cj = p & 3, ci = p >> 2;
+  const bool ok = grid_ray(G, a, X, a.views + (size_t)min(t0 + v, a.nviews - 1) * FC_VIEW_DOUBLES, v,
+                           p, (double)min(j0 + (cj >> 1) * 8 + (cj & 1) * 7, a.nw - 1),
+                           (double)min(i0 + (ci >> 1) * 8 + (ci & 1) * 7, a.nh - 1));
+  if (!__all(ok)) return;  // goes to fp_lds_kernel in any case
+  __syncthreads();
+  // items (kind, slab), kind 0-1: the two halves over all four views, 2-5: each view's whole
+  // tile, over every fourth slab (brick sizes change slowly from slab to slab); consecutive
+  // lanes take consecutive slabs of one kind; a brick over its budget counts 4x
+  unsigned long long csh = 0ull, csi = 0ull;
+  const int nsub = (X.nslabs + 3) / 4;
+  for (int w = threadIdx.x; w < 6 * nsub; w += 64) {
+    const int kind = w / nsub, m = 4 * (w - kind * nsub);
+    if (kind >= 2 && t0 + kind - 2 >= a.nviews) continue;  // a missing view of the last quad
+    const int4 B = kind < 2 ? slab_box<S>(G, X, 0, kQuad, 0, kind * 2, 2, 0, m)
+                            : slab_box<S>(G, X, kind - 2, 1, 0, 0, 2, 2, m);
+    if (B.z > 0 && B.w > 0) {
+      const unsigned long long ne = brick_elems(DP, (uint32_t)B.z, (uint32_t)B.w);
+      const int cap = kind < 2 ? cap_shared : a.lds_cap;
+      const unsigned long long c = ne > (unsigned long long)cap ? 4ull * ne : ne;
+      if (kind < 2) csh += c; else csi += c;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    csh += __shfl_xor(csh, off);
+    csi += __shfl_xor(csi, off);
+  }
+  if (threadIdx.x == 0) {
+    atomicAdd(total, csh);
+    atomicAdd(total + 1, csi);
+  }
+}
+
+// Shared mode for the call (`total` null: forced). The line lies at 0.65 of single mode's elements:
+// shared / single mode (ms) at ratio 0.42 6.85 / 8.34 (bf16, 181 views of 301 x 250 x 203), 0.44 8.2 /
+// 9.5 (180 of 256^3), 0.57 19.0 / 23.1 (160 of 384^3), 0.61 3.33 / 3.47 (90 of 256^3, whole steps),
+// 0.63 25.2 / 28.5 (144 of 384^3), 0.70 0.52 / 0.33 (40 of 128^3), 0.74 30.4 / 24.6 (120 of 384^3),
+// 1.1 105 / 61 (120 of 512^3): beyond it the shared bricks stop fitting the LDS as pairs, then at all.
+// One decision for the call, not one per quad: a call that mixes the modes runs two kernels of which
+// each leaves part of the XCDs idle (90 views of 512^3 53 ms mixed, 45 single; 181 bf16 views as above
+// 8.35 mixed, 6.97 shared).
+__device__ __forceinline__ bool shared_layout(const unsigned long long* total) {
+  return !total || 20ull * total[0] <= 13ull * total[1];
+}
+
+// Shared-mode quads. Blocks (quad, half) record whether they take their quad; the others are
+// left to fp_lds_kernel. Launched with half as many
 // blocks as fp_lds_kernel: block b covers "virtual view" 2 q + h (quad q, half h), so the tile
 // order of fp_tile_origin (groups, XCD dealing) applies with half the group size.
 template <int DT, int S>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(8, 8)))
-void fp_quad_kernel(FpArgs a, uint8_t* __restrict__ quad_mode, int mode) {
-  constexpr int DP = S + 3;
+void fp_quad_kernel(FpArgs a, uint8_t* __restrict__ quad_mode,
+                    const unsigned long long* __restrict__ total) {
   __shared__ float brick[kHalfCap];
   __shared__ int4 tab[kSlabTab];
   __shared__ QuadGrid G;
-  __shared__ unsigned long long cost[2];
+  if (!shared_layout(total)) return;
   const int nvq = (a.nviews + kQuad - 1) / kQuad * kQuad;
   int tv, j0, i0;
   fp_tile_origin(a.tiles_w, a.tiles_per_view, a.group / 2, nvq / 2, &tv, &j0, &i0);
@@ -768,45 +829,11 @@ void fp_quad_kernel(FpArgs a, uint8_t* __restrict__ quad_mode, int mode) {
                     (double)min(j0 + (cj >> 1) * 8 + (cj & 1) * 7, a.nw - 1),
                     (double)min(i0 + (ci >> 1) * 8 + (ci & 1) * 7, a.nh - 1));
   }
-  if (threadIdx.x < 2) cost[threadIdx.x] = 0ull;
-  const bool quad_bad = __syncthreads_or(bad);
-  // items (kind, slab), kind 0-1: the two halves over all four views, 2-5: each view's whole
-  // tile, over every fourth slab (brick sizes change slowly from slab to slab); consecutive
-  // lanes take consecutive slabs of one kind; a brick over its budget counts 4x. Sums stay in
-  // registers and are reduced across the wave, so each wave adds once to each LDS total.
-  if (!quad_bad && mode == 0) {
-    unsigned long long csh = 0ull, csi = 0ull;
-    const int nsub = (X.nslabs + 3) / 4;
-    for (int w = threadIdx.x; w < 6 * nsub; w += 512) {
-      const int kind = w / nsub, m = 4 * (w - kind * nsub);
-      if (kind >= 2 && t0 + kind - 2 >= a.nviews) continue;  // a missing view of the last quad
-      const int4 B = kind < 2 ? slab_box<S>(G, X, 0, kQuad, 0, kind * 2, 2, 0, m)
-                              : slab_box<S>(G, X, kind - 2, 1, 0, 0, 2, 2, m);
-      if (B.z > 0 && B.w > 0) {
-        const unsigned long long ne = brick_elems(DP, (uint32_t)B.z, (uint32_t)B.w);
-        const int cap = kind < 2 ? cap_shared : a.lds_cap;
-        const unsigned long long c = ne > (unsigned long long)cap ? 4ull * ne : ne;
-        if (kind < 2) csh += c; else csi += c;
-      }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      csh += __shfl_xor(csh, off);
-      csi += __shfl_xor(csi, off);
-    }
-    if (lane == 0) {
-      atomicAdd(&cost[0], csh);
-      atomicAdd(&cost[1], csi);
-    }
-  }
-  __syncthreads();
   // A quad whose grid rays do not all advance along the dominant axis goes to fp_lds_kernel,
-  // which checks each view's tile on its own. The last quad of a view count that is not a
-  // multiple of four is decided like the others (its missing views' waves idle in shared mode;
-  // left to fp_lds_kernel, whose block order keeps one view group on one XCD, its tiles would
-  // run on one eighth of the GPU after this kernel). Both halves' blocks evaluate the same
-  // decision from the same inputs.
-  const bool shared = mode == 1 || (!quad_bad && cost[0] <= cost[1]);
+  // which checks each view's tile on its own (unless shared mode is forced). Both halves' blocks
+  // find the same from the same inputs.
+  const bool quad_bad = __syncthreads_or(bad);
+  const bool shared = !total || !quad_bad;
   const int tile = (i0 / kTile) * a.tiles_w + j0 / kTile;
   if (half == 0 && threadIdx.x == 0)
     quad_mode[(size_t)(t0 / kQuad) * a.tiles_per_view + tile] = shared ? kQuadShared : 0;
@@ -838,14 +865,15 @@ void fp_quad_kernel(FpArgs a, uint8_t* __restrict__ quad_mode, int mode) {
 // view tg.
 template <int DT, int S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8)))
-void fp_lds_kernel(FpArgs a, const uint8_t* __restrict__ quad_mode) {
+void fp_lds_kernel(FpArgs a, const uint8_t* __restrict__ quad_mode,
+                   const unsigned long long* __restrict__ total) {
   __shared__ float brick[kLdsCap];
   __shared__ int4 tab[kSlabTab];
   __shared__ QuadGrid G;
   const int nvq = (a.nviews + kQuad - 1) / kQuad * kQuad;
   int t, j0, i0;
   fp_tile_origin(a.tiles_w, a.tiles_per_view, a.group, nvq, &t, &j0, &i0);
-  if (quad_mode) {
+  if (quad_mode && shared_layout(total)) {
     const int tile = (i0 / kTile) * a.tiles_w + j0 / kTile;
     if (quad_mode[(size_t)(t / kQuad) * a.tiles_per_view + tile] == kQuadShared) return;
   }
@@ -1446,25 +1474,40 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   FC_CHECK_ARG((size_t)PX * PY * PZ < (1ull << 32), "volume too large for 32-bit voxel offsets");
   FC_CHECK_ARG(max_steps_for(vs, h) <= (1 << 24), "step %g too small for the volume: over 2^24 "
                "samples per ray (the sample loops count in FP32)", h);
-  // one mode byte per quad of the LDS projector after the staged volume
-  const size_t flags_off = (bytes + 255) & ~(size_t)255;
+  // the LDS projector's cost totals and one mode byte per quad after the staged volume
+  const size_t total_off = (bytes + 255) & ~(size_t)255, flags_off = total_off + 256;
   const size_t nquads = (size_t)((ps[0] + kTile - 1) / kTile) * ((ps[1] + kTile - 1) / kTile) *
                         (size_t)((ps[2] + kQuad - 1) / kQuad);
   if (layout == FP_LDS) bytes = flags_off + nquads;
   void* ws = nullptr;
   int rc = acquire_ws(device, SLOT_OCTET, bytes, stream, &ws);
   if (rc) return rc;
+  // FASTCONE_FP_QUAD = "never" / "always" forces single / shared mode for every quad, "auto" the
+  // decision of fp_decide (tests). Otherwise volumes of up to 64 voxels a side are projected in
+  // single mode without asking: few slabs and blocks, for which the decision and a second kernel
+  // cost more than the layouts differ (us, shared / single: 45 views of 48 x 52 x 50 68 / 52, 60 of
+  // 64^3 70 / 71, 84 with the decision; 180 of 64^3 at half steps 198 / 197).
+  const char* qe = std::getenv("FASTCONE_FP_QUAD");
+  const int qmode = qe && std::strcmp(qe, "never") == 0    ? -1
+                    : qe && std::strcmp(qe, "always") == 0 ? 1
+                    : qe && std::strcmp(qe, "auto") == 0   ? 0
+                    : std::max(nx, std::max(ny, nz)) <= 64 ? -1
+                                                           : 0;
+  unsigned long long* total =
+      layout == FP_LDS && qmode == 0
+          ? reinterpret_cast<unsigned long long*>(static_cast<char*>(ws) + total_off)
+          : nullptr;
   dim3 sg((PX + 255) / 256, PY, PZ);
   if (layout == FP_OCTET) {
     if (dt == FC_F32) stage_octets<FC_F32><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, ws, PX, PY);
     else if (dt == FC_BF16) stage_octets<FC_BF16><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, ws, PX, PY);
     else stage_octets<FC_F16><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, ws, PX, PY);
   } else if (layout == FP_PLAIN || dt == FC_F32) {
-    stage_plain<FC_F32><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, (float*)ws, PX, PY);
+    stage_plain<FC_F32><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, (float*)ws, PX, PY, total);
   } else if (dt == FC_BF16) {
-    stage_plain16<FC_BF16><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, (uint16_t*)ws, PX, PY);
+    stage_plain16<FC_BF16><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, (uint16_t*)ws, PX, PY, total);
   } else {
-    stage_plain16<FC_F16><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, (uint16_t*)ws, PX, PY);
+    stage_plain16<FC_F16><<<sg, 256, 0, stream>>>(vol, nx, ny, nz, (uint16_t*)ws, PX, PY, total);
   }
   FC_HIP(hipGetLastError());
   FpArgs a;
@@ -1495,10 +1538,6 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   const long long nblocks = (long long)a.tiles_per_view * (layout == FP_LDS ? nvq : a.nviews);
   FC_CHECK_ARG(nblocks < (1ll << 31), "too many projection tiles");
   if (layout == FP_LDS) a.group = std::min((a.group + kQuad - 1) / kQuad * kQuad, nvq);
-  // FASTCONE_FP_QUAD = "never" / "always" forces single / shared mode for every quad (tests)
-  const char* qe = std::getenv("FASTCONE_FP_QUAD");
-  const int qmode = qe && std::strcmp(qe, "never") == 0 ? -1
-                    : (qe && std::strcmp(qe, "always") == 0 ? 1 : 0);
   uint8_t* quad_mode = qmode < 0 ? nullptr : static_cast<uint8_t*>(ws) + flags_off;
   if (nblocks > 0) {
     int tok = prof_begin("project", stream);
@@ -1511,16 +1550,18 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
       fp_kernel<FC_F32, FP_PLAIN><<<nb, 256, 0, stream>>>(a);
     } else {
       if (qmode >= 0) {
+        if (qmode == 0)
+          fp_decide<8><<<(int)std::min<long long>(kSamples, nquads), 64, 0, stream>>>(a, total);
         // two 512-thread blocks per quad and tile (nb = tiles x nvq is a multiple of four)
         const int nh = nb / 2;
-        if (dt == FC_F32) fp_quad_kernel<FC_F32, 8><<<nh, 512, 0, stream>>>(a, quad_mode, qmode);
-        else if (dt == FC_BF16) fp_quad_kernel<FC_BF16, 8><<<nh, 512, 0, stream>>>(a, quad_mode, qmode);
-        else fp_quad_kernel<FC_F16, 8><<<nh, 512, 0, stream>>>(a, quad_mode, qmode);
+        if (dt == FC_F32) fp_quad_kernel<FC_F32, 8><<<nh, 512, 0, stream>>>(a, quad_mode, total);
+        else if (dt == FC_BF16) fp_quad_kernel<FC_BF16, 8><<<nh, 512, 0, stream>>>(a, quad_mode, total);
+        else fp_quad_kernel<FC_F16, 8><<<nh, 512, 0, stream>>>(a, quad_mode, total);
       }
       if (qmode <= 0) {
-        if (dt == FC_F32) fp_lds_kernel<FC_F32, 8><<<nb, 256, 0, stream>>>(a, quad_mode);
-        else if (dt == FC_BF16) fp_lds_kernel<FC_BF16, 8><<<nb, 256, 0, stream>>>(a, quad_mode);
-        else fp_lds_kernel<FC_F16, 8><<<nb, 256, 0, stream>>>(a, quad_mode);
+        if (dt == FC_F32) fp_lds_kernel<FC_F32, 8><<<nb, 256, 0, stream>>>(a, quad_mode, total);
+        else if (dt == FC_BF16) fp_lds_kernel<FC_BF16, 8><<<nb, 256, 0, stream>>>(a, quad_mode, total);
+        else fp_lds_kernel<FC_F16, 8><<<nb, 256, 0, stream>>>(a, quad_mode, total);
       }
     }
     prof_end(tok, stream);
@@ -1651,7 +1692,7 @@ int launch_gather_bench_fp(int device, int dt, int plain, double* samples_per_s)
   void* ws = nullptr;
   FC_HIP(hipMalloc(&ws, bytes));
   dim3 sg((PX + 255) / 256, PY, PZ);
-  if (plain) stage_plain<FC_F32><<<sg, 256>>>(src, n, n, n, (float*)ws, PX, PY);
+  if (plain) stage_plain<FC_F32><<<sg, 256>>>(src, n, n, n, (float*)ws, PX, PY, nullptr);
   else if (dt == FC_F32) stage_octets<FC_F32><<<sg, 256>>>(src, n, n, n, ws, PX, PY);
   else if (dt == FC_BF16) stage_octets<FC_BF16><<<sg, 256>>>(src, n, n, n, ws, PX, PY);
   else stage_octets<FC_F16><<<sg, 256>>>(src, n, n, n, ws, PX, PY);

@@ -599,3 +599,27 @@ def test_adjoint_of_non_finite_data_is_nan_and_cgls_raises(gpu):
     y[2, 13, 15] = float("nan")
     with pytest.raises(FloatingPointError):
         cgls.cgls(lambda x: ops.project(x, g, 0.5), lambda r: ops.adjoint(r, g, 0.5), y, iters=3)
+
+
+@pytest.mark.parametrize("nviews,arc", [(1, 0.0), (5, 4.0), (13, 6.0), (40, 360.0), (6, 360.0),
+                                        (66, 33.0)])
+@pytest.mark.parametrize("side", [22, 70])
+def test_project_layout_decision(gpu, nviews, arc, side, monkeypatch):
+    # dense and sparse views (shared and single layout), missing views in the last quad, fewer and
+    # more quads than are sampled, volumes on both sides of the size that is not asked; tolerance as
+    # for the forced modes above
+    from fastcone_amd import ops
+    rng = np.random.default_rng(80 + nviews + side)
+    ang = np.deg2rad(30.0 + arc * np.arange(nviews) / nviews)
+    det = (24, 40) if nviews < 66 else (40, 112)
+    g, prob = _setup(rng, ang=ang, vol=(16, side, side - 3), vol_dim=(16, side, side - 3), det=det,
+                     det_dim=det)
+    x = rng.standard_normal(g.vol_shape).astype(np.float32)
+    ref = oracle.project(prob, x, window=g.det_shape[::-1], h=0.5)
+    for mode in ("auto", None):
+        if mode is None:
+            monkeypatch.delenv("FASTCONE_FP_QUAD", raising=False)
+        else:
+            monkeypatch.setenv("FASTCONE_FP_QUAD", mode)
+        p = ops.project(torch.from_numpy(x).to(gpu), g, step=0.5).cpu()
+        assert rel(p, ref) < 5e-5
