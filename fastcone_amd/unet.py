@@ -161,6 +161,21 @@ class _UpCat(torch.autograd.Function):
         return ga, g[..., ca:]
 
 
+class _UpCatConv(torch.autograd.Function):
+    """conv3d of _UpCat in one kernel, for calls that keep nothing for a backward pass."""
+
+    @staticmethod
+    def forward(ctx, a, b, w32, b32, relu):
+        N, D, H, W, cb = b.shape
+        cout, _, cin = w32.shape
+        wb = w32.to(torch.bfloat16).contiguous()
+        y = torch.empty((N, D, H, W, cout), dtype=b.dtype, device=b.device)
+        _native.check(_native.lib().fc_net_up_cat_conv_dev(
+            b.device.index, a.data_ptr(), b.data_ptr(), wb.data_ptr(), b32.data_ptr(),
+            y.data_ptr(), N, D, H, W, cin - cb, cb, cout, 1 if relu else 0, _stream(b)))
+        return y
+
+
 class UNet3D(torch.nn.Module):
     SCALE = 50.0  # attenuation per voxel ~ 0.02 -> O(1) activations
 
@@ -178,6 +193,12 @@ class UNet3D(torch.nn.Module):
         _, cin, cout, relu = next(L for L in LAYERS if L[0] == name)
         return conv3d(x, self.w[name], self.b[name], relu)
 
+    def _up(self, a, b, name):
+        relu = next(L for L in LAYERS if L[0] == name)[3]
+        if torch.is_grad_enabled():
+            return self._c(_UpCat.apply(a, b), name)
+        return _UpCatConv.apply(a, b, self.w[name], self.b[name], relu)
+
     def forward(self, vol):
         """vol: [N, D, H, W] (or [D, H, W]) FP32 FDK reconstruction -> FP32 prediction of the
         same shape."""
@@ -191,8 +212,8 @@ class UNet3D(torch.nn.Module):
         e1, p1 = _Pool.apply(self._c(self._c(x, "e1a"), "e1b"))
         e2, p2 = _Pool.apply(self._c(self._c(p1, "e2a"), "e2b"))
         bt = self._c(self._c(p2, "b_a"), "b_b")
-        d2 = self._c(self._c(_UpCat.apply(bt, e2), "d2a"), "d2b")
-        d1 = self._c(self._c(_UpCat.apply(d2, e1), "d1a"), "d1b")
+        d2 = self._c(self._up(bt, e2, "d2a"), "d2b")
+        d1 = self._c(self._up(d2, e1, "d1a"), "d1b")
         out = vol + self._c(d1, "out")[..., 0] / self.SCALE
         return out[0] if single else out
 

@@ -208,6 +208,12 @@ int fc_conv3d_dgrad_dev(int device, const void* dy, const void* w, void* wt, voi
 /* dw (FP32 [cout][27][cin]) += weight gradient for input x and output gradient dy. */
 int fc_conv3d_wgrad_dev(int device, const void* x, const void* dy, float* dw, int N, int D, int H,
                         int W, int cin, int cout, void* stream);
+/* fc_conv3d_fwd_dev of the concatenation (a upsampled by 2, nearest; b) along the channels, which is
+ * not formed: ca + cb -> cout = 64 + 32 -> 32 or 32 + 16 -> 16; D, H, W even, the fine sizes; bit for
+ * bit the result of fc_net_up_cat_dev and the convolution. No counterpart in the reference. */
+int fc_net_up_cat_conv_dev(int device, const void* a, const void* b, const void* w,
+                           const float* bias, void* y, int N, int D, int H, int W, int ca, int cb,
+                           int cout, int relu, void* stream);
 /* The network's element-wise steps on the same BF16 layout (16-byte aligned; D, H, W even and the
  * fine sizes). fc_net_pool_dev: y = mean over 2x2x2 voxels, c = 16 or 32. fc_net_up_cat_dev: out =
  * (a upsampled by 2, nearest; b) along the channels, ca + cb = 64 + 32 or 32 + 16.

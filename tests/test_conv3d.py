@@ -356,3 +356,36 @@ def test_one_channel_layers(gpu, shape):
         assert rel(wg.grad.cpu(), wr.grad.permute(0, 2, 3, 4, 1).reshape(cout, 27, cin)) < 1e-5
         if cin != 1:
             assert rel(xg.grad.cpu(), xr.grad.permute(0, 2, 3, 4, 1)) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("shape,ca,cb,cout", [((1, 2, 2, 2), 32, 16, 16), ((2, 6, 10, 36), 32, 16, 16),
+                                              ((1, 34, 18, 16), 32, 16, 16), ((1, 4, 8, 34), 64, 32, 32),
+                                              ((3, 2, 22, 14), 64, 32, 32)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_up_cat_conv_matches_its_parts(gpu, shape, ca, cb, cout, offset):
+    # tiles cut by every side of the volume, several batches and z chunks, operands that start at an
+    # odd element: bit for bit the convolution of the concatenation
+    from fastcone_amd.unet import _UpCatConv, conv3d, upsample2
+    N, D, H, W = shape
+    g = torch.Generator().manual_seed(ca + sum(shape))
+
+    def bf(*s):
+        n = int(np.prod(s))
+        t = torch.randn(n + offset, generator=g).to(torch.bfloat16).to(gpu)
+        return t[offset:].view(s)
+    a, b = bf(N, D // 2, H // 2, W // 2, ca), bf(N, D, H, W, cb)
+    w = torch.randn((cout, 27, ca + cb), generator=g).to(gpu) * 0.05
+    bias = torch.randn(cout, generator=g).to(gpu)
+    with torch.no_grad():
+        for relu in (True, False):
+            ref = conv3d(torch.cat([upsample2(a), b], dim=-1).contiguous(), w, bias, relu)
+            assert torch.equal(_UpCatConv.apply(a, b, w, bias, relu), ref)
+
+
+def test_unet_without_gradients_is_the_same_network(gpu):
+    from fastcone_amd.unet import UNet3D
+    net = UNet3D(3).to(gpu)
+    vol = torch.rand((2, 12, 20, 16), generator=torch.Generator().manual_seed(1)).to(gpu) * 0.02
+    with torch.no_grad():
+        y = net(vol)
+    assert torch.equal(y, net(vol).detach())
