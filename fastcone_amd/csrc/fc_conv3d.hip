@@ -61,7 +61,9 @@ __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint
 // by the weights' way from L1 in the 64- and 96-channel ones. Before, a wave owned one group and
 // read patches and weights from L1 for every instruction. Time at 256^3: 16 -> 16 channels 1.49 ->
 // 0.32 ms (1.07 GB of activations: 0.23 ms at the rate of a large copy), 48 -> 16 5.29 -> 0.98 ms;
-// at 128^3: 96 -> 32 2.26 -> 0.96 ms, 32 -> 32 0.64 -> 0.17 ms; at 64^3: 64 -> 64 0.47 -> 0.21 ms.
+// at 128^3: 96 -> 32 2.26 -> 0.96 ms, 32 -> 32 0.64 -> 0.17 ms; at 64^3: 64 -> 64 0.47 -> 0.21 ms
+// (the layers with whole 32-channel steps have since got a kernel of their own for large inputs,
+// conv_fwd_stream).
 template <int CIN, int COUT>
 struct ConvTile {
   static constexpr int XT = (CIN == 16 && COUT <= 32) || (CIN == 32 && COUT >= 32) ? 32 : 16;
@@ -258,6 +260,166 @@ __global__ __launch_bounds__(256, 2) void conv_fwd_mfma(const uint16_t* __restri
       slot[0] = slot[1];
       slot[1] = slot[2];
       slot[2] = s0;
+      __syncthreads();
+    }
+  }
+}
+
+// The same convolution for whole 32-channel steps (Cin a multiple of 32) and many tiles, plane by
+// plane: one input plane is in LDS, and a patch read from it feeds the three output planes z - 1, z,
+// z + 1 at once (their dz = 2, 1, 0 weights), whose sums are all in registers. Every output still
+// adds its terms in ascending order of k, 32 per instruction: dz = 0 comes with its first plane. A
+// wave owns one block of 16 output channels and V rows of 16 voxels, so a step's three weight
+// fragments (from L1, a step ahead) feed 3 V instructions; the next plane is loaded into registers
+// meanwhile.
+//
+// conv_fwd_mfma is bound by the weights' way from L1 in these layers: two instructions per fragment
+// of 1 KB, which takes L1 16 clocks for each wave as the instruction takes its SIMD. Here it is 24
+// (12 for 96 channels, whose next plane needs the registers), and a third of the patch reads. Time
+// before and now: 96 -> 32 channels at 128^3 0.92 -> 0.58 ms, 64 -> 64 at 64^3 0.20 -> 0.09, 32 -> 32
+// at 128^3 0.15 -> 0.12, 64 -> 32 at 4 x 32^3 0.055 -> 0.037 ms. With all of a row's channel blocks
+// in one wave (6 or 12 fragments a step) it was slower than before.
+template <int CIN, int COUT>
+struct StreamTile {
+  static constexpr int NB = COUT / 16;          // channel blocks; a wave owns one
+  static constexpr int V = CIN == 96 ? 4 : 8;    // and this many rows of 16 voxels
+  static constexpr int XT = 16, YT = 4 / NB * V, PITCH = 2 * CIN + 16;
+  static constexpr int ROWB = (XT + 2) * PITCH, PLANEB = (YT + 2) * ROWB;
+  static constexpr int C32 = CIN / 32, STEPS = 9 * C32, K = 27 * CIN;
+};
+
+template <int CIN, int COUT, bool RELU, bool UPCAT>
+__global__ __launch_bounds__(256, 2) void conv_fwd_stream(const uint16_t* __restrict__ x,
+                                                          const uint16_t* __restrict__ skip,
+                                                          const uint16_t* __restrict__ w,
+                                                          const float* __restrict__ bias,
+                                                          uint16_t* __restrict__ y, int D, int H,
+                                                          int W, int tx, int ty, int zc, int nzc) {
+  using T = StreamTile<CIN, COUT>;
+  constexpr int XT = T::XT, YT = T::YT, V = T::V, PITCH = T::PITCH, ROWB = T::ROWB, NB = T::NB;
+  constexpr int C8 = CIN / 8, UNITS = (XT + 2) * (YT + 2) * C8, NU = (UNITS + 255) / 256;
+  constexpr int CA = 2 * CIN / 3, STEPS = T::STEPS, K = T::K;
+  __shared__ __align__(16) char plane[T::PLANEB];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int bx = b % tx; b /= tx;
+  const int by = b % ty; b /= ty;
+  const int bz = b % nzc, n = b / nzc;
+  const int xb = bx * XT, yb = by * YT, z0 = bz * zc, z1 = min(D, z0 + zc);
+
+  // plane units as in conv_fwd_mfma
+  int vox[NU];
+#pragma unroll
+  for (int q = 0; q < NU; ++q) {
+    const int u = (int)threadIdx.x + 256 * q;
+    const int v = u / C8, ch = 8 * (u - v * C8), yy = v / (XT + 2), xx = v - yy * (XT + 2);
+    const int gx = xb + xx - 1, gy = yb + yy - 1;
+    vox[q] = -1;
+    if (u < UNITS && gx >= 0 && gx < W && gy >= 0 && gy < H)
+      vox[q] = !UPCAT    ? yy * W + xx
+               : ch < CA ? ((gy >> 1) * (W >> 1) + (gx >> 1)) * CA + ch
+                         : (gy * W + gx) * (CIN - CA) + ch - CA;
+  }
+  u32x4 pf[NU];
+  auto fetch = [&](int z) {
+    const uint16_t* p = x + ((((long long)n * D + z) * H + (yb - 1)) * W + (xb - 1)) * CIN;
+    const bool zin = z >= 0 && z < D;
+    const long long pl = (long long)n * D + z;
+    const uint16_t *pa = nullptr, *pb = nullptr;
+    if constexpr (UPCAT) {
+      pa = x + (pl >> 1) * (H >> 1) * (W >> 1) * CA;  // D is even
+      pb = skip + pl * H * W * (CIN - CA);
+    }
+#pragma unroll
+    for (int q = 0; q < NU; ++q) {
+      const int ch = 8 * (((int)threadIdx.x + 256 * q) % C8);
+      pf[q] = u32x4{0u, 0u, 0u, 0u};
+      if (zin && vox[q] >= 0)
+        pf[q] = *reinterpret_cast<const u32x4_a2*>(UPCAT ? (ch < CA ? pa : pb) + vox[q]
+                                                         : p + (long long)vox[q] * CIN + ch);
+    }
+  };
+  auto put = [&]() {
+#pragma unroll
+    for (int q = 0; q < NU; ++q) {
+      const int u = (int)threadIdx.x + 256 * q, v = u / C8;
+      if (u < UNITS) *reinterpret_cast<u32x4*>(plane + v * PITCH + 16 * (u - v * C8)) = pf[q];
+    }
+  };
+  const int cb = wave % NB, rows = wave / NB * V;  // this wave's channel block and first row
+  f32x4 bb;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bb[r] = bias ? bias[cb * 16 + 4 * g + r] : 0.0f;
+  const char* lane0 = plane + (rows * (XT + 2) + m) * PITCH + 16 * g;
+  const uint32_t wlane = 2u * (uint32_t)((cb * 16 + m) * K + g * 8);
+  bf16x8 wr[2][3];
+  auto weights = [&](int s) {
+    uint32_t from = wlane;
+    const uint16_t* ws = w;
+    asm volatile("" : "+v"(from), "+s"(ws));  // loads and addresses not earlier than a step ahead
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const char* at = reinterpret_cast<const char*>(ws + (d * 9 * CIN + s * 32));
+      wr[s & 1][d] =
+          __builtin_bit_cast(bf16x8, (u32x4)*reinterpret_cast<const u32x4_a2*>(at + from));
+    }
+  };
+  f32x4 acc[3][V];  // output planes p - 1, p, p + 1
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[d][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+  fetch(z0 - 1);
+  put();
+  __syncthreads();
+  for (int p = z0 - 1; p <= z1; ++p) {
+    if (p < z1) fetch(p + 1);
+    // planes at the ends of the chunk serve one or two outputs
+    const bool use[3] = {p + 1 < z1, p >= z0 && p < z1, p > z0};
+    weights(0);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 < STEPS) weights(s + 1);
+      const int tap = s / T::C32, o = (tap / 3 * (XT + 2) + tap % 3) * PITCH + s % T::C32 * 64;
+      bf16x8 f[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+        f[v] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lane0 + o + v * ROWB));
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        if (use[d])
+#pragma unroll
+          for (int v = 0; v < V; ++v)
+            acc[2 - d][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[s & 1][d], f[v],
+                                                                    acc[2 - d][v], 0, 0, 0);
+    }
+    if (p > z0) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const int vy = yb + rows + v, vx = xb + m;
+        if (vy < H && vx < W) {
+          float f[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            f[r] = acc[0][v][r] + bb[r];
+            if (RELU) f[r] = fmaxf(f[r], 0.0f);
+          }
+          uint16_t* o = y + ((((size_t)n * D + (p - 1)) * H + vy) * W + vx) * COUT + cb * 16 + 4 * g;
+          *reinterpret_cast<u32x2_a2*>(o) = u32x2_a2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
+        }
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      acc[0][v] = acc[1][v];
+      acc[1][v] = acc[2][v];
+      acc[2][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();  // the plane is no longer read
+    if (p < z1) {
+      put();
       __syncthreads();
     }
   }
@@ -850,20 +1012,35 @@ __global__ __launch_bounds__(64) void mfma_probe(const uint16_t* __restrict__ A3
 template <int CIN, int COUT, bool UPCAT>
 void launch_fwd_t(const void* x, const void* skip, const void* w, const float* b, void* y, int N,
                   int D, int H, int W, int relu, hipStream_t s) {
-  using T = ConvTile<CIN, COUT>;
-  const int tx = (W + T::XT - 1) / T::XT, ty = (H + T::YT - 1) / T::YT;
+  const auto run = [&](auto tile, auto with_relu, auto without, int blocks, int zmin) {
+    using T = decltype(tile);
+    const int tx = (W + T::XT - 1) / T::XT, ty = (H + T::YT - 1) / T::YT;
+    const long long tiles = (long long)tx * ty * N;
+    const int zc = (int)std::max((long long)zmin, std::min(32LL, tiles * D / blocks));
+    const int nzc = (D + zc - 1) / zc;
+    (relu ? with_relu : without)<<<(unsigned)(tiles * nzc), 256, 0, s>>>(
+        (const uint16_t*)x, (const uint16_t*)skip, (const uint16_t*)w, b, (uint16_t*)y, D, H, W, tx,
+        ty, zc, nzc);
+  };
+  // conv_fwd_stream wants its 512 resident blocks (two per CU) and at least two planes per block (the
+  // two halo planes are loaded besides): below 512 tile planes the smaller tiles of conv_fwd_mfma are
+  // faster (us, before / stream): 96 -> 32 at 32^3 (256 tile planes) 18 / 32, 32 -> 32 at 48^3 (432)
+  // 18 / 16, 64 -> 32 at 4 x 32^3 (512) 55 / 37, 64 -> 64 at 40^3 (600) 78 / 55; for 16 output channels
+  // always (32 -> 16 at 128^3 64 / 86).
+  if constexpr (CIN % 32 == 0 && (COUT == 32 || COUT == 64)) {
+    using T = StreamTile<CIN, COUT>;
+    const long long planes =
+        (long long)((W + T::XT - 1) / T::XT) * ((H + T::YT - 1) / T::YT) * N * D;
+    if (planes >= 512) {
+      run(T(), conv_fwd_stream<CIN, COUT, true, UPCAT>, conv_fwd_stream<CIN, COUT, false, UPCAT>, 512,
+          2);
+      return;
+    }
+  }
   // planes per block: as many as leave about 2048 blocks (eight per CU), at most 32 (the two halo
   // planes are then 6 % of the planes loaded)
-  const long long tiles = (long long)tx * ty * N;
-  const int zc = (int)std::max(1LL, std::min(32LL, tiles * D / 2048));
-  const int nzc = (D + zc - 1) / zc;
-  const unsigned grid = (unsigned)(tiles * nzc);
-  const auto launch = [&](auto kernel) {
-    kernel<<<grid, 256, 0, s>>>((const uint16_t*)x, (const uint16_t*)skip, (const uint16_t*)w, b,
-                                (uint16_t*)y, D, H, W, tx, ty, zc, nzc);
-  };
-  if (relu) launch(conv_fwd_mfma<CIN, COUT, true, UPCAT>);
-  else launch(conv_fwd_mfma<CIN, COUT, false, UPCAT>);
+  run(ConvTile<CIN, COUT>(), conv_fwd_mfma<CIN, COUT, true, UPCAT>,
+      conv_fwd_mfma<CIN, COUT, false, UPCAT>, 2048, 1);
 }
 
 // Supported (Cin, Cout) pairs of the MFMA kernels: the network's layers and their transposes.

@@ -389,3 +389,29 @@ def test_unet_without_gradients_is_the_same_network(gpu):
     with torch.no_grad():
         y = net(vol)
     assert torch.equal(y, net(vol).detach())
+
+
+@pytest.mark.parametrize("cin,cout", [(32, 32), (32, 64), (64, 64), (96, 32), (64, 32)])
+@pytest.mark.parametrize("shape", [(1, 32, 64, 129), (2, 67, 33, 50), (1, 130, 20, 36), (3, 3, 120, 340)])
+def test_conv_large_layers(gpu, cin, cout, shape):
+    # inputs with enough tiles for the plane-by-plane kernel: tiles cut in x and y, chunks of 2 to 32
+    # planes with a remainder, several batches. Every output adds its terms in the order of the tiled
+    # kernel, which the same volume in pieces of few tiles runs: bit for bit (each piece with the
+    # planes around it)
+    from fastcone_amd.unet import conv3d
+    N, D, H, W = shape
+    g = torch.Generator().manual_seed(cin + cout + D)
+    x = torch.randn((N, D, H, W, cin), generator=g).to(torch.bfloat16).to(gpu)
+    w = torch.randn((cout, 27, cin), generator=g).to(gpu) * 0.05
+    b = torch.randn(cout, generator=g).to(gpu)
+    with torch.no_grad():
+        y = conv3d(x, w, b, True)
+        zs = torch.randint(0, D, (4,), generator=g).tolist() + [0, D - 1]
+        for n in range(N):
+            for z in zs:
+                lo, hi = max(z - 1, 0), min(z + 2, D)
+                for y0 in range(0, H, 16):
+                    ya, yb = max(y0 - 1, 0), min(y0 + 17, H)
+                    part = x[n:n + 1, lo:hi, ya:yb].contiguous()
+                    ref = conv3d(part, w, b, True)[0, z - lo, y0 - ya:min(y0 + 16, H) - ya]
+                    assert torch.equal(y[n, z, y0:y0 + 16], ref)
