@@ -182,7 +182,7 @@ def main():
                "gather_peak_Gtap_per_s": peak_bp * 4 / 1e9,
                "gather_frac": bp_taps / (bp_ms * 1e-3) / (peak_bp * 4),
                "gather_random_positions_Gtap_per_s": peak_bp_random * 4 / 1e9},
-        "filter": {"ms": flt_ms, "kernel": "row_filter_kernel (cosine weight + ramp, FFT in LDS)",
+        "filter": {"ms": flt_ms, "kernel": "row_filter_kernel (cosine weight + ramp, FFT in registers)",
                    "hbm_GBps": 2 * 4 * nv * NDET * NDET / (flt_ms * 1e-3) / 1e9 if flt_ms else None},
         "R_kernels_only": W / ((fp_ms + bp_ms) * 1e-3) / 1e9,
     }

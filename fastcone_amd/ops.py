@@ -198,7 +198,7 @@ def cone_adjoint(proj, geom, step=1.0):
 # ---- FDK ------------------------------------------------------------------------------------
 def fdk_filter(proj, geom, D=None, pw=1.0, out_dtype=torch.float32, out=None, cosine=True):
     """Cosine pre-weighting and ramp filtering of a projection stack on the device (one HIP kernel,
-    fc_fdk_filter_dev: FFT convolution of every detector row in LDS, FP32 arithmetic).
+    fc_fdk_filter_dev: FFT convolution of every detector row, FP32 arithmetic).
 
     The ramp is the reference's (fastcone.py:272-292, cycles per pixel) divided by pw, so that
     FDK returns the attenuation per voxel (the reference's fbp() returns pw times it); the cosine
