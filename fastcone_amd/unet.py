@@ -195,7 +195,8 @@ class UNet3D(torch.nn.Module):
 
     def _up(self, a, b, name):
         relu = next(L for L in LAYERS if L[0] == name)[3]
-        if torch.is_grad_enabled():
+        # the fused kernel counts a plane's elements in 32 bits
+        if torch.is_grad_enabled() or b.shape[2] * b.shape[3] * a.shape[4] >= 2 ** 31:
             return self._c(_UpCat.apply(a, b), name)
         return _UpCatConv.apply(a, b, self.w[name], self.b[name], relu)
 
