@@ -1487,11 +1487,12 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   // single mode without asking: few slabs and blocks, for which the decision and a second kernel
   // cost more than the layouts differ (us, shared / single: 45 views of 48 x 52 x 50 68 / 52, 60 of
   // 64^3 70 / 71, 84 with the decision; 180 of 64^3 at half steps 198 / 197).
+  const bool small = std::max(nx, std::max(ny, nz)) <= 64;
   const char* qe = std::getenv("FASTCONE_FP_QUAD");
   const int qmode = qe && std::strcmp(qe, "never") == 0    ? -1
                     : qe && std::strcmp(qe, "always") == 0 ? 1
                     : qe && std::strcmp(qe, "auto") == 0   ? 0
-                    : std::max(nx, std::max(ny, nz)) <= 64 ? -1
+                    : small                                ? -1
                                                            : 0;
   unsigned long long* total =
       layout == FP_LDS && qmode == 0
@@ -1529,10 +1530,16 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   // FASTCONE_FP_LDS_CAP lowers the LDS brick budget (testing the global-gather fallback)
   const char* cap = std::getenv("FASTCONE_FP_LDS_CAP");
   a.lds_cap = cap ? std::max(0, std::min(kLdsCap, std::atoi(cap))) : kLdsCap;
-  // FASTCONE_FP_PAIRS=0 keeps every LDS brick in plain values (testing that the pair bricks and
-  // their cell reuse give the same bits)
+  // Bricks of (value, difference) pairs pay where samples follow each other within a cell, so that a
+  // lane keeps its cell's pairs; otherwise their fill and its LDS cost more than the interpolation
+  // saves. Pairs / plain: 180 views of 256^3 at step 0.6 7.59 / 7.98 ms, 0.8 6.55 / 6.67, 0.9 6.28 /
+  // 6.23; whole steps, 90 of 256^3 3.43 / 3.36, 160 of 384^3 19.4 / 19.2, 120 of 96^3 0.291 / 0.283.
+  // The small volumes' short slabs never gain: 60 views of 64^3 71.7 / 68.8 us at whole and 91.1 /
+  // 88.9 at half steps (pairs stay where the layout is forced). FASTCONE_FP_PAIRS=0 keeps every brick
+  // in plain values (testing that the pairs and their cell reuse give the same bits).
   const char* pe = std::getenv("FASTCONE_FP_PAIRS");
-  a.pairs = pe && std::strcmp(pe, "0") == 0 ? 0 : 1;
+  const bool gain = h < 0.85 && (qe || !small);
+  a.pairs = !(pe && std::strcmp(pe, "0") == 0) && gain ? 1 : 0;
   // The LDS projector deals quads of four views; `group` stays a multiple of four.
   const int nvq = (a.nviews + kQuad - 1) / kQuad * kQuad;
   const long long nblocks = (long long)a.tiles_per_view * (layout == FP_LDS ? nvq : a.nviews);

@@ -623,3 +623,21 @@ def test_project_layout_decision(gpu, nviews, arc, side, monkeypatch):
             monkeypatch.setenv("FASTCONE_FP_QUAD", mode)
         p = ops.project(torch.from_numpy(x).to(gpu), g, step=0.5).cpu()
         assert rel(p, ref) < 5e-5
+
+
+@pytest.mark.parametrize("side,step", [(22, 0.5), (22, 1.0), (70, 0.5), (70, 0.84), (70, 0.86)])
+def test_project_brick_kind_is_bit_identical(gpu, side, step, monkeypatch):
+    # volumes and steps on both sides of the rule that chooses pair bricks, against plain bricks
+    # and against forced single mode, which keeps the pairs of small volumes
+    from fastcone_amd import ops
+    rng = np.random.default_rng(side)
+    g, _ = _setup(rng, ang=np.deg2rad(10.0 + 25.0 * np.arange(9)), vol=(20, side, side - 3),
+                  vol_dim=(20, side, side - 3), det=(30, 44), det_dim=(30, 44))
+    x = torch.from_numpy(rng.standard_normal(g.vol_shape).astype(np.float32)).to(gpu)
+    p = ops.project(x, g, step=step)
+    monkeypatch.setenv("FASTCONE_FP_PAIRS", "0")
+    assert torch.equal(p, ops.project(x, g, step=step)) and float(p.abs().max()) > 0.0
+    if side <= 64:
+        monkeypatch.delenv("FASTCONE_FP_PAIRS")
+        monkeypatch.setenv("FASTCONE_FP_QUAD", "never")
+        assert torch.equal(p, ops.project(x, g, step=step))
