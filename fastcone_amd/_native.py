@@ -57,6 +57,7 @@ def _declare(lib):
         "fc_conv3d_wgrad_dev": (i, [i, _vp, _vp, _vp, i, i, i, i, i, i, _vp]),
         "fc_net_pool_dev": (i, [i, _vp, _vp, i, i, i, i, i, _vp]),
         "fc_net_up_cat_conv_dev": (i, [i, _vp, _vp, _vp, _vp, _vp, i, i, i, i, i, i, i, i, _vp]),
+        "fc_net_up_cat_wgrad_dev": (i, [i, _vp, _vp, _vp, _vp, i, i, i, i, i, i, i, _vp]),
         "fc_net_up_cat_dev": (i, [i, _vp, _vp, _vp, i, i, i, i, i, i, _vp]),
         "fc_net_up_cat_grad_dev": (i, [i, _vp, _vp, i, i, i, i, i, i, _vp]),
         "fc_net_skip_pool_grad_dev": (i, [i, _vp, i, _vp, _vp, i, i, i, i, i, _vp]),

@@ -452,12 +452,18 @@ __global__ __launch_bounds__(256) void flip_transpose_weights(const uint16_t* __
 // accumulator registers). Before, every lane gathered its eight voxels one by one for each tap:
 // a training step's seven layers (4 x 128^3) took 19.1 ms; 48 -> 16 channels at 4 x 128^3 7.88 ->
 // 0.52 ms, 16 -> 16 2.24 -> 0.17 ms, 96 -> 32 at 4 x 64^3 2.12 -> 0.22 ms.
+// A block's input channels are one aligned group of 16, so for the decoder's layers they lie in one
+// of the two tensors that are concatenated, and the rows are loaded from there: with the forward
+// pass doing the same, a training step at 4 x 128^3 forms none of its 1.0 GB of concatenations (6.17
+// -> 5.68 ms).
 constexpr int kWgSeg = 32;                        // input voxels per wave and row
 constexpr int kWgWaveB = 3 * kWgSeg * 32 + 34 * 32;  // LDS bytes per wave: three rows, gradient row
 constexpr int kWgRed = 4;                         // accumulators reduced at once
 
 struct WgArgs {
-  const uint16_t* x;
+  const uint16_t* x;     // the input, or its first ca channels at half the size (skip: the others)
+  const uint16_t* skip;
+  int ca;                // 0: x is the input
   const uint16_t* dy;
   float* dw;
   long long units;  // (n, z, y chunk, x segment)
@@ -509,6 +515,10 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
     const int xv = x0 + (lane >> 1);                     // input voxel of this lane's 16 bytes
     const int gv0 = x0 - 1 + (lane >> 1), gv1 = gv0 + 32;  // gradient voxels (gv1: lanes 0 - 3)
     const bool xok = xv < a.W, g0ok = gv0 >= 0 && gv0 < a.W, g1ok = lane < 4 && gv1 < a.W;
+    // where this block's input channels are: in x, or of a concatenation (x upsampled, skip)
+    const int up = a.ca && ci0 < a.ca, xc = !a.ca ? a.cin : (up ? a.ca : a.cin - a.ca);
+    const uint16_t* xp = !a.ca || up ? a.x + ci0 : a.skip + (ci0 - a.ca);
+    const long long xh = a.H >> up, xw = a.W >> up;
     u32x4 px[3], pg0, pg1;
     // input rows yy of the three planes, and gradient row yg, as zeros outside the volume
     auto fetch_x = [&](int yy) {
@@ -518,7 +528,7 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
         px[d] = u32x4{0u, 0u, 0u, 0u};
         if (xok && zz >= 0 && zz < a.D && yy >= 0 && yy < a.H)
           px[d] = *reinterpret_cast<const u32x4_a2*>(
-              a.x + (((n * a.D + zz) * a.H + yy) * a.W + xv) * a.cin + ci0 + 8 * (lane & 1));
+              xp + ((((n * a.D + zz) >> up) * xh + (yy >> up)) * xw + (xv >> up)) * xc + 8 * (lane & 1));
       }
     };
     auto fetch_g = [&](int yg) {
@@ -1059,7 +1069,7 @@ bool launch_fwd(int cin, int cout, const void* x, const void* w, const float* b,
 }
 
 bool launch_wgrad(int cin, int cout, const void* x, const void* dy, float* dw, int N, int D,
-                  int H, int W, hipStream_t s) {
+                  int H, int W, hipStream_t s, const void* skip = nullptr, int ca = 0) {
   bool known = false;  // the network's layers
   for (const auto& p : {std::pair<int, int>{16, 16}, {16, 32}, {32, 32}, {32, 64}, {64, 64},
                         {96, 32}, {48, 16}})
@@ -1067,6 +1077,8 @@ bool launch_wgrad(int cin, int cout, const void* x, const void* dy, float* dw, i
   if (!known) return false;
   WgArgs a;
   a.x = (const uint16_t*)x;
+  a.skip = (const uint16_t*)skip;
+  a.ca = ca;
   a.dy = (const uint16_t*)dy;
   a.dw = dw;
   a.D = D; a.H = H; a.W = W; a.cin = cin; a.cout = cout;
@@ -1188,6 +1200,24 @@ int fc_conv3d_wgrad_dev(int device, const void* x, const void* dy, float* dw, in
     prof_end(tok, s);
     FC_CHECK_ARG(false, "unsupported channel pair %d -> %d", cin, cout);
   }
+  prof_end(tok, s);
+  FC_HIP(hipGetLastError());
+  return FC_OK;
+}
+
+int fc_net_up_cat_wgrad_dev(int device, const void* a, const void* b, const void* dy, float* dw,
+                            int N, int D, int H, int W, int ca, int cb, int cout, void* stream) {
+  clear_error();
+  FC_CHECK_ARG(a && b && dy && dw, "null pointer argument");
+  FC_CHECK_ARG(N > 0 && D > 0 && H > 0 && W > 0, "bad activation shape");
+  FC_CHECK_ARG(D % 2 == 0 && H % 2 == 0 && W % 2 == 0, "sides must be even");
+  FC_CHECK_ARG((ca == 64 && cb == 32 && cout == 32) || (ca == 32 && cb == 16 && cout == 16),
+               "unsupported channel counts %d + %d -> %d", ca, cb, cout);
+  int rc = select_device(device);
+  if (rc) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  int tok = prof_begin("conv3d_wgrad", s);
+  launch_wgrad(ca + cb, cout, a, dy, dw, N, D, H, W, s, b, ca);
   prof_end(tok, s);
   FC_HIP(hipGetLastError());
   return FC_OK;

@@ -61,34 +61,41 @@ class _Conv(torch.autograd.Function):
         x, wb, y = ctx.saved_tensors
         cin, cout, relu = ctx.cfg
         N, D, H, W, _ = x.shape
-        L = _native.lib()
-        db = None
-        if relu and gy.dtype == torch.bfloat16 and not torch.is_grad_enabled():
-            # mask and bias gradient in one pass
-            g0, gy = _packed(gy), torch.empty_like(y)
-            db = torch.zeros(cout, dtype=torch.float32, device=y.device)
-            _native.check(L.fc_net_relu_grad_dev(y.device.index, g0.data_ptr(), y.data_ptr(),
-                                                 gy.data_ptr(), db.data_ptr(), N * D * H * W,
-                                                 cout, _stream(y)))
-        else:
-            if relu:
-                gy = gy * (y > 0)
-            gy = gy.to(torch.float32 if cout == 1 else torch.bfloat16).contiguous()
+        gy, db = _masked(gy, y, cout, relu)
         dw = torch.zeros((cout, 27, cin), dtype=torch.float32, device=x.device)
-        rc = L.fc_conv3d_wgrad_dev(x.device.index, x.data_ptr(), gy.data_ptr(), dw.data_ptr(),
-                                   N, D, H, W, cin, cout, _stream(x))
+        rc = _native.lib().fc_conv3d_wgrad_dev(x.device.index, x.data_ptr(), gy.data_ptr(),
+                                               dw.data_ptr(), N, D, H, W, cin, cout, _stream(x))
         _native.check(rc)
         if db is None:
             db = gy.float().sum(dim=(0, 1, 2, 3))
-        dx = None
-        if ctx.needs_input_grad[0]:
-            dx = torch.empty_like(x)
-            wt = torch.empty((cin * 27 * cout,), dtype=torch.bfloat16, device=x.device)
-            rc = L.fc_conv3d_dgrad_dev(x.device.index, gy.data_ptr(), wb.data_ptr(),
-                                       wt.data_ptr(), dx.data_ptr(), N, D, H, W, cin, cout,
-                                       _stream(x))
-            _native.check(rc)
+        dx = _dgrad(gy, wb, x.shape, cout) if ctx.needs_input_grad[0] else None
         return dx, dw, db, None, None, None
+
+
+def _masked(gy, y, cout, relu):
+    """The gradient at the convolution's sum, and the bias gradient (None: not yet summed)."""
+    if relu and gy.dtype == torch.bfloat16 and not torch.is_grad_enabled():
+        # mask and bias gradient in one pass
+        g0, gy = _packed(gy), torch.empty_like(y)
+        db = torch.zeros(cout, dtype=torch.float32, device=y.device)
+        _native.check(_native.lib().fc_net_relu_grad_dev(
+            y.device.index, g0.data_ptr(), y.data_ptr(), gy.data_ptr(), db.data_ptr(),
+            y.numel() // cout, cout, _stream(y)))
+        return gy, db
+    if relu:
+        gy = gy * (y > 0)
+    return gy.to(torch.float32 if cout == 1 else torch.bfloat16).contiguous(), None
+
+
+def _dgrad(gy, wb, shape, cout):
+    N, D, H, W, cin = shape
+    dx = torch.empty(shape, dtype=torch.bfloat16, device=gy.device)
+    wt = torch.empty((cin * 27 * cout,), dtype=torch.bfloat16, device=gy.device)
+    rc = _native.lib().fc_conv3d_dgrad_dev(gy.device.index, gy.data_ptr(), wb.data_ptr(),
+                                           wt.data_ptr(), dx.data_ptr(), N, D, H, W, cin, cout,
+                                           _stream(gy))
+    _native.check(rc)
+    return dx
 
 
 def conv3d(x, w, b, relu):
@@ -151,18 +158,19 @@ class _UpCat(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        N, D, H, W, C = g.shape
-        ca = ctx.ca
-        g = _packed(g)
-        ga = torch.empty((N, D // 2, H // 2, W // 2, ca), dtype=g.dtype, device=g.device)
-        _native.check(_native.lib().fc_net_up_cat_grad_dev(g.device.index, g.data_ptr(),
-                                                           ga.data_ptr(), N, D, H, W, ca, C - ca,
-                                                           _stream(g)))
-        return ga, g[..., ca:]
+        return _up_cat_grad(_packed(g), ctx.ca)
+
+
+def _up_cat_grad(g, ca):
+    N, D, H, W, C = g.shape
+    ga = torch.empty((N, D // 2, H // 2, W // 2, ca), dtype=g.dtype, device=g.device)
+    _native.check(_native.lib().fc_net_up_cat_grad_dev(g.device.index, g.data_ptr(), ga.data_ptr(),
+                                                       N, D, H, W, ca, C - ca, _stream(g)))
+    return ga, g[..., ca:]
 
 
 class _UpCatConv(torch.autograd.Function):
-    """conv3d of _UpCat in one kernel, for calls that keep nothing for a backward pass."""
+    """conv3d of _UpCat; the concatenation is not formed, the kernels load from both tensors."""
 
     @staticmethod
     def forward(ctx, a, b, w32, b32, relu):
@@ -173,7 +181,26 @@ class _UpCatConv(torch.autograd.Function):
         _native.check(_native.lib().fc_net_up_cat_conv_dev(
             b.device.index, a.data_ptr(), b.data_ptr(), wb.data_ptr(), b32.data_ptr(),
             y.data_ptr(), N, D, H, W, cin - cb, cb, cout, 1 if relu else 0, _stream(b)))
+        ctx.save_for_backward(a, b, wb, y if relu else torch.empty(0, device=b.device))
+        ctx.relu = relu
         return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        a, b, wb, y = ctx.saved_tensors
+        N, D, H, W, cb = b.shape
+        cout, _, cin = wb.shape
+        gy, db = _masked(gy, y, cout, ctx.relu)
+        dw = torch.zeros((cout, 27, cin), dtype=torch.float32, device=b.device)
+        _native.check(_native.lib().fc_net_up_cat_wgrad_dev(
+            b.device.index, a.data_ptr(), b.data_ptr(), gy.data_ptr(), dw.data_ptr(), N, D, H, W,
+            cin - cb, cb, cout, _stream(b)))
+        if db is None:
+            db = gy.float().sum(dim=(0, 1, 2, 3))
+        ga = gb = None
+        if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
+            ga, gb = _up_cat_grad(_dgrad(gy, wb, (N, D, H, W, cin), cout), cin - cb)
+        return ga, gb, dw, db, None
 
 
 class UNet3D(torch.nn.Module):
@@ -195,8 +222,8 @@ class UNet3D(torch.nn.Module):
 
     def _up(self, a, b, name):
         relu = next(L for L in LAYERS if L[0] == name)[3]
-        # the fused kernel counts a plane's elements in 32 bits
-        if torch.is_grad_enabled() or b.shape[2] * b.shape[3] * a.shape[4] >= 2 ** 31:
+        # the kernel that forms no concatenation counts a plane's elements in 32 bits
+        if b.shape[2] * b.shape[3] * a.shape[4] >= 2 ** 31:
             return self._c(_UpCat.apply(a, b), name)
         return _UpCatConv.apply(a, b, self.w[name], self.b[name], relu)
 

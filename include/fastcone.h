@@ -214,6 +214,9 @@ int fc_conv3d_wgrad_dev(int device, const void* x, const void* dy, float* dw, in
 int fc_net_up_cat_conv_dev(int device, const void* a, const void* b, const void* w,
                            const float* bias, void* y, int N, int D, int H, int W, int ca, int cb,
                            int cout, int relu, void* stream);
+/* fc_conv3d_wgrad_dev for that input. */
+int fc_net_up_cat_wgrad_dev(int device, const void* a, const void* b, const void* dy, float* dw,
+                            int N, int D, int H, int W, int ca, int cb, int cout, void* stream);
 /* The network's element-wise steps on the same BF16 layout (16-byte aligned; D, H, W even and the
  * fine sizes). fc_net_pool_dev: y = mean over 2x2x2 voxels, c = 16 or 32. fc_net_up_cat_dev: out =
  * (a upsampled by 2, nearest; b) along the channels, ca + cb = 64 + 32 or 32 + 16.

@@ -382,6 +382,39 @@ def test_up_cat_conv_matches_its_parts(gpu, shape, ca, cb, cout, offset):
             assert torch.equal(_UpCatConv.apply(a, b, w, bias, relu), ref)
 
 
+@pytest.mark.parametrize("shape,ca,cb,cout", [((1, 2, 2, 2), 32, 16, 16), ((2, 6, 10, 36), 32, 16, 16),
+                                              ((1, 34, 18, 70), 32, 16, 16), ((3, 4, 38, 34), 64, 32, 32)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("relu", [True, False])
+def test_up_cat_conv_gradients_match_their_parts(gpu, shape, ca, cb, cout, offset, relu):
+    # rows and x segments cut by the volume, several batches and y chunks. Whole numbers: every
+    # sum of the weight and bias gradients is exact in FP32 in any order, so all bits are the same
+    from fastcone_amd.unet import _UpCat, _UpCatConv, conv3d
+    N, D, H, W = shape
+    g = torch.Generator().manual_seed(cb + sum(shape))
+
+    def whole(*s, lim, off=0):
+        n = int(np.prod(s))
+        t = torch.randint(-lim, lim + 1, (n + off,), generator=g).to(torch.bfloat16).to(gpu)
+        return t[off:].view(s)
+    a = whole(N, D // 2, H // 2, W // 2, ca, lim=2, off=offset)
+    b = whole(N, D, H, W, cb, lim=2, off=offset)
+    w = whole(cout, 27, ca + cb, lim=1).float()
+    bias = whole(cout, lim=3).float()
+    gy = whole(N, D, H, W, cout, lim=1)
+    res = []
+    for ours in (True, False):
+        p = [t.detach().requires_grad_(True) for t in (a, b, w, bias)]
+        if ours:
+            y = _UpCatConv.apply(*p, relu)
+        else:  # the concatenation's operands must start on 16 bytes
+            y = conv3d(_UpCat.apply(p[0].clone(), p[1].clone()), p[2], p[3], relu)
+        y.backward(gy)
+        res.append([y.detach()] + [t.grad for t in p])
+    for u, v in zip(*res):
+        assert torch.equal(u, v)
+
+
 def test_unet_without_gradients_is_the_same_network(gpu):
     from fastcone_amd.unet import UNet3D
     net = UNet3D(3).to(gpu)
