@@ -55,6 +55,8 @@ def _declare(lib):
         "fc_conv3d_fwd_dev": (i, [i, _vp, _vp, _vp, _vp, i, i, i, i, i, i, i, _vp]),
         "fc_conv3d_dgrad_dev": (i, [i, _vp, _vp, _vp, _vp, i, i, i, i, i, i, _vp]),
         "fc_conv3d_wgrad_dev": (i, [i, _vp, _vp, _vp, i, i, i, i, i, i, _vp]),
+        "fc_net_weights_dev": (i, [i, ctypes.POINTER(_vp), ctypes.POINTER(ctypes.c_longlong), i,
+                                   _vp, _vp]),
         "fc_net_pool_dev": (i, [i, _vp, _vp, i, i, i, i, i, _vp]),
         "fc_net_up_cat_conv_dev": (i, [i, _vp, _vp, _vp, _vp, _vp, i, i, i, i, i, i, i, i, _vp]),
         "fc_net_up_cat_wgrad_dev": (i, [i, _vp, _vp, _vp, _vp, i, i, i, i, i, i, i, _vp]),

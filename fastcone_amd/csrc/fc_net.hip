@@ -182,6 +182,25 @@ int net_check(int device, int N, int D, int H, int W, bool even) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// The network's weights as the convolutions read them: up to kMaxTensors FP32 tensors rounded to
+// BF16 into one buffer, a column of blocks per tensor. 0.4 M elements: bound by its launch. In
+// place of a launch per tensor an inference takes 254 instead of 274 us at 64^3 and 361 instead of
+// 382 at 96^3; at 256^3 the difference is 0.3 %.
+constexpr int kMaxTensors = 16;
+
+struct WeightArgs {
+  const float* src[kMaxTensors];
+  long long begin[kMaxTensors + 1];
+};
+
+__global__ __launch_bounds__(256) void round_weights(WeightArgs a, uint16_t* __restrict__ out) {
+  const float* src = a.src[blockIdx.y];
+  uint16_t* dst = out + a.begin[blockIdx.y];
+  const long long n = a.begin[blockIdx.y + 1] - a.begin[blockIdx.y];
+  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll)
+    dst[i] = f32_to_bf16_bits(src[i]);
+}
+
 }  // namespace
 }  // namespace fc
 
@@ -291,6 +310,28 @@ int fc_net_relu_grad_dev(int device, const void* gy, const void* y, void* gm, fl
   if (c == 16) relu_grad_kernel<2><<<blocks, 256, 0, s>>>(pg, py, po, db, units);
   else if (c == 32) relu_grad_kernel<4><<<blocks, 256, 0, s>>>(pg, py, po, db, units);
   else relu_grad_kernel<8><<<blocks, 256, 0, s>>>(pg, py, po, db, units);
+  FC_HIP(hipGetLastError());
+  return FC_OK;
+}
+
+int fc_net_weights_dev(int device, const float* const* src, const long long* counts, int n,
+                       void* dst, void* stream) {
+  clear_error();
+  FC_CHECK_ARG(src && counts && dst, "null pointer argument");
+  FC_CHECK_ARG(n > 0 && n <= kMaxTensors, "1 to %d tensors", kMaxTensors);
+  WeightArgs a;
+  a.begin[0] = 0;
+  long long most = 0;
+  for (int q = 0; q < n; ++q) {
+    FC_CHECK_ARG(src[q] && counts[q] > 0, "empty tensor %d", q);
+    a.src[q] = src[q];
+    a.begin[q + 1] = a.begin[q] + counts[q];
+    most = std::max(most, counts[q]);
+  }
+  int rc = select_device(device);
+  if (rc) return rc;
+  const dim3 grid((unsigned)std::min(256LL, (most + 255) / 256), n);
+  round_weights<<<grid, 256, 0, static_cast<hipStream_t>(stream)>>>(a, static_cast<uint16_t*>(dst));
   FC_HIP(hipGetLastError());
   return FC_OK;
 }

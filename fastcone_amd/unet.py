@@ -11,6 +11,7 @@ upsampling with concatenation, their gradients and the ReLU mask with the bias g
 fc_net_*; the loss is torch's. Master weights and
 Adam state are FP32; the kernels read BF16 copies.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -29,7 +30,6 @@ LAYERS = [  # (name, cin, cout, relu)
 
 
 def _stream(t):
-    import ctypes
     return ctypes.c_void_p(int(torch.cuda.current_stream(t.device).cuda_stream))
 
 
@@ -39,12 +39,26 @@ def _packed(t):
     return t.clone() if t.data_ptr() % 16 else t
 
 
+def _bf16_weights(ws, device):
+    """The BF16 copies the kernels read, by one launch (None each: the convolutions make theirs)."""
+    if len(ws) > 16 or any(w.dtype != torch.float32 or w.device != device or
+                           not w.is_contiguous() or not w.numel() for w in ws):
+        return [None] * len(ws)
+    n = [w.numel() for w in ws]
+    out = torch.empty(sum(n), dtype=torch.bfloat16, device=device)
+    _native.check(_native.lib().fc_net_weights_dev(
+        device.index, (ctypes.c_void_p * len(n))(*[w.data_ptr() for w in ws]),
+        (ctypes.c_longlong * len(n))(*n), len(n), out.data_ptr(), _stream(out)))
+    return [t.view(w.shape) for t, w in zip(out.split(n), ws)]
+
+
 class _Conv(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w32, b32, cin, cout, relu):
+    def forward(ctx, x, w32, b32, cin, cout, relu, wb=None):
         N, D, H, W, C = x.shape
         assert C == cin and x.dtype == torch.bfloat16 and x.is_contiguous()
-        wb = w32.to(torch.bfloat16).contiguous()
+        if wb is None:
+            wb = w32.to(torch.bfloat16).contiguous()
         odt = torch.float32 if cout == 1 else torch.bfloat16
         y = torch.empty((N, D, H, W, cout), dtype=odt, device=x.device)
         L = _native.lib()
@@ -69,7 +83,7 @@ class _Conv(torch.autograd.Function):
         if db is None:
             db = gy.float().sum(dim=(0, 1, 2, 3))
         dx = _dgrad(gy, wb, x.shape, cout) if ctx.needs_input_grad[0] else None
-        return dx, dw, db, None, None, None
+        return dx, dw, db, None, None, None, None
 
 
 def _masked(gy, y, cout, relu):
@@ -98,10 +112,10 @@ def _dgrad(gy, wb, shape, cout):
     return dx
 
 
-def conv3d(x, w, b, relu):
-    """x: [N, D, H, W, Cin] BF16; w: [Cout, 27, Cin] FP32; b: [Cout] FP32."""
+def conv3d(x, w, b, relu, wb=None):
+    """x: [N, D, H, W, Cin] BF16; w: [Cout, 27, Cin] FP32 (wb: its BF16 copy); b: [Cout] FP32."""
     cout, _, cin = w.shape
-    return _Conv.apply(x, w, b, cin, cout, relu)
+    return _Conv.apply(x, w, b, cin, cout, relu, wb)
 
 
 def avgpool2(x):
@@ -173,10 +187,11 @@ class _UpCatConv(torch.autograd.Function):
     """conv3d of _UpCat; the concatenation is not formed, the kernels load from both tensors."""
 
     @staticmethod
-    def forward(ctx, a, b, w32, b32, relu):
+    def forward(ctx, a, b, w32, b32, relu, wb=None):
         N, D, H, W, cb = b.shape
         cout, _, cin = w32.shape
-        wb = w32.to(torch.bfloat16).contiguous()
+        if wb is None:
+            wb = w32.to(torch.bfloat16).contiguous()
         y = torch.empty((N, D, H, W, cout), dtype=b.dtype, device=b.device)
         _native.check(_native.lib().fc_net_up_cat_conv_dev(
             b.device.index, a.data_ptr(), b.data_ptr(), wb.data_ptr(), b32.data_ptr(),
@@ -200,7 +215,7 @@ class _UpCatConv(torch.autograd.Function):
         ga = gb = None
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
             ga, gb = _up_cat_grad(_dgrad(gy, wb, (N, D, H, W, cin), cout), cin - cb)
-        return ga, gb, dw, db, None
+        return ga, gb, dw, db, None, None
 
 
 class UNet3D(torch.nn.Module):
@@ -216,16 +231,16 @@ class UNet3D(torch.nn.Module):
             self.w[name] = torch.nn.Parameter(torch.randn((cout, 27, cin), generator=g) * std)
             self.b[name] = torch.nn.Parameter(torch.zeros(cout))
 
-    def _c(self, x, name):
+    def _c(self, x, name, wb):
         _, cin, cout, relu = next(L for L in LAYERS if L[0] == name)
-        return conv3d(x, self.w[name], self.b[name], relu)
+        return conv3d(x, self.w[name], self.b[name], relu, wb[name])
 
-    def _up(self, a, b, name):
+    def _up(self, a, b, name, wb):
         relu = next(L for L in LAYERS if L[0] == name)[3]
         # the kernel that forms no concatenation counts a plane's elements in 32 bits
         if b.shape[2] * b.shape[3] * a.shape[4] >= 2 ** 31:
-            return self._c(_UpCat.apply(a, b), name)
-        return _UpCatConv.apply(a, b, self.w[name], self.b[name], relu)
+            return self._c(_UpCat.apply(a, b), name, wb)
+        return _UpCatConv.apply(a, b, self.w[name], self.b[name], relu, wb[name])
 
     def forward(self, vol):
         """vol: [N, D, H, W] (or [D, H, W]) FP32 FDK reconstruction -> FP32 prediction of the
@@ -237,12 +252,14 @@ class UNet3D(torch.nn.Module):
             if s % 4:
                 raise ValueError("volume sides must be multiples of 4")
         x = (vol * self.SCALE).to(torch.bfloat16)[..., None].contiguous()
-        e1, p1 = _Pool.apply(self._c(self._c(x, "e1a"), "e1b"))
-        e2, p2 = _Pool.apply(self._c(self._c(p1, "e2a"), "e2b"))
-        bt = self._c(self._c(p2, "b_a"), "b_b")
-        d2 = self._c(self._up(bt, e2, "d2a"), "d2b")
-        d1 = self._c(self._up(d2, e1, "d1a"), "d1b")
-        out = vol + self._c(d1, "out")[..., 0] / self.SCALE
+        names = [L[0] for L in LAYERS]
+        wb = dict(zip(names, _bf16_weights([self.w[n] for n in names], x.device)))
+        e1, p1 = _Pool.apply(self._c(self._c(x, "e1a", wb), "e1b", wb))
+        e2, p2 = _Pool.apply(self._c(self._c(p1, "e2a", wb), "e2b", wb))
+        bt = self._c(self._c(p2, "b_a", wb), "b_b", wb)
+        d2 = self._c(self._up(bt, e2, "d2a", wb), "d2b", wb)
+        d1 = self._c(self._up(d2, e1, "d1a", wb), "d1b", wb)
+        out = vol + self._c(d1, "out", wb)[..., 0] / self.SCALE
         return out[0] if single else out
 
     def save(self, path):

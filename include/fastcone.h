@@ -217,6 +217,10 @@ int fc_net_up_cat_conv_dev(int device, const void* a, const void* b, const void*
 /* fc_conv3d_wgrad_dev for that input. */
 int fc_net_up_cat_wgrad_dev(int device, const void* a, const void* b, const void* dy, float* dw,
                             int N, int D, int H, int W, int ca, int cb, int cout, void* stream);
+/* n (1 to 16) FP32 device tensors src[q] of counts[q] elements, rounded to BF16 one after the other
+ * into dst; src and counts are host arrays. */
+int fc_net_weights_dev(int device, const float* const* src, const long long* counts, int n,
+                       void* dst, void* stream);
 /* The network's element-wise steps on the same BF16 layout (16-byte aligned; D, H, W even and the
  * fine sizes). fc_net_pool_dev: y = mean over 2x2x2 voxels, c = 16 or 32. fc_net_up_cat_dev: out =
  * (a upsampled by 2, nearest; b) along the channels, ca + cb = 64 + 32 or 32 + 16.

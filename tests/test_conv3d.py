@@ -415,6 +415,19 @@ def test_up_cat_conv_gradients_match_their_parts(gpu, shape, ca, cb, cout, offse
         assert torch.equal(u, v)
 
 
+def test_bf16_weights_are_rounded_like_torch(gpu):
+    # counts around a block and above one grid, special values, tensors that the kernel does not take
+    from fastcone_amd.unet import _bf16_weights
+    g = torch.Generator().manual_seed(4)
+    ws = [torch.randn(n, generator=g).to(gpu) * 10.0 ** e
+          for n, e in ((1, 0), (255, -3), (256, 3), (257, -40), (70000, 0), (7, 38))]
+    ws[1][:4] = torch.tensor([float("inf"), -float("inf"), 1 + 2.0 ** -8, -0.0])
+    for w, b in zip(ws, _bf16_weights(ws, gpu)):
+        assert torch.equal(w.to(torch.bfloat16), b)
+    assert _bf16_weights([ws[0], ws[2].double()], gpu) == [None, None]
+    assert _bf16_weights([ws[0], ws[2][::2]], gpu) == [None, None]
+
+
 def test_unet_without_gradients_is_the_same_network(gpu):
     from fastcone_amd.unet import UNet3D
     net = UNet3D(3).to(gpu)
