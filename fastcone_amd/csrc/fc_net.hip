@@ -5,10 +5,11 @@
 //
 // All are bound by memory: a thread moves 16 bytes (8 channels of a voxel) per access, every tensor
 // is read or written once, and one launch takes the place of a chain of element-wise operations
-// that stored FP32 or strided copies in between. At 256^3 (inference) the concatenation at full size
-// takes 0.44 ms (1.6 GB written, 0.8 GB read), the pooling 0.12 ms, and all steps 0.7 instead of
-// 3.7 ms; at 4 x 128^3 (training) the mask with the bias gradient takes 0.14 ms a layer (0.8 GB) and
-// all steps 1.8 instead of 6.6 ms.
+// that stored FP32 or strided copies in between. At 256^3 (inference) the pooling takes 0.12 ms; the
+// concatenation at full size would take 0.44 ms (1.6 GB written, 0.8 GB read), so it is formed only
+// for planes of 2^31 elements and more, and the convolutions load its parts elsewhere. At 4 x 128^3
+// (training) the mask with the bias gradient takes 0.14 ms a layer (0.8 GB) and all steps 1.3 instead
+// of 6.6 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

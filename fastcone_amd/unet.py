@@ -6,9 +6,10 @@ nearest-neighbour upsampling up with channel concatenation of the skip connectio
 3x3x3 convolution to one FP32 channel added to the (scaled) input: the network predicts the
 correction from the FDK reconstruction to the CGLS reconstruction.
 
-Convolutions (forward, input gradient, weight gradient) run in fc_conv3d_* (MFMA); pooling,
-upsampling with concatenation, their gradients and the ReLU mask with the bias gradient in
-fc_net_*; the loss is torch's. Master weights and
+Convolutions (forward, input gradient, weight gradient) run in fc_conv3d_* (MFMA), the decoder's,
+whose concatenated input is not formed, in fc_net_up_cat_conv_dev and fc_net_up_cat_wgrad_dev;
+pooling, upsampling, their gradients and the ReLU mask with the bias gradient in fc_net_*; the loss
+is torch's. Master weights and
 Adam state are FP32; the kernels read BF16 copies.
 """
 import ctypes
