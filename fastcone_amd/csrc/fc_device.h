@@ -123,19 +123,23 @@ __device__ __forceinline__ float lerp(float a, float b, float t) { return fmaf(t
 // the LDS it writes must be read only after an explicit s_waitcnt vmcnt(0) and a barrier.
 // Loads complete in order, so the compiler's own vmcnt waits stay conservative with these loads
 // outstanding. M0 is declared clobbered; the compiler reports that it reserves M0, and it uses M0
-// nowhere else in the kernels that copy this way.
+// nowhere else in the kernels that copy this way. A load to LDS reads the old M0 if it directly
+// follows the write of M0 (one wait state; the compiler puts an s_nop or another instruction between
+// the two for the builtin, but nothing inside an asm statement), hence the s_nop. A scalar base
+// written by a vector instruction would need five wait states before the load; here every base ends
+// in scalar arithmetic. tests/test_load_to_lds.py checks both in the generated code.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void copy_units_to_lds(const void* base, uint32_t lane_bytes,
                                                   uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(
                    __builtin_amdgcn_readfirstlane(lds_dst)),
                "v"(lane_bytes), "s"(base)
                : "memory", "m0");
 }
 __device__ __forceinline__ void copy_dword_to_lds(const void* base, uint32_t lane_bytes,
                                                   uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(
                    __builtin_amdgcn_readfirstlane(lds_dst)),
                "v"(lane_bytes), "s"(base)
                : "memory", "m0");
