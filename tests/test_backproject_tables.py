@@ -62,3 +62,27 @@ def test_several_tables_per_block(gpu, dt):
                               vol_start=(0, 0, z0), proj_dim=det[::-1])
         ref = oracle.backproject(prob, y.float().numpy(), (2, n, n), mode=2, norm=np.ones(nv))
         assert rel(out[z0:z0 + 2], ref) < 5e-5
+
+
+@pytest.mark.parametrize("nv", [1, 50])
+@pytest.mark.parametrize("mode,mis", [(2, None), (0, [0.6, -0.8, 1.5, 0.02, -0.03, 0.01])])
+@pytest.mark.parametrize("dt", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("pw,det", [(0.33, (40, 110)), (0.15, (100, 200))])
+def test_windows_wider_than_the_tile(gpu, nv, mode, mis, dt, pw, det):
+    # fine pixels: whole cubes gather all their views from global memory, partial ones some, with taps
+    # over every edge of the detector; 50 views are two tables
+    from fastcone_amd import ops
+    from fastcone_amd.geometry import Geometry
+    rng = np.random.default_rng(nv + mode + det[0])
+    ang = np.sort(rng.uniform(0, 2 * np.pi, nv))
+    vol = (18, 33, 20)
+    hmid = rng.uniform(7, 11, nv)
+    g = Geometry.circular(ang, 70.0, pw, vol, det, hmid=hmid, misalign=mis)
+    prob = oracle.Problem(ang, hmid, 70.0, pw, vol_dim=vol[::-1], proj_dim=det[::-1], mis=mis)
+    y = torch.from_numpy(rng.standard_normal(g.proj_shape).astype(np.float32)).to(
+        getattr(torch, dt))
+    base = torch.from_numpy(rng.standard_normal(vol).astype(np.float32)).to(gpu)
+    norm = rng.uniform(0.5, 1.5, nv).astype(np.float32)
+    out = ops.backproject(y.to(gpu), g, mode, norm=norm, out=base.clone())
+    ref = oracle.backproject(prob, y.float().numpy(), vol, mode=mode, norm=norm)
+    assert rel((out.double() - base.double()).cpu(), ref) < 5e-5
