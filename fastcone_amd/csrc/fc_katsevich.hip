@@ -281,7 +281,7 @@ typedef const __attribute__((address_space(3))) f2* lds_f2;
 template <bool LDS, class P>
 __device__ __forceinline__ void kat_samples(float* acc, P at, uint32_t pitch, float au, float dr,
                                             float r0, int qa, float lo, float hi, float wgt) {
-  constexpr int B = LDS ? 4 : 1;  // samples in flight; the rare global path gets no registers
+  constexpr int B = 4;  // samples in flight
 #pragma unroll
   for (int q0 = 0; q0 < kZR; q0 += B) {
     f2 p[B], n[B];
@@ -316,6 +316,10 @@ __device__ __forceinline__ void kat_samples(float* acc, P at, uint32_t pitch, fl
 // 256 voxels, 4320 views of 64 x 512: 15.2 ms against 38.9 ms for gathering 16-byte quads of every
 // visited view from global memory (20 L1 accesses per wave and sample: L1-bound at best, 21.6 ms, once
 // the views outside the window were skipped).
+// Views whose window does not fit the buffers are gathered from global memory, slabs outside the
+// window left out, four samples in flight. 256 x 256 x 128 voxels of twice the size on the same
+// detector (89 % of the blocks' views), whole reconstruction: 9.7 ms, of 128 x 64 x 64 of four times the
+// size 5.2; one sample in flight and every slab 20.4 and 6.7, the quads' gather 12.6 and 9.9 ms.
 template <int SLABS>
 __global__ __launch_bounds__(256, 4) void kat_bp_kernel(KatBpArgs a) {
   constexpr int NZ = SLABS * kZR, ROWS = win_rows(SLABS), SLOTS = (ROWS * kWinW / 2 + 255) / 256;
@@ -426,11 +430,13 @@ __global__ __launch_bounds__(256, 4) void kat_bp_kernel(KatBpArgs a) {
           if (big || !__any(ra <= rtop && rb >= rbot)) continue;  // the rows rise with z
           kat_samples<true>(acc + s * kZR, at, 0, au, dr, r0, qa, lo, hi, wgt);
         }
-        if (big) {
+        if (big) {  // windows wider than the LDS buffers: columns finer than about half a voxel
           const char* src = pairs + (size_t)t.k * viewB + pitchB + (size_t)(uint32_t)iu * 8u;
 #pragma unroll
           for (int s = 0; s < SLABS; ++s) {
             const float r0 = row0(z0 + s * kZR, qa);
+            const float ra = fmaf((float)qa, dr, r0), rb = fmaf((float)(qa + kZR - 1), dr, r0);
+            if (!__any(ra <= rtop && rb >= rbot)) continue;
             kat_samples<false>(acc + s * kZR, src, pitchB, au, dr, r0, qa, lo, hi, wgt);
           }
         }

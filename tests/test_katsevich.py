@@ -190,3 +190,25 @@ def test_katsevich_backprojector_branches(gpu, nw, nh, dg, drow, nz, ny, nx, ori
         tol = rel * (np.abs(row) + np.abs(edge) * (1 + np.abs(np.tan(gam)))
                      + SDD * hp / R / drow / np.cos(gam))
         assert (np.abs(row - edge) < tol).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dg,drow", [(0.0009, 0.5), (0.0016, 1.0)])
+def test_katsevich_wide_windows_by_parts(gpu, dg, drow):
+    """Views whose windows are wider than the LDS buffers (all, or those near the source), in blocks of
+    four slabs, against the same volume in parts of a slab per block: the same samples in the same
+    order, so the same bits."""
+    import torch
+    from fastcone_amd.katsevich import HelixScan, katsevich
+    n, nz, nh, vpt = 240, 128, 64, 200
+    nw = int(0.72 / dg)
+    hp = 0.8 * nh * drow * 500.0 / 900.0 / (2 * math.pi)
+    dl = 2 * math.pi / vpt
+    views = 3 * vpt
+    scan = HelixScan(views, dl, 0.0, -hp * dl * (views - 1) / 2, hp, 500.0, 900.0, dg, drow, nw, nh)
+    proj = torch.randn((views, nh, nw), generator=torch.Generator().manual_seed(nw)).to(gpu)
+    whole = katsevich(proj, scan, (nz, n, n))
+    for z in (0, 64):
+        part = katsevich(proj, scan, (64, n, n), origin=(-(n // 2), -(n // 2), z - nz // 2))
+        assert torch.equal(whole[z:z + 64], part)
+    assert bool(whole.abs().sum() > 0)
