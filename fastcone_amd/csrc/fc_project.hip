@@ -1483,11 +1483,17 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   int rc = acquire_ws(device, SLOT_OCTET, bytes, stream, &ws);
   if (rc) return rc;
   // FASTCONE_FP_QUAD = "never" / "always" forces single / shared mode for every quad, "auto" the
-  // decision of fp_decide (tests). Otherwise volumes of up to 64 voxels a side are projected in
-  // single mode without asking: few slabs and blocks, for which the decision and a second kernel
-  // cost more than the layouts differ (us, shared / single: 45 views of 48 x 52 x 50 68 / 52, 60 of
-  // 64^3 70 / 71, 84 with the decision; 180 of 64^3 at half steps 198 / 197).
-  const bool small = std::max(nx, std::max(ny, nz)) <= 64;
+  // decision of fp_decide (tests). Otherwise calls of little work (16 x 16 pixel tiles, times views,
+  // times the longest side of the volume, as 1e3) are projected in single mode without asking: the
+  // decision and a second kernel cost 13 to 30 us, which is more than the layouts differ there. Single
+  // mode with plain bricks / with the decision (us, half steps): 60 views of 64^3 (138) 89 / 103, 30 of
+  // 80^3 (154) 94 / 166, 60 of 80^3 (307) 149 / 174, 180 of 64^3 (415) 194 / 197, 120 of 72^3 (423) 195 /
+  // 201, 60 of 96^3 (467) 218 / 235; 120 of 80^3 (614) 253 / 254, 360 of 64^3 (829) 358 / 343, 120 of 96^3
+  // (933) 393 / 382, 120 of 112^3 (1626) 598 / 571. (Few views gain beyond the line, 60 of 128^3 (1106) 448 /
+  // 476, but how far apart views are is not known here.)
+  const bool small = (long long)((ps[0] + kTile - 1) / kTile) * ((ps[1] + kTile - 1) / kTile) *
+                         ps[2] * std::max(nx, std::max(ny, nz)) <=
+                     500000;
   const char* qe = std::getenv("FASTCONE_FP_QUAD");
   const int qmode = qe && std::strcmp(qe, "never") == 0    ? -1
                     : qe && std::strcmp(qe, "always") == 0 ? 1
@@ -1534,9 +1540,10 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   // lane keeps its cell's pairs; otherwise their fill and its LDS cost more than the interpolation
   // saves. Pairs / plain: 180 views of 256^3 at step 0.6 7.59 / 7.98 ms, 0.8 6.55 / 6.67, 0.9 6.28 /
   // 6.23; whole steps, 90 of 256^3 3.43 / 3.36, 160 of 384^3 19.4 / 19.2, 120 of 96^3 0.291 / 0.283.
-  // The small volumes' short slabs never gain: 60 views of 64^3 71.7 / 68.8 us at whole and 91.1 /
-  // 88.9 at half steps (pairs stay where the layout is forced). FASTCONE_FP_PAIRS=0 keeps every brick
-  // in plain values (testing that the pairs and their cell reuse give the same bits).
+  // In calls of little work (single mode unasked) they never gain: 60 views of 64^3 71.7 / 68.8 us at
+  // whole and 91.1 / 88.9 at half steps, 60 of 96^3 at half steps 223 / 218 (pairs stay where the layout
+  // is forced, for tests of both kinds). FASTCONE_FP_PAIRS=0 keeps every brick in plain values (testing
+  // that the pairs and their cell reuse give the same bits).
   const char* pe = std::getenv("FASTCONE_FP_PAIRS");
   const bool gain = h < 0.85 && (qe || !small);
   a.pairs = !(pe && std::strcmp(pe, "0") == 0) && gain ? 1 : 0;

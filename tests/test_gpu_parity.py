@@ -641,3 +641,20 @@ def test_project_brick_kind_is_bit_identical(gpu, side, step, monkeypatch):
         monkeypatch.delenv("FASTCONE_FP_PAIRS")
         monkeypatch.setenv("FASTCONE_FP_QUAD", "never")
         assert torch.equal(p, ops.project(x, g, step=step))
+
+
+@pytest.mark.parametrize("nviews,step", [(177, 0.5), (179, 0.5), (224, 0.84), (224, 0.86)])
+def test_project_little_work_rule(gpu, nviews, step, monkeypatch):
+    # calls on both sides of the work that is projected without a layout decision (28 tiles x 100
+    # voxels x 178.6 views), with the steps on both sides of the rule for pair bricks: against the
+    # oracle, with plain bricks the same bits
+    from fastcone_amd import ops
+    rng = np.random.default_rng(nviews)
+    g, prob = _setup(rng, ang=np.deg2rad(2.0 * np.arange(nviews)), vol=(20, 60, 100),
+                     vol_dim=(20, 60, 100), det=(57, 112), det_dim=(57, 112))
+    x = rng.standard_normal(g.vol_shape).astype(np.float32)
+    p = ops.project(torch.from_numpy(x).to(gpu), g, step=step)
+    ref = oracle.project(prob, x, window=g.det_shape[::-1], h=step)
+    assert rel(p.cpu(), ref) < 5e-5
+    monkeypatch.setenv("FASTCONE_FP_PAIRS", "0")
+    assert torch.equal(p, ops.project(torch.from_numpy(x).to(gpu), g, step=step))
