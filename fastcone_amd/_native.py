@@ -64,6 +64,7 @@ def _declare(lib):
         "fc_net_up_cat_grad_dev": (i, [i, _vp, _vp, i, i, i, i, i, i, _vp]),
         "fc_net_skip_pool_grad_dev": (i, [i, _vp, i, _vp, _vp, i, i, i, i, i, _vp]),
         "fc_net_relu_grad_dev": (i, [i, _vp, _vp, _vp, _vp, ll, i, _vp]),
+        "fc_net_relu_grad_parts_dev": (i, [i, _vp, _vp, _vp, _vp, i, _vp, ll, i, _vp]),
         "fc_mfma_layout_probe": (i, [i, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
         "fc_katsevich_dev": (i, [i, _vp, i, i, i, i, d, d, d, d, d, d, d, d, d, d, i, _vp,
                                  _c_int_p, _c_dbl_p, _vp, _vp]),

@@ -131,12 +131,15 @@ __global__ __launch_bounds__(256) void skip_pool_grad_kernel(const u32x4* __rest
   }
 }
 
-// gm = gy (y > 0) and db[c] += sum over voxels of gm. A thread keeps its 8 channels: the stride of
-// its units is a multiple of C8. Every block adds its sums with one float atomic per channel.
+// gm = gy (y > 0) and the sums over voxels of gm. A thread keeps its 8 channels: the stride of its
+// units is a multiple of C8. Every block stores its sums in `part` (bias_sum adds them in order, so
+// that equal inputs give equal bits), or adds them to db with one float atomic per channel if part is
+// null.
 template <int C8>
 __global__ __launch_bounds__(256) void relu_grad_kernel(const u32x4* __restrict__ gy,
                                                         const u32x4* __restrict__ y,
                                                         u32x4* __restrict__ gm,
+                                                        float* __restrict__ part,
                                                         float* __restrict__ db, long long units) {
   __shared__ float red[4][8 * C8];
   float s[8];
@@ -164,10 +167,36 @@ __global__ __launch_bounds__(256) void relu_grad_kernel(const u32x4* __restrict_
     if (lane < C8) red[wave][lane * 8 + q] = s[q];
   }
   __syncthreads();
-  if (threadIdx.x < 8 * C8)
-    unsafeAtomicAdd(db + threadIdx.x, red[0][threadIdx.x] + red[1][threadIdx.x] +
-                                          red[2][threadIdx.x] + red[3][threadIdx.x]);
+  if (threadIdx.x < 8 * C8) {
+    const float v = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] +
+                    red[3][threadIdx.x];
+    if (part) part[(size_t)blockIdx.x * (8 * C8) + threadIdx.x] = v;
+    else unsafeAtomicAdd(db + threadIdx.x, v);
+  }
 }
+
+// db[c] = sum over the rows of part, in an order that depends on their number only. A block sums
+// sixteen channels with 64 rows at a time; bound by its latency.
+__global__ __launch_bounds__(1024) void bias_sum(const float* __restrict__ part, int rows, int c,
+                                                 float* __restrict__ db) {
+  __shared__ float red[16][16];
+  const int ch = threadIdx.x & 15;
+  const float* p = part + blockIdx.x * 16 + ch;
+  float s = 0.0f;
+  for (int r = threadIdx.x >> 4; r < rows; r += 64) s += p[(size_t)r * c];
+  s += __shfl_xor(s, 16, 64);
+  s += __shfl_xor(s, 32, 64);
+  if ((threadIdx.x & 63) < 16) red[threadIdx.x >> 6][ch] = s;
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    s = red[0][ch];
+    for (int w = 1; w < 16; ++w) s += red[w][ch];
+    db[blockIdx.x * 16 + ch] = s;
+  }
+}
+
+// Blocks of relu_grad_kernel at most: four per CU.
+constexpr int kReluRows = 1024;
 
 dim3 row_grid(long long units_per_row, long long rows) {
   return dim3((unsigned)((units_per_row + 255) / 256),
@@ -292,8 +321,9 @@ int fc_net_skip_pool_grad_dev(int device, const void* gs, int gs_pitch, const vo
   return FC_OK;
 }
 
-int fc_net_relu_grad_dev(int device, const void* gy, const void* y, void* gm, float* db,
-                         long long voxels, int c, void* stream) {
+// fc_net_relu_grad_dev and fc_net_relu_grad_parts_dev: `rows` is the most blocks that `part` holds.
+static int relu_grad(int device, const void* gy, const void* y, void* gm, float* part, long long rows,
+                     float* db, long long voxels, int c, void* stream) {
   clear_error();
   FC_CHECK_ARG(gy && y && gm && db, "null pointer argument");
   FC_CHECK_ARG(aligned16(gy) && aligned16(y) && aligned16(gm),
@@ -304,15 +334,28 @@ int fc_net_relu_grad_dev(int device, const void* gy, const void* y, void* gm, fl
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const long long units = voxels * (c / 8);
-  // at least 16 units per thread, so that a block's atomics are few beside its loads
-  const unsigned blocks = (unsigned)std::max(1LL, std::min(1024LL, units / (256 * 16)));
+  // at least 16 units per thread, so that a block's sums are few beside its loads
+  const unsigned blocks = (unsigned)std::max(1LL, std::min(rows, units / (256 * 16)));
   const u32x4 *pg = static_cast<const u32x4*>(gy), *py = static_cast<const u32x4*>(y);
   u32x4* po = static_cast<u32x4*>(gm);
-  if (c == 16) relu_grad_kernel<2><<<blocks, 256, 0, s>>>(pg, py, po, db, units);
-  else if (c == 32) relu_grad_kernel<4><<<blocks, 256, 0, s>>>(pg, py, po, db, units);
-  else relu_grad_kernel<8><<<blocks, 256, 0, s>>>(pg, py, po, db, units);
+  if (c == 16) relu_grad_kernel<2><<<blocks, 256, 0, s>>>(pg, py, po, part, db, units);
+  else if (c == 32) relu_grad_kernel<4><<<blocks, 256, 0, s>>>(pg, py, po, part, db, units);
+  else relu_grad_kernel<8><<<blocks, 256, 0, s>>>(pg, py, po, part, db, units);
+  if (part) bias_sum<<<c / 16, 1024, 0, s>>>(part, (int)blocks, c, db);
   FC_HIP(hipGetLastError());
   return FC_OK;
+}
+
+int fc_net_relu_grad_dev(int device, const void* gy, const void* y, void* gm, float* db,
+                         long long voxels, int c, void* stream) {
+  return relu_grad(device, gy, y, gm, nullptr, kReluRows, db, voxels, c, stream);
+}
+
+int fc_net_relu_grad_parts_dev(int device, const void* gy, const void* y, void* gm, float* part,
+                               int rows, float* db, long long voxels, int c, void* stream) {
+  clear_error();
+  FC_CHECK_ARG(part && rows > 0, "null or empty scratch");
+  return relu_grad(device, gy, y, gm, part, std::min(rows, kReluRows), db, voxels, c, stream);
 }
 
 int fc_net_weights_dev(int device, const float* const* src, const long long* counts, int n,

@@ -90,12 +90,13 @@ class _Conv(torch.autograd.Function):
 def _masked(gy, y, cout, relu):
     """The gradient at the convolution's sum, and the bias gradient (None: not yet summed)."""
     if relu and gy.dtype == torch.bfloat16 and not torch.is_grad_enabled():
-        # mask and bias gradient in one pass
+        # mask and bias gradient in one pass, the bias's sums in a fixed order
         g0, gy = _packed(gy), torch.empty_like(y)
-        db = torch.zeros(cout, dtype=torch.float32, device=y.device)
-        _native.check(_native.lib().fc_net_relu_grad_dev(
-            y.device.index, g0.data_ptr(), y.data_ptr(), gy.data_ptr(), db.data_ptr(),
-            y.numel() // cout, cout, _stream(y)))
+        part = torch.empty((1024, cout), dtype=torch.float32, device=y.device)
+        db = torch.empty(cout, dtype=torch.float32, device=y.device)
+        _native.check(_native.lib().fc_net_relu_grad_parts_dev(
+            y.device.index, g0.data_ptr(), y.data_ptr(), gy.data_ptr(), part.data_ptr(),
+            part.shape[0], db.data_ptr(), y.numel() // cout, cout, _stream(y)))
         return gy, db
     if relu:
         gy = gy * (y > 0)

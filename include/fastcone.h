@@ -227,7 +227,10 @@ int fc_net_weights_dev(int device, const float* const* src, const long long* cou
  * fc_net_up_cat_grad_dev: ga = the gradient with respect to a for output gradient g (b's is a channel
  * slice of g). fc_net_skip_pool_grad_dev: g = gs + the pooling's gradient for gp, gs holding c
  * channels of every gs_pitch. fc_net_relu_grad_dev: gm = gy where y > 0, else 0, and db[c] (FP32) +=
- * its sum over the voxels, c = 16, 32 or 64. No counterpart in the reference. */
+ * its sum over the voxels, c = 16, 32 or 64, by float atomics (the last bits depend on the order in
+ * which blocks end). fc_net_relu_grad_parts_dev: the same with db[c] = the sum, added in a fixed order
+ * by way of `part`, scratch of rows x c floats (rows up to 1024 are used): equal inputs and rows give
+ * equal bits. No counterpart in the reference. */
 int fc_net_pool_dev(int device, const void* x, void* y, int N, int D, int H, int W, int c,
                     void* stream);
 int fc_net_up_cat_dev(int device, const void* a, const void* b, void* out, int N, int D, int H,
@@ -238,6 +241,8 @@ int fc_net_skip_pool_grad_dev(int device, const void* gs, int gs_pitch, const vo
                               int N, int D, int H, int W, int c, void* stream);
 int fc_net_relu_grad_dev(int device, const void* gy, const void* y, void* gm, float* db,
                          long long voxels, int c, void* stream);
+int fc_net_relu_grad_parts_dev(int device, const void* gy, const void* y, void* gm, float* part,
+                               int rows, float* db, long long voxels, int c, void* stream);
 /* One 16x16x32 BF16 and one 16x16x4 FP32 MFMA product of row-major A, B (single wave): checks the
  * operand / result lane layouts the convolution kernels assume. */
 int fc_mfma_layout_probe(int device, const void* A32, const void* B32, const float* A4,

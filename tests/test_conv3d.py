@@ -461,3 +461,41 @@ def test_conv_large_layers(gpu, cin, cout, shape):
                     part = x[n:n + 1, lo:hi, ya:yb].contiguous()
                     ref = conv3d(part, w, b, True)[0, z - lo, y0 - ya:min(y0 + 16, H) - ya]
                     assert torch.equal(y[n, z, y0:y0 + 16], ref)
+
+
+def test_bias_gradients_are_reproducible(gpu):
+    # two passes over the same batch: the ReLU layers' bias gradients bit for bit (many blocks add to
+    # each; the weight gradients are float atomics)
+    from fastcone_amd.unet import UNet3D
+    net = UNet3D(seed=5).to(gpu)
+    x = torch.rand((2, 48, 64, 64), generator=torch.Generator().manual_seed(1)).to(gpu) * 0.02
+    runs = []
+    for _ in range(3):
+        net.zero_grad(set_to_none=True)
+        ((net(x) - 0.9 * x) ** 2).mean().mul(UNet3D.SCALE ** 2).backward()
+        runs.append({k: p.grad.clone() for k, p in net.b.items()})
+    for r in runs[1:]:
+        assert all(torch.equal(r[k], runs[0][k]) for k in r)
+
+
+@pytest.mark.parametrize("voxels", [1, 127, 4097, 70001])
+@pytest.mark.parametrize("c,rows", [(16, 1024), (32, 3), (64, 65), (64, 5000)])
+def test_ordered_bias_gradient(gpu, voxels, c, rows):
+    # fewer and more rows of scratch than blocks, rows that are no multiple of a block's 64; bound as
+    # in test_relu_gradient_kernel, and nothing written past the rows that were given
+    import ctypes
+    from fastcone_amd import _native
+    g = torch.Generator().manual_seed(voxels + c)
+    gy = torch.randn((voxels, c), generator=g).to(torch.bfloat16)
+    y = torch.randn((voxels, c), generator=g).to(torch.bfloat16)
+    ref = gy * (y > 0)
+    gd, yd = gy.to(gpu), y.to(gpu)
+    gm, part, db = torch.empty_like(gd), torch.full((rows + 1, c), 7.0, device=gpu), \
+        torch.full((c,), 3.0, device=gpu)
+    _native.check(_native.lib().fc_net_relu_grad_parts_dev(
+        gpu.index, gd.data_ptr(), yd.data_ptr(), gm.data_ptr(), part.data_ptr(), rows,
+        db.data_ptr(), voxels, c, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.equal(gm.cpu(), ref)
+    bound = ref.double().abs().sum(0) * (voxels ** 0.5 + 1.0) * 2.0 ** -24 + 1e-30
+    assert bool(((db.double().cpu() - ref.double().sum(0)).abs() <= bound).all())
+    assert bool((part[rows] == 7.0).all())
