@@ -534,8 +534,8 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
     auto fetch_g = [&](int yg) {
       const uint16_t* p = a.dy + ((n * a.D + z) * a.H + yg) * a.W * a.cout + co0 + 8 * (lane & 1);
       pg0 = pg1 = u32x4{0u, 0u, 0u, 0u};
-      if (g0ok) pg0 = *reinterpret_cast<const u32x4*>(p + (long long)gv0 * a.cout);
-      if (g1ok) pg1 = *reinterpret_cast<const u32x4*>(p + (long long)gv1 * a.cout);
+      if (g0ok) pg0 = *reinterpret_cast<const u32x4_a2*>(p + (long long)gv0 * a.cout);
+      if (g1ok) pg1 = *reinterpret_cast<const u32x4_a2*>(p + (long long)gv1 * a.cout);
     };
     auto put_x = [&]() {
 #pragma unroll

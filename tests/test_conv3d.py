@@ -499,3 +499,32 @@ def test_ordered_bias_gradient(gpu, voxels, c, rows):
     bound = ref.double().abs().sum(0) * (voxels ** 0.5 + 1.0) * 2.0 ** -24 + 1e-30
     assert bool(((db.double().cpu() - ref.double().sum(0)).abs() <= bound).all())
     assert bool((part[rows] == 7.0).all())
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 32), (48, 16), (1, 16), (16, 1)])
+def test_output_gradient_at_an_odd_element(gpu, cin, cout):
+    # without a ReLU the gradient is read where it lies: one that starts off 16 bytes gives the bits
+    # of an aligned copy (whole numbers: every sum is exact)
+    from fastcone_amd.unet import _UpCatConv, conv3d
+    g = torch.Generator().manual_seed(cin)
+    whole = lambda n, lim: torch.randint(-lim, lim + 1, (n,), generator=g).float().to(gpu)
+    shape = (2, 4, 6, 34)
+    x = whole(int(np.prod(shape)) * cin, 2).to(torch.bfloat16).view(shape + (cin,))
+    w, b = whole(cout * 27 * cin, 1).view(cout, 27, cin), whole(cout, 2)
+    gy = whole(int(np.prod(shape)) * cout + 1, 1).to(torch.float32 if cout == 1 else torch.bfloat16)
+    gy = gy[1:].view(shape + (cout,))
+    assert gy.is_contiguous() and gy.data_ptr() % 16
+    coarse = whole(int(np.prod(shape)) // 8 * 32, 2).to(torch.bfloat16).view(2, 2, 3, 17, 32)
+    res = []
+    for grad in (gy, gy.clone()):
+        if cin == 48:
+            p = [t.detach().requires_grad_(True) for t in (coarse, x[..., 32:].contiguous(), w, b)]
+            y = _UpCatConv.apply(*p, False)
+        else:
+            # the first layer's input has no gradient
+            p = [t.detach().requires_grad_(t is not x or cin > 1) for t in (x, w, b)]
+            y = conv3d(*p, False)
+        y.backward(grad)
+        res.append([t.grad for t in p if t.requires_grad])
+    for u, v in zip(*res):
+        assert torch.equal(u, v)
