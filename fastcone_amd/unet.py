@@ -53,6 +53,22 @@ def _bf16_weights(ws, device):
     return [t.view(w.shape) for t, w in zip(out.split(n), ws)]
 
 
+def _activation(t):
+    return t.dim() == 5 and t.dtype == torch.bfloat16 and t.is_contiguous()
+
+
+def _check_weights(w32, wb):
+    assert wb is None or (wb.dtype == torch.bfloat16 and wb.is_contiguous() and
+                          wb.shape == w32.shape and wb.device == w32.device)
+
+
+def _check_up_cat(a, b):
+    N, D, H, W, _ = b.shape
+    assert _activation(a) and _activation(b) and a.device == b.device
+    n, d, h, w, _ = a.shape
+    assert n == N and 2 * d == D and 2 * h == H and 2 * w == W
+
+
 class _Conv(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w32, b32, cin, cout, relu, wb=None):
@@ -117,6 +133,7 @@ def _dgrad(gy, wb, shape, cout):
 def conv3d(x, w, b, relu, wb=None):
     """x: [N, D, H, W, Cin] BF16; w: [Cout, 27, Cin] FP32 (wb: its BF16 copy); b: [Cout] FP32."""
     cout, _, cin = w.shape
+    _check_weights(w, wb)
     return _Conv.apply(x, w, b, cin, cout, relu, wb)
 
 
@@ -138,6 +155,7 @@ class _Pool(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x):
         N, D, H, W, C = x.shape
+        assert _activation(x)
         y = torch.empty((N, D // 2, H // 2, W // 2, C), dtype=x.dtype, device=x.device)
         _native.check(_native.lib().fc_net_pool_dev(x.device.index, x.data_ptr(), y.data_ptr(), N,
                                                     D, H, W, C, _stream(x)))
@@ -165,6 +183,7 @@ class _UpCat(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b):
         N, D, H, W, cb = b.shape
+        _check_up_cat(a, b)
         ctx.ca = a.shape[4]
         out = torch.empty((N, D, H, W, ctx.ca + cb), dtype=b.dtype, device=b.device)
         _native.check(_native.lib().fc_net_up_cat_dev(b.device.index, a.data_ptr(), b.data_ptr(),
@@ -192,6 +211,9 @@ class _UpCatConv(torch.autograd.Function):
     def forward(ctx, a, b, w32, b32, relu, wb=None):
         N, D, H, W, cb = b.shape
         cout, _, cin = w32.shape
+        _check_up_cat(a, b)
+        assert a.shape[4] + cb == cin
+        _check_weights(w32, wb)
         if wb is None:
             wb = w32.to(torch.bfloat16).contiguous()
         y = torch.empty((N, D, H, W, cout), dtype=b.dtype, device=b.device)
@@ -235,7 +257,7 @@ class UNet3D(torch.nn.Module):
 
     def _c(self, x, name, wb):
         _, cin, cout, relu = next(L for L in LAYERS if L[0] == name)
-        return conv3d(x, self.w[name], self.b[name], relu, wb[name])
+        return _Conv.apply(x, self.w[name], self.b[name], cin, cout, relu, wb[name])
 
     def _up(self, a, b, name, wb):
         relu = next(L for L in LAYERS if L[0] == name)[3]
