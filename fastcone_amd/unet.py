@@ -167,7 +167,7 @@ class _Pool(torch.autograd.Function):
         # the skip gradient is a channel slice of the concatenation's: voxels at a fixed pitch
         pitch = gs.stride(3)
         if gs.stride() != (D * H * W * pitch, H * W * pitch, W * pitch, pitch, 1) or pitch % 8 \
-                or gs.data_ptr() % 16:
+                or pitch < C or gs.data_ptr() % 16:
             gs, pitch = _packed(gs), C
         gp = _packed(gp)
         g = torch.empty((N, D, H, W, C), dtype=gs.dtype, device=gs.device)

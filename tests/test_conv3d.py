@@ -528,3 +528,25 @@ def test_output_gradient_at_an_odd_element(gpu, cin, cout):
         res.append([t.grad for t in p if t.requires_grad])
     for u, v in zip(*res):
         assert torch.equal(u, v)
+
+
+@pytest.mark.parametrize("skip", ["expanded", "transposed", "none"])
+@pytest.mark.parametrize("pooled", ["expanded", "dense"])
+def test_pool_gradient_layouts(gpu, skip, pooled):
+    # gradients as autograd hands them over: one value per channel for all voxels (the gradient of a
+    # sum over voxels), another order of the axes, none at all; against avgpool2 and the tensor itself
+    from fastcone_amd.unet import _Pool, avgpool2
+    g = torch.Generator().manual_seed(3)
+    bf = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).to(gpu)
+    shape, coarse = (2, 4, 6, 8, 16), (2, 2, 3, 4, 16)
+    e = bf(*shape)
+    gs = {"expanded": bf(16).expand(shape), "none": None,
+          "transposed": bf(2, 4, 8, 6, 16).transpose(2, 3)}[skip]
+    gp = bf(16).expand(coarse) if pooled == "expanded" else bf(*coarse)
+    grads = []
+    for ours in (True, False):
+        x = e.clone().requires_grad_(True)
+        y, p = _Pool.apply(x) if ours else (x * 1.0, avgpool2(x))
+        torch.autograd.backward([p] if gs is None else [y, p], [gp] if gs is None else [gs, gp])
+        grads.append(x.grad)
+    assert rel(grads[0].cpu(), grads[1].cpu()) < 2.0 ** -8
