@@ -45,3 +45,32 @@ def test_chunked_host_volume(gpu):
     cone.backproject(rec, proj, np.array([0.0, 1.0, 2.0], np.float32), 500.0,
                      np.full(3, 50.0, np.float32), pixelWidth=0.8)
     assert np.array_equal(rec, before)
+
+
+@pytest.mark.parametrize("shape,nv,nh,nw", [((100, 111, 119), 130, 96, 96), ((64, 128, 129), 131, 89, 91)])
+def test_chunked_backprojection(gpu, shape, nv, nh, nw):
+    # a random volume and projections, both above the size that is copied in chunks, up and down,
+    # against slabs and view batches small enough for plain copies: the sums are split otherwise, so
+    # equal up to a few FP32 roundings of a voxel's sum of nv terms (sqrt(nv) 2^-24 < 1e-6)
+    from fastcone_amd import fastcone as cone
+    rng = np.random.default_rng(nv)
+    start = rng.standard_normal(shape).astype(np.float32)
+    proj = rng.standard_normal((nv, nh, nw)).astype(np.float32)
+    assert start.nbytes >= 4 << 20 and proj.nbytes >= 4 << 20
+    given = proj.copy()
+    out = []
+    try:
+        for voxels, views in ((0, 0), (16 * shape[1] * shape[2], 40)):
+            assert 4 * voxels < 4 << 20 and 4 * views * nh * nw < 4 << 20
+            cone.set_tile_limits(voxels, views)
+            rec = start.copy()
+            cone.backproject(rec, proj, np.linspace(0.0, 6.0, nv).astype(np.float32), 500.0,
+                             np.full(nv, shape[0] / 2, np.float32), pixelWidth=0.9,
+                             norm=np.ones(nv, np.float32))
+            out.append(rec.astype(np.float64))
+    finally:
+        cone.set_tile_limits(0, 0)
+    added = out[1] - start
+    assert np.linalg.norm(added) > np.linalg.norm(start)
+    assert np.abs(out[0] - out[1]).max() < 1e-5 * np.abs(added).max()
+    assert np.array_equal(proj, given)
