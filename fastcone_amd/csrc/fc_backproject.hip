@@ -280,7 +280,7 @@ __device__ __forceinline__ void column_samples(float* acc, uint32_t col, float a
 
 // The same for a tilted detector: column, row and weight by voxel, from the view's forms at the
 // column's first voxel.
-template <int MODE, bool CLAMP>
+template <int MODE>
 __device__ __forceinline__ void tilted_samples(float* acc, uint32_t T0, float A, float B, float C,
                                                const ViewEntry& E, float umax, float vmax) {
 #pragma unroll
@@ -288,8 +288,8 @@ __device__ __forceinline__ void tilted_samples(float* acc, uint32_t T0, float A,
     if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four samples at a time in registers
     const float kf = (float)k;
     const float rc = __builtin_amdgcn_rcpf(fmaf(kf, E.c[3], C));  // 1 ulp, as the positions
-    float u = fmaf(kf, E.a[3], A) * rc, v = fmaf(kf, E.b[3], B) * rc;
-    if (CLAMP) u = clampf(u, 0.0f, umax), v = clampf(v, 0.0f, vmax);
+    const float u = clampf(fmaf(kf, E.a[3], A) * rc, 0.0f, umax);
+    const float v = clampf(fmaf(kf, E.b[3], B) * rc, 0.0f, vmax);
     float wt = E.s;
     if constexpr (MODE == FC_BP_FDK) wt = E.s * rc * rc;
     if constexpr (MODE == FC_BP_KATSEVICH) wt = E.s * rc;
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
         if (inner) column_samples<false>(acc, col0, au, vb, dv, wt, 0.0f);
         else column_samples<true>(acc, col0, au, vb, dv, wt, vmax);
       } else {
-        tilted_samples<MODE, true>(acc, T0, A, B, C, E, umax, vmax);
+        tilted_samples<MODE>(acc, T0, A, B, C, E, umax, vmax);
       }
     }
   }

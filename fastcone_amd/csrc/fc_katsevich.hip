@@ -43,16 +43,6 @@ __device__ __forceinline__ double kappa_w(const KatGeom& g, double gam, double p
   return g.SDD * g.hp / g.R * (psi * cos(gam) + pc * sin(gam));
 }
 
-// Linear interpolation along a row of nw values at column coordinate c, zero outside.
-__device__ __forceinline__ float row_lerp(const float* row, int nw, float c) {
-  float fc = floorf(c);
-  int j0 = (int)fc;
-  float t = c - fc, s = 0.0f;
-  if (j0 >= 0 && j0 < nw) s += (1.0f - t) * row[j0];
-  if (j0 + 1 >= 0 && j0 + 1 < nw) s += t * row[j0 + 1];
-  return s;
-}
-
 // Tables: fwd[m][j] = detector row coordinate of kappa line m at column j;
 // bwd[i][j] = (m + t) with w_k(g_j, psi_m..m+1) bracketing row i's height, or -1 outside;
 // cone[i] = the cone-angle weight of row i.
@@ -209,9 +199,11 @@ __global__ __launch_bounds__(256) void kat_view_table(KatGeom g, float4* __restr
   vt[k] = make_float4((float)cos(l), (float)sin(l), (float)(g.zs0 + k * g.dl * g.hp), 0.0f);
 }
 
-// 1 / b, a / b and the square root of x, correctly rounded like the operators, in 3, 3 more and 8
-// instructions (the operators' 10, 10 and 14 also scale against overflow and underflow of their
-// intermediate values, which no volume and helix of finite voxel coordinates gets near).
+// 1 / b, a / b and the square root of x in 3, 3 more and 8 instructions (the operators' 10, 10 and 14
+// also scale against overflow and underflow of their intermediate values, which no volume and helix of
+// finite voxel coordinates gets near). That one Newton step rounds correctly is a property of this
+// GPU's v_rcp_f32 and v_rsq_f32, not of any 1-ulp start: compared on gfx950, the results equal the
+// operators' for all 2^23 mantissas b, all floats x in [1, 4) and 2^30 random pairs (a, b).
 __device__ __forceinline__ float recip(float b) {
   const float y = __builtin_amdgcn_rcpf(b);
   return fmaf(fmaf(-b, y, 1.0f), y, y);
@@ -274,8 +266,7 @@ __device__ __forceinline__ bool kat_entry(const KatBpArgs& a, int k, float X, fl
 
 // kZR voxels of a column at rows rr = (q + qa) dr + r0: acc[q] += wgt * sample if rbot <= rr <= rtop. The
 // sample is bilinear between the elements at `at` + row * pitch and the next row's, `at` standing for
-// row 0 of the column, an LDS or a global address. [lo, hi] is the window within the copied rows;
-// INSIDE: all rows of all lanes are inside it.
+// row 0 of the column, an LDS or a global address. [lo, hi] is the window within the copied rows.
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef const __attribute__((address_space(3))) f2* lds_f2;
 template <bool LDS, class P>
