@@ -173,13 +173,16 @@ __device__ __forceinline__ void global_samples(float* acc, const BpArgs& a, size
       wt[g] = s;
       if constexpr (MODE == FC_BP_FDK) wt[g] = s * rc * rc;
       if constexpr (MODE == FC_BP_KATSEVICH) wt[g] = s * rc;
-      const float fu = floorf(u), fv = floorf(v);
+      const bool on = u > -1.0f && u < (float)a.nw && v > -1.0f && v < (float)a.nh;
+      // off the detector u and v may be anything, infinite or NaN on the source's plane: bounded
+      // before they become integers
+      const float fu = fminf(fmaxf(floorf(u), -1.0f), (float)a.nw);
+      const float fv = fminf(fmaxf(floorf(v), -1.0f), (float)a.nh);
       au[g] = u - fu, av[g] = v - fv;
       const int iu = (int)fu, iv = (int)fv;
-      const bool on = u > -1.0f && u < (float)a.nw && v > -1.0f && v < (float)a.nh;
-      const int c0 = min(max(iu, 0), a.nw - 1), c1 = min(max(iu, -1) + 1, a.nw - 1);
+      const int c0 = min(max(iu, 0), a.nw - 1), c1 = min(iu + 1, a.nw - 1);
       const size_t r0 = vbase + (size_t)min(max(iv, 0), a.nh - 1) * a.nw;
-      const size_t r1 = vbase + (size_t)min(max(iv, -1) + 1, a.nh - 1) * a.nw;
+      const size_t r1 = vbase + (size_t)min(iv + 1, a.nh - 1) * a.nw;
       const bool x0 = on && iu >= 0, x1 = on && iu + 1 < a.nw, y0 = iv >= 0, y1 = iv + 1 < a.nh;
       p[g][0] = load_elem<DT>(a.proj, r0 + c0);
       p[g][1] = load_elem<DT>(a.proj, r0 + c1);

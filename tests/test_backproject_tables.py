@@ -86,3 +86,27 @@ def test_windows_wider_than_the_tile(gpu, nv, mode, mis, dt, pw, det):
     out = ops.backproject(y.to(gpu), g, mode, norm=norm, out=base.clone())
     ref = oracle.backproject(prob, y.float().numpy(), vol, mode=mode, norm=norm)
     assert rel((out.double() - base.double()).cpu(), ref) < 5e-5
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+def test_source_inside_the_volume(gpu, mode, dt):
+    # the source's plane passes through voxels, whose detector coordinates are infinite there; those a
+    # voxel and more from every view's plane are compared
+    from fastcone_amd import ops
+    from fastcone_amd.geometry import Geometry
+    rng = np.random.default_rng(mode)
+    ang = np.array([0.0, 0.5, 1.0, 1.5, 0.27]) * np.pi
+    vol, det, D = (18, 33, 20), (30, 40), 8.0
+    hmid = np.full(5, 9.0)
+    g = Geometry.circular(ang, D, 0.5, vol, det, hmid=hmid)
+    prob = oracle.Problem(ang, hmid, D, 0.5, vol_dim=vol[::-1], proj_dim=det[::-1])
+    y = torch.from_numpy(rng.standard_normal(g.proj_shape).astype(np.float32)).to(
+        getattr(torch, dt))
+    out = ops.backproject(y.to(gpu), g, mode, norm=np.ones(5, np.float32)).cpu().numpy()
+    ref = oracle.backproject(prob, y.float().numpy(), vol, mode=mode, norm=np.ones(5))
+    yy, xx = np.meshgrid(np.arange(33) - 16, np.arange(20) - 10, indexing="ij")
+    c = D + xx[..., None] * np.cos(ang) + yy[..., None] * np.sin(ang)
+    far = np.abs(c).min(axis=-1) >= 1.0
+    assert (np.abs(c).min(axis=-1) == 0.0).any() and far.sum() > 300
+    assert rel(out[:, far], ref[:, far]) < 5e-5
