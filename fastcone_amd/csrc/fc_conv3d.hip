@@ -587,6 +587,35 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
         ++y;
       }
     }
+    // A product of a padding zero with an infinite value is NaN, where the sum has no such term: a
+    // unit with a NaN is summed again, term by term
+    float sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 27 * 4; ++q) sum += 0.0f * acc[q / 36][q / 12 % 3][q / 4 % 3][q % 4];
+    if (__any(sum != 0.0f)) {
+#pragma unroll
+      for (int q = 0; q < 27; ++q) acc[q / 9][q / 3 % 3][q % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int y = y0; y < y1; ++y)
+        for (int x = x0; x < min(x0 + kWgSeg, a.W); ++x) {
+          const uint16_t* gp = a.dy + ((n * a.D + z) * a.H + y) * a.W * a.cout + co0 + 4 * g;
+#pragma unroll
+          for (int q = 0; q < 9; ++q) {
+            const int zz = z + q / 3 - 1, yy = y + q % 3 - 1;
+            if (zz < 0 || zz >= a.D || yy < 0 || yy >= a.H) continue;
+            const float f =
+                bf2f(xp[((((n * a.D + zz) >> up) * xh + (yy >> up)) * xw + (x >> up)) * xc + m]);
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) {
+              const int gx = x + 1 - dx;
+              if (gx < 0 || gx >= a.W) continue;
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                acc[q / 3][q % 3][dx][r] =
+                    fmaf(bf2f(gp[(long long)gx * a.cout + r]), f, acc[q / 3][q % 3][dx][r]);
+            }
+          }
+        }
+    }
   }
   // sum over the block's waves, kWgRed taps at a time: part[wave][tap][co][ci]
   float* part = reinterpret_cast<float*>(lds);
@@ -948,6 +977,34 @@ __global__ __launch_bounds__(64 * kNrWaves) void conv_wgrad_narrow(WgNarrowArgs 
         wave_sync();
         ++y;
       }
+    }
+    // As in conv_wgrad_mfma, and for the zero parts of a value that is multiplied by an infinite one.
+    // The sums go to the rows of the first part.
+    float sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < MT * 12; ++q) sum += 0.0f * acc[q / 12][q / 4 % 3][q % 4];
+    if (__any(sum != 0.0f)) {
+#pragma unroll
+      for (int q = 0; q < 3 * MT; ++q) acc[q / 3][q % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int y = y0; y < y1; ++y)
+        for (int x = x0; x < min(x0 + kWgSeg, a.W); ++x) {
+          const uint16_t* wp = a.wide + ((n * a.D + z) * a.H + y) * a.W * 16 + m;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int d = 4 * g + r;
+            const int zz = z + (FLIP ? 1 - d / 3 : d / 3 - 1), yy = y + (FLIP ? 1 - d % 3 : d % 3 - 1);
+            if (d >= 9 || zz < 0 || zz >= a.D || yy < 0 || yy >= a.H) continue;
+            const long long i = ((n * a.D + zz) * a.H + yy) * a.W + x;
+            const float f = FLIP ? static_cast<const float*>(a.narrow)[i]
+                                 : bf2f(static_cast<const uint16_t*>(a.narrow)[i]);
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) {
+              const int wx = FLIP ? x + dx - 1 : x + 1 - dx;
+              if (wx >= 0 && wx < a.W)
+                acc[0][dx][r] = fmaf(f, bf2f(wp[(long long)wx * 16]), acc[0][dx][r]);
+            }
+          }
+        }
     }
   }
   // sum over the block's waves and the parts, one shift at a time: part[wave][row][channel]

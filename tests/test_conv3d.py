@@ -550,3 +550,35 @@ def test_pool_gradient_layouts(gpu, skip, pooled):
         torch.autograd.backward([p] if gs is None else [y, p], [gp] if gs is None else [gs, gp])
         grads.append(x.grad)
     assert rel(grads[0].cpu(), grads[1].cpu()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("cin,cout", [(1, 16), (16, 1), (16, 32), (48, 16)])
+@pytest.mark.parametrize("where", [(0, 0, 0, 0), (1, 2, 16, 33), (0, 1, 16, 0), (1, 1, 7, 31)])
+@pytest.mark.parametrize("operand", ["input", "gradient"])
+def test_weight_gradients_of_infinite_values(gpu, cin, cout, where, operand):
+    # an infinite value reaches the taps that it is a term of, and not those that lie in the padding
+    # there; segments of 32 voxels and one past, volume borders and none. Reference: FP64 sums over
+    # the voxels of each tap that lie in the volume; finite ones < 1e-5 as above
+    from fastcone_amd.unet import conv3d
+    g = torch.Generator().manual_seed(cin + sum(where))
+    shape = (2, 3, 17, 34)
+    _, D, H, W = shape
+    x = torch.randn(shape + (cin,), generator=g).to(torch.bfloat16)
+    gy = torch.randn(shape + (cout,), generator=g)
+    gy = gy.to(torch.bfloat16) if cout != 1 else gy
+    (x if operand == "input" else gy)[where + (0,)] = float("inf")
+    w = torch.zeros((cout, 27, cin), device=gpu, requires_grad=True)
+    conv3d(x.to(gpu), w, torch.zeros(cout, device=gpu), False).backward(gy.to(gpu))
+    dw = w.grad.cpu().double()
+    ref = torch.empty_like(dw)
+    cut = lambda d, n: (slice(max(0, -d), n - max(0, d)), slice(max(0, d), n + min(0, d)))
+    for tap in range(27):
+        z, y, xx = (cut(tap // 9 - 1, D), cut(tap // 3 % 3 - 1, H), cut(tap % 3 - 1, W))
+        a = gy[:, z[0], y[0], xx[0]].double()
+        b = x[:, z[1], y[1], xx[1]].double()
+        ref[:, tap] = (a[..., :, None] * b[..., None, :]).sum((0, 1, 2, 3))
+    finite = ref.isfinite()
+    assert not bool(finite.all())
+    assert torch.equal(dw[~finite], ref[~finite])
+    if bool(finite.any()):  # not with one input channel and its infinite value inside
+        assert rel(dw[finite], ref[finite]) < 1e-5
