@@ -490,6 +490,22 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Mask of the eight BF16 voxels x .. x + 7 of a fragment that lie in [0, W), as do those `shift` on.
+__device__ __forceinline__ u32x4 pairs_inside(int x, int shift, int W) {
+  u32x4 in;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int v = x + 2 * q;
+    const bool lo = v < W && v + shift >= 0 && v + shift < W;
+    const bool hi = v + 1 < W && v + 1 + shift >= 0 && v + 1 + shift < W;
+    in[q] = (lo ? 0xffffu : 0u) | (hi ? 0xffff0000u : 0u);
+  }
+  return in;
+}
+__device__ __forceinline__ bf16x8 masked(bf16x8 v, u32x4 mask) {
+  return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & mask);
+}
+
 __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
   __shared__ __align__(16) char lds[4 * kWgWaveB];
   static_assert(4 * kWgRed * 1024 <= 4 * kWgWaveB, "the reduction reuses the rows' LDS");
@@ -587,34 +603,41 @@ __global__ __launch_bounds__(256, 2) void conv_wgrad_mfma(WgArgs a) {
         ++y;
       }
     }
-    // A product of a padding zero with an infinite value is NaN, where the sum has no such term: a
-    // unit with a NaN is summed again, term by term
+    // A product of a padding zero with an infinite value is NaN, where the sum has no such term: sums
+    // with a NaN are formed once more, with both factors of these products zero, row by row.
     float sum = 0.0f;
 #pragma unroll
     for (int q = 0; q < 27 * 4; ++q) sum += 0.0f * acc[q / 36][q / 12 % 3][q / 4 % 3][q % 4];
     if (__any(sum != 0.0f)) {
 #pragma unroll
       for (int q = 0; q < 27; ++q) acc[q / 9][q / 3 % 3][q % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int y = y0; y < y1; ++y)
-        for (int x = x0; x < min(x0 + kWgSeg, a.W); ++x) {
-          const uint16_t* gp = a.dy + ((n * a.D + z) * a.H + y) * a.W * a.cout + co0 + 4 * g;
+#pragma unroll 1
+      for (int y = y0; y < y1; ++y) {
+        fetch_g(y);
+        *reinterpret_cast<u32x4*>(gr + lane * 16) = pg0;
+        if (lane < 4) *reinterpret_cast<u32x4*>(gr + (64 + lane) * 16) = pg1;
 #pragma unroll
-          for (int q = 0; q < 9; ++q) {
-            const int zz = z + q / 3 - 1, yy = y + q % 3 - 1;
-            if (zz < 0 || zz >= a.D || yy < 0 || yy >= a.H) continue;
-            const float f =
-                bf2f(xp[((((n * a.D + zz) >> up) * xh + (yy >> up)) * xw + (x >> up)) * xc + m]);
+        for (int dy = 0; dy < 3; ++dy) {
+          const int yy = y + dy - 1;
+          if (yy < 0 || yy >= a.H) continue;
+          fetch_x(yy);
+          put_x();
+          wave_sync();
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx) {
-              const int gx = x + 1 - dx;
-              if (gx < 0 || gx >= a.W) continue;
+          for (int dx = 0; dx < 3; ++dx) {
+            int xs = x0 + 8 * g;
+            asm volatile("" : "+v"(xs));  // a mask at a time in registers
+            const u32x4 in = pairs_inside(xs, 1 - dx, a.W);
+            const bf16x8 A = masked(read_channel(gr + (2 - dx) * 32, lane), in);
 #pragma unroll
-              for (int r = 0; r < 4; ++r)
-                acc[q / 3][q % 3][dx][r] =
-                    fmaf(bf2f(gp[(long long)gx * a.cout + r]), f, acc[q / 3][q % 3][dx][r]);
-            }
+            for (int d = 0; d < 3; ++d)
+              if (z + d - 1 >= 0 && z + d - 1 < a.D)
+                acc[d][dy][dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    A, masked(read_channel(xr + d * kWgSeg * 32, lane), in), acc[d][dy][dx], 0, 0, 0);
           }
+          wave_sync();
         }
+      }
     }
   }
   // sum over the block's waves, kWgRed taps at a time: part[wave][tap][co][ci]
@@ -866,6 +889,17 @@ struct WgNarrowArgs {
   int nseg, nyc, yc;
 };
 
+// Mask of a fragment's finite values.
+__device__ __forceinline__ u32x4 finite_values(bf16x8 v) {
+  const u32x4 u = __builtin_bit_cast(u32x4, v);
+  u32x4 m;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    m[q] = ((u[q] & 0x7f80u) != 0x7f80u ? 0xffffu : 0u) |
+           ((u[q] & 0x7f800000u) != 0x7f800000u ? 0xffff0000u : 0u);
+  return m;
+}
+
 template <bool FLIP>
 __global__ __launch_bounds__(64 * kNrWaves) void conv_wgrad_narrow(WgNarrowArgs a) {
   constexpr int PARTS = FLIP ? 3 : 1, ROWS = 9 * PARTS, MT = (ROWS + 15) / 16;
@@ -978,33 +1012,49 @@ __global__ __launch_bounds__(64 * kNrWaves) void conv_wgrad_narrow(WgNarrowArgs 
         ++y;
       }
     }
-    // As in conv_wgrad_mfma, and for the zero parts of a value that is multiplied by an infinite one.
-    // The sums go to the rows of the first part.
+    // As in conv_wgrad_mfma. A narrow row outside the volume is a row of A, so its products are left out
+    // of the sums instead, and an infinite wide value is multiplied by a narrow value's first part only
+    // (the others may be zero where the value is not).
     float sum = 0.0f;
 #pragma unroll
     for (int q = 0; q < MT * 12; ++q) sum += 0.0f * acc[q / 12][q / 4 % 3][q % 4];
     if (__any(sum != 0.0f)) {
 #pragma unroll
       for (int q = 0; q < 3 * MT; ++q) acc[q / 3][q % 3] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int y = y0; y < y1; ++y)
-        for (int x = x0; x < min(x0 + kWgSeg, a.W); ++x) {
-          const uint16_t* wp = a.wide + ((n * a.D + z) * a.H + y) * a.W * 16 + m;
+#pragma unroll 1
+      for (int y = y0; y < y1; ++y) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int d = 4 * g + r;
-            const int zz = z + (FLIP ? 1 - d / 3 : d / 3 - 1), yy = y + (FLIP ? 1 - d % 3 : d % 3 - 1);
-            if (d >= 9 || zz < 0 || zz >= a.D || yy < 0 || yy >= a.H) continue;
-            const long long i = ((n * a.D + zz) * a.H + yy) * a.W + x;
-            const float f = FLIP ? static_cast<const float*>(a.narrow)[i]
-                                 : bf2f(static_cast<const uint16_t*>(a.narrow)[i]);
+        for (int r = 0; r < 3; ++r) {
+          fetch_n(y + r - 1);
+          put_n(r);
+        }
+        fetch_w(y);
+        *reinterpret_cast<u32x4*>(wr + lane * 16) = pw0;
+        if (lane < 4) *reinterpret_cast<u32x4*>(wr + (64 + lane) * 16) = pw1;
+        wave_sync();
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx) {
-              const int wx = FLIP ? x + dx - 1 : x + 1 - dx;
-              if (wx >= 0 && wx < a.W)
-                acc[0][dx][r] = fmaf(f, bf2f(wp[(long long)wx * 16]), acc[0][dx][r]);
-            }
+        for (int q = 0; q < 3 * MT; ++q) {
+          const int dx = q / MT, i = q % MT;
+          int xs = x0 + 8 * g;
+          asm volatile("" : "+v"(xs));  // a mask at a time in registers
+          const u32x4 in = pairs_inside(xs, FLIP ? dx - 1 : 1 - dx, a.W);
+          const bf16x8 A =
+              masked(__builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(nr + arow[i][0])), in);
+          const bf16x8 B = masked(read_channel(wr + (FLIP ? dx : 2 - dx) * 32, lane), in);
+          const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+          const f32x4 all = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, zero, 0, 0, 0);
+          const f32x4 fin = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, masked(B, finite_values(B)),
+                                                                    zero, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = 16 * i + 4 * g + e, d = j % 9;
+            const int zz = z + (FLIP ? 1 - d / 3 : d / 3 - 1),
+                      yy = y + (FLIP ? 1 - d % 3 : d % 3 - 1);
+            if (zz >= 0 && zz < a.D && yy >= 0 && yy < a.H) acc[i][dx][e] += j < 9 ? all[e] : fin[e];
           }
         }
+        wave_sync();
+      }
     }
   }
   // sum over the block's waves and the parts, one shift at a time: part[wave][row][channel]
