@@ -25,9 +25,12 @@
 // View table: every kTab views the block computes, one thread per view and in FP64, the window of its
 // cube — the projective image of a box lies in the box of its eight corners' images, so the corners'
 // (u, v) widened by a pixel each side bound every tap — and the view's projective forms relative to
-// the window's and the cube's corner, A' = A - u0 C, B' = B - v0 C and C as linear functions of the
-// offset in the cube. There they are small (|A'| < 64 |C|), so rounding them to FP32 moves a tile
-// coordinate by about 4e-6 pixel, less than the FP32 rounding of an absolute coordinate. A view whose
+// the window's and the cube's corners, A' = (A - u0 C) / Cm, B' = (B - v0 C) / Cm and q = C / Cm - 1 as
+// linear functions of the offset in the cube, Cm being the largest C of its lowest plane. There they
+// are small (|A'| < 64, -1 < q <= 0), so rounding them to FP32 moves a tile coordinate by 1.1e-6 pixel
+// (rms; FP64 terms rounded to an absolute coordinate 7e-6), and Cm / C = 1 - q / (1 + q) and the weight
+// have the error of their last rounding (weight 3.6e-8 of it, rms, as from FP64 terms; the square of an
+// FP32 reciprocal of C 1.1e-7). A view whose
 // window does not fit the LDS tile (pixels below about a third of a voxel, very short source
 // distances) is gathered from global memory with explicit bounds, after the views that fit; a view
 // that misses the detector entirely is skipped.
@@ -81,10 +84,11 @@ struct BpArgs {
 };
 
 // One view for one cube: with (dx, dy, dz) a voxel's offset from the cube's first voxel,
-// A' = a0 + a1 dx + a2 dy + a3 dz, likewise B' and C; u - u0 = A' / C, v - v0 = B' / C.
+// A' = a0 + a1 dx + a2 dy + a3 dz, likewise B' and q; u - u0 = A' / (1 + q), v - v0 = B' / (1 + q). For
+// tilted detectors q stands for 1 + q.
 struct ViewEntry {
-  float a[4], b[4], c[4];
-  float s;       // norm
+  float a[4], b[4], q[4];
+  float s;       // norm times the mode's weight at q = 0
   uint32_t org;  // window origin u0 | v0 << 16 (int16 each)
   uint32_t size; // Wu | Wv << 16, or kWinSkip / kWinGlobal
   uint32_t tilted;  // a3 or c3 nonzero
@@ -92,6 +96,7 @@ struct ViewEntry {
 
 // Window pixels [u0, u0 + Wu) x [v0, v0 + Wv) with u0 = floor(min u) - 1 and Wu = floor(max u) - u0
 // + 3, so every tap (iu, iu + 1) of a voxel in the cube lies at least one pixel inside; likewise v.
+template <int MODE>
 __device__ __forceinline__ ViewEntry view_entry(const BpArgs& a, int t, int x0, int y0, int z0) {
   const double* M = a.views + (size_t)t * FC_VIEW_DOUBLES + 12;
   const double X0 = x0 + a.ox, Y0 = y0 + a.oy, Z0 = z0 + a.oz;
@@ -116,7 +121,6 @@ __device__ __forceinline__ ViewEntry view_entry(const BpArgs& a, int t, int x0, 
     vmin = fmin(vmin, v); vmax = fmax(vmax, v);
   }
   ViewEntry e;
-  e.s = a.norm ? a.norm[t] : 1.0f;
   e.org = 0u;
   e.size = kWinGlobal;
   e.tilted = M[2] != 0.0 || M[10] != 0.0;
@@ -135,14 +139,17 @@ __device__ __forceinline__ ViewEntry view_entry(const BpArgs& a, int t, int x0, 
       }
     }
   }
-  e.a[0] = (float)(A0 - u0 * C0);
-  e.b[0] = (float)(B0 - v0 * C0);
-  e.c[0] = (float)C0;
+  const double Cm = C0 + fmax(M[8], 0.0) * ex + fmax(M[9], 0.0) * ey, rm = 1.0 / Cm;
+  const double s = a.norm ? a.norm[t] : 1.0f;
+  e.s = (float)(MODE == FC_BP_FDK ? s * rm * rm : MODE == FC_BP_KATSEVICH ? s * rm : s);
+  e.a[0] = (float)((A0 - u0 * C0) * rm);
+  e.b[0] = (float)((B0 - v0 * C0) * rm);
+  e.q[0] = (float)((e.tilted ? C0 : C0 - Cm) * rm);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    e.a[1 + k] = (float)(M[k] - u0 * M[8 + k]);
-    e.b[1 + k] = (float)(M[4 + k] - v0 * M[8 + k]);
-    e.c[1 + k] = (float)M[8 + k];
+    e.a[1 + k] = (float)((M[k] - u0 * M[8 + k]) * rm);
+    e.b[1 + k] = (float)((M[4 + k] - v0 * M[8 + k]) * rm);
+    e.q[1 + k] = (float)(M[8 + k] * rm);
   }
   return e;
 }
@@ -212,7 +219,7 @@ __device__ __forceinline__ void gather_views(float* acc, const BpArgs& a, ViewEn
   for (int tb = tbeg; tb < tend; tb += kTab) {
     const int n = min(kTab, tend - tb);
     __syncthreads();  // the previous table is no longer read
-    if ((int)threadIdx.x < n) tab[threadIdx.x] = view_entry(a, tb + (int)threadIdx.x, bx0, by0, z0);
+    if ((int)threadIdx.x < n) tab[threadIdx.x] = view_entry<MODE>(a, tb + (int)threadIdx.x, bx0, by0, z0);
     __syncthreads();
     for (int i = 0; i < n; ++i) {
       if ((__builtin_amdgcn_readfirstlane(tab[i].size) & 0xffffu) != kWinGlobal) continue;
@@ -222,7 +229,7 @@ __device__ __forceinline__ void gather_views(float* acc, const BpArgs& a, ViewEn
                                (float)(M[0] * X + M[1] * Y + M[2] * Z0 + M[3]),
                                (float)(M[4] * X + M[5] * Y + M[6] * Z0 + M[7]),
                                (float)(M[8] * X + M[9] * Y + M[10] * Z0 + M[11]), (float)M[2],
-                               (float)M[6], (float)M[10], tab[i].s);
+                               (float)M[6], (float)M[10], a.norm ? a.norm[t] : 1.0f);
     }
   }
 }
@@ -290,7 +297,7 @@ __device__ __forceinline__ void tilted_samples(float* acc, uint32_t T0, float A,
   for (int k = 0; k < kZR; ++k) {
     if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four samples at a time in registers
     const float kf = (float)k;
-    const float rc = __builtin_amdgcn_rcpf(fmaf(kf, E.c[3], C));  // 1 ulp, as the positions
+    const float rc = __builtin_amdgcn_rcpf(fmaf(kf, E.q[3], C));  // 1 ulp, as the positions
     const float u = clampf(fmaf(kf, E.a[3], A) * rc, 0.0f, umax);
     const float v = clampf(fmaf(kf, E.b[3], B) * rc, 0.0f, vmax);
     float wt = E.s;
@@ -430,7 +437,7 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
     __syncthreads();  // the previous table is no longer read
     // one entry more than the table's views: the next view's window
     if ((int)threadIdx.x <= n && tb + (int)threadIdx.x < tend)
-      tab[threadIdx.x] = view_entry(a, tb + (int)threadIdx.x, bx0, by0, z0);
+      tab[threadIdx.x] = view_entry<MODE>(a, tb + (int)threadIdx.x, bx0, by0, z0);
     __syncthreads();
     if (tb == tbeg) {
       const uint32_t org = __builtin_amdgcn_readfirstlane(tab[0].org),
@@ -476,17 +483,15 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
       const uint32_t T0 = lds_address(T);
       const float A = fmaf(dx, E.a[1], fmaf(dy, E.a[2], E.a[0]));
       const float B = fmaf(dx, E.b[1], fmaf(dy, E.b[2], E.b[0]));
-      const float C = fmaf(dx, E.c[1], fmaf(dy, E.c[2], E.c[0]));
+      const float q = fmaf(dx, E.q[1], fmaf(dy, E.q[2], E.q[0]));
       if (__builtin_amdgcn_readfirstlane(E.tilted) == 0u) {
         // Columns independent of z: u and the weight are per column, the row is linear in z.
-        // A 1-ulp reciprocal refined by one Newton step
-        float rc = __builtin_amdgcn_rcpf(C);
-        rc = fmaf(rc, fmaf(-C, rc, 1.0f), rc);
+        const float p = -q * __builtin_amdgcn_rcpf(1.0f + q), rc = 1.0f + p;  // Cm / C
         const float u = clampf(A * rc, 0.0f, umax);
         const float vb = B * rc, dv = E.b[3] * rc;
         float wt = E.s;
-        if constexpr (MODE == FC_BP_FDK) wt = E.s * rc * rc;
-        if constexpr (MODE == FC_BP_KATSEVICH) wt = E.s * rc;
+        if constexpr (MODE == FC_BP_FDK) wt = fmaf(E.s, p * (p + 2.0f), E.s);
+        if constexpr (MODE == FC_BP_KATSEVICH) wt = fmaf(E.s, p, E.s);
         const uint32_t col0 = T0 + 4u * (uint32_t)(int)u;
         const float au = __builtin_amdgcn_fractf(u);
         // Voxels outside the volume (partial cubes) are kept inside the buffer by clamping; in whole
@@ -494,7 +499,7 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
         if (inner) column_samples<false>(acc, col0, au, vb, dv, wt, 0.0f);
         else column_samples<true>(acc, col0, au, vb, dv, wt, vmax);
       } else {
-        tilted_samples<MODE>(acc, T0, A, B, C, E, umax, vmax);
+        tilted_samples<MODE>(acc, T0, A, B, q, E, umax, vmax);
       }
     }
   }
