@@ -990,7 +990,9 @@ __global__ __launch_bounds__(256) void adj_rays(AdjVArgs a) {
   __shared__ float red[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int per_view = a.tiles_w * a.tiles_h;
-  const int t = (int)(blockIdx.x / (unsigned)per_view), tile = (int)blockIdx.x - t * per_view;
+  const unsigned b = blockIdx.y * gridDim.x + blockIdx.x;
+  const int t = (int)(b / (unsigned)per_view), tile = (int)(b - (unsigned)t * (unsigned)per_view);
+  if (t >= a.nviews) return;
   const int ty = tile / a.tiles_w, tx = tile - ty * a.tiles_w;
   const int j = tx * kTile + (wave & 1) * 8 + (lane >> 3);
   const int i = ty * kTile + (wave >> 1) * 8 + (lane & 7);
@@ -1441,6 +1443,16 @@ __global__ __launch_bounds__(256) void gather_bench_lds_ray(FpArgs a, int reps,
   if (acc == 12345.678f) sink[0] = acc;
 }
 
+// The most blocks of a launch in x: with 2^32 threads and more the launch takes their number modulo
+// 2^32, without an error.
+constexpr long long kMaxBlocks = 1 << 22;
+
+// Grid of n blocks, numbered blockIdx.y * gridDim.x + blockIdx.x; the last row may have more than n.
+dim3 block_grid(long long n) {
+  const long long x = std::min(n, kMaxBlocks);
+  return dim3((unsigned)x, (unsigned)((n + x - 1) / x));
+}
+
 int max_steps_for(const int vs[3], double h) {
   double diag = sqrt((double)(vs[0] + 2) * (vs[0] + 2) + (double)(vs[1] + 2) * (vs[1] + 2) +
                      (double)(vs[2] + 2) * (vs[2] + 2));
@@ -1651,6 +1663,10 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
   FC_CHECK_ARG((long long)a.nbz * a.nsplit <= 65535, "volume too large for the adjoint grid");
   const size_t nwin = (size_t)a.nbx * a.nby * a.nbz * a.nviews;
   const size_t nrays = (size_t)a.nw * a.nh * a.nviews;
+  a.tiles_w = (a.nw + kTile - 1) / kTile;
+  a.tiles_h = (a.nh + kTile - 1) / kTile;
+  FC_CHECK_ARG((long long)a.tiles_w * a.tiles_h * a.nviews < (1ll << 32) - kMaxBlocks,
+               "too many projection tiles");
   void* ws = nullptr;
   // ray records (32 B each), window words, then one 256-byte-aligned word for max |y|
   const size_t woff = nrays * 2 * sizeof(float4);
@@ -1663,9 +1679,7 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
   a.ymax = reinterpret_cast<unsigned int*>(static_cast<char*>(ws) + moff);
   int tok = prof_begin("adjoint", stream);
   zero_fill<unsigned int><<<1, 256, 0, stream>>>(a.ymax, 2);  // max |y| bits, non-finite flag
-  a.tiles_w = (a.nw + kTile - 1) / kTile;
-  a.tiles_h = (a.nh + kTile - 1) / kTile;
-  const unsigned rblocks = (unsigned)((long long)a.tiles_w * a.tiles_h * a.nviews);
+  const dim3 rblocks = block_grid((long long)a.tiles_w * a.tiles_h * a.nviews);
   if (dt == FC_F32) adj_rays<FC_F32><<<rblocks, 256, 0, stream>>>(a);
   else if (dt == FC_BF16) adj_rays<FC_BF16><<<rblocks, 256, 0, stream>>>(a);
   else adj_rays<FC_F16><<<rblocks, 256, 0, stream>>>(a);

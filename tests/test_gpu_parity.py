@@ -658,3 +658,20 @@ def test_project_little_work_rule(gpu, nviews, step, monkeypatch):
     assert rel(p.cpu(), ref) < 5e-5
     monkeypatch.setenv("FASTCONE_FP_PAIRS", "0")
     assert torch.equal(p, ops.project(torch.from_numpy(x).to(gpu), g, step=step))
+
+
+def test_adjoint_of_more_tiles_than_a_launch_counts(gpu):
+    # 2^24 + 1 views of one row: as many 16 x 16 pixel tiles, 2^32 threads and more. Against the views
+    # that hold data: the fixed-point sums of a block are exact and those of its up to 17 blocks with
+    # data are rounded to FP32 and added, in one call or the other by other splits: rel. L2 < 17 x 2^-24
+    from fastcone_amd import ops
+    from fastcone_amd.geometry import Geometry
+    nv, every = 2 ** 24 + 1, 2 ** 20
+    ang = np.linspace(0.0, 2 * np.pi, nv)
+    y = torch.zeros((nv, 1, 3), device=gpu)
+    y[::every] = 1.0
+    g = Geometry.circular(ang, 60.0, 1.0, (8, 8, 8), (1, 3))
+    few = Geometry.circular(ang[::every], 60.0, 1.0, (8, 8, 8), (1, 3))
+    out = ops.adjoint(y, g, step=0.5)
+    ref = ops.adjoint(y[::every].contiguous(), few, step=0.5)
+    assert float(ref.abs().max()) > 1.0 and rel(out.cpu(), ref.cpu()) < 17 * 2.0 ** -24
