@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(256) void adj_rays(AdjVArgs a) {
 // not wholly in front of the source, or a cylindrical detector, gets the whole detector.
 __global__ __launch_bounds__(256) void adj_windows(AdjVArgs a, uint2* __restrict__ out) {
   const size_t total = (size_t)a.nbx * a.nby * a.nbz * a.nviews;
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t idx = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
   if (idx >= total) return;
   const int t = (int)(idx % (size_t)a.nviews);
   const size_t b = idx / (size_t)a.nviews;
@@ -1443,9 +1443,9 @@ __global__ __launch_bounds__(256) void gather_bench_lds_ray(FpArgs a, int reps,
   if (acc == 12345.678f) sink[0] = acc;
 }
 
-// The most blocks of a launch in x: with 2^32 threads and more the launch takes their number modulo
-// 2^32, without an error.
-constexpr long long kMaxBlocks = 1 << 22;
+// The most blocks (of 256 threads) of a launch in x: with 2^32 threads and more the launch takes their
+// number modulo 2^32, without an error.
+constexpr long long kMaxBlocks = (1 << 24) - 1;
 
 // Grid of n blocks, numbered blockIdx.y * gridDim.x + blockIdx.x; the last row may have more than n.
 dim3 block_grid(long long n) {
@@ -1559,25 +1559,38 @@ int launch_project(int device, const void* vol, int dt, const int vs[3], const d
   const char* pe = std::getenv("FASTCONE_FP_PAIRS");
   const bool gain = h < 0.85 && (qe || !small);
   a.pairs = !(pe && std::strcmp(pe, "0") == 0) && gain ? 1 : 0;
-  // The LDS projector deals quads of four views; `group` stays a multiple of four.
-  const int nvq = (a.nviews + kQuad - 1) / kQuad * kQuad;
-  const long long nblocks = (long long)a.tiles_per_view * (layout == FP_LDS ? nvq : a.nviews);
-  FC_CHECK_ARG(nblocks < (1ll << 31), "too many projection tiles");
-  if (layout == FP_LDS) a.group = std::min((a.group + kQuad - 1) / kQuad * kQuad, nvq);
-  uint8_t* quad_mode = qmode < 0 ? nullptr : static_cast<uint8_t*>(ws) + flags_off;
+  const long long nblocks = (long long)a.tiles_per_view * a.nviews;
+  FC_CHECK_ARG(nblocks < (1ll << 31) && kQuad * (long long)a.tiles_per_view <= kMaxBlocks,
+               "too many projection tiles");
   if (nblocks > 0) {
     int tok = prof_begin("project", stream);
-    const int nb = (int)nblocks;
-    if (layout == FP_OCTET) {
-      if (dt == FC_F32) fp_kernel<FC_F32, FP_OCTET><<<nb, 256, 0, stream>>>(a);
-      else if (dt == FC_BF16) fp_kernel<FC_BF16, FP_OCTET><<<nb, 256, 0, stream>>>(a);
-      else fp_kernel<FC_F16, FP_OCTET><<<nb, 256, 0, stream>>>(a);
-    } else if (layout == FP_PLAIN) {
-      fp_kernel<FC_F32, FP_PLAIN><<<nb, 256, 0, stream>>>(a);
-    } else {
+    if (total)
+      fp_decide<8><<<(int)std::min<long long>(kSamples, nquads), 64, 0, stream>>>(a, total);
+    // the views of a launch: whole quads, as the LDS projector deals them
+    const int most = (int)(kMaxBlocks / (kQuad * a.tiles_per_view)) * kQuad, group = a.group;
+    for (int t0 = 0; t0 < ps[2]; t0 += a.nviews) {
+      a.nviews = std::min(most, ps[2] - t0);
+      a.views = views + (size_t)t0 * FC_VIEW_DOUBLES;
+      a.norm = norm ? norm + t0 : nullptr;
+      a.proj = proj + (size_t)t0 * a.nw * a.nh;
+      a.group = std::min(group, a.nviews);
+      const int nvq = (a.nviews + kQuad - 1) / kQuad * kQuad;
+      const int nb = a.tiles_per_view * (layout == FP_LDS ? nvq : a.nviews);
+      if (layout == FP_OCTET) {
+        if (dt == FC_F32) fp_kernel<FC_F32, FP_OCTET><<<nb, 256, 0, stream>>>(a);
+        else if (dt == FC_BF16) fp_kernel<FC_BF16, FP_OCTET><<<nb, 256, 0, stream>>>(a);
+        else fp_kernel<FC_F16, FP_OCTET><<<nb, 256, 0, stream>>>(a);
+        continue;
+      }
+      if (layout == FP_PLAIN) {
+        fp_kernel<FC_F32, FP_PLAIN><<<nb, 256, 0, stream>>>(a);
+        continue;
+      }
+      a.group = std::min((a.group + kQuad - 1) / kQuad * kQuad, nvq);  // a multiple of four
+      uint8_t* quad_mode = qmode < 0 ? nullptr
+                                     : static_cast<uint8_t*>(ws) + flags_off +
+                                           (size_t)(t0 / kQuad) * a.tiles_per_view;
       if (qmode >= 0) {
-        if (qmode == 0)
-          fp_decide<8><<<(int)std::min<long long>(kSamples, nquads), 64, 0, stream>>>(a, total);
         // two 512-thread blocks per quad and tile (nb = tiles x nvq is a multiple of four)
         const int nh = nb / 2;
         if (dt == FC_F32) fp_quad_kernel<FC_F32, 8><<<nh, 512, 0, stream>>>(a, quad_mode, total);
@@ -1628,14 +1641,23 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
     a.nw = ps[0]; a.nh = ps[1]; a.nviews = ps[2];
     a.tiles_w = (a.nw + kTile - 1) / kTile;
     a.tiles_per_view = a.tiles_w * ((a.nh + kTile - 1) / kTile);
-    a.group = std::min(8, std::max(1, a.nviews));
     a.max_steps = max_steps_for(vs, h);
-    long long nblocks = (long long)a.tiles_per_view * a.nviews;
-    FC_CHECK_ARG(nblocks < (1ll << 31), "too many projection tiles");
+    const long long nblocks = (long long)a.tiles_per_view * a.nviews;
+    FC_CHECK_ARG(nblocks < (1ll << 31) && a.tiles_per_view <= kMaxBlocks, "too many projection tiles");
     int tok = prof_begin("adjoint", stream);
-    if (dt == FC_F32) adjoint_kernel<FC_F32><<<(int)nblocks, 256, 0, stream>>>(a);
-    else if (dt == FC_BF16) adjoint_kernel<FC_BF16><<<(int)nblocks, 256, 0, stream>>>(a);
-    else adjoint_kernel<FC_F16><<<(int)nblocks, 256, 0, stream>>>(a);
+    const size_t view_bytes = (size_t)a.nw * a.nh * dtype_size(dt);
+    const int most = (int)(kMaxBlocks / a.tiles_per_view);
+    for (int t0 = 0; t0 < ps[2]; t0 += a.nviews) {  // views of a launch
+      a.nviews = std::min(most, ps[2] - t0);
+      a.group = std::min(8, a.nviews);
+      a.views = views + (size_t)t0 * FC_VIEW_DOUBLES;
+      a.norm = norm ? norm + t0 : nullptr;
+      a.proj = static_cast<const char*>(proj) + (size_t)t0 * view_bytes;
+      const int nb = a.tiles_per_view * a.nviews;
+      if (dt == FC_F32) adjoint_kernel<FC_F32><<<nb, 256, 0, stream>>>(a);
+      else if (dt == FC_BF16) adjoint_kernel<FC_BF16><<<nb, 256, 0, stream>>>(a);
+      else adjoint_kernel<FC_F16><<<nb, 256, 0, stream>>>(a);
+    }
     prof_end(tok, stream);
     FC_HIP(hipGetLastError());
     dim3 ug((nx + 255) / 256, ny, nz);
@@ -1683,7 +1705,7 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
   if (dt == FC_F32) adj_rays<FC_F32><<<rblocks, 256, 0, stream>>>(a);
   else if (dt == FC_BF16) adj_rays<FC_BF16><<<rblocks, 256, 0, stream>>>(a);
   else adj_rays<FC_F16><<<rblocks, 256, 0, stream>>>(a);
-  adj_windows<<<(unsigned)((nwin + 255) / 256), 256, 0, stream>>>(a, win);
+  adj_windows<<<block_grid((long long)((nwin + 255) / 256)), 256, 0, stream>>>(a, win);
   const dim3 grid(a.nbx, a.nby, a.nbz * a.nsplit);
   if (a.h >= 0.25) adjoint_vox_kernel<false><<<grid, kAT, 0, stream>>>(a);
   else adjoint_vox_kernel<true><<<grid, kAT, 0, stream>>>(a);

@@ -675,3 +675,20 @@ def test_adjoint_of_more_tiles_than_a_launch_counts(gpu):
     out = ops.adjoint(y, g, step=0.5)
     ref = ops.adjoint(y[::every].contiguous(), few, step=0.5)
     assert float(ref.abs().max()) > 1.0 and rel(out.cpu(), ref.cpu()) < 17 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("layout", ["lds", "plain"])
+def test_project_of_more_tiles_than_a_launch_counts(gpu, layout, monkeypatch):
+    # 2^24 + 5 views of one pixel, in two launches: the bits of the last views projected by themselves
+    from fastcone_amd import ops
+    from fastcone_amd.geometry import Geometry
+    monkeypatch.setenv("FASTCONE_FP_LAYOUT", layout)
+    nv, last = 2 ** 24 + 5, 77
+    ang = np.linspace(0.0, 2 * np.pi, nv)
+    vol = torch.rand((4, 4, 4), device=gpu, generator=torch.Generator(gpu).manual_seed(1))
+    g = Geometry.circular(ang, 20.0, 1.0, (4, 4, 4), (1, 1))
+    out = ops.project(vol, g, step=0.5)
+    for part in (slice(0, last), slice(nv // 2, nv // 2 + last), slice(nv - last, nv)):
+        few = Geometry.circular(ang[part], 20.0, 1.0, (4, 4, 4), (1, 1))
+        ref = ops.project(vol, few, step=0.5)
+        assert float(ref.min()) > 0.0 and torch.equal(out[part], ref)
