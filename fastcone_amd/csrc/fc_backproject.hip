@@ -22,7 +22,7 @@
 // z (untilted detectors) each voxel then costs one FMA for its row and a bilinear interpolation from
 // LDS (two ds_read2 pairs, one multiply-add for the address).
 //
-// View table: every kTab views the block computes, one thread per view and in FP64, the window of its
+// View table: every kTab views the block computes, eight threads per view and in FP64, the window of its
 // cube — the projective image of a box lies in the box of its eight corners' images, so the corners'
 // (u, v) widened by a pixel each side bound every tap — and the view's projective forms relative to
 // the window's and the cube's corners, A' = (A - u0 C) / Cm, B' = (B - v0 C) / Cm and q = C / Cm - 1 as
@@ -94,64 +94,80 @@ struct ViewEntry {
   uint32_t tilted;  // a3 or c3 nonzero
 };
 
+// Entries of the views [t0, t0 + n) for the cube at (x0, y0, z0), eight lanes of a block's threads per
+// view: each projects a corner of the cube, and four of them form the constants and slopes.
 // Window pixels [u0, u0 + Wu) x [v0, v0 + Wv) with u0 = floor(min u) - 1 and Wu = floor(max u) - u0
 // + 3, so every tap (iu, iu + 1) of a voxel in the cube lies at least one pixel inside; likewise v.
 template <int MODE>
-__device__ __forceinline__ ViewEntry view_entry(const BpArgs& a, int t, int x0, int y0, int z0) {
-  const double* M = a.views + (size_t)t * FC_VIEW_DOUBLES + 12;
+__device__ __forceinline__ void view_table(const BpArgs& a, ViewEntry* tab, int t0, int n, int x0,
+                                           int y0, int z0) {
+  int c = threadIdx.x & 7;
+  asm volatile("" : "+v"(c), "+s"(x0), "+s"(y0), "+s"(z0));  // nothing of this stays in registers
   const double X0 = x0 + a.ox, Y0 = y0 + a.oy, Z0 = z0 + a.oz;
   const double ex = min(kBXY - 1, a.nx - 1 - x0), ey = min(kBXY - 1, a.ny - 1 - y0),
                ez = min(kZR - 1, a.nz - 1 - z0);
-  const double A0 = M[0] * X0 + M[1] * Y0 + M[2] * Z0 + M[3];
-  const double B0 = M[4] * X0 + M[5] * Y0 + M[6] * Z0 + M[7];
-  const double C0 = M[8] * X0 + M[9] * Y0 + M[10] * Z0 + M[11];
-  double umin = 1e300, umax = -1e300, vmin = 1e300, vmax = -1e300;
-  bool ok = true;
-  // the matrix is reread per corner: held in registers, it would spill the block's accumulators
 #pragma unroll 1
-  for (int c = 0; c < 8; ++c) {
-    asm volatile("" : "+v"(M));
-    const double dx = c & 1 ? ex : 0.0, dy = c & 2 ? ey : 0.0, dz = c & 4 ? ez : 0.0;
-    const double C = C0 + M[8] * dx + M[9] * dy + M[10] * dz;
-    ok = ok && C > 0.0;
-    const double rc = 1.0 / C;
-    const double u = (A0 + M[0] * dx + M[1] * dy + M[2] * dz) * rc;
-    const double v = (B0 + M[4] * dx + M[5] * dy + M[6] * dz) * rc;
-    umin = fmin(umin, u); umax = fmax(umax, u);
-    vmin = fmin(vmin, v); vmax = fmax(vmax, v);
-  }
-  ViewEntry e;
-  e.org = 0u;
-  e.size = kWinGlobal;
-  e.tilted = M[2] != 0.0 || M[10] != 0.0;
-  int u0 = 0, v0 = 0;
-  if (ok && umin > -1e6 && umax < 1e6 && vmin > -1e6 && vmax < 1e6) {
-    if (umax <= -1.0 || umin >= (double)a.nw || vmax <= -1.0 || vmin >= (double)a.nh) {
-      e.size = kWinSkip;  // zero-extended data: every sample of the cube is 0
-    } else {
-      u0 = (int)floor(umin) - 1;
-      v0 = (int)floor(vmin) - 1;
-      const int Wu = (int)floor(umax) - u0 + 3, Wv = (int)floor(vmax) - v0 + 3;
-      if (Wu <= kTileW && Wv <= kTileH && u0 >= -32768 && u0 <= 32767 && v0 >= -32768 &&
-          v0 <= 32767) {
-        e.org = ((uint32_t)u0 & 0xffffu) | ((uint32_t)v0 << 16);
-        e.size = (uint32_t)Wu | ((uint32_t)Wv << 16);
+  for (int i = threadIdx.x >> 3; i < n; i += 32) {
+    const double* M = a.views + (size_t)(t0 + i) * FC_VIEW_DOUBLES + 12;
+    // the matrix is reread where it is used: held in registers, it would spill the block's accumulators
+    auto form = [&](int r, double x, double y, double z) {
+      asm volatile("" : "+v"(M));
+      return M[4 * r] * x + M[4 * r + 1] * y + M[4 * r + 2] * z + M[4 * r + 3];
+    };
+    const double X = X0 + (c & 1 ? ex : 0.0), Y = Y0 + (c & 2 ? ey : 0.0), Z = Z0 + (c & 4 ? ez : 0.0);
+    const double C = form(2, X, Y, Z), rc = 1.0 / C;
+    int ok = C > 0.0;
+    // least and greatest whole pixel of the corners in one direction; ok: within the integers' reach
+    // and, if the detector's n pixels are nowhere near, hit = false
+    bool hit = true;
+    int lo[2], hi[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      double least = form(d, X, Y, Z) * rc, most = least;
+#pragma unroll
+      for (int m = 1; m < 8; m <<= 1) {
+        least = fmin(least, __shfl_xor(least, m));
+        most = fmax(most, __shfl_xor(most, m));
+      }
+      ok &= least > -1e6 && most < 1e6;
+      hit = hit && !(most <= -1.0 || least >= (double)(d ? a.nh : a.nw));
+      lo[d] = (int)floor(fmax(least, -1e6));
+      hi[d] = (int)floor(fmin(most, 1e6));
+    }
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1) ok &= __shfl_xor(ok, m);
+    uint32_t org = 0u, size = kWinGlobal;
+    int u0 = 0, v0 = 0;
+    if (ok && !hit) {
+      size = kWinSkip;  // zero-extended data: every sample of the cube is 0
+    } else if (ok) {
+      u0 = lo[0] - 1;
+      v0 = lo[1] - 1;
+      const int Wu = hi[0] - u0 + 3, Wv = hi[1] - v0 + 3;
+      if (Wu <= kTileW && Wv <= kTileH && u0 >= -32768 && u0 <= 32767 && v0 >= -32768 && v0 <= 32767) {
+        org = ((uint32_t)u0 & 0xffffu) | ((uint32_t)v0 << 16);
+        size = (uint32_t)Wu | ((uint32_t)Wv << 16);
       }
     }
+    asm volatile("" : "+v"(M));
+    const bool tilted = M[2] != 0.0 || M[10] != 0.0;
+    const double C0 = form(2, X0, Y0, Z0);
+    const double Cm = C0 + fmax(M[8], 0.0) * ex + fmax(M[9], 0.0) * ey, rm = 1.0 / Cm;
+    ViewEntry& e = tab[i];
+    if (c < 4) {
+      const double fa = c ? M[c - 1] : form(0, X0, Y0, Z0), fb = c ? M[c + 3] : form(1, X0, Y0, Z0),
+                   fc = c ? M[c + 7] : C0;
+      e.a[c] = (float)((fa - u0 * fc) * rm);
+      e.b[c] = (float)((fb - v0 * fc) * rm);
+      e.q[c] = (float)((c || tilted ? fc : C0 - Cm) * rm);
+    } else if (c == 4) {
+      const double s = a.norm ? a.norm[t0 + i] : 1.0f;
+      e.s = (float)(MODE == FC_BP_FDK ? s * rm * rm : MODE == FC_BP_KATSEVICH ? s * rm : s);
+      e.org = org;
+      e.size = size;
+      e.tilted = tilted;
+    }
   }
-  const double Cm = C0 + fmax(M[8], 0.0) * ex + fmax(M[9], 0.0) * ey, rm = 1.0 / Cm;
-  const double s = a.norm ? a.norm[t] : 1.0f;
-  e.s = (float)(MODE == FC_BP_FDK ? s * rm * rm : MODE == FC_BP_KATSEVICH ? s * rm : s);
-  e.a[0] = (float)((A0 - u0 * C0) * rm);
-  e.b[0] = (float)((B0 - v0 * C0) * rm);
-  e.q[0] = (float)((e.tilted ? C0 : C0 - Cm) * rm);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    e.a[1 + k] = (float)((M[k] - u0 * M[8 + k]) * rm);
-    e.b[1 + k] = (float)((M[4 + k] - v0 * M[8 + k]) * rm);
-    e.q[1 + k] = (float)(M[8 + k] * rm);
-  }
-  return e;
 }
 
 // Zero-extended bilinear samples of one view straight from global memory, for windows that do not fit
@@ -219,7 +235,7 @@ __device__ __forceinline__ void gather_views(float* acc, const BpArgs& a, ViewEn
   for (int tb = tbeg; tb < tend; tb += kTab) {
     const int n = min(kTab, tend - tb);
     __syncthreads();  // the previous table is no longer read
-    if ((int)threadIdx.x < n) tab[threadIdx.x] = view_entry<MODE>(a, tb + (int)threadIdx.x, bx0, by0, z0);
+    view_table<MODE>(a, tab, tb, n, bx0, by0, z0);
     __syncthreads();
     for (int i = 0; i < n; ++i) {
       if ((__builtin_amdgcn_readfirstlane(tab[i].size) & 0xffffu) != kWinGlobal) continue;
@@ -436,8 +452,7 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
     const int n = min(kTab, tend - tb);
     __syncthreads();  // the previous table is no longer read
     // one entry more than the table's views: the next view's window
-    if ((int)threadIdx.x <= n && tb + (int)threadIdx.x < tend)
-      tab[threadIdx.x] = view_entry<MODE>(a, tb + (int)threadIdx.x, bx0, by0, z0);
+    view_table<MODE>(a, tab, tb, min(n + 1, tend - tb), bx0, by0, z0);
     __syncthreads();
     if (tb == tbeg) {
       const uint32_t org = __builtin_amdgcn_readfirstlane(tab[0].org),
