@@ -268,20 +268,17 @@ __device__ __forceinline__ float tile_bilinear(uint32_t col, float au, float v) 
   return lerp(lerp(p[0], p[1], au), lerp(p[kTileP], p[kTileP + 1], au), av);
 }
 
-// acc[k] += wt times the bilinear sample at row vb + k dv of the column at LDS byte address `col`;
-// rows clamped to [0, vmax] if CLAMP. Two samples' reads are issued before the previous two are
-// used.
-template <bool CLAMP>
-__device__ __forceinline__ void column_samples(float* acc, uint32_t col, float au, float vb,
-                                               float dv, float wt, float vmax) {
+// acc[k] += wt times the bilinear sample at row vb + kz[k] dv of the column at LDS byte address `col`.
+// Two samples' reads are issued before the previous two are used.
+__device__ __forceinline__ void column_samples(float* acc, const float* kz, uint32_t col, float au,
+                                               float vb, float dv, float wt) {
   typedef __attribute__((address_space(3))) const float* lds_p;
   constexpr int kG = 2;
   float p[2][kG][4], av[2][kG];
   auto read = [&](int g) {
 #pragma unroll
     for (int q = 0; q < kG; ++q) {
-      float v = fmaf((float)(g * kG + q), dv, vb);
-      if (CLAMP) v = clampf(v, 0.0f, vmax);
+      const float v = fmaf(kz[g * kG + q], dv, vb);
       av[g & 1][q] = __builtin_amdgcn_fractf(v);
       const lds_p a = (lds_p)mad_u24((uint32_t)(int)v, 4u * kTileP, col);
       p[g & 1][q][0] = a[0];
@@ -307,15 +304,13 @@ __device__ __forceinline__ void column_samples(float* acc, uint32_t col, float a
 // The same for a tilted detector: column, row and weight by voxel, from the view's forms at the
 // column's first voxel.
 template <int MODE>
-__device__ __forceinline__ void tilted_samples(float* acc, uint32_t T0, float A, float B, float C,
-                                               const ViewEntry& E, float umax, float vmax) {
+__device__ __forceinline__ void tilted_samples(float* acc, const float* kz, uint32_t T0, float A,
+                                               float B, float C, const ViewEntry& E) {
 #pragma unroll
   for (int k = 0; k < kZR; ++k) {
-    if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four samples at a time in registers
-    const float kf = (float)k;
-    const float rc = __builtin_amdgcn_rcpf(fmaf(kf, E.q[3], C));  // 1 ulp, as the positions
-    const float u = clampf(fmaf(kf, E.a[3], A) * rc, 0.0f, umax);
-    const float v = clampf(fmaf(kf, E.b[3], B) * rc, 0.0f, vmax);
+    if (k % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two samples at a time in registers
+    const float rc = __builtin_amdgcn_rcpf(fmaf(kz[k], E.q[3], C));  // 1 ulp, as the positions
+    const float u = fmaf(kz[k], E.a[3], A) * rc, v = fmaf(kz[k], E.b[3], B) * rc;
     float wt = E.s;
     if constexpr (MODE == FC_BP_FDK) wt = E.s * rc * rc;
     if constexpr (MODE == FC_BP_KATSEVICH) wt = E.s * rc;
@@ -341,11 +336,20 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
   const int bx0 = blockIdx.x * kBXY, by0 = blockIdx.y * kBXY;
   const int split = blockIdx.z / a.nbz, z0 = (int)(blockIdx.z - split * a.nbz) * kZR;
   const int x = bx0 + ix, y = by0 + iy;
-  const float dx = (float)ix, dy = (float)iy;
+  // Columns and voxels beyond the volume (partial cubes) repeat its last ones, so that every sample's
+  // taps lie >= 1 pixel inside the window; their sums are not stored. kz in scalar registers.
+  const float dx = (float)min(ix, a.nx - 1 - bx0), dy = (float)min(iy, a.ny - 1 - by0);
+  const uint32_t last = __builtin_amdgcn_readfirstlane(__float_as_uint((float)(a.nz - 1 - z0)));
+  float kz[kZR];
+  kz[0] = 0.0f;
+#pragma unroll
+  for (int k = 1; k < kZR; ++k) {
+    // the smaller of two non-negative floats
+    kz[k] = __uint_as_float(
+        __builtin_amdgcn_readfirstlane(min(__builtin_bit_cast(uint32_t, (float)k), last)));
+  }
   const int tbeg = (int)((long long)a.nviews * split / a.nsplit);
   const int tend = (int)((long long)a.nviews * (split + 1) / a.nsplit);
-  // the whole 16 x 16 x 16 cube lies in the volume (no clamping of tile coordinates needed)
-  const bool inner = bx0 + kBXY <= a.nx && by0 + kBXY <= a.ny && z0 + kZR <= a.nz;
   float acc[kZR];
 #pragma unroll
   for (int k = 0; k < kZR; ++k) acc[k] = 0.0f;
@@ -492,9 +496,6 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
         gather = true;
         continue;
       }
-      // Tile coordinates. Valid voxels lie >= 1 pixel inside the window; the clamps only keep
-      // voxels outside the volume (partial blocks) and NaN inside the buffer.
-      const float umax = (float)Wu - 2.0f, vmax = (float)Wv - 2.0f;
       const uint32_t T0 = lds_address(T);
       const float A = fmaf(dx, E.a[1], fmaf(dy, E.a[2], E.a[0]));
       const float B = fmaf(dx, E.b[1], fmaf(dy, E.b[2], E.b[0]));
@@ -502,19 +503,15 @@ __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a)
       if (__builtin_amdgcn_readfirstlane(E.tilted) == 0u) {
         // Columns independent of z: u and the weight are per column, the row is linear in z.
         const float p = -q * __builtin_amdgcn_rcpf(1.0f + q), rc = 1.0f + p;  // Cm / C
-        const float u = clampf(A * rc, 0.0f, umax);
-        const float vb = B * rc, dv = E.b[3] * rc;
+        const float u = A * rc, vb = B * rc, dv = E.b[3] * rc;
         float wt = E.s;
         if constexpr (MODE == FC_BP_FDK) wt = fmaf(E.s, p * (p + 2.0f), E.s);
         if constexpr (MODE == FC_BP_KATSEVICH) wt = fmaf(E.s, p, E.s);
         const uint32_t col0 = T0 + 4u * (uint32_t)(int)u;
         const float au = __builtin_amdgcn_fractf(u);
-        // Voxels outside the volume (partial cubes) are kept inside the buffer by clamping; in whole
-        // cubes every voxel's taps lie >= 1 pixel inside the window
-        if (inner) column_samples<false>(acc, col0, au, vb, dv, wt, 0.0f);
-        else column_samples<true>(acc, col0, au, vb, dv, wt, vmax);
+        column_samples(acc, kz, col0, au, vb, dv, wt);
       } else {
-        tilted_samples<MODE>(acc, T0, A, B, q, E, umax, vmax);
+        tilted_samples<MODE>(acc, kz, T0, A, B, q, E);
       }
     }
   }
