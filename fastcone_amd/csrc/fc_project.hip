@@ -974,7 +974,8 @@ struct AdjVArgs {
   int nbx, nby, nbz;
   int nsplit;          // view ranges per brick (grid z = nbz * nsplit)
   int max_steps;
-  int tiles_w, tiles_h;  // 16 x 16 pixel tiles of a view (adj_rays)
+  int tiles_w, tiles_h;  // tiles of 256 pixels of a view (adj_rays)
+  int tile_rows;         // log2 of their rows, at most 4
 };
 
 // One thread per ray (view, row, column): the ray's FP32 first sample, step and sample count
@@ -984,7 +985,8 @@ struct AdjVArgs {
 // block-wide maximum, then one integer atomic per block that exceeds the maximum so far (an atomic
 // from every block serialises on its one address). Records lie column by column, [view][column][row],
 // as the bricks read them; a block takes a 16 x 16 pixel tile, so a wave reads eight row pieces of 32
-// bytes and writes eight column pieces of 256.
+// bytes and writes eight column pieces of 256. Detectors of eight rows or fewer: all rows (rounded up to
+// a power of two) of as many columns as make 256 pixels.
 template <int DT>
 __global__ __launch_bounds__(256) void adj_rays(AdjVArgs a) {
   __shared__ float red[4];
@@ -994,8 +996,12 @@ __global__ __launch_bounds__(256) void adj_rays(AdjVArgs a) {
   const int t = (int)(b / (unsigned)per_view), tile = (int)(b - (unsigned)t * (unsigned)per_view);
   if (t >= a.nviews) return;
   const int ty = tile / a.tiles_w, tx = tile - ty * a.tiles_w;
-  const int j = tx * kTile + (wave & 1) * 8 + (lane >> 3);
-  const int i = ty * kTile + (wave >> 1) * 8 + (lane & 7);
+  int j = tx * (256 >> a.tile_rows) + ((int)threadIdx.x >> a.tile_rows);
+  int i = ((int)threadIdx.x & ((1 << a.tile_rows) - 1));
+  if (a.tile_rows == 4) {
+    j = tx * kTile + (wave & 1) * 8 + (lane >> 3);
+    i = ty * kTile + (wave >> 1) * 8 + (lane & 7);
+  }
   float m = 0.0f;
   if (j < a.nw && i < a.nh) {
     const float y = load_elem<DT>(a.proj, ((size_t)t * a.nh + i) * a.nw + j) *
@@ -1069,8 +1075,10 @@ __global__ __launch_bounds__(256) void adj_windows(AdjVArgs a, uint2* __restrict
   out[idx] = w;
 }
 
-// CAPRUN: cap a run at kRun samples (steps below 0.25 voxel; see the run merging below).
-template <bool CAPRUN>
+// CAPRUN: cap a run at kRun samples (steps below 0.25 voxel; see the run merging below). SLAB: windows
+// may be walked along their rows (detectors of at most kSlabRows rows; the choice costs the others 1 %).
+constexpr int kSlabRows = 12;
+template <bool CAPRUN, bool SLAB>
 __global__ __launch_bounds__(kAT) void adjoint_vox_kernel(AdjVArgs a) {
   __shared__ unsigned long long acc[kAL3];
   for (int e = threadIdx.x; e < kAL3; e += kAT) acc[e] = 0ull;
@@ -1111,26 +1119,36 @@ __global__ __launch_bounds__(kAT) void adjoint_vox_kernel(AdjVArgs a) {
   // diagonal. Two rows apart they rarely add to the same LDS word at once (same-address atomics
   // serialise). Timed at 256^3 x 360 views x 384^2, this kernel and its rays: along rows 2 apart 76.7
   // ms, along columns 1, 2, 3 and 4 apart 88.3, 61.2, 72.0 and 69.3 ms (columns also 2 apart: 63.4).
+  // Windows of slabs' detectors run along their rows: their columns are too short for the lanes of a
+  // wave, and the rays of neighbouring columns, less than a voxel apart, meet in the same words. 180
+  // views of nz x 200^2, rows / columns (us) at half and whole steps: 4 278 / 327 and 185 / 246; 7 509 / 501
+  // and 329 / 389; 8 (12 rows of 20 to 28 pixels) 549 / 537 and 351 / 390; 10 734 / 624 and 463 / 432. (Windows
+  // that the edge of a tall detector cuts are better left alone: 128^3 x 90 views 1.89 / 1.91 ms.)
   const int perm =
       ((threadIdx.x >> 7) << 7) | ((threadIdx.x & 63) << 1) | ((threadIdx.x >> 6) & 1);
   for (int g = perm;; g += kAT) {
-    int Wi = (int)(w.y >> 16), npix = Wi * (int)(w.y & 0xffffu);
+    int Wi = (int)(w.y >> 16), Wj = (int)(w.y & 0xffffu), npix = Wi * Wj;
     while (t < tend && g >= start + npix) {
       start += npix;
       if (++t < tend) {
         w = W[t];
         Wi = (int)(w.y >> 16);
-        npix = Wi * (int)(w.y & 0xffffu);
+        Wj = (int)(w.y & 0xffffu);
+        npix = Wi * Wj;
       }
     }
     if (t >= tend) break;
     const int p = g - start;
-    // p / Wi from a 1-ulp reciprocal, exact for p < 2^21: (p + 0.5) / Wi lies at least 0.5 / Wi
-    // from an integer and the roundings move it by less than 2^-2 / Wi (integer division for
+    const bool flat = SLAB && 20 * a.nh < 9 * Wj;
+    const int len = flat ? Wj : Wi;
+    // p / len from a 1-ulp reciprocal, exact for p < 2^21: (p + 0.5) / len lies at least 0.5 / len
+    // from an integer and the roundings move it by less than 2^-2 / len (integer division for
     // larger windows)
-    const int pj = p < (1 << 21) ? (int)(((float)p + 0.5f) * __builtin_amdgcn_rcpf((float)Wi))
-                                 : p / Wi;
-    const int j = (int)(w.x & 0xffffu) + pj, i = (int)(w.x >> 16) + (p - pj * Wi);
+    const int line = p < (1 << 21) ? (int)(((float)p + 0.5f) * __builtin_amdgcn_rcpf((float)len))
+                                   : p / len;
+    const int along = p - line * len;
+    const int j = (int)(w.x & 0xffffu) + (flat ? along : line);
+    const int i = (int)(w.x >> 16) + (flat ? line : along);
     const size_t ray = ((size_t)t * a.nw + j) * a.nh + i;
     const float4 r1 = a.rays[2 * ray + 1];
     if (r1.w == 0.0f) continue;  // zero datum or a ray that misses the block
@@ -1685,8 +1703,10 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
   FC_CHECK_ARG((long long)a.nbz * a.nsplit <= 65535, "volume too large for the adjoint grid");
   const size_t nwin = (size_t)a.nbx * a.nby * a.nbz * a.nviews;
   const size_t nrays = (size_t)a.nw * a.nh * a.nviews;
-  a.tiles_w = (a.nw + kTile - 1) / kTile;
-  a.tiles_h = (a.nh + kTile - 1) / kTile;
+  a.tile_rows = 0;
+  while (a.tile_rows < 4 && 1 << a.tile_rows < a.nh) ++a.tile_rows;
+  a.tiles_w = (a.nw + (256 >> a.tile_rows) - 1) / (256 >> a.tile_rows);
+  a.tiles_h = (a.nh + (1 << a.tile_rows) - 1) >> a.tile_rows;
   FC_CHECK_ARG((long long)a.tiles_w * a.tiles_h * a.nviews < (1ll << 32) - kMaxBlocks,
                "too many projection tiles");
   void* ws = nullptr;
@@ -1707,8 +1727,11 @@ int launch_adjoint(int device, float* vol, const int vs[3], const double origin[
   else adj_rays<FC_F16><<<rblocks, 256, 0, stream>>>(a);
   adj_windows<<<block_grid((long long)((nwin + 255) / 256)), 256, 0, stream>>>(a, win);
   const dim3 grid(a.nbx, a.nby, a.nbz * a.nsplit);
-  if (a.h >= 0.25) adjoint_vox_kernel<false><<<grid, kAT, 0, stream>>>(a);
-  else adjoint_vox_kernel<true><<<grid, kAT, 0, stream>>>(a);
+  const bool slab = a.nh <= kSlabRows;
+  if (a.h >= 0.25 && slab) adjoint_vox_kernel<false, true><<<grid, kAT, 0, stream>>>(a);
+  else if (a.h >= 0.25) adjoint_vox_kernel<false, false><<<grid, kAT, 0, stream>>>(a);
+  else if (slab) adjoint_vox_kernel<true, true><<<grid, kAT, 0, stream>>>(a);
+  else adjoint_vox_kernel<true, false><<<grid, kAT, 0, stream>>>(a);
   prof_end(tok, stream);
   FC_HIP(hipGetLastError());
   return release_ws(device, SLOT_OCTET, stream);

@@ -692,3 +692,21 @@ def test_project_of_more_tiles_than_a_launch_counts(gpu, layout, monkeypatch):
         few = Geometry.circular(ang[part], 20.0, 1.0, (4, 4, 4), (1, 1))
         ref = ops.project(vol, few, step=0.5)
         assert float(ref.min()) > 0.0 and torch.equal(out[part], ref)
+
+
+@pytest.mark.parametrize("det", [(1, 300), (2, 40), (3, 129), (4, 64), (5, 70), (8, 33), (9, 40), (17, 16), (300, 1)])
+def test_adjoint_of_few_rows(gpu, det):
+    # ray tiles of 1 to 16 rows with remainders, windows walked along rows and along columns
+    from fastcone_amd import ops
+    from fastcone_amd.geometry import Geometry
+    rng = np.random.default_rng(det[0])
+    n = 9
+    ang = np.sort(rng.uniform(0, 2 * np.pi, n))
+    vol = (max(2, det[0] * 2 // 3), 20, 34) if det[0] < 100 else (90, 20, 6)
+    g = Geometry.circular(ang, 90.0, 0.9, vol, det)
+    prob = oracle.Problem(ang, np.full(n, vol[0] / 2), 90.0, 0.9, vol_dim=vol[::-1],
+                          proj_dim=det[::-1])
+    y = rng.standard_normal(g.proj_shape).astype(np.float32)
+    aty = ops.adjoint(torch.from_numpy(y).to(gpu), g, step=0.5).cpu().numpy()
+    ref = oracle.adjoint(prob, y, g.vol_shape, h=0.5)
+    assert rel(aty, ref) < 5e-5
