@@ -30,10 +30,9 @@
 // are small (|A'| < 64, -1 < q <= 0), so rounding them to FP32 moves a tile coordinate by 1.1e-6 pixel
 // (rms; FP64 terms rounded to an absolute coordinate 7e-6), and Cm / C = 1 - q / (1 + q) and the weight
 // have the error of their last rounding (weight 3.6e-8 of it, rms, as from FP64 terms; the square of an
-// FP32 reciprocal of C 1.1e-7). A view whose
-// window does not fit the LDS tile (pixels below about a third of a voxel, very short source
-// distances) is gathered from global memory with explicit bounds, after the views that fit; a view
-// that misses the detector entirely is skipped.
+// FP32 reciprocal of C 1.1e-7). A view whose window does not fit the LDS tile (pixels below about a
+// third of a voxel, very short source distances) is gathered from global memory with explicit bounds,
+// after the views that fit; a view that misses the detector entirely is skipped.
 //
 // Small volumes leave compute units idle or the last round of blocks nearly empty: the views are
 // then split over several blocks per cube, whose sums go to partial volumes that bp_reduce adds in
@@ -320,12 +319,13 @@ __device__ __forceinline__ void tilted_samples(float* acc, const float* kz, uint
 
 typedef uint32_t fc_u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
 
-// Bound by VALU issue (0.95-1.0 instructions per CU clock, 15.8 -> 13.4 per voxel-view at 512^3 x 720)
-// with the LDS busy 64 % of the time; five blocks per CU for FP32 storage (96 registers), four for
-// 16-bit storage, whose staging registers would spill at five. Against per-view FP64 terms by column
-// and dword copies row by row: 512^3 x 720 FP32 39.2 -> 37.0 ms, 256^3 x 360 BF16 3.3 -> 3.1 ms,
-// 150 x 333 x 290 x 275 tilted FP16 2.84 -> 2.75 ms. Keeping two samples' reads ahead (column_samples)
-// is part of that: with four ahead the registers allow only four blocks (38.0 ms).
+// Bound by VALU issue (1.02 instructions per CU clock, 14.1 per voxel-view at 512^3 x 720) with the LDS
+// busy 72 % of the time; five blocks per CU for FP32 storage (96 registers, of which two to four and one
+// scalar one spill, outside the samples), four for 16-bit storage (113), which at five spills and is 1 to
+// 6 % slower. Against per-view FP64 terms by column and dword copies row by row (17.5 instructions, 49 %):
+// 512^3 x 720 FP32 39.2 -> 36.9 ms, 256^3 x 360 BF16 2.85 -> 2.72 ms, 150 x 333 x 290 x 275 tilted FP16 2.84 ->
+// 2.66 ms. Keeping two samples' reads ahead (column_samples) is part of that: with four ahead the
+// registers allow only four blocks (38.0 against 37.0 ms).
 template <int DT, int MODE>
 __global__ __launch_bounds__(256, DT == FC_F32 ? 5 : 4) void bp_kernel(BpArgs a) {
   __shared__ __align__(16) float tile[2][kTileCap];
@@ -613,10 +613,10 @@ int dispatch_bp(const BpArgs& a, int mode, dim3 grid, hipStream_t s) {
 
 // Splits of the views. Blocks run in rounds of five per CU (1280): fewer cubes than that leave CUs
 // idle, and a few rounds waste much of the last one. A split costs its partial volume's write and
-// read, so it needs enough views. Timed (1 split against the number chosen): 64^3 x 60 views 92 -> 31
-// us (12 splits), 96^3 x 120 176 -> 82 (8), 128^3 x 180 289 -> 212 (4), 150 x 200 x 210 x 200 701 ->
-// 653 (3), 256^3 x 360 2649 -> 2513 (3), 240 x 300^2 x 360 3324 -> 3233 (3); at 320 x 400^2 x 200
-// (12500 cubes) 2 and 3 splits lose 3 and 5 %.
+// read, so it needs enough views. Timed (us, 1 split / 2 / the number chosen): 64^3 x 60 views 81 / 47 / 26
+// (12 splits), 96^3 x 120 152 / 99 / 73 (11), 128^3 x 180 247 / 188 / 193 (5), 150 x 200 x 210 x 200 658 / 619 /
+// 598 (3), 256^3 x 360 2319 / 2339 / 2317 (3), 240 x 300^2 x 360 3148 / 3093 / 3070 (3); at 320 x 400^2 x 200
+// (12500 cubes) 3768 / 3933.
 int bp_splits(long long nblocks, int nviews) {
   if (nblocks < 1280) return (int)std::max(1LL, std::min<long long>(2560 / nblocks, nviews / 5));
   return nblocks < 8192 && nviews >= 128 ? 3 : 1;

@@ -278,7 +278,8 @@ __global__ __launch_bounds__(256, 2) void conv_fwd_mfma(const uint16_t* __restri
 // (12 for 96 channels, whose next plane needs the registers), and a third of the patch reads. Time
 // before and now: 96 -> 32 channels at 128^3 0.92 -> 0.58 ms, 64 -> 64 at 64^3 0.20 -> 0.09, 32 -> 32
 // at 128^3 0.15 -> 0.12, 64 -> 32 at 4 x 32^3 0.055 -> 0.037 ms. With all of a row's channel blocks
-// in one wave (6 or 12 fragments a step) it was slower than before.
+// in one wave (6 or 12 fragments a step) it was slower than before. (64 -> 32 channels spill 23 of 256
+// registers, and are 1.5 times as fast as conv_fwd_mfma all the same.)
 template <int CIN, int COUT>
 struct StreamTile {
   static constexpr int NB = COUT / 16;          // channel blocks; a wave owns one

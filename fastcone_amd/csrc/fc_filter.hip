@@ -353,7 +353,7 @@ constexpr int filt_threads(int L) { return L / kE > 64 ? L / kE : 64; }
 
 // Per pair and wave (2048 points, cosine weights): about 1600 VALU and 72 double LDS instructions
 // against 32 to 48 memory ones. Three waves per SIMD hide the exchanges' and loads' latency best
-// (166 registers; 3.46 GB of FP32 rows of 768 columns, in ms: two waves 2.27, three 2.14, three with
+// (166 registers, two spilled at 512 and 8192 points; 3.46 GB of FP32 rows of 768 columns, in ms: two waves 2.27, three 2.14, three with
 // the loads issued after the round begins 2.18); about 60 % VALU busy, 1.6 TB/s. The radix-8
 // Stockham stages with every exchange, load and the spectrum product through LDS that this replaces
 // took 3.82 ms; rows of 384 columns 0.56 -> 0.29, 3000 columns 1.36 -> 0.67, and 200000 rows of 31
